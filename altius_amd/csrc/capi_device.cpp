@@ -591,7 +591,8 @@ int ahip_conv2d(ahip_ctx *ctx, float *out, const float *x, const float *w, const
     REQUIRE_CTX(ctx, "ahip_conv2d");
     if (!kh || !kw || !stride_h || !stride_w || !dilation_h || !dilation_w)
         return ctx->d.fail(AHIP_ERR_ARG, "ahip_conv2d: kernel, stride and dilation must be positive");
-    return altius::launch_conv2d(ctx->d, out, x, w, bias, col, batch, c, ih, iw, oc, oh, ow, kh, kw, stride_h, stride_w,
+    if (batch && oc && oh && ow && !col) return ctx->d.fail(AHIP_ERR_ARG, "conv2d: null pointer");
+    return altius::launch_conv2d(ctx->d, out, x, w, bias, batch, c, ih, iw, oc, oh, ow, kh, kw, stride_h, stride_w,
                                  dilation_h, dilation_w, pad_top, pad_left, group);
 } catch (...) {
     return altius::caught_at_boundary("ahip_conv2d");

@@ -1411,13 +1411,10 @@ bool HipSession::run_device_op(const Node &node, const Op &op, const std::vector
             if (in[2]->elem_ty != TensorElemType::F32 || in[2]->dims.total_elems() != w[0]) return fail(err, SessionError::Shape, "Conv2d: bias must hold one f32 per output channel");
             bias = f(in[2]);
         }
-        DeviceTensor col;
-        const size_t oh = out.dims[2], ow = out.dims[3];
-        if (!allocate(TypedFixedShape{FixedDimensions({x[0], x[1], w[2], w[3], oh, ow}), TensorElemType::F32}, &col, err)) return false;
-        rc = launch_conv2d(ctx_, o, f(in[0]), f(in[1]), bias, static_cast<float *>(col.ptr), x[0], x[1], x[2], x[3], w[0], oh, ow, w[2], w[3],
+        rc = launch_conv2d(ctx_, o, f(in[0]), f(in[1]), bias, x[0], x[1], x[2], x[3], w[0], out.dims[2], out.dims[3], w[2], w[3],
                            (size_t)op.strides[0], (size_t)op.strides[1], (size_t)op.dilations[0], (size_t)op.dilations[1],
                            (size_t)op.padding[0], (size_t)op.padding[1], group);
-        break;  // `col` goes back to the pool here; stream order keeps it intact until the GEMMs have read it
+        break;
     }
     case OpKind::MaxPool: {  // compute_max_pool (session.rs:324-382)
         if (!need(1) || !need_f32({0})) return false;

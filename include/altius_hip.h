@@ -376,9 +376,8 @@ int ahip_xcd_round_robin_holds(int cu_count, const uint32_t *xcc_of_block, size_
 int ahip_gemm_register_constant(ahip_ctx *ctx, const void *ptr, size_t bytes);
 int ahip_gemm_unregister_constant(ahip_ctx *ctx, const void *ptr);
 
-/* Conv2d on NCHW (crates/session_interpreter/src/conv2d.rs:26-211): im2col into `col`
- * (scratch of batch*c*kh*kw*oh*ow floats, the reference's layout [b][c][kh][kw][oh][ow]) and one
- * batched GEMM per group.  w is [oc, c/group, kh, kw]; bias ([oc]) may be NULL.  oh / ow are the
+/* Conv2d on NCHW (crates/session_interpreter/src/conv2d.rs:26-211), which unfolds the input into `col`;
+ * the kernels here read x in place: `col` must not be NULL, and is neither read nor written.  w is [oc, c/group, kh, kw]; bias ([oc]) may be NULL.  oh / ow are the
  * output extents the caller inferred (shape.rs:38-88).
  * MaxPool (compute_max_pool, session.rs:324-382) over [planes, ih, iw] -> [planes, oh, ow]. */
 int ahip_conv2d(ahip_ctx *ctx, float *out, const float *x, const float *w, const float *bias, float *col, size_t batch,

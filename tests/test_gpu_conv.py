@@ -36,6 +36,39 @@ def test_conv2d(ctx, case, case_):
     assert np.allclose(got, O.conv2d(xr, wr, bias, **args), rtol=1e-5, atol=1e-5 * np.sqrt(k))
 
 
+@pytest.mark.parametrize("x, w, args", [
+    # depthwise: planes of one, several planes per block, rows and columns cut into tiles, one and four rows per thread
+    ((1, 5, 1, 1), (5, 1, 3, 3), dict(pads=(1, 1, 1, 1), group=5)),
+    ((3, 37, 7, 7), (37, 1, 5, 5), dict(pads=(2, 2, 2, 2), group=37)),
+    ((2, 3, 67, 131), (3, 1, 5, 5), dict(pads=(2, 2, 2, 2), group=3)),
+    ((40, 96, 29, 30), (96, 1, 3, 3), dict(pads=(1, 1, 1, 1), group=96)),
+    ((40, 96, 29, 31), (96, 1, 5, 5), dict(pads=(2, 2, 2, 2), strides=(2, 2), group=96)),
+    ((40, 96, 29, 31), (96, 1, 5, 5), dict(pads=(2, 2, 2, 2), group=96)),
+    ((40, 96, 28, 31), (96, 1, 3, 3), dict(pads=(1, 1, 1, 1), strides=(2, 2), group=96)),
+    ((2, 6, 20, 23), (12, 1, 3, 5), dict(pads=(1, 2, 3, 0), strides=(1, 3), dilations=(2, 1), group=6)),
+    ((1, 2, 9, 300), (2, 1, 9, 150), dict(group=2)),
+    # products: edges of the 16, 32 and 64 x 128 tiles, k below, at and past a step, images that end inside a tile
+    ((1, 1, 1, 1), (1, 1, 1, 1), dict()),
+    ((1, 16, 4, 4), (16, 16, 1, 1), dict()),
+    ((2, 17, 5, 5), (33, 17, 1, 1), dict()),
+    ((1, 576, 7, 7), (96, 576, 1, 1), dict()),
+    ((9, 40, 64, 64), (65, 40, 1, 1), dict()),
+    ((33, 15, 47, 43), (63, 15, 1, 1), dict()),
+    ((70, 3, 57, 53), (16, 3, 3, 3), dict(pads=(1, 1, 1, 1), strides=(2, 2))),
+    ((1, 24, 19, 21), (36, 12, 3, 3), dict(pads=(1, 1, 1, 1), group=2)),
+    ((1, 64, 30, 30), (40, 64, 1, 1), dict(strides=(2, 2))),
+    ((33, 8, 33, 33), (130, 8, 3, 3), dict(pads=(0, 1, 0, 1), dilations=(2, 1))),
+])
+def test_conv2d_kernel_edges(ctx, case, x, w, args):
+    """Small integers: every product and partial sum is exact in fp32 whatever the order, so the result is the oracle's."""
+    case(f"conv2d edges {x} {w} {args}")
+    args = {**dict(strides=(1, 1), pads=(0, 0, 0, 0), dilations=(1, 1), group=1), **args}
+    xi, wi = RNG.integers(-3, 4, size=x).astype(np.float32), RNG.integers(-3, 4, size=w).astype(np.float32)
+    bias = RNG.integers(-3, 4, size=w[0]).astype(np.float32)
+    for b in (bias, None):
+        assert_bits_equal(ctx.conv2d(xi, wi, b, **args), O.conv2d(xi, wi, b, **args), "vs oracle")
+
+
 def test_max_pool(ctx, case):
     case("maxpool")
     x = RNG.standard_normal((2, 5, 33, 31)).astype(np.float32)
