@@ -68,8 +68,9 @@ int create_device_ctx(int device, hipStream_t stream, bool own_stream, DeviceCtx
     ctx->scratch = static_cast<float *>(scratch);
     ctx->scratch_floats = SCRATCH_FLOATS;
     void *flags = nullptr;
-    e = hipMalloc(&flags, 256);
-    if (e == hipSuccess) e = hipMemset(flags, 0, 256);
+    constexpr size_t FLAG_BYTES = 256;  // the error flags, and behind them the counters of tiles that products cut along k
+    e = hipMalloc(&flags, FLAG_BYTES + GEMM_COUNTERS * sizeof(int));
+    if (e == hipSuccess) e = hipMemset(flags, 0, FLAG_BYTES + GEMM_COUNTERS * sizeof(int));
     if (e != hipSuccess) {
         if (flags) (void)hipFree(flags);
         (void)hipFree(scratch);
@@ -79,6 +80,7 @@ int create_device_ctx(int device, hipStream_t stream, bool own_stream, DeviceCtx
         return fail(e, "hipMalloc(flags)");
     }
     ctx->flags = static_cast<int *>(flags);
+    ctx->gemm_counters = ctx->flags + FLAG_BYTES / sizeof(int);
     ctx->flags_armed = false;
     // Where do blocks run?  Decides whether the bf16 GEMM may combine the slices of a tile inside one XCD's L2.
     // A probe that cannot run leaves the answer at "not shown", which only switches that cut off.
@@ -125,6 +127,7 @@ void destroy_device_ctx(DeviceCtx *ctx) {
     ctx->scratch = nullptr;
     if (ctx->flags) (void)hipFree(ctx->flags);
     ctx->flags = nullptr;
+    ctx->gemm_counters = nullptr;
     if (ctx->owns_stream) (void)hipStreamDestroy(ctx->stream);
     ctx->stream = nullptr;
 }

@@ -60,7 +60,7 @@ struct DeviceCtx {
     void *gemm_ws = nullptr;
     size_t gemm_ws_bytes = 0;
     uint64_t gemm_ws_generation = 0;
-    // Partial sums and arrival counters of tiles the bf16 GEMM cuts along k (device memory, owned).
+    // Partial sums (device memory, owned) and arrival counters (behind the flags) of tiles that products cut along k.
     void *gemm_partials = nullptr;
     size_t gemm_partials_bytes = 0;
     int *gemm_counters = nullptr;
@@ -212,6 +212,10 @@ int launch_layernorm_planes(DeviceCtx &ctx, void *planes, float *sum_out, const 
 bool layernorm_planes_fits(size_t rows, size_t len);
 // The context's grow-only GEMM workspace, at least `bytes` large (stream-ordered use only).
 int gemm_workspace(DeviceCtx &ctx, size_t bytes, void **p);
+// Room for the partial sums of tiles that a product cuts along k (ctx.gemm_partials, at least `bytes`, grow-only) and the
+// counters of such tiles (ctx.gemm_counters, GEMM_COUNTERS of them, zero between launches).
+constexpr size_t GEMM_COUNTERS = 2048;
+int gemm_partials(DeviceCtx &ctx, size_t bytes);
 // Row sums (optionally times `scale`) or maxima of a [rows, len] matrix through LDS-staged groups of rows (rows.hip): for
 // rows that are short or not whole float4s.  Returns -1 without launching when the shape is not one it is meant for.
 int launch_reduce_rows_lds(DeviceCtx &ctx, bool is_max, float *out, const float *in, size_t rows, size_t len, float scale, bool scaled);

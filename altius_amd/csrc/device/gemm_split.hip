@@ -182,7 +182,6 @@ __global__ __launch_bounds__(LNP_THREADS) void layernorm_planes(u32x4 *__restric
 // ---------------------------------------------------------------- the product
 
 constexpr int TM = 256, TN = 256, THREADS = 512;
-constexpr size_t GEMM_COUNTERS = 256;  // tiles cut along k per launch: at most 8 XCDs x 31
 
 // One k step of 16 (two k groups of 8) of both operand tiles.
 struct Stage {
@@ -544,18 +543,9 @@ int ensure_workspace(DeviceCtx &ctx, size_t bytes) {
     return AHIP_OK;
 }
 
-int ensure_partials(DeviceCtx &ctx, size_t bytes) {
-    if (!ctx.gemm_counters) {
-        void *c = nullptr;
-        // Zeroed once, in stream order ahead of the first kernel that counts in it; the kernels leave it zeroed.
-        if (hipMalloc(&c, GEMM_COUNTERS * sizeof(int)) != hipSuccess ||
-            hipMemsetAsync(c, 0, GEMM_COUNTERS * sizeof(int), ctx.stream) != hipSuccess) {
-            (void)hipGetLastError();
-            if (c) (void)hipFree(c);
-            return ctx.fail(AHIP_ERR_OOM, "gemm: no memory for the slice counters");
-        }
-        ctx.gemm_counters = static_cast<int *>(c);
-    }
+}  // namespace
+
+int gemm_partials(DeviceCtx &ctx, size_t bytes) {
     if (bytes <= ctx.gemm_partials_bytes) return AHIP_OK;
     int rc = ctx.check(hipStreamSynchronize(ctx.stream), "hipStreamSynchronize");
     if (rc) return rc;
@@ -572,8 +562,6 @@ int ensure_partials(DeviceCtx &ctx, size_t bytes) {
     ctx.gemm_partials_bytes = bytes;
     return AHIP_OK;
 }
-
-}  // namespace
 
 int gemm_workspace(DeviceCtx &ctx, size_t bytes, void **p) {
     const int rc = ensure_workspace(ctx, bytes);
@@ -667,10 +655,10 @@ int launch_gemm_split(DeviceCtx &ctx, float *c, const float *a, const float *b, 
     if (g.sf > 1) {
         if (!g.misplaced) return ctx.fail(AHIP_ERR_HIP, "gemm: the context has no error flags");
         ctx.flags_armed = true;
-        rc = ensure_partials(ctx, (size_t)8 * (g.chunk - g.full) * g.sf * TM * TN * sizeof(float));
+        rc = gemm_partials(ctx, (size_t)8 * (g.chunk - g.full) * g.sf * TM * TN * sizeof(float));
         if (rc) return rc;
         g.partials = static_cast<float *>(ctx.gemm_partials);
-        g.counters = ctx.gemm_counters;  // allocated by ensure_partials on first use
+        g.counters = ctx.gemm_counters;
         if (!g.partials || !g.counters) return ctx.fail(AHIP_ERR_HIP, "gemm: the buffers for tiles cut along k are missing");
     }
     const uint32_t slots = g.full + (g.chunk - g.full) * g.sf;
@@ -760,8 +748,6 @@ void gemm_release_all(DeviceCtx &ctx) {
     if (ctx.gemm_partials) (void)hipFree(ctx.gemm_partials);
     ctx.gemm_partials = nullptr;
     ctx.gemm_partials_bytes = 0;
-    if (ctx.gemm_counters) (void)hipFree(ctx.gemm_counters);
-    ctx.gemm_counters = nullptr;
 }
 
 }  // namespace altius

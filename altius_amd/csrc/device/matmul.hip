@@ -3,18 +3,28 @@
 // (crates/session_interpreter/src/session.rs:621-684) and compute_gemm (686-794), both of which
 // call sgemm (crates/session_interpreter/src/gemm.rs: the `matrixmultiply` crate or CBLAS).
 //
-// This is the one MFMA-bound kernel of the library.  A 256-thread block (4 wavefronts in a 2 x 2
-// grid) owns a 128 x 128 tile of C; each wavefront accumulates a 64 x 64 sub-tile in four
-// 32 x 32 accumulators with v_mfma_f32_32x32x2_f32 (fp32 in, fp32 accumulate: 256 flop per cycle
-// per CU, 157 Tflop/s on the part).  K advances 16 at a time through double-buffered LDS tiles
-// stored k-major ([k][m] and [k][n], pitch 132 floats) so that a fragment read is 32 consecutive
-// floats per half-wave and the transposing store of a k-contiguous operand spreads over all banks.
-// The global loads of tile t+1 are issued before the MFMA loop of tile t and land in LDS after it:
-// one barrier per K tile.
+// One kernel, gemm_f32_tiles, with v_mfma_f32_32x32x2_f32 (fp32 in, fp32 accumulate: 256 flop per cycle per CU, 157 Tflop/s
+// on the part).  A block's wavefronts form a WM x WN grid over its tile of C, each with TA x TB tiles of 32 x 32, and WK such
+// grids take different values of k (their sums are added in LDS at the end): small tiles for products with few of them, whose
+// time is a chain of loads that WK cuts, large tiles where the chip is full and traffic per operation counts.
+//
+// Operand tiles go from memory to LDS directly (buffer loads, which read zeros behind an operand's end and wherever k is past
+// its end), S - 1 tiles ahead, with one barrier per tile.  Nothing is transposed on the way: an operand whose k is the
+// contiguous axis lies in LDS as [row][16], its 16-byte pieces exchanged by piece ^= (row / 4) % 4 so that a column of pieces
+// covers the banks, and a lane reads four values of k at once; one whose rows are contiguous lies as [k][row], and a lane reads
+// TA (TB) neighbouring rows, one for each of its tiles.  The instruction takes two values of k, one per half of the wavefront;
+// a half takes k = 8 i + 4 half + 0 .. 3 in turn, the same for both layouts, so that a product does not depend on them.
+//
+// Measured against 128 x 128 and 128 x 64 tiles staged through registers, cut along k into batches whose sums a second kernel
+// added, with activations and residuals in a pass of their own (us, whole layers' products in sessions):
+//   [197,768] x [768,768 / 2304 / 3072]: 17 -> 10, 23 -> 14, 29 -> 20 (latency: 168 to 672 tiles of 32 x 32)
+//   [1024,768] x [768,768]: 27 -> 16;  [1024,768] x [768,3072] with Gelu: 76 -> 50
+//   [6304,768] x [768,2304]: 229 -> 200 (112 Tflop/s);  x [768,3072] with Gelu: 323 -> 269
+//   [197,197] x [197,64], 12 heads: 19 -> 7 (single-value loads: rows of 197 start anywhere)
+// What is left on large shapes is power (2.1 GHz under load, where the rate is quoted for 2.4) and the gaps around barriers.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <type_traits>
 
 #include "common.h"
 #include "ctx.h"
@@ -25,248 +35,395 @@ namespace altius {
 namespace {
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) void *lds_ptr;
 
-constexpr int BM = 128, BN = 128, BK = 16;
-constexpr int PITCH = BM + 4;  // floats; (4k + m) mod 64 is a bijection over a transposing store's lanes
-constexpr int THREADS = 256;
+constexpr int BK = 16;  // values of k a wavefront multiplies between two barriers
 
 struct GemmArgs {
-    const float *a, *b, *c0;
+    const float *a, *b, *c0, *residual;
     float *c;
     uint32_t m, n, k;
-    // Element (i, kk) of op(A) is a[i * a_rs + kk * a_cs]; (kk, j) of op(B) is b[kk * b_rs + j * b_cs].
-    // One of the two strides of each operand is 1.
-    uint32_t a_rs, a_cs, b_rs, b_cs;
-    uint32_t ldc;
-    // C0 (Gemm's third input) is read as c0[i * c0_rs + j * c0_cs]; either stride may be 0.
-    uint32_t c0_rs, c0_cs;
-    // Batch z = blockIdx.z is (z / batch_inner, z % batch_inner); operand X starts at
-    // x + (z / batch_inner) * x_bs + (z % batch_inner) * x_bs2 (strides in elements, 0 = shared).
+    // Row pitches of the stored matrices.  C0 (Gemm's third input) is read as c0[i * c0_rs + j * c0_cs]; either stride may be 0.
+    uint32_t lda, ldb, ldc, c0_rs, c0_cs;
+    // Batch z is (z / batch_inner, z % batch_inner); operand X starts at x + (z / batch_inner) * x_bs + (z % batch_inner) * x_bs2
+    // (strides in elements, 0 = shared).
     uint64_t a_bs, b_bs, c_bs, a_bs2, b_bs2, c_bs2;
     uint32_t batch_inner;
-    // Single-batch launches are one-dimensional: consecutive block ids go to the eight XCDs in turn, and
-    // each XCD (one L2) is given a contiguous run of tiles, so the blocks it runs together share panels.
-    // Within that order tiles go by groups of group_n tile columns, each group walked row of tiles by row of tiles,
-    // so that the blocks an XCD runs together cover few columns of B (they stay in its L2) and many rows of A.
-    uint32_t tiles_n, tiles_m, tiles, chunk, group_n;  // chunk = 0: the grid is (n tiles, m tiles, batches)
+    // Consecutive block ids go to the eight XCDs in turn, and each XCD (one L2) is given a contiguous run of `chunk` tiles, so
+    // that the blocks it runs together share panels.  Within that order tiles go by groups of group_n tile columns, each group
+    // walked row of tiles by row of tiles, so that those blocks cover few columns of B (they stay in its L2) and many rows of A.
+    uint32_t tiles_m, tiles_n, tiles, chunk, group_n;  // tiles: of all batches
+    // A tile's k cut into `slices` of slice_k values (whole steps of the block; the last one takes the rest): see the epilogue.
+    uint32_t slices, slice_k;
+    float *partials;
+    int *counters;
     float alpha, beta;
-    int a_vec, b_vec;  // 16-byte loads are legal for this operand (alignment of base, strides, batch stride)
+    int act;
 };
 
-__device__ __forceinline__ float post_ops(float v, int act, const float *__restrict__ residual, size_t at) {
-    if (act == AHIP_GELU) v = dev::gelu_elem(v);
-    else if (act == AHIP_RELU) v = dev::relu_elem(v);
-    if (residual) v = v + residual[at];
+__device__ __forceinline__ float activation(float v, int act) {
+    if (act == AHIP_GELU) return dev::gelu_elem(v);
+    if (act == AHIP_RELU) return dev::relu_elem(v);
     return v;
 }
 
-// Loads this thread's share of a BK x 128 operand tile into registers.
-// K_CONTIG: the operand's k axis is the contiguous one (A without transA, B with transB).
-// `mn` is the tile's first row (A) or column (B), `lim` the extent of that axis.
-// INSIDE: 16-byte loads are legal, the K tile is whole, and an operand whose mn axis is the contiguous one
-// has an extent that is a multiple of 4 (decided per block and K tile, a scalar branch): no per-lane bounds
-// checks, edge tiles clamp their addresses instead.
-template <bool K_CONTIG, int WIDTH, bool INSIDE>
-__device__ __forceinline__ void load_tile(float4 (&r)[WIDTH / 64], const float *__restrict__ p, uint32_t mn0, uint32_t lim,
-                                          uint32_t k0, uint32_t kdim, uint32_t s_mn, uint32_t s_k, int vec, int tid) {
-#pragma unroll
-    for (int u = 0; u < WIDTH / 64; u++) {
-        const int f = tid + THREADS * u;
-        uint32_t mn, kk;
-        if (K_CONTIG) {  // WIDTH rows of 16 floats: 4 float4 per row
-            mn = mn0 + (f >> 2);
-            kk = k0 + ((f & 3) << 2);
-        } else {  // 16 rows of WIDTH floats: WIDTH / 4 float4 per row
-            kk = k0 + f / (WIDTH / 4);
-            mn = mn0 + ((f % (WIDTH / 4)) << 2);
-        }
-        if (INSIDE) {
-            // Rows (or float4 columns) past the operand's edge re-read its last one: in bounds, and what they
-            // contribute only reaches elements of C that are never stored.
-            const uint32_t last = K_CONTIG ? lim - 1 : (lim - 4) & ~3u;
-            if (mn > last) mn = last;
-            r[u] = *reinterpret_cast<const float4 *>(K_CONTIG ? p + (size_t)mn * s_mn + kk : p + (size_t)kk * s_k + mn);
-            continue;
-        }
-        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (K_CONTIG) {
-            if (mn < lim) {
-                const float *q = p + (size_t)mn * s_mn + kk;
-                if (vec && kk + 3 < kdim) {
-                    v = *reinterpret_cast<const float4 *>(q);
-                } else {
-                    if (kk < kdim) v.x = q[0];
-                    if (kk + 1 < kdim) v.y = q[1];
-                    if (kk + 2 < kdim) v.z = q[2];
-                    if (kk + 3 < kdim) v.w = q[3];
-                }
-            }
-        } else {
-            if (kk < kdim) {
-                const float *q = p + (size_t)kk * s_k + mn;
-                if (vec && mn + 3 < lim) {
-                    v = *reinterpret_cast<const float4 *>(q);
-                } else {
-                    if (mn < lim) v.x = q[0];
-                    if (mn + 1 < lim) v.y = q[1];
-                    if (mn + 2 < lim) v.z = q[2];
-                    if (mn + 3 < lim) v.w = q[3];
-                }
-            }
-        }
-        r[u] = v;
-    }
+// Four floats that blocks on any XCD read and write.
+struct Halves {
+    unsigned long long h[2];
+};
+__device__ __forceinline__ void store_shared(f32x4 *p, const f32x4 &v) {
+    const Halves b = __builtin_bit_cast(Halves, v);
+    unsigned long long *q = reinterpret_cast<unsigned long long *>(p);
+    __hip_atomic_store(q, b.h[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(q + 1, b.h[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ f32x4 load_shared(const f32x4 *p) {
+    const unsigned long long *q = reinterpret_cast<const unsigned long long *>(p);
+    Halves b;
+    b.h[0] = __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    b.h[1] = __hip_atomic_load(q + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return __builtin_bit_cast(f32x4, b);
 }
 
-// Stores the registers into the k-major LDS tile [BK][PITCH].
-template <bool K_CONTIG, int WIDTH>
-__device__ __forceinline__ void store_tile(float *__restrict__ t, const float4 (&r)[WIDTH / 64], int tid) {
-#pragma unroll
-    for (int u = 0; u < WIDTH / 64; u++) {
-        const int f = tid + THREADS * u;
-        if (K_CONTIG) {
-            const int mn = f >> 2, kk = (f & 3) << 2;
-            t[(kk + 0) * PITCH + mn] = r[u].x;
-            t[(kk + 1) * PITCH + mn] = r[u].y;
-            t[(kk + 2) * PITCH + mn] = r[u].z;
-            t[(kk + 3) * PITCH + mn] = r[u].w;
-        } else {
-            const int kk = f / (WIDTH / 4), mn = (f % (WIDTH / 4)) << 2;
-            *reinterpret_cast<float4 *>(t + kk * PITCH + mn) = r[u];
-        }
-    }
-}
+// What a lane holds of T tiles of an operand for BK values of k: at(tile, step).  KC: k is the operand's contiguous axis.
+template <bool KC, int T> struct FragRegs;
+template <> struct FragRegs<true, 1> { f32x4 v[2]; __device__ float at(int, int s) const { return v[s >> 2][s & 3]; } };
+template <> struct FragRegs<true, 2> { f32x4 v[4]; __device__ float at(int t, int s) const { return v[t * 2 + (s >> 2)][s & 3]; } };
+template <> struct FragRegs<false, 1> { float v[8]; __device__ float at(int, int s) const { return v[s]; } };
+template <> struct FragRegs<false, 2> { f32x2 v[8]; __device__ float at(int t, int s) const { return v[s][t]; } };
 
-// TN = 128: wavefronts in a 2 x 2 grid, 64 x 64 each.  TN = 64 (narrow outputs such as attention's
-// P x V with 64 columns): wavefronts stacked 4 x 1, 32 x 64 each.
-template <bool A_KC, bool B_KC, int TN>
-__global__ __launch_bounds__(THREADS) void gemm_f32_mfma(GemmArgs g) {
-    constexpr int WI = TN == 128 ? 2 : 1;  // 32-row MFMA tiles per wavefront
-    __shared__ __align__(16) float As[2][BK * PITCH];
-    __shared__ __align__(16) float Bs[2][BK * PITCH];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = TN == 128 ? wave >> 1 : wave, wn = TN == 128 ? wave & 1 : 0;
-    uint32_t tile_m = blockIdx.y, tile_n = blockIdx.x;
-    if (g.chunk) {
-        const uint32_t tile = (blockIdx.x & 7) * g.chunk + (blockIdx.x >> 3);
-        if (tile >= g.tiles) return;
-        const uint32_t per_group = g.tiles_m * g.group_n, grp = tile / per_group, r = tile - grp * per_group;
-        const uint32_t width = min(g.group_n, g.tiles_n - grp * g.group_n);  // the last group may be narrower
-        tile_m = r / width, tile_n = grp * g.group_n + r % width;
-    }
-    const uint32_t m0 = tile_m * BM, n0 = tile_n * TN;
-    const uint32_t zo = blockIdx.z / g.batch_inner, zi = blockIdx.z % g.batch_inner;
-    const float *a = g.a + (size_t)zo * g.a_bs + (size_t)zi * g.a_bs2;
-    const float *b = g.b + (size_t)zo * g.b_bs + (size_t)zi * g.b_bs2;
-    // Strides of the tile's mn axis and k axis for each operand.
-    const uint32_t a_smn = g.a_rs, a_sk = g.a_cs, b_smn = g.b_cs, b_sk = g.b_rs;
+// A stage's fragments of both operands, read and waited for in one asm statement: the compiler's wait-count pass drains every
+// outstanding memory -> LDS load before an LDS read that it cannot prove independent of them, which would undo the prefetch.
+#define RD_K1(X) "ds_read_b128 %[" X "0], %[p" X "0]\n\tds_read_b128 %[" X "1], %[p" X "1]\n\t"
+#define RD_K2(X) RD_K1(X) "ds_read_b128 %[" X "2], %[p" X "0] offset:2048\n\tds_read_b128 %[" X "3], %[p" X "1] offset:2048\n\t"
+#define RD_M8(X, W) \
+    "ds_read_" W " %[" X "0], %[p" X "0]\n\tds_read_" W " %[" X "1], %[p" X "0] offset:%c[s" X "1]\n\t" \
+    "ds_read_" W " %[" X "2], %[p" X "0] offset:%c[s" X "2]\n\tds_read_" W " %[" X "3], %[p" X "0] offset:%c[s" X "3]\n\t" \
+    "ds_read_" W " %[" X "4], %[p" X "0] offset:%c[s" X "4]\n\tds_read_" W " %[" X "5], %[p" X "0] offset:%c[s" X "5]\n\t" \
+    "ds_read_" W " %[" X "6], %[p" X "0] offset:%c[s" X "6]\n\tds_read_" W " %[" X "7], %[p" X "0] offset:%c[s" X "7]\n\t"
+#define RD_M1(X) RD_M8(X, "b32")
+#define RD_M2(X) RD_M8(X, "b64")
+#define OUT_K1(X, F) [X##0] "=&v"(F.v[0]), [X##1] "=&v"(F.v[1])
+#define OUT_K2(X, F) OUT_K1(X, F), [X##2] "=&v"(F.v[2]), [X##3] "=&v"(F.v[3])
+#define OUT_M1(X, F) OUT_K2(X, F), [X##4] "=&v"(F.v[4]), [X##5] "=&v"(F.v[5]), [X##6] "=&v"(F.v[6]), [X##7] "=&v"(F.v[7])
+#define OUT_M2(X, F) OUT_M1(X, F)
+#define IN_K1(X, P, PITCH) [p##X##0] "v"(P[0]), [p##X##1] "v"(P[1])
+#define IN_K2(X, P, PITCH) IN_K1(X, P, PITCH)
+#define IN_M1(X, P, PITCH)                                                                                                             \
+    [p##X##0] "v"(P[0]), [s##X##1] "i"((PITCH) * 4), [s##X##2] "i"((PITCH) * 8), [s##X##3] "i"((PITCH) * 12), [s##X##4] "i"((PITCH) * 32), \
+        [s##X##5] "i"((PITCH) * 36), [s##X##6] "i"((PITCH) * 40), [s##X##7] "i"((PITCH) * 44)
+#define IN_M2(X, P, PITCH) IN_M1(X, P, PITCH)
 
-    floatx16 acc[WI][2];
-#pragma unroll
-    for (int i = 0; i < WI; i++)
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
+template <bool AK, int TA, bool BKC, int TB, int PA, int PB> struct Reader;
+#define READER(AK_, TA_, AKIND, BK_, TB_, BKIND)                                                                                       \
+    template <int PA, int PB> struct Reader<AK_, TA_, BK_, TB_, PA, PB> {                                                              \
+        static __device__ __forceinline__ void read(FragRegs<AK_, TA_> &fa, FragRegs<BK_, TB_> &fb, const uint32_t (&pa)[2], const uint32_t (&pb)[2]) { \
+            asm volatile(RD_##AKIND("a") RD_##BKIND("b") "s_waitcnt lgkmcnt(0)"                                                         \
+                         : OUT_##AKIND(a, fa), OUT_##BKIND(b, fb)                                                                       \
+                         : IN_##AKIND(a, pa, PA), IN_##BKIND(b, pb, PB)                                                                 \
+                         : "memory");                                                                                                   \
+        }                                                                                                                               \
+    };
+READER(true, 1, K1, true, 1, K1)
+READER(true, 1, K1, true, 2, K2)
+READER(true, 2, K2, true, 1, K1)
+READER(true, 2, K2, true, 2, K2)
+READER(true, 1, K1, false, 1, M1)
+READER(true, 1, K1, false, 2, M2)
+READER(true, 2, K2, false, 1, M1)
+READER(true, 2, K2, false, 2, M2)
+READER(false, 1, M1, true, 1, K1)
+READER(false, 1, M1, true, 2, K2)
+READER(false, 2, M2, true, 1, K1)
+READER(false, 2, M2, true, 2, K2)
+READER(false, 1, M1, false, 1, M1)
+READER(false, 1, M1, false, 2, M2)
+READER(false, 2, M2, false, 1, M1)
+READER(false, 2, M2, false, 2, M2)
 
-    // Operands that allow 16-byte loads everywhere run a loop without any bounds check on all K tiles but a
-    // ragged last one (edge tiles clamp their addresses); the choice is a scalar branch around the whole
-    // loop, so the loop is straight-line code between its barriers.
-    const bool inside = g.a_vec && g.b_vec && (A_KC || (g.m & 3) == 0) && (B_KC || (g.n & 3) == 0);
-    const int lr = lane & 31, lk = lane >> 5;
-    auto main_loop = [&](auto inside_tag) {
-        constexpr bool INSIDE = decltype(inside_tag)::value;
-        float4 ra[BM / 64], rb[TN / 64];
-        auto load = [&](uint32_t k0) {
-            if (INSIDE && k0 + BK <= g.k) {
-                load_tile<A_KC, BM, true>(ra, a, m0, g.m, k0, g.k, a_smn, a_sk, 1, tid);
-                load_tile<B_KC, TN, true>(rb, b, n0, g.n, k0, g.k, b_smn, b_sk, 1, tid);
+template <int N> __device__ __forceinline__ void wait_loads_and_barrier() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory"); }
+
+// Copies an operand's tiles to LDS: [WK][W][BK] (KC, pieces exchanged) or [WK][BK][W], VEC floats per lane and instruction.  The
+// operand is addressed as a buffer that ends behind its last element; p walks along k.  A lane whose k lies past the end asks for
+// an offset behind any buffer, and lanes of rows past the edge for zeros or for values that only reach sums nobody stores.
+template <bool KC, int W, int WK, int WAVES, int VEC> struct Loader {
+    static constexpr int PER = 64 * VEC, TILE = W * BK, COUNT = TILE * WK / PER / WAVES;
+    static_assert(COUNT * PER * WAVES == TILE * WK, "whole instructions");
+    uint32_t off[COUNT], kk[COUNT];  // of this lane's pieces: byte offset from p, value of k
+    const float *p;
+    uint64_t left, step;             // floats from p to the operand's end; floats to the next tile
+    __device__ __forceinline__ void init(const float *base, uint64_t floats, uint32_t ld, int wave, int lane) {
+        p = base, left = floats, step = KC ? (uint64_t)(BK * WK) : (uint64_t)(BK * WK) * ld;
+#pragma unroll
+        for (int u = 0; u < COUNT; u++) {
+            const uint32_t f = ((u * WAVES + wave) * 64 + lane) * VEC, sub = f / TILE, q = f % TILE;
+            if (KC) {
+                const uint32_t row = q / BK, piece = (q % BK) / 4, k = sub * BK + ((piece ^ ((row >> 2) & 3)) * 4) + (q & 3);
+                off[u] = (row * ld + k) * 4, kk[u] = k;
             } else {
-                load_tile<A_KC, BM, false>(ra, a, m0, g.m, k0, g.k, a_smn, a_sk, g.a_vec, tid);
-                load_tile<B_KC, TN, false>(rb, b, n0, g.n, k0, g.k, b_smn, b_sk, g.b_vec, tid);
+                const uint32_t row = q / W, k = sub * BK + row;
+                off[u] = (k * ld + q % W) * 4, kk[u] = k;
             }
-        };
-        load(0);
-        store_tile<A_KC, BM>(As[0], ra, tid);
-        store_tile<B_KC, TN>(Bs[0], rb, tid);
-        __syncthreads();
+        }
+    }
+    // k_left: values of k from this tile on
+    __device__ __forceinline__ void issue(float *stage, int wave, uint32_t k_left) {
+        const uint32_t bytes = (uint32_t)min(left, (uint64_t)0x3fffffff) * 4u;
+        const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p), 0, (int)bytes, 0x00020000);
+#pragma unroll
+        for (int u = 0; u < COUNT; u++) {
+            const uint32_t o = kk[u] < k_left ? off[u] : 0xffffffffu;
+            if constexpr (VEC == 4) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr)(stage + (u * WAVES + wave) * PER), 16, (int)o, 0, 0, 0);
+            else __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr)(stage + (u * WAVES + wave) * PER), 4, (int)o, 0, 0, 0);
+        }
+        const uint64_t s = min(step, left);
+        p += s;
+        left -= s;
+    }
+};
 
-        const uint32_t nk = (g.k + BK - 1) / BK;
-        for (uint32_t kt = 0; kt < nk; kt++) {
-            const int cur = kt & 1;
-            const bool more = kt + 1 < nk;
-            if (more) load((kt + 1) * BK);
-            const float *at = As[cur] + wm * (32 * WI) + lr;
-            const float *bt = Bs[cur] + wn * 64 + lr;
+template <bool AKC, bool BKC, int WM, int WN, int WK, int TA, int TB, int VEC>
+__global__ __launch_bounds__(64 * WM * WN * WK) void gemm_f32_tiles(GemmArgs g) {
+    constexpr int S = 3;  // stages; a fourth is 3 to 10 % slower, it costs a block per CU
+    constexpr int WAVES = WM * WN * WK, THREADS = 64 * WAVES, BM = 32 * WM * TA, BN = 32 * WN * TB, BKT = BK * WK;
+    constexpr int STAGE_A = BM * BKT, STAGE = (BM + BN) * BKT;
+    constexpr int CP = BN + 4, PASS_ROWS = 32 * WM, SUMS = WK * PASS_ROWS * CP;  // the epilogue's [WK][PASS_ROWS][CP]
+    __shared__ __align__(16) float lds[S * STAGE > SUMS ? S * STAGE : SUMS];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wk = wave / (WM * WN), wmn = wave % (WM * WN), wm = wmn / WN, wn = wmn % WN;
+    const int lr = lane & 31, lk = lane >> 5;
+
+    // block id -> (slice, tile): an XCD gets a run of consecutive tiles, the slices of a tile next to each other in it
+    const uint32_t xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
+    const uint32_t in_run = local / g.slices, slice = local - in_run * g.slices;
+    const uint32_t tile = xcd * g.chunk + in_run;
+    if (tile >= g.tiles) return;
+    const uint32_t per_batch = g.tiles_m * g.tiles_n, z = tile / per_batch, t = tile - z * per_batch;
+    const uint32_t per_group = g.tiles_m * g.group_n, grp = t / per_group, r = t - grp * per_group;
+    const uint32_t width = min(g.group_n, g.tiles_n - grp * g.group_n);
+    const uint32_t m0 = (r / width) * BM, n0 = (grp * g.group_n + r % width) * BN;
+    const uint32_t zo = z / g.batch_inner, zi = z - zo * g.batch_inner;
+    const uint32_t k0 = slice * g.slice_k, k = min(g.slice_k, g.k - k0);
+    const float *a = g.a + (size_t)zo * g.a_bs + (size_t)zi * g.a_bs2 + (AKC ? (size_t)m0 * g.lda + k0 : (size_t)k0 * g.lda + m0);
+    const float *b = g.b + (size_t)zo * g.b_bs + (size_t)zi * g.b_bs2 + (BKC ? (size_t)n0 * g.ldb + k0 : (size_t)k0 * g.ldb + n0);
+
+    Loader<AKC, BM, WK, WAVES, VEC> la;
+    Loader<BKC, BN, WK, WAVES, VEC> lb;
+    la.init(a, k == 0 ? 0 : AKC ? (uint64_t)(min(g.m - m0, (uint32_t)BM) - 1) * g.lda + k : (uint64_t)(k - 1) * g.lda + (g.m - m0), g.lda, wave, lane);
+    lb.init(b, k == 0 ? 0 : BKC ? (uint64_t)(min(g.n - n0, (uint32_t)BN) - 1) * g.ldb + k : (uint64_t)(k - 1) * g.ldb + (g.n - n0), g.ldb, wave, lane);
+    constexpr int LOADS = decltype(la)::COUNT + decltype(lb)::COUNT;
+
+    floatx16 acc[TA][TB];
 #pragma unroll
-            for (int kk = 0; kk < BK; kk += 2) {
-                float av[WI];
+    for (int i = 0; i < TA; i++)
 #pragma unroll
-                for (int i = 0; i < WI; i++) av[i] = at[(kk + lk) * PITCH + 32 * i];
-                const float b0 = bt[(kk + lk) * PITCH], b1 = bt[(kk + lk) * PITCH + 32];
+        for (int j = 0; j < TB; j++)
 #pragma unroll
-                for (int i = 0; i < WI; i++) {
-                    acc[i][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i], b0, acc[i][0], 0, 0, 0);
-                    acc[i][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i], b1, acc[i][1], 0, 0, 0);
-                }
+            for (int e = 0; e < 16; e++) acc[i][j][e] = 0.0f;
+
+    const uint32_t nk = (k + BKT - 1) / BKT;
+    uint32_t k_left = k;
+    auto issue = [&](uint32_t s) {
+        la.issue(lds + s * STAGE, wave, k_left);
+        lb.issue(lds + s * STAGE + STAGE_A, wave, k_left);
+        k_left -= min(k_left, (uint32_t)BKT);
+    };
+#pragma unroll
+    for (int s = 0; s < S - 1; s++) issue(s);
+
+    // Byte addresses of this lane's fragments in stage 0.
+    uint32_t pa[2], pb[2];
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr)lds;
+    if (AKC) {
+        const uint32_t row = wm * (32 * TA) + lr, sw = (row >> 2) & 3;
+        pa[0] = lds0 + ((wk * BM + row) * BK + ((uint32_t)(lk ^ sw) << 2)) * 4, pa[1] = lds0 + ((wk * BM + row) * BK + ((uint32_t)((2 + lk) ^ sw) << 2)) * 4;
+    } else {
+        pa[0] = lds0 + ((wk * BK + 4 * lk) * BM + wm * (32 * TA) + TA * lr) * 4, pa[1] = 0;
+    }
+    if (BKC) {
+        const uint32_t row = wn * (32 * TB) + lr, sw = (row >> 2) & 3;
+        pb[0] = lds0 + (STAGE_A + (wk * BN + row) * BK + ((uint32_t)(lk ^ sw) << 2)) * 4, pb[1] = lds0 + (STAGE_A + (wk * BN + row) * BK + ((uint32_t)((2 + lk) ^ sw) << 2)) * 4;
+    } else {
+        pb[0] = lds0 + (STAGE_A + (wk * BK + 4 * lk) * BN + wn * (32 * TB) + TB * lr) * 4, pb[1] = 0;
+    }
+
+    uint32_t cur = 0, put = S - 1;
+    for (uint32_t kt = 0; kt < nk; kt++) {
+        wait_loads_and_barrier<(S - 2) * LOADS>();
+        issue(put);
+        if (++put == S) put = 0;
+        FragRegs<AKC, TA> fa;
+        FragRegs<BKC, TB> fb;
+        const uint32_t so = cur * (STAGE * 4);
+        const uint32_t qa[2] = {pa[0] + so, pa[1] + so}, qb[2] = {pb[0] + so, pb[1] + so};
+        Reader<AKC, TA, BKC, TB, BM, BN>::read(fa, fb, qa, qb);
+        if (++cur == S) cur = 0;
+#pragma unroll
+        for (int s = 0; s < 8; s++)
+#pragma unroll
+            for (int i = 0; i < TA; i++)
+#pragma unroll
+                for (int j = 0; j < TB; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa.at(i, s), fb.at(j, s), acc[i][j], 0, 0, 0);
+    }
+    wait_loads_and_barrier<0>();
+
+    // Epilogue, TA passes of PASS_ROWS rows: accumulator e of lane l is row 8 (e / 4) + 4 (l / 32) + e % 4, column l % 32 of its
+    // tile; through LDS the WK sums of an element meet and rows of C are stored 16 bytes per lane.
+    float *c = g.c + (size_t)zo * g.c_bs + (size_t)zi * g.c_bs2;
+    constexpr int PIECES = PASS_ROWS * BN / 4 / THREADS;  // per thread and pass
+    static_assert(PIECES * THREADS * 4 == PASS_ROWS * BN, "whole pieces");
+    // A thread's pieces lie in the same columns: a bias row is read once.
+    static_assert(THREADS % (BN / 4) == 0, "a thread keeps its columns");
+    const uint32_t col = n0 + tid % (BN / 4) * 4, w = col < g.n ? min(g.n - col, 4u) : 0;
+    const bool bias = g.c0 && g.c0_rs == 0;
+    f32x4 bias4 = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (bias) {
+#pragma unroll
+        for (uint32_t e = 0; e < 4; e++)
+            if (e < w) bias4[e] = g.beta * g.c0[(size_t)(col + e) * g.c0_cs];
+    }
+    auto finish = [&](f32x4 v, int pass, int u) {
+        const int pr = (u * THREADS + tid) / (BN / 4);
+        const uint32_t row = m0 + (pr >> 5) * (32 * TA) + (AKC ? 32 * pass + (pr & 31) : TA * (pr & 31) + pass);
+        if (row >= g.m || w == 0) return;
+        const size_t at = (size_t)row * g.ldc + col;
+        v = g.alpha * v;
+        if (bias) v += bias4;
+        if (w == 4) {
+            if (g.c0 && !bias) {
+                const float *q = g.c0 + (size_t)row * g.c0_rs + (size_t)col * g.c0_cs;
+                const f32x4 x = {q[0], q[g.c0_cs], q[2 * (size_t)g.c0_cs], q[3 * (size_t)g.c0_cs]};
+                v += g.beta * x;
             }
-            if (more) {
-                store_tile<A_KC, BM>(As[cur ^ 1], ra, tid);
-                store_tile<B_KC, TN>(Bs[cur ^ 1], rb, tid);
+            if (g.act) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) v[e] = activation(v[e], g.act);
             }
-            __syncthreads();
+            if (g.residual) v += *reinterpret_cast<const dev::v4f_dword *>(g.residual + at);
+            *reinterpret_cast<dev::v4f_dword *>(c + at) = v;
+        } else {
+            for (uint32_t e = 0; e < w; e++) {
+                float x = e == 0 ? v.x : e == 1 ? v.y : v.z;
+                if (g.c0 && !bias) x += g.beta * g.c0[(size_t)row * g.c0_rs + (size_t)(col + e) * g.c0_cs];
+                x = activation(x, g.act);
+                if (g.residual) x += g.residual[at + e];
+                c[at + e] = x;
+            }
         }
     };
-    if (inside) main_loop(std::true_type{});
-    else main_loop(std::false_type{});
-
-    // Accumulator r of lane l is C[8 * (r / 4) + 4 * (l / 32) + r % 4][l % 32] of its 32 x 32 tile.
-    float *c = g.c + (size_t)zo * g.c_bs + (size_t)zi * g.c_bs2;
+    const uint32_t idx = xcd * g.chunk + in_run;
+    f32x4 *parts = reinterpret_cast<f32x4 *>(g.partials) + (size_t)idx * g.slices * (BM * BN / 4) + tid;
 #pragma unroll
-    for (int i = 0; i < WI; i++)
+    for (int i = 0; i < TA; i++) {
+        float *ct = lds + (size_t)wk * (PASS_ROWS * CP);
+        if (i) __syncthreads();
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const uint32_t col = n0 + wn * 64 + j * 32 + lr;
+        for (int e = 0; e < 16; e++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const uint32_t row = m0 + wm * (32 * WI) + i * 32 + 8 * (r >> 2) + 4 * lk + (r & 3);
-                if (row < g.m && col < g.n) {
-                    float v = g.alpha * acc[i][j][r];
-                    if (g.c0) v += g.beta * g.c0[(size_t)row * g.c0_rs + (size_t)col * g.c0_cs];
-                    c[(size_t)row * g.ldc + col] = v;
-                }
-            }
+            for (int j = 0; j < TB; j++)
+                ct[(wm * 32 + 8 * (e >> 2) + 4 * lk + (e & 3)) * CP + wn * (32 * TB) + (BKC ? 32 * j + lr : TB * lr + j)] = acc[i][j][e];
+        __syncthreads();
+        auto sum_at = [&](int u) {
+            const int f = u * THREADS + tid;
+            const float *s = lds + f / (BN / 4) * CP + f % (BN / 4) * 4;
+            f32x4 v = *reinterpret_cast<const f32x4 *>(s);
+#pragma unroll
+            for (int w = 1; w < WK; w++) v += *reinterpret_cast<const f32x4 *>(s + w * (PASS_ROWS * CP));
+            return v;
+        };
+        if (g.slices > 1) {
+#pragma unroll
+            for (int u = 0; u < PIECES; u++) store_shared(parts + (size_t)slice * (BM * BN / 4) + (i * PIECES + u) * THREADS, sum_at(u));
+        } else if (g.act) {  // one copy of the activation's code: unrolled, it slowed every launch down
+#pragma unroll 1
+            for (int u = 0; u < PIECES; u++) finish(sum_at(u), i, u);
+        } else {
+#pragma unroll
+            for (int u = 0; u < PIECES; u++) finish(sum_at(u), i, u);
         }
-}
+    }
+    if (g.slices == 1) return;
 
-// C = alpha * (sum over k slices, in slice order) + beta * C0: the second half of a product cut along k.
-__global__ __launch_bounds__(256) void splitk_finish(float *__restrict__ c, const float *__restrict__ partials, uint32_t slices,
-                                                     uint32_t m, uint32_t n, uint32_t ldc, const float *__restrict__ c0, uint32_t c0_rs,
-                                                     uint32_t c0_cs, float alpha, float beta, int act,
-                                                     const float *__restrict__ residual) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x, total = (size_t)m * n;
-    if (i >= total) return;
-    float sum = partials[i];
-    for (uint32_t s = 1; s < slices; s++) sum += partials[(size_t)s * total + i];
-    const uint32_t row = (uint32_t)(i / n), col = (uint32_t)(i % n);
-    float v = alpha * sum;
-    if (c0) v += beta * c0[(size_t)row * c0_rs + (size_t)col * c0_cs];
-    c[(size_t)row * ldc + col] = post_ops(v, act, residual, (size_t)row * ldc + col);
-}
-
-// c = act(c) + residual in place, for products that were not cut along k (their kernel's epilogue stays free of it:
-// sixty-four inlined activations per thread slowed every launch down).
-__global__ __launch_bounds__(256) void post_in_place(float *__restrict__ c, uint32_t m, uint32_t n, uint32_t ldc, int act,
-                                                     const float *__restrict__ residual) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= (size_t)m * n) return;
-    const size_t at = (i / n) * ldc + i % n;
-    c[at] = post_ops(c[at], act, residual, at);
+    // A tile cut along k: the block that arrives last adds the slices' sums up in slice order, so the result does not depend on who
+    // was last.  The sums pass by the L2s (agent-scope accesses), so it does not matter on which XCD a slice ran; vmcnt(0) says
+    // that this block's are where the others look.
+    __shared__ int arrived;
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (tid == 0) arrived = atomicAdd(&g.counters[idx], 1);
+    __syncthreads();
+    if (arrived != (int)g.slices - 1) return;
+    if (tid == 0) atomicExch(&g.counters[idx], 0);  // ready for the next launch
+#pragma unroll 1
+    for (int p = 0; p < TA * PIECES; p++) {
+        f32x4 v = load_shared(parts + p * THREADS);
+        for (uint32_t q = 1; q < g.slices; q++) v += load_shared(parts + (size_t)q * (BM * BN / 4) + p * THREADS);
+        finish(v, p / PIECES, p % PIECES);
+    }
 }
 
 inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-thread_local int split_k_inner = 0;  // the batched launch of the slices must not cut again (1), and keeps the tile width chosen for the whole product (2: the narrow one)
+// The block tiles, and what a round of blocks (one per CU) costs over 768 values of k, in us, launch and epilogue (3.5 us, and
+// where k is cut 2 us, 0.5 us a slice and the partial sums written and read at 2.5 TB/s) apart.  Fitted to [197, 768] x [768, 768 .. 3072] (32 x 32: 8.1, 11.9 and 16.1 us for 1, 2 and 3
+// rounds), [1024, 768] x [768, 3072] (64 x 64, 3 rounds: 48.5 us), [6304, 768] x [768, 2304 .. 3072] (64 x 64, 14 rounds: 207 us;
+// 128 x 64, 10 rounds: 273 us; 128 x 128, 4 rounds: 219 us).  Per value of C a small tile costs more (each of its operands serves
+// fewer products), but its rounds come in smaller units.
+struct Shape {
+    uint32_t bm, bn, step;  // step: values of k per barrier
+    double round_us;
+};
+constexpr Shape SHAPES[] = {{32, 32, 64, 4.1}, {64, 64, 32, 14.6}, {128, 64, 16, 27.0}, {128, 128, 16, 52.5}};
+constexpr int N_SHAPES = 4;
+
+struct Choice {
+    int shape = 0;
+    uint32_t slices = 1, slice_k = 0;
+};
+
+// Decided by the sizes alone, so that a product and the same product with an operand stored the other way round add up alike.
+// cut: k may be cut into slices.
+Choice choose(size_t batch, size_t m, size_t n, size_t k, size_t cus_per_xcd, bool cut) {
+    Choice best;
+    double best_us = 0.0;
+    for (int s = 0; s < N_SHAPES; s++) {
+        const Shape &sh = SHAPES[s];
+        const size_t chunk = (((m + sh.bm - 1) / sh.bm) * ((n + sh.bn - 1) / sh.bn) * batch + 7) / 8;
+        for (uint32_t want = 1; want <= 8; want *= 2) {
+            if (want > 1 && (!cut || batch != 1 || k < 128 * (size_t)want || chunk * 8 > GEMM_COUNTERS)) break;
+            const size_t slice_k = ((k + want - 1) / want + sh.step - 1) / sh.step * sh.step, slices = slice_k ? (k + slice_k - 1) / slice_k : 1;
+            if (want > 1 && slices != want) continue;
+            const size_t rounds = (chunk * want + cus_per_xcd - 1) / cus_per_xcd;
+            // A CU's only block has nothing to fill its gaps with.
+            const double us = (double)rounds * sh.round_us * (rounds == 1 ? 1.2 : 1.0) * (double)std::max<size_t>(slice_k, sh.step) / 768.0 +
+                              (want > 1 ? 2.0 + 0.5 * want + (double)m * (double)n * 8.0 * want / 2.5e6 : 0.0);
+            if (best_us == 0.0 || us < best_us) {
+                best_us = us;
+                best.shape = s, best.slices = want, best.slice_k = (uint32_t)slice_k;
+            }
+        }
+    }
+    return best;
+}
+
+template <bool AKC, bool BKC> void launch_tiles(const DeviceCtx &ctx, const GemmArgs &g, int shape, bool vec) {
+    const dim3 grid(g.chunk * 8 * g.slices), block(256);
+#define TILES(...)                                                                                                                      \
+    do {                                                                                                                                \
+        if (vec) hipLaunchKernelGGL((gemm_f32_tiles<AKC, BKC, __VA_ARGS__, 4>), grid, block, 0, ctx.stream, g);                         \
+        else hipLaunchKernelGGL((gemm_f32_tiles<AKC, BKC, __VA_ARGS__, 1>), grid, block, 0, ctx.stream, g);                             \
+    } while (0)
+    switch (shape) {
+    case 0: TILES(1, 1, 4, 1, 1); break;
+    case 1: TILES(2, 1, 2, 1, 2); break;
+    case 2: TILES(4, 1, 1, 1, 2); break;
+    default: TILES(2, 2, 1, 2, 2); break;
+    }
+#undef TILES
+}
+
+constexpr size_t TILE_SPAN = (size_t)1 << 30;  // floats from a tile's first element to its last: byte offsets are 32 bits
 
 }  // namespace
 
@@ -281,6 +438,44 @@ int launch_gemm(DeviceCtx &ctx, float *c, const float *a, const float *b, const 
     const size_t a_bs[2] = {a_batch_stride, 0}, b_bs[2] = {b_batch_stride, 0}, c_bs[2] = {c_batch_stride, 0};
     return launch_gemm_batch2(ctx, c, a, b, c0, batch, 1, m, n, k, trans_a, trans_b, lda, ldb, ldc, a_bs, b_bs, c_bs, c0_row_stride,
                               c0_col_stride, alpha, beta);
+}
+
+// The product in parts of at most `part` values of m (axis 0), n (1) or k (2; the parts' sums meet in C).
+static int launch_gemm_far_rows(DeviceCtx &ctx, int axis, size_t part, float *c, const float *a, const float *b, const float *c0, size_t batch_outer,
+                                size_t batch_inner, size_t m, size_t n, size_t k, int trans_a, int trans_b, size_t lda, size_t ldb, size_t ldc,
+                                const size_t a_bs[2], const size_t b_bs[2], const size_t c_bs[2], size_t c0_rs, size_t c0_cs, float alpha, float beta,
+                                const GemmPost *post) {
+    const size_t none[2] = {0, 0};
+    if (axis == 2 && batch_outer * batch_inner > 1) {  // C0 of the second part on is C, which has batches of its own
+        for (size_t z = 0; z < batch_outer * batch_inner; z++) {
+            const size_t zo = z / batch_inner, zi = z % batch_inner;
+            const int rc = launch_gemm_far_rows(ctx, axis, part, c + zo * c_bs[0] + zi * c_bs[1], a + zo * a_bs[0] + zi * a_bs[1],
+                                                b + zo * b_bs[0] + zi * b_bs[1], c0, 1, 1, m, n, k, trans_a, trans_b, lda, ldb, ldc, none, none, none,
+                                                c0_rs, c0_cs, alpha, beta, post);
+            if (rc) return rc;
+        }
+        return AHIP_OK;
+    }
+    const size_t extent = axis == 0 ? m : axis == 1 ? n : k;
+    for (size_t i = 0; i < extent; i += part) {
+        const size_t w = std::min(part, extent - i);
+        int rc;
+        if (axis == 2) {
+            const bool last = i + w == extent;
+            rc = launch_gemm_batch2(ctx, c, a + (trans_a ? i * lda : i), b + (trans_b ? i : i * ldb), i ? c : c0, 1, 1, m, n, w, trans_a, trans_b, lda, ldb,
+                                    ldc, none, none, none, i ? ldc : c0_rs, i ? 1 : c0_cs, alpha, i ? 1.0f : beta, last ? post : nullptr);
+        } else {
+            const size_t r = axis == 0 ? i : 0, q = axis == 1 ? i : 0;
+            GemmPost p;
+            if (post) p = *post;
+            if (p.residual) p.residual += r * ldc + q;
+            rc = launch_gemm_batch2(ctx, c + r * ldc + q, a + (trans_a ? r : r * lda), b + (trans_b ? q * ldb : q), c0 ? c0 + r * c0_rs + q * c0_cs : nullptr,
+                                    batch_outer, batch_inner, axis == 0 ? w : m, axis == 1 ? w : n, k, trans_a, trans_b, lda, ldb, ldc, a_bs, b_bs, c_bs,
+                                    c0_rs, c0_cs, alpha, beta, post ? &p : nullptr);
+        }
+        if (rc) return rc;
+    }
+    return AHIP_OK;
 }
 
 int launch_gemm_batch2(DeviceCtx &ctx, float *c, const float *a, const float *b, const float *c0, size_t batch_outer,
@@ -302,49 +497,23 @@ int launch_gemm_batch2(DeviceCtx &ctx, float *c, const float *a, const float *b,
     // Hundreds of small matrices (attention's two products per head): one block per matrix.
     // (its fetchers address a head's operand with 32-bit byte offsets: 2^29 floats per head at most)
     const size_t a_extent = (m - 1) * lda + k, b_extent = trans_b ? (n - 1) * ldb + k : (k ? k - 1 : 0) * ldb + n;
-    if (!has_post && !trans_a && alpha == 1.0f && (!c0 || beta == 0.0f) && !split_k_inner && gemm_small_batched_fits(batch, m, n, k) &&
+    if (!has_post && !trans_a && alpha == 1.0f && (!c0 || beta == 0.0f) && gemm_small_batched_fits(batch, m, n, k) &&
         a_extent < ((size_t)1 << 29) && b_extent < ((size_t)1 << 29))
         return launch_gemm_small_batched(ctx, c, a, b, batch_outer, batch_inner, m, n, k, trans_b, lda, ldb, ldc, a_batch_strides, b_batch_strides,
                                          c_batch_strides);
-    // The 128 x 64 tile when it leaves fewer idle columns (n = 64: 64 instead of 128 computed), and for long
-    // K loops: with half the accumulators per wavefront more blocks fit a CU and the last round of blocks
-    // is fuller (measured at [50432,3072]x[3072,768]: 120.9 against 110.3 TFLOP/s; the wide tile stays ahead
-    // only where K is short and the tile's fixed costs weigh more, as in attention's 64-deep products).
-    // ... and when the wide tile would leave CUs without a block (the slices of a product cut along k).
-    const size_t cus = ctx.cus_per_xcd ? (size_t)ctx.cus_per_xcd * 8 : 256;
-    const bool narrow = split_k_inner ? split_k_inner == 2
-                                      : n <= 64 || (n < 512 && n % 128 != 0 && n % 128 <= 64) || k >= 256 ||
-                                            ((m + BM - 1) / BM) * ((n + BN - 1) / BN) * batch < cus;
-    const size_t tn = narrow ? 64 : BN;
-    const size_t gy = (m + BM - 1) / BM, gx = (n + tn - 1) / tn;
-    if (gy > 65535 || batch > 65535) return ctx.fail(AHIP_ERR_UNSUPPORTED, "gemm: more than 65535 row tiles or batches");
-    // A single product with few tiles and a long k (one image through a transformer layer) leaves most CUs idle
-    // while each block walks all of k: cut k into slices that run as batches into a workspace, and add the
-    // slices up in order afterwards (the bias and alpha / beta go there).
-    if (batch == 1 && ctx.gemm_split_k && gx * gy <= cus && k >= 512 && !split_k_inner) {
-        size_t slices = std::min<size_t>(std::min<size_t>((2 * cus + gx * gy - 1) / (gx * gy), k / 128), 16);
-        while (slices > 1 && k % (slices * 16) != 0) slices--;  // equal slices of whole k tiles
-        if (slices >= 2) {
-            void *ws = nullptr;
-            int rc = gemm_workspace(ctx, slices * m * n * sizeof(float), &ws);
-            if (rc) return rc;
-            const size_t ks = k / slices;
-            // slice z of op(A) starts ks columns (or rows, transposed) further on; likewise op(B)
-            const size_t a_bs[2] = {trans_a ? ks * lda : ks, 0}, b_bs[2] = {trans_b ? ks : ks * ldb, 0}, c_bs[2] = {m * n, 0};
-            split_k_inner = narrow ? 2 : 1;
-            rc = launch_gemm_batch2(ctx, static_cast<float *>(ws), a, b, nullptr, slices, 1, m, n, ks, trans_a, trans_b, lda, ldb, n, a_bs, b_bs,
-                                    c_bs, 0, 0, 1.0f, 0.0f);
-            split_k_inner = 0;
-            if (rc) return rc;
-            const size_t total = m * n;
-            hipLaunchKernelGGL(splitk_finish, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, ctx.stream, c, static_cast<const float *>(ws),
-                               (uint32_t)slices, (uint32_t)m, (uint32_t)n, (uint32_t)ldc, (c0 && beta != 0.0f) ? c0 : nullptr,
-                               (uint32_t)c0_row_stride, (uint32_t)c0_col_stride, alpha, beta, has_post ? post->act : 0,
-                               has_post ? post->residual : nullptr);
-            return ctx.check(hipGetLastError(), "gemm split-k finish launch");
-        }
-    }
-    GemmArgs g;
+    const bool a_kc = !trans_a, b_kc = trans_b != 0;
+    // Rows so far apart that a tile's would not lie within 32-bit offsets: fewer of them at a time.
+    const size_t a_rows = a_kc ? std::min<size_t>(m, 128) : std::min<size_t>(k, 64), b_rows = b_kc ? std::min<size_t>(n, 128) : std::min<size_t>(k, 64);
+    if (a_rows > 1 && a_rows * lda > TILE_SPAN)
+        return launch_gemm_far_rows(ctx, a_kc ? 0 : 2, std::max<size_t>(1, TILE_SPAN / lda), c, a, b, c0, batch_outer, batch_inner, m, n, k, trans_a, trans_b,
+                                    lda, ldb, ldc, a_batch_strides, b_batch_strides, c_batch_strides, c0_row_stride, c0_col_stride, alpha, beta, post);
+    if (b_rows > 1 && b_rows * ldb > TILE_SPAN)
+        return launch_gemm_far_rows(ctx, b_kc ? 1 : 2, std::max<size_t>(1, TILE_SPAN / ldb), c, a, b, c0, batch_outer, batch_inner, m, n, k, trans_a, trans_b,
+                                    lda, ldb, ldc, a_batch_strides, b_batch_strides, c_batch_strides, c0_row_stride, c0_col_stride, alpha, beta, post);
+    const size_t cus = ctx.cus_per_xcd ? (size_t)ctx.cus_per_xcd : 32;
+    const Choice ch = choose(batch, m, n, k, cus, ctx.gemm_split_k);
+    const Shape &sh = SHAPES[ch.shape];
+    GemmArgs g = {};
     g.a = a;
     g.b = b;
     g.c0 = (c0 && beta != 0.0f) ? c0 : nullptr;
@@ -352,10 +521,8 @@ int launch_gemm_batch2(DeviceCtx &ctx, float *c, const float *a, const float *b,
     g.m = (uint32_t)m;
     g.n = (uint32_t)n;
     g.k = (uint32_t)k;
-    g.a_rs = trans_a ? 1u : (uint32_t)lda;
-    g.a_cs = trans_a ? (uint32_t)lda : 1u;
-    g.b_rs = trans_b ? 1u : (uint32_t)ldb;
-    g.b_cs = trans_b ? (uint32_t)ldb : 1u;
+    g.lda = (uint32_t)lda;
+    g.ldb = (uint32_t)ldb;
     g.ldc = (uint32_t)ldc;
     g.c0_rs = (uint32_t)c0_row_stride;
     g.c0_cs = (uint32_t)c0_col_stride;
@@ -368,37 +535,38 @@ int launch_gemm_batch2(DeviceCtx &ctx, float *c, const float *a, const float *b,
     g.batch_inner = (uint32_t)batch_inner;
     g.alpha = alpha;
     g.beta = beta;
-    g.a_vec = aligned16(a) && lda % 4 == 0 && a_batch_strides[0] % 4 == 0 && a_batch_strides[1] % 4 == 0;
-    g.b_vec = aligned16(b) && ldb % 4 == 0 && b_batch_strides[0] % 4 == 0 && b_batch_strides[1] % 4 == 0;
+    g.act = has_post ? post->act : 0;
+    g.residual = has_post ? post->residual : nullptr;
+    // 16-byte loads: every piece aligned, and whole inside its row.
+    auto vec = [&](const float *p, size_t contiguous, size_t ld, const size_t bs[2]) {
+        return aligned16(p) && contiguous % 4 == 0 && ld % 4 == 0 && bs[0] % 4 == 0 && bs[1] % 4 == 0;
+    };
+    const bool both = vec(a, a_kc ? k : m, lda, a_batch_strides) && vec(b, b_kc ? k : n, ldb, b_batch_strides);
+    const size_t gy = (m + sh.bm - 1) / sh.bm, gx = (n + sh.bn - 1) / sh.bn, tiles = gx * gy * batch;
+    if (gx * gy >= lim || batch >= lim || tiles >= lim / 16) return ctx.fail(AHIP_ERR_UNSUPPORTED, "gemm: too many tiles");
     g.tiles_n = (uint32_t)gx;
     g.tiles_m = (uint32_t)gy;
-    g.tiles = (uint32_t)(gx * gy);
+    g.tiles = (uint32_t)tiles;
+    g.chunk = (uint32_t)((tiles + 7) / 8);
     {
         // Groups of about 768 columns (measured on [50432,768]x[768,2304..3072] and 4096^3 .. 8192^3: widths of
         // 6 to 16 tile columns are within 1 % of each other and up to 3 % ahead of whole rows of tiles; a single
         // column is 3-6 % behind), all groups equally wide.
-        const size_t group = std::max<size_t>(1, 768 / tn), groups = (gx + group - 1) / group;
+        const size_t group = 768 / sh.bn, groups = (gx + group - 1) / group;
         g.group_n = (uint32_t)((gx + groups - 1) / groups);
     }
-    g.chunk = batch == 1 && gx * gy >= 64 && gx * gy < lim / 8 ? (uint32_t)((gx * gy + 7) / 8) : 0;
-    const dim3 grid = g.chunk ? dim3(g.chunk * 8) : dim3((unsigned)gx, (unsigned)gy, (unsigned)batch);
-    const bool a_kc = !trans_a, b_kc = trans_b != 0;
-#define GEMM(AK, BK_, TN_) hipLaunchKernelGGL((gemm_f32_mfma<AK, BK_, TN_>), grid, dim3(THREADS), 0, ctx.stream, g)
-    if (narrow) {
-        if (a_kc && b_kc) GEMM(true, true, 64);
-        else if (a_kc) GEMM(true, false, 64);
-        else if (b_kc) GEMM(false, true, 64);
-        else GEMM(false, false, 64);
-    } else {
-        if (a_kc && b_kc) GEMM(true, true, 128);
-        else if (a_kc) GEMM(true, false, 128);
-        else if (b_kc) GEMM(false, true, 128);
-        else GEMM(false, false, 128);
+    g.slices = ch.slices;
+    g.slice_k = ch.slices > 1 ? ch.slice_k : (uint32_t)k;
+    if (g.slices > 1) {
+        const int rc = gemm_partials(ctx, (size_t)g.chunk * 8 * g.slices * sh.bm * sh.bn * sizeof(float));
+        if (rc) return rc;
+        g.partials = static_cast<float *>(ctx.gemm_partials);
+        g.counters = ctx.gemm_counters;
     }
-#undef GEMM
-    if (has_post)
-        hipLaunchKernelGGL(post_in_place, dim3((unsigned)((m * n + 255) / 256)), dim3(256), 0, ctx.stream, c, (uint32_t)m, (uint32_t)n,
-                           (uint32_t)ldc, post->act, post->residual);
+    if (a_kc && b_kc) launch_tiles<true, true>(ctx, g, ch.shape, both);
+    else if (a_kc) launch_tiles<true, false>(ctx, g, ch.shape, both);
+    else if (b_kc) launch_tiles<false, true>(ctx, g, ch.shape, both);
+    else launch_tiles<false, false>(ctx, g, ch.shape, both);
     return ctx.check(hipGetLastError(), "gemm launch");
 }
 

@@ -1,0 +1,100 @@
+"""The fp32 product's block tiles (32 x 32 with k over four wavefronts, 64 x 64 with k over two, 128 x 64, 128 x 128), k cut
+into slices, 16-byte and single-value loads, all four storage orders: integer operands, whose sums are exact in fp32 in any
+order.  The operands lie between NaNs, so that a value read from outside them and used shows."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from conftest import assert_bits_equal
+
+pytestmark = pytest.mark.gpu
+
+# Sizes around the tiles' edges and k around the steps of 16, 32 and 64 values; in the second row few tiles with a long k
+# (slices), in the third enough tiles for the 64 x 64, 128 x 64 and 128 x 128 blocks, last ones ragged.
+SIZES = [(1, 1, 1), (31, 33, 15), (32, 32, 64), (33, 31, 65), (65, 63, 17), (40, 36, 44),
+         (1, 1000, 1024), (77, 768, 3072), (5, 130, 2052), (100, 40, 1031),
+         (1024, 3072, 48), (1025, 3071, 33), (6304, 2300, 20), (6300, 3073, 37)]
+
+
+def padded(rng, rows, cols, pad, offset):
+    """A [rows, cols] matrix of small integers with pitch cols + pad, `offset` floats into a buffer of NaNs."""
+    x = rng.integers(-3, 4, size=(rows, cols)).astype(np.float32)
+    ld = cols + pad
+    buf = np.full(offset + rows * ld + 64, np.nan, np.float32)
+    buf[offset:offset + rows * ld].reshape(rows, ld)[:, :cols] = x
+    return x, buf, ld
+
+
+@pytest.mark.parametrize("trans_a", [False, True])
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("pad,offset", [(0, 0), (8, 16), (3, 1)])
+def test_every_tile_and_storage_order(ctx, case, trans_a, trans_b, pad, offset):
+    rng = np.random.default_rng(5)
+    for m, n, k in SIZES:
+        case(f"gemm [{m},{k}] x [{k},{n}] trans {trans_a} {trans_b} pad {pad} offset {offset}")
+        a, abuf, lda = padded(rng, *((k, m) if trans_a else (m, k)), pad, offset)
+        b, bbuf, ldb = padded(rng, *((n, k) if trans_b else (k, n)), pad, offset)
+        bias = rng.integers(-3, 4, size=n).astype(np.float32)
+        da, db, dbias = ctx.upload(abuf), ctx.upload(bbuf), ctx.upload(bias)
+        ldc = n + pad
+        dc = ctx.upload(np.full(m * ldc, 7.0, np.float32))
+        try:
+            for _ in range(2):  # a cut tile's counters are ready for the next launch
+                ctx.gemm_raw(dc.ptr, da.ptr + 4 * offset, db.ptr + 4 * offset, dbias.ptr, 1, m, n, k, trans_a, trans_b, lda, ldb, ldc,
+                             c0_rs=0, c0_cs=1, alpha=2.0, beta=1.0)
+                got = ctx.download(dc, (m, ldc))
+                want = 2.0 * np.matmul((a.T if trans_a else a).astype(np.float64), (b.T if trans_b else b).astype(np.float64)) + bias
+                assert_bits_equal(np.ascontiguousarray(got[:, :n]), want.astype(np.float32), "product")
+                assert np.all(got[:, n:] == 7.0), "a store outside the result"
+        finally:
+            for x in (da, db, dc, dbias):
+                ctx.free(x)
+
+
+def test_batches_with_two_strides_and_infinities(ctx, case):
+    case("gemm batches [3, 4] of [70, 20] x [20, 40], an infinity against zeros past k")
+    rng = np.random.default_rng(6)
+    bo, bi, m, n, k = 3, 4, 70, 40, 20
+    a = rng.integers(-3, 4, size=(bo, m, bi, k)).astype(np.float32)  # heads side by side in a row
+    b = rng.integers(-3, 4, size=(bi, k, n)).astype(np.float32)      # shared by the outer axis
+    a[0, 0, 0, 0], a[0, 1, 0, k - 1] = np.inf, np.inf
+    b[:, 0, :] = np.abs(b[:, 0, :]) + 1
+    b[:, k - 1, :] = np.abs(b[:, k - 1, :]) + 1
+    da, db, dc = ctx.upload(a), ctx.upload(b), ctx.alloc(4 * bo * bi * m * n)
+    S = ctypes.c_size_t * 2
+    try:
+        rc = ctx.L.ahip_gemm_batch2(ctx.handle, dc.ptr, da.ptr, db.ptr, None, bo, bi, m, n, k, 0, 0, bi * k, n, n, S(m * bi * k, k), S(0, k * n),
+                                    S(bi * m * n, m * n), 0, 0, 1.0, 0.0)
+        assert rc == 0
+        want = np.matmul(a.transpose(0, 2, 1, 3).astype(np.float64), b.astype(np.float64)).astype(np.float32)
+        assert_bits_equal(ctx.download(dc, want.shape), want, "product")
+    finally:
+        for x in (da, db, dc):
+            ctx.free(x)
+
+
+@pytest.mark.parametrize("axis", ["m", "k"])
+def test_rows_too_far_apart_for_32_bit_offsets(ctx, case, axis):
+    """Rows 2 GiB apart: taken a few at a time (m), or summed in parts (k)."""
+    case(f"gemm rows 2 GiB apart along {axis}")
+    rows, w, n = 3, 6, 5
+    ld = (1 << 29) + 64
+    da = ctx.alloc(4 * ((rows - 1) * ld + w))
+    rng = np.random.default_rng(7)
+    x = rng.integers(-3, 4, size=(rows, w)).astype(np.float32)
+    m, k, trans = (rows, w, False) if axis == "m" else (w, rows, True)
+    b = rng.integers(-3, 4, size=(k, n)).astype(np.float32)
+    c0 = rng.integers(-3, 4, size=(m, n)).astype(np.float32)
+    db, dc0, dc = ctx.upload(b), ctx.upload(c0), ctx.alloc(4 * m * n)
+    try:
+        for r in range(rows):
+            row = np.ascontiguousarray(x[r])
+            assert ctx.L.ahip_h2d_async(ctx.handle, da.ptr + 4 * r * ld, row.ctypes.data, row.nbytes) == 0
+            ctx.sync()
+        ctx.gemm_raw(dc.ptr, da.ptr, db.ptr, dc0.ptr, 1, m, n, k, trans, False, ld, n, n, c0_rs=n, c0_cs=1, alpha=1.0, beta=1.0)
+        want = np.matmul((x.T if trans else x).astype(np.float64), b.astype(np.float64)) + c0
+        assert_bits_equal(ctx.download(dc, (m, n)), want.astype(np.float32), "product")
+    finally:
+        for d in (da, db, dc0, dc):
+            ctx.free(d)
