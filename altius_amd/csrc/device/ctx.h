@@ -121,6 +121,10 @@ int launch_softmax_prologue(DeviceCtx &ctx, float *out, const float *in, size_t 
                             const float *mask, size_t rows_per_mask);
 int launch_layernorm(DeviceCtx &ctx, float *out, const float *in, const float *gamma,
                      const float *beta, size_t rows, size_t len, float eps);
+// The nine operators of a written-out LayerNormalization (ReduceMean, Sub, Pow 2, ReduceMean, Add eps, Sqrt, Div, Mul, Add) in one
+// pass, each rounding as its own kernel does (rows.hip).  Only where norm_chain_fits says so.
+int launch_norm_chain(DeviceCtx &ctx, float *out, const float *in, const float *gamma, const float *beta, size_t rows, size_t len, float eps);
+bool norm_chain_fits(const float *out, const float *in, const float *gamma, const float *beta, size_t rows, size_t len);
 int launch_reduce(DeviceCtx &ctx, int kind, float *out, const float *in, size_t outer, size_t red,
                   size_t inner);
 // The same reduction for callers that may not allocate: partial results go to a fixed array in the code

@@ -116,6 +116,7 @@ std::unique_ptr<HipSession> HipSessionBuilder::build(SessionError *err) {
     }
     s->plan_ = create_execution_plan(s->model_);
     if (strided_views_) s->plan_views(fused_attention_);
+    if (strided_views_ && !enable_profiling_) s->plan_norm_chains();  // a profile names every node
 
     std::string derr;
     int rc = create_device_ctx(device_, nullptr, true, &s->ctx_, &derr);
@@ -297,6 +298,7 @@ bool HipSession::run(const std::vector<Tensor> &inputs, std::vector<Tensor> *out
     copies_avoided_ = 0;
     pending_attn_.clear();
     absorbed_add_.clear();
+    passed_over_.clear();
     std::vector<hipEvent_t> events;
     // Nothing may still read a block when it goes back to the pool for another run, and input
     // tensors must outlive their uploads: every exit path synchronises first.
@@ -400,6 +402,7 @@ bool HipSession::run_device(const std::vector<DeviceTensor> &inputs, std::vector
     copies_avoided_ = 0;
     pending_attn_.clear();
     absorbed_add_.clear();
+    passed_over_.clear();
     for (size_t i = 0; i < g.inputs.size(); i++) {
         if (!inputs[i].ptr && inputs[i].nbytes())
             return fail(err, SessionError::Argument, "run_device: input " + std::to_string(i) + " has no device pointer");
@@ -474,6 +477,7 @@ bool HipSession::try_capture(const std::string &key, const std::vector<Tensor> &
     copies_avoided_ = 0;
     pending_attn_.clear();
     absorbed_add_.clear();
+    passed_over_.clear();
     for (size_t i = 0; i < g.inputs.size(); i++) {
         DeviceTensor d;
         if (!allocate(TypedFixedShape{inputs[i].dims(), inputs[i].elem_ty()}, &d, err)) return false;
@@ -594,6 +598,7 @@ bool HipSession::replay(CapturedRun &run, const std::vector<Tensor> &inputs, std
 }
 
 bool HipSession::run_node(NodeId id, std::map<ValueId, DeviceTensor> &values, SessionError *err) {
+    if (passed_over_.count(id)) return true;
     const Node &node = model_.graph.nodes[id];
     auto opname = [&]() { return std::string(node.op.name()); };  // for messages only
 
@@ -637,6 +642,12 @@ bool HipSession::run_node(NodeId id, std::map<ValueId, DeviceTensor> &values, Se
             !(in[i]->pending_op == PENDING_ATTENTION && i == 0 && attn_softmax_.count(id)) &&
             !(in[i]->pending_op == PENDING_ATTENTION ? flush_attention(node.inputs[i], in[i], err) : apply_pending(in[i], err)))
             return false;
+
+    if (norm_chains_.count(id) && in[0]) {
+        bool done = false;
+        if (!run_norm_chain(id, *in[0], values, &done, err)) return false;
+        if (done) return true;
+    }
 
     // Output shapes: inferred at build time if possible, else now (session.rs:149-158).  Operands
     // whose contents decide a shape are read from their host copy, fetched on demand.

@@ -285,6 +285,18 @@ private:
     std::map<NodeId, PlanesPlan> attn_planes_;
     std::set<NodeId> planes_pass_;
     std::map<NodeId, NodeId> add_into_ln_;  // Add nodes (a residual connection) -> the planes-writing LayerNormalization that reads the sum
+    // A LayerNormalization written out as nine operators whose intermediate results nobody else reads, by its first node: one
+    // kernel computes the last node's result when the first one is due, and the nodes between are passed over.
+    struct NormChainPlan {
+        std::vector<NodeId> rest;  // the eight nodes behind the first
+        ValueId gamma = 0, beta = 0, result = 0;
+        float eps = 0.0f;
+    };
+    std::map<NodeId, NormChainPlan> norm_chains_;
+    std::set<NodeId> passed_over_;  // nodes of this run that a norm chain's kernel has done
+    void plan_norm_chains();
+    // Runs the chain that starts at node `id` if its operands allow it; *done tells.
+    bool run_norm_chain(NodeId id, const DeviceTensor &x, std::map<ValueId, DeviceTensor> &values, bool *done, SessionError *err);
     // Runs a deferred Add into the tensor's block.
     bool flush_add(DeviceTensor *t, SessionError *err);
     std::set<NodeId> lazy_views_;                               // Split / Transpose nodes whose outputs are views

@@ -430,4 +430,94 @@ void HipSession::plan_views(bool fused_attention) {
     }
 }
 
+void HipSession::plan_norm_chains() {
+    const auto users = model_.get_value_users();
+    const Graph &g = model_.graph;
+    auto listed = [](const std::vector<ValueId> &l, ValueId v) { return std::find(l.begin(), l.end(), v) != l.end(); };
+    // An initializer no input of the graph can stand in for.
+    auto constant = [&](ValueId v) -> const Tensor * {
+        auto it = g.inits.find(v);
+        return it == g.inits.end() || listed(g.inputs, v) || it->second.elem_ty() != TensorElemType::F32 || !it->second.has_data() ? nullptr : &it->second;
+    };
+    auto scalar = [&](ValueId v) -> const Tensor * {
+        const Tensor *t = constant(v);
+        return t && t->dims().total_elems() == 1 && t->dims().len() <= 1 ? t : nullptr;
+    };
+    auto row = [&](ValueId v, size_t len) {
+        const Tensor *t = constant(v);
+        return t && t->dims().len() == 1 && t->dims()[0] == len;
+    };
+    // The node of kind `k` that reads v, where v has exactly `readers` readers and is no output of the graph.
+    auto reader = [&](ValueId v, OpKind k, size_t readers, NodeId *id) -> const Node * {
+        auto it = users.find(v);
+        if (it == users.end() || it->second.size() != readers || listed(g.outputs, v)) return nullptr;
+        const Node *found = nullptr;
+        for (NodeId u : it->second)
+            if (g.nodes[u].op.kind == k && g.nodes[u].inputs.size() == (k == OpKind::Sqrt || k == OpKind::ReduceMean ? 1u : 2u) && g.nodes[u].outputs.size() == 1) {
+                if (found) return nullptr;
+                found = &g.nodes[u], *id = u;
+            }
+        return found;
+    };
+    for (const NodeExecutionPlan &step : plan_) {
+        const Node &mean = g.nodes[step.node_id];
+        if (mean.op.kind != OpKind::ReduceMean || mean.inputs.size() != 1 || mean.outputs.size() != 1) continue;
+        const ValueId x = mean.inputs[0];
+        auto inferred = inferred_.find(step.node_id);
+        if (inferred == inferred_.end() || inferred->second.second.empty()) continue;
+        const int64_t rank = (int64_t)inferred->second.second[0].dims.len();  // of x as well: the axis is kept
+        auto last_axis = [&](const Node &n) {
+            return n.op.keep_dims && n.op.axes.size() == 1 && (n.op.axes[0] == -1 || n.op.axes[0] == rank - 1);
+        };
+        if (rank < 1 || !last_axis(mean)) continue;
+        NormChainPlan c;
+        c.rest.resize(8);
+        const Node *sub = reader(mean.outputs[0], OpKind::Sub, 1, &c.rest[0]);
+        if (!sub || sub->inputs[0] != x || sub->inputs[1] != mean.outputs[0] || x == mean.outputs[0]) continue;
+        const ValueId d = sub->outputs[0];
+        const Node *pow = reader(d, OpKind::Pow, 2, &c.rest[1]), *div = reader(d, OpKind::Div, 2, &c.rest[6]);
+        if (!pow || !div || pow->inputs[0] != d || div->inputs[0] != d || div->inputs[1] == d) continue;
+        const Tensor *two = scalar(pow->inputs[1]);
+        if (!two || two->data_f32()[0] != 2.0f) continue;
+        const Node *var = reader(pow->outputs[0], OpKind::ReduceMean, 1, &c.rest[2]);
+        if (!var || !last_axis(*var)) continue;
+        const Node *add = reader(var->outputs[0], OpKind::Add, 1, &c.rest[3]);
+        if (!add) continue;
+        const Tensor *eps = scalar(add->inputs[add->inputs[0] == var->outputs[0] ? 1 : 0]);
+        const Node *sqrt = eps ? reader(add->outputs[0], OpKind::Sqrt, 1, &c.rest[4]) : nullptr;
+        NodeId div_id = 0;
+        if (!sqrt || reader(sqrt->outputs[0], OpKind::Div, 1, &div_id) != div || div->inputs[1] != sqrt->outputs[0]) continue;
+        const Node *mul = reader(div->outputs[0], OpKind::Mul, 1, &c.rest[5]);
+        if (!mul) continue;
+        const Node *shift = reader(mul->outputs[0], OpKind::Add, 1, &c.rest[7]);
+        if (!shift) continue;
+        // The row length: gamma's, checked against x when the chain runs.
+        c.gamma = mul->inputs[mul->inputs[0] == div->outputs[0] ? 1 : 0];
+        c.beta = shift->inputs[shift->inputs[0] == mul->outputs[0] ? 1 : 0];
+        const Tensor *gamma = constant(c.gamma);
+        if (!gamma || gamma->dims().len() != 1 || !row(c.beta, gamma->dims()[0])) continue;
+        c.result = shift->outputs[0];
+        c.eps = eps->data_f32()[0];
+        norm_chains_[step.node_id] = std::move(c);
+    }
+}
+
+bool HipSession::run_norm_chain(NodeId id, const DeviceTensor &x, std::map<ValueId, DeviceTensor> &values, bool *done, SessionError *err) {
+    const NormChainPlan &c = norm_chains_[id];
+    const DeviceTensor &gamma = inits_.at(c.gamma), &beta = inits_.at(c.beta);
+    const size_t rank = x.dims.len(), len = rank ? x.dims[rank - 1] : 0;
+    if (x.elem_ty != TensorElemType::F32 || len == 0 || gamma.dims[0] != len || !x.strides.empty()) return true;
+    const size_t rows = x.dims.total_elems() / len;
+    DeviceTensor out;
+    const float *in = static_cast<const float *>(x.ptr), *gp = static_cast<const float *>(gamma.ptr), *bp = static_cast<const float *>(beta.ptr);
+    if (!norm_chain_fits(in, in, gp, bp, rows, len)) return true;  // the result's block is aligned like every other
+    if (!allocate({x.dims, x.elem_ty}, &out, err)) return false;
+    const int rc = launch_norm_chain(ctx_, static_cast<float *>(out.ptr), in, gp, bp, rows, len, c.eps);
+    if (rc) return fail_code(err, rc, ctx_.last_error);
+    values[c.result] = std::move(out);
+    passed_over_.insert(c.rest.begin(), c.rest.end());
+    *done = true;
+    return true;
+}
+
 }  // namespace altius
