@@ -21,6 +21,7 @@ namespace {
 using namespace dev;
 
 constexpr int BLOCK = 256;
+constexpr size_t MAX_GRID_Y = 65535;
 constexpr size_t DW_LDS_FLOATS = 8192;  // 32 KB: five blocks to a CU
 
 struct DepthwiseArgs {
@@ -238,9 +239,9 @@ __device__ __forceinline__ floatx4 weights4(const float *row, uint32_t k0, uint3
 }
 
 // One block per 16 MT x 16 NT tile; its wavefronts take every 16 th chunk of k in turn, straight from memory (nothing is
-// shared between them, so nothing goes through LDS but the final sum, in wavefront order).  With the small products of
-// one image (96 x 49 over k = 576: 3.8 us, against 3.0 for im2col and 5 to 10 for a general product of it) the whole time is the latency of one chain of loads; cutting k shortens the chain and
-// brings more of them into flight.
+// shared between them, so nothing goes through LDS but the final sum, in wavefront order).  With the small products of one
+// image the whole time is the latency of one chain of loads; cutting k shortens the chain and brings more of them into
+// flight: 96 x 49 over k = 576 takes 3.8 us, against 3.0 for an im2col and 5 to 10 for the general product of its result.
 // (Requesting the next chunk ahead of the products was measured: equal for one tile, 9.1 -> 11.5 us for 2 x 2.)
 // The k of an MFMA may be any four as long as both operands agree: lane q of four takes k0 + 4 q + j in step j, so that
 // a lane's share of w is one 16-byte load per four steps.
@@ -406,11 +407,10 @@ int launch_conv2d(DeviceCtx &ctx, float *out, const float *x, const float *w, co
     if (group == c && launch_depthwise(ctx, out, x, w, bias, batch, c, ih, iw, oc, oh, ow, kh, kw, sh, sw, dh, dw, pad_t, pad_l))
         return ctx.check(hipGetLastError(), "conv2d launch");
     const size_t lim = (size_t)1 << 31, cg = c / group, m = oc / group, k = cg * kh * kw, n = batch * oh * ow;
-    if (n >= lim || k >= lim || m >= lim || c >= lim || oc >= lim || ih >= lim || iw >= lim || group > 65535 || (oh - 1) * sh + pad_t >= lim ||
+    if (n >= lim || k >= lim || m >= lim || c >= lim || oc >= lim || ih >= lim || iw >= lim || (oh - 1) * sh + pad_t >= lim ||
         (ow - 1) * sw + pad_l >= lim || (oh - 1) * sh + (kh - 1) * dh >= lim || (ow - 1) * sw + (kw - 1) * dw >= lim)
         return ctx.fail(AHIP_ERR_UNSUPPORTED, "conv2d: extent above 2^31");
     ConvGemmArgs g;
-    g.x = x, g.w = w, g.bias = bias, g.out = out;
     g.ohw = make_fastdiv((uint32_t)(oh * ow)), g.ow = make_fastdiv((uint32_t)ow);
     g.taps = make_fastdiv((uint32_t)(kh * kw)), g.kw = make_fastdiv((uint32_t)kw);
     g.m = (uint32_t)m, g.n = (uint32_t)n, g.k = (uint32_t)k;
@@ -427,20 +427,18 @@ int launch_conv2d(DeviceCtx &ctx, float *out, const float *x, const float *w, co
         g.tiles_n = (uint32_t)up(n, bn);
         return up(m, bm) * up(n, bn);
     };
-    size_t blocks = grid(TM, TN);
-    if (blocks * group >= 2 * cus) {
-        if (blocks >= lim) return ctx.fail(AHIP_ERR_UNSUPPORTED, "conv2d: more than 2^31 tiles");
-        const dim3 dim((unsigned)blocks, (unsigned)group);
-        if (pointwise) hipLaunchKernelGGL((conv_gemm_tiled<true>), dim, dim3(BLOCK), 0, ctx.stream, g);
-        else hipLaunchKernelGGL((conv_gemm_tiled<false>), dim, dim3(BLOCK), 0, ctx.stream, g);
-    } else {
-        const size_t waves = std::min<size_t>(8, std::max<size_t>(1, up(k, 16)));
-        blocks = grid(32, 32);
-        const bool wide = blocks * group >= 2 * cus;
-        if (!wide) blocks = grid(16, 16);
-        const dim3 dim((unsigned)blocks, (unsigned)group), block((unsigned)(64 * waves));
-        const size_t lds = waves * (wide ? 1024 : 256) * sizeof(float);
-        if (pointwise && wide) hipLaunchKernelGGL((conv_gemm_small<true, 2, 2>), dim, block, lds, ctx.stream, g);
+    const bool tiled = grid(TM, TN) * group >= 2 * cus, wide = !tiled && grid(32, 32) * group >= 2 * cus;
+    const size_t blocks = tiled ? grid(TM, TN) : wide ? grid(32, 32) : grid(16, 16);
+    if (blocks >= lim) return ctx.fail(AHIP_ERR_UNSUPPORTED, "conv2d: more than 2^31 tiles");
+    const size_t waves = std::min<size_t>(8, std::max<size_t>(1, up(k, 16))), lds = waves * (wide ? 1024 : 256) * sizeof(float);
+    const dim3 block((unsigned)(tiled ? BLOCK : 64 * waves));
+    // Groups lie along the grid's second axis, which ends at 65535.
+    for (size_t g0 = 0; g0 < group; g0 += MAX_GRID_Y) {
+        const dim3 dim((unsigned)blocks, (unsigned)std::min(group - g0, MAX_GRID_Y));
+        g.x = x + g0 * cg * ih * iw, g.w = w + g0 * m * k, g.bias = bias ? bias + g0 * m : nullptr, g.out = out + g0 * m * oh * ow;
+        if (tiled && pointwise) hipLaunchKernelGGL((conv_gemm_tiled<true>), dim, block, 0, ctx.stream, g);
+        else if (tiled) hipLaunchKernelGGL((conv_gemm_tiled<false>), dim, block, 0, ctx.stream, g);
+        else if (pointwise && wide) hipLaunchKernelGGL((conv_gemm_small<true, 2, 2>), dim, block, lds, ctx.stream, g);
         else if (pointwise) hipLaunchKernelGGL((conv_gemm_small<true, 1, 1>), dim, block, lds, ctx.stream, g);
         else if (wide) hipLaunchKernelGGL((conv_gemm_small<false, 2, 2>), dim, block, lds, ctx.stream, g);
         else hipLaunchKernelGGL((conv_gemm_small<false, 1, 1>), dim, block, lds, ctx.stream, g);

@@ -1,4 +1,4 @@
-"""Conv2d (im2col + MFMA GEMM) and MaxPool through the C ABI and the session: exact on integer-valued
+"""Conv2d and MaxPool through the C ABI and the session: exact on integer-valued
 data against the oracle and the definition, bounded on random data; padding forms, strides, dilation,
 groups, SAME_UPPER, and the ViT patch embedding feeding the token layout."""
 import numpy as np
@@ -132,3 +132,13 @@ def test_resize(ctx, case):
         (got,) = HipSessionBuilder(m).build().run([x])
         want = O.resize(x, (26, 34), True) if mode == "nearest" else O.resize(x, (30, 40), False)
         assert_bits_equal(got, want, f"session resize {mode}")
+
+
+def test_more_groups_than_a_grid_has_rows(ctx, case):
+    groups = 65535 + 7
+    case(f"conv2d of {groups} groups of two channels")
+    x = RNG.integers(-3, 4, size=(2, 2 * groups, 1, 3)).astype(np.float32)
+    w = RNG.integers(-3, 4, size=(groups, 2, 1, 1)).astype(np.float32)
+    bias = RNG.integers(-3, 4, size=groups).astype(np.float32)
+    want = (x.reshape(2, groups, 2, 1, 3) * w[None, :, :, :, :]).sum(axis=2) + bias[None, :, None, None]
+    assert_bits_equal(ctx.conv2d(x, w, bias, group=groups), want, "against the definition")
