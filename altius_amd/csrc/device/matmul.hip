@@ -394,6 +394,8 @@ Choice choose(size_t batch, size_t m, size_t n, size_t k, size_t cus_per_xcd, bo
             if (want > 1 && (!cut || batch != 1 || k < 128 * (size_t)want || chunk * 8 > GEMM_COUNTERS)) break;
             const size_t slice_k = ((k + want - 1) / want + sh.step - 1) / sh.step * sh.step, slices = slice_k ? (k + slice_k - 1) / slice_k : 1;
             if (want > 1 && slices != want) continue;
+            // A grid ends at 2^32 threads: a few rows with 2^29 columns are more blocks of 32 x 32 than that.
+            if (s < N_SHAPES - 1 && chunk * 8 * want * 256 > 0xffffffffu) break;
             const size_t rounds = (chunk * want + cus_per_xcd - 1) / cus_per_xcd;
             // A CU's only block has nothing to fill its gaps with.
             const double us = (double)rounds * sh.round_us * (rounds == 1 ? 1.2 : 1.0) * (double)std::max<size_t>(slice_k, sh.step) / 768.0 +

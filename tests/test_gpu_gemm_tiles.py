@@ -98,3 +98,21 @@ def test_rows_too_far_apart_for_32_bit_offsets(ctx, case, axis):
     finally:
         for d in (da, db, dc0, dc):
             ctx.free(d)
+
+
+def test_more_columns_than_a_grid_of_small_tiles_holds(ctx, case):
+    """2^29 columns are 2^24 tiles of 32 x 32, 2^32 threads: one more than a grid holds."""
+    n, period = 1 << 29, 1 << 22
+    case(f"gemm [1,1] x [1,{n}]")
+    x = np.random.default_rng(8).integers(-9, 10, size=period).astype(np.float32)
+    da, db, dc = ctx.upload(np.full(1, 3.0, np.float32)), ctx.alloc(4 * n), ctx.alloc(4 * n)
+    try:
+        for start in range(0, n, period):
+            assert ctx.L.ahip_h2d_async(ctx.handle, db.ptr + 4 * start, x.ctypes.data, x.nbytes) == 0
+        ctx.sync()
+        ctx.gemm_raw(dc.ptr, da.ptr, db.ptr, None, 1, 1, n, 1, False, False, 1, n, n, c0_rs=0, c0_cs=0, alpha=1.0, beta=0.0)
+        for start in (0, n // 2 - period, n // 2, n - period):
+            assert_bits_equal(ctx.download(dc, (period,), offset_bytes=4 * start), 3.0 * x, f"columns from {start}")
+    finally:
+        for d in (da, db, dc):
+            ctx.free(d)
