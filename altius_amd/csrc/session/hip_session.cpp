@@ -1013,6 +1013,26 @@ bool HipSession::run_fused_elemwise(const Node &node, const Op &op, const std::v
     return true;
 }
 
+GemmPost HipSession::gemm_post(const MatMulPost &mp, const FixedDimensions &product) const {
+    GemmPost post;
+    post.act = mp.act;
+    if (!mp.has_add || !values_) return post;
+    const FixedDimensions *dims = &product;
+    if (mp.reshaped) {  // the shape under which the Add reads the product
+        auto sh = inferred_.find(mp.reshape);
+        if (sh == inferred_.end() || sh->second.second.empty()) return post;
+        dims = &sh->second.second[0].dims;
+        if (dims->total_elems() != product.total_elems()) return post;
+    }
+    const DeviceTensor *x = nullptr;
+    auto xv = values_->find(mp.residual);
+    if (xv != values_->end()) x = &xv->second;
+    else if (auto xi = inits_.find(mp.residual); xi != inits_.end()) x = &xi->second;
+    if (x && x->ptr && x->elem_ty == TensorElemType::F32 && x->strides.empty() && x->pending_op < 0 && x->applied_op < 0 && x->dims == *dims)
+        post.residual = static_cast<const float *>(x->ptr);
+    return post;
+}
+
 bool HipSession::run_device_op(const Node &node, const Op &op, const std::vector<DeviceTensor *> &in,
                                const std::vector<TypedFixedShape> &shapes, std::vector<DeviceTensor> *outs, SessionError *err) {
     struct LazyName {  // the operator's name, made where a message needs it
@@ -1524,18 +1544,7 @@ bool HipSession::run_device_op(const Node &node, const Op &op, const std::vector
             // On the fp32 kernel, the activation or the residual Add behind the product is done as it is written.
             auto mp = matmul_post_.find(current_node_);
             if (!a_op && mp != matmul_post_.end() && !gemm_takes_split(ctx_, batch * m, n, k)) {
-                GemmPost post;
-                if (mp->second.act) {
-                    post.act = mp->second.act;
-                } else if (mp->second.has_add && values_) {
-                    const DeviceTensor *x = nullptr;
-                    auto xv = values_->find(mp->second.residual);
-                    if (xv != values_->end()) x = &xv->second;
-                    else if (auto xi = inits_.find(mp->second.residual); xi != inits_.end()) x = &xi->second;
-                    if (x && x->ptr && x->elem_ty == TensorElemType::F32 && x->strides.empty() && x->pending_op < 0 && x->applied_op < 0 &&
-                        x->dims == out.dims)
-                        post.residual = static_cast<const float *>(x->ptr);
-                }
+                const GemmPost post = gemm_post(mp->second, out.dims);
                 if (post.act || post.residual) {
                     const size_t none[2] = {0, 0};
                     rc = launch_gemm_batch2(ctx_, o, f(in[0]), f(in[1]), bias, 1, 1, batch * m, n, k, 0, tb, A.ld, B.ld, n, none, none, none, 0, 1, 1.0f,
@@ -1617,6 +1626,18 @@ bool HipSession::run_device_op(const Node &node, const Op &op, const std::vector
             rs = (*st)[0];
             cs = (*st)[1];
             c0 = f(in[2]);
+        }
+        auto mp = matmul_post_.find(current_node_);
+        if (mp != matmul_post_.end() && !gemm_takes_split(ctx_, m, n, k)) {
+            const GemmPost post = gemm_post(mp->second, out.dims);
+            if (post.act || post.residual) {
+                const size_t none[2] = {0, 0};
+                rc = launch_gemm_batch2(ctx_, o, f(in[0]), f(in[1]), c0, 1, 1, m, n, k, op.trans_a, op.trans_b, a[1], b[1], n, none, none, none, rs, cs,
+                                        op.alpha, c0 ? op.beta : 0.0f, &post);
+                if (!rc && post.act) out.applied_op = post.act;
+                if (!rc && post.residual) absorbed_add_[mp->second.add_node] = mp->second.add_input;
+                break;
+            }
         }
         rc = launch_gemm(ctx_, o, f(in[0]), f(in[1]), c0, 1, m, n, k, op.trans_a, op.trans_b, a[1], b[1], n, 0, 0, 0, rs, cs, op.alpha,
                          c0 ? op.beta : 0.0f);

@@ -259,15 +259,20 @@ private:
     std::map<NodeId, AttentionPlan> attn_head_;                  // first MatMul of a fusable attention -> the rest
     std::set<NodeId> attn_softmax_, attn_tail_;
     std::map<ValueId, PendingAttention> pending_attn_;
-    // What follows a MatMul whose result has one reader and can be done while the product is written (fp32 kernel):
-    // a Gelu / Relu node, or an Add of a tensor of the result's shape (a residual connection).
+    // What follows a MatMul or a Gemm whose result has one reader and can be done while the product is written (fp32 kernel):
+    // a Gelu / Relu node, or an Add of a tensor of the result's shape (a residual connection); a Gemm's may stand behind the
+    // Reshape that gives it back the axes exporters fold for it.
     struct MatMulPost {
         int act = 0;            // AHIP_GELU / AHIP_RELU, 0: none
         bool has_add = false;
         NodeId add_node = 0;
         size_t add_input = 0;   // which input of the Add is the product
         ValueId residual = 0;   // the Add's other input
+        bool reshaped = false;
+        NodeId reshape = 0;
     };
+    // What of a plan can be done for a product of this shape now: nothing, an activation, or a residual of the same shape.
+    GemmPost gemm_post(const MatMulPost &mp, const FixedDimensions &product) const;
     std::map<NodeId, MatMulPost> matmul_post_;
     std::map<NodeId, size_t> absorbed_add_;                     // Add nodes whose sum a MatMul wrote in this run -> input holding it
     const std::map<ValueId, DeviceTensor> *values_ = nullptr;   // the running call's values, for run_device_op

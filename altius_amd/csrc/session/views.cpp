@@ -284,6 +284,24 @@ void HipSession::plan_views(bool fused_attention) {
         }
         return true;
     };
+    // Product -> Gelu / Relu, or product -> Add(residual): done by the product's own kernel when it is the fp32 one.
+    // v: the product as that node reads it.
+    auto plan_post = [&](NodeId id, ValueId v, MatMulPost mp) {
+        auto it = users.find(v);
+        if (it == users.end() || it->second.size() != 1 || is_output(v)) return;
+        const NodeId uid = *it->second.begin();
+        const Node &u = g.nodes[uid];
+        if ((u.op.kind == OpKind::Gelu || u.op.kind == OpKind::ReLU) && u.inputs.size() == 1 && u.outputs.size() == 1) {
+            mp.act = u.op.kind == OpKind::Gelu ? AHIP_GELU : AHIP_RELU;
+            matmul_post_[id] = mp;
+        } else if (u.op.kind == OpKind::Add && u.inputs.size() == 2 && u.outputs.size() == 1 && u.inputs[0] != u.inputs[1]) {
+            mp.has_add = true;
+            mp.add_node = uid;
+            mp.add_input = u.inputs[0] == v ? 0 : 1;
+            mp.residual = u.inputs[1 - mp.add_input];
+            matmul_post_[id] = mp;
+        }
+    };
     for (const NodeExecutionPlan &step : plan_) {
         const NodeId id = step.node_id;
         const Node &n = g.nodes[id];
@@ -323,25 +341,20 @@ void HipSession::plan_views(bool fused_attention) {
                 if (add.op.kind == OpKind::Add && add.inputs.size() == 2 && add.outputs.size() == 1 && add.inputs[0] != add.inputs[1])
                     add_into_ln_[par->second] = id;
             }
+        } else if (n.op.kind == OpKind::Gemm && n.outputs.size() == 1) {
+            auto it = users.find(n.outputs[0]);
+            if (it == users.end() || it->second.size() != 1 || is_output(n.outputs[0])) continue;
+            const Node &r = g.nodes[*it->second.begin()];
+            MatMulPost mp;
+            if (r.op.kind == OpKind::Reshape && !r.inputs.empty() && r.inputs[0] == n.outputs[0] && r.outputs.size() == 1) {
+                mp.reshaped = true;
+                mp.reshape = *it->second.begin();
+            }
+            plan_post(id, mp.reshaped ? r.outputs[0] : n.outputs[0], mp);
         } else if (n.op.kind == OpKind::MatMul && n.outputs.size() == 1 && !is_output(n.outputs[0])) {
             auto it = users.find(n.outputs[0]);
             if (it == users.end() || it->second.size() != 1) continue;
-            // MatMul -> Gelu / Relu, or MatMul -> Add(residual): done by the product's own kernel when it is the fp32 one.
-            {
-                const NodeId uid = *it->second.begin();
-                const Node &u = g.nodes[uid];
-                MatMulPost mp;
-                if ((u.op.kind == OpKind::Gelu || u.op.kind == OpKind::ReLU) && u.inputs.size() == 1 && u.outputs.size() == 1) {
-                    mp.act = u.op.kind == OpKind::Gelu ? AHIP_GELU : AHIP_RELU;
-                    matmul_post_[id] = mp;
-                } else if (u.op.kind == OpKind::Add && u.inputs.size() == 2 && u.outputs.size() == 1 && u.inputs[0] != u.inputs[1]) {
-                    mp.has_add = true;
-                    mp.add_node = uid;
-                    mp.add_input = u.inputs[0] == n.outputs[0] ? 0 : 1;
-                    mp.residual = u.inputs[1 - mp.add_input];
-                    matmul_post_[id] = mp;
-                }
-            }
+            plan_post(id, n.outputs[0], MatMulPost());
             // MatMul -> Softmax(last axis, optional scalar scale, no mask) -> MatMul(first operand): one attention kernel.
             if (fused_attention) {
                 const NodeId sid = *it->second.begin();
