@@ -1028,7 +1028,9 @@ GemmPost HipSession::gemm_post(const MatMulPost &mp, const FixedDimensions &prod
     auto xv = values_->find(mp.residual);
     if (xv != values_->end()) x = &xv->second;
     else if (auto xi = inits_.find(mp.residual); xi != inits_.end()) x = &xi->second;
-    if (x && x->ptr && x->elem_ty == TensorElemType::F32 && x->strides.empty() && x->pending_op < 0 && x->applied_op < 0 && x->dims == *dims)
+    // The product's node does not list the residual, so nothing has run an Add that it still owes: its block holds no sum yet.
+    if (x && x->ptr && x->elem_ty == TensorElemType::F32 && x->strides.empty() && x->pending_op < 0 && x->applied_op < 0 && !x->owes_add() &&
+        !x->planes && x->dims == *dims)
         post.residual = static_cast<const float *>(x->ptr);
     return post;
 }

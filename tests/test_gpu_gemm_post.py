@@ -3,6 +3,7 @@ it returns the bits of the session that runs the nodes apart, and leaves apart w
 import numpy as np
 import pytest
 
+from altius_amd import device as D
 from altius_amd.graph import Model, Op
 from altius_amd.session import HipSessionBuilder
 from conftest import assert_bits_equal
@@ -64,3 +65,46 @@ def test_behind_a_gemm(case, after, reshape, form):
                     assert_bits_equal(a, w, "the nodes together and apart")
             if form in ("first", "second") or (form in ("row", "wide") and after != Op.Add):
                 assert together.copies_avoided() > apart.copies_avoided()
+
+
+@pytest.mark.parametrize("product", ["MatMul", "Gemm", "Gemm and Reshape"])
+def test_behind_a_residual_that_is_still_owed(case, product):
+    """s = a + b stands in front of a LayerNormalization that leaves the sum to its own kernel, which runs behind the product
+    (its scale is computed by a later node): the product's kernel must not read s before anybody has written it."""
+    case(f"{product} + a sum that waits for a LayerNormalization")
+    b, t, k, n, wide = 2, 512, 64, 768, 3072
+    rows, rng = b * t, np.random.default_rng(11)
+    normal = lambda *shape: rng.standard_normal(shape).astype(np.float32)  # noqa: E731
+    m = Model(opset_version=17)
+    const = lambda *shape: m.new_initializer(normal(*shape))  # noqa: E731
+
+    def op(kind, inputs, **attrs):
+        out = m.new_val()
+        m.add_node(kind, inputs, [out], **attrs)
+        return out
+
+    shape = [rows, n] if product == "Gemm" else [b, t, n]
+    u_shape = [b, t, k] if product == "MatMul" else [rows, k]
+    shapes = {"a": shape, "b": shape, "u": u_shape, "p": [n], "q": [n]}
+    v = {name: m.new_val_named_and_shaped(name, dims) for name, dims in shapes.items()}
+    for x in v.values():
+        m.add_input(x)
+    s = op(Op.Add, [v["a"], v["b"]])
+    if product == "MatMul":
+        g = op(Op.MatMul, [v["u"], const(k, n)])
+    else:
+        g = op(Op.Gemm, [v["u"], const(k, n), const(n)])
+        if product != "Gemm":
+            g = op(Op.Reshape, [g, m.new_initializer(np.array(shape, np.int64))])
+    y = op(Op.Add, [g, s])
+    gamma = op(Op.Add, [v["p"], v["q"]])
+    h = op(Op.LayerNormalization, [s, gamma, const(n)], axis=-1)
+    z = op(Op.MatMul, [h, const(n, wide)])
+    m.add_output(y)
+    m.add_output(z)
+    sessions = [HipSessionBuilder(m).with_gemm_algorithm(D.GEMM_AUTO).with_strided_views(views).build() for views in (True, False)]
+    for _ in range(3):
+        inputs = [normal(*dims) for dims in shapes.values()]
+        (y0, z0), (y1, z1) = (x.run(inputs) for x in sessions)
+        assert_bits_equal(y0, y1, "the product and the sum")
+        assert_bits_equal(z0, z1, "the product behind the LayerNormalization")
