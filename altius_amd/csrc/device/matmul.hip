@@ -365,46 +365,68 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_f32_tiles(GemmArgs g) 
 
 inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-// The block tiles, and what a round of blocks (one per CU) costs over 768 values of k, in us, launch and epilogue (3.5 us, and
-// where k is cut 2 us, 0.5 us a slice and the partial sums written and read at 2.5 TB/s) apart.  Fitted to [197, 768] x [768, 768 .. 3072] (32 x 32: 8.1, 11.9 and 16.1 us for 1, 2 and 3
-// rounds), [1024, 768] x [768, 3072] (64 x 64, 3 rounds: 48.5 us), [6304, 768] x [768, 2304 .. 3072] (64 x 64, 14 rounds: 207 us;
-// 128 x 64, 10 rounds: 273 us; 128 x 128, 4 rounds: 219 us).  Per value of C a small tile costs more (each of its operands serves
-// fewer products), but its rounds come in smaller units.
+// The block tiles, and what a launch of them takes: launch_us + rounds * (block_us + k_us * k / 768), rounds being the blocks that
+// the busiest CU runs (dealt to the XCDs in turn), times `lone` where that is one: a CU's only block has nothing to fill its gaps
+// with.  Where k is cut, 0.8 us more, slice_us for each slice and the partial sums at 2.5 TB/s.  Fitted to 222 products of 1e8 to
+// 5e11 multiplications with every tile (within 3 % rms of the first three's times and, but for tail_rounds, the fourth's) and to 210
+// of up to 2e7 sums with every tile and cut; of those the choice is 0.7 % behind the best one on average.  Per value of C a small
+// tile costs more (each of its operands serves fewer products), but its rounds come in smaller units.
 struct Shape {
     uint32_t bm, bn, step;  // step: values of k per barrier
-    double round_us;
+    double launch_us, block_us, k_us, lone, slice_us;
 };
-constexpr Shape SHAPES[] = {{32, 32, 64, 4.1}, {64, 64, 32, 14.6}, {128, 64, 16, 27.0}, {128, 128, 16, 52.5}};
+constexpr Shape SHAPES[] = {{32, 32, 64, 3.0, 0.81, 3.71, 1.29, 0.3},
+                            {64, 64, 32, 3.7, 1.15, 12.7, 1.14, 0.9},
+                            {128, 64, 16, 4.9, 1.18, 24.7, 1.16, 1.8},
+                            {128, 128, 16, 4.9, 2.06, 46.5, 1.12, 4.0}};
 constexpr int N_SHAPES = 4;
+
+double cost_us(const Shape &sh, size_t rounds, size_t k) {
+    return sh.launch_us + (double)rounds * (sh.block_us + sh.k_us * (double)k / 768.0) * (rounds == 1 ? sh.lone : 1.0);
+}
+
+// Three 128 x 128 blocks fit a CU.  Those that run together end together where k is cut, or where an operand of 16-byte loads has its
+// rows along m or n, and the blocks left over then fill the slots of few CUs: a fourth or fifth round takes as long as three more, a
+// seventh as two (4096^3: 1440 us for four rounds, 128 x 64 tiles 1070; with both operands' k contiguous 1025 and 1045).
+size_t tail_rounds(size_t rounds) { return rounds == 4 || rounds == 5 ? 6 : rounds == 7 ? 8 : rounds; }
 
 struct Choice {
     int shape = 0;
     uint32_t slices = 1, slice_k = 0;
 };
 
-// Decided by the sizes alone, so that a product and the same product with an operand stored the other way round add up alike.
-// cut: k may be cut into slices.
-Choice choose(size_t batch, size_t m, size_t n, size_t k, size_t cus_per_xcd, bool cut) {
+// What a product adds up in which order is decided by the sizes alone, so that a product and the same product with an operand stored
+// the other way round add up alike (the last two tiles do, as long as k is whole).
+// cut: k may be cut into slices.  tail: an operand of 16-byte loads has its rows along m or n.
+Choice choose(size_t batch, size_t m, size_t n, size_t k, size_t cus_per_xcd, bool cut, bool tail) {
     Choice best;
     double best_us = 0.0;
+    auto chunk_of = [&](const Shape &sh) { return (((m + sh.bm - 1) / sh.bm) * ((n + sh.bn - 1) / sh.bn) * batch + 7) / 8; };
+    auto rounds_of = [&](size_t blocks_per_xcd) { return (blocks_per_xcd + cus_per_xcd - 1) / cus_per_xcd; };
     for (int s = 0; s < N_SHAPES; s++) {
         const Shape &sh = SHAPES[s];
-        const size_t chunk = (((m + sh.bm - 1) / sh.bm) * ((n + sh.bn - 1) / sh.bn) * batch + 7) / 8;
+        const size_t chunk = chunk_of(sh);
         for (uint32_t want = 1; want <= 8; want *= 2) {
             if (want > 1 && (!cut || batch != 1 || k < 128 * (size_t)want || chunk * 8 > GEMM_COUNTERS)) break;
             const size_t slice_k = ((k + want - 1) / want + sh.step - 1) / sh.step * sh.step, slices = slice_k ? (k + slice_k - 1) / slice_k : 1;
             if (want > 1 && slices != want) continue;
             // A grid ends at 2^32 threads: a few rows with 2^29 columns are more blocks of 32 x 32 than that.
             if (s < N_SHAPES - 1 && chunk * 8 * want * 256 > 0xffffffffu) break;
-            const size_t rounds = (chunk * want + cus_per_xcd - 1) / cus_per_xcd;
-            // A CU's only block has nothing to fill its gaps with.
-            const double us = (double)rounds * sh.round_us * (rounds == 1 ? 1.2 : 1.0) * (double)std::max<size_t>(slice_k, sh.step) / 768.0 +
-                              (want > 1 ? 2.0 + 0.5 * want + (double)m * (double)n * 8.0 * want / 2.5e6 : 0.0);
+            size_t rounds = rounds_of(chunk * want);
+            if (want > 1 && s == N_SHAPES - 1) rounds = tail_rounds(rounds);
+            const double us = cost_us(sh, rounds, std::max<size_t>(slice_k, sh.step)) +
+                              (want > 1 ? 0.8 + want * (sh.slice_us + (double)(chunk * 8) * sh.bm * sh.bn * sizeof(float) / 2.5e6) : 0.0);
             if (best_us == 0.0 || us < best_us) {
                 best_us = us;
                 best.shape = s, best.slices = want, best.slice_k = (uint32_t)slice_k;
             }
         }
+    }
+    if (best.shape == N_SHAPES - 1 && best.slices == 1 && tail) {
+        const Shape &large = SHAPES[N_SHAPES - 1], &half = SHAPES[N_SHAPES - 2];
+        const size_t blocks = chunk_of(half);
+        if (blocks * 8 * 256 <= 0xffffffffu && cost_us(half, rounds_of(blocks), k) < cost_us(large, tail_rounds(rounds_of(chunk_of(large))), k))
+            best.shape = N_SHAPES - 2;
     }
     return best;
 }
@@ -513,8 +535,6 @@ int launch_gemm_batch2(DeviceCtx &ctx, float *c, const float *a, const float *b,
         return launch_gemm_far_rows(ctx, b_kc ? 1 : 2, std::max<size_t>(1, TILE_SPAN / ldb), c, a, b, c0, batch_outer, batch_inner, m, n, k, trans_a, trans_b,
                                     lda, ldb, ldc, a_batch_strides, b_batch_strides, c_batch_strides, c0_row_stride, c0_col_stride, alpha, beta, post);
     const size_t cus = ctx.cus_per_xcd ? (size_t)ctx.cus_per_xcd : 32;
-    const Choice ch = choose(batch, m, n, k, cus, ctx.gemm_split_k);
-    const Shape &sh = SHAPES[ch.shape];
     GemmArgs g = {};
     g.a = a;
     g.b = b;
@@ -544,6 +564,8 @@ int launch_gemm_batch2(DeviceCtx &ctx, float *c, const float *a, const float *b,
         return aligned16(p) && contiguous % 4 == 0 && ld % 4 == 0 && bs[0] % 4 == 0 && bs[1] % 4 == 0;
     };
     const bool both = vec(a, a_kc ? k : m, lda, a_batch_strides) && vec(b, b_kc ? k : n, ldb, b_batch_strides);
+    const Choice ch = choose(batch, m, n, k, cus, ctx.gemm_split_k, both && !(a_kc && b_kc));
+    const Shape &sh = SHAPES[ch.shape];
     const size_t gy = (m + sh.bm - 1) / sh.bm, gx = (n + sh.bn - 1) / sh.bn, tiles = gx * gy * batch;
     if (gx * gy >= lim || batch >= lim || tiles >= lim / 16) return ctx.fail(AHIP_ERR_UNSUPPORTED, "gemm: too many tiles");
     g.tiles_n = (uint32_t)gx;

@@ -67,6 +67,18 @@ def test_behind_a_gemm(case, after, reshape, form):
                 assert together.copies_avoided() > apart.copies_avoided()
 
 
+@pytest.mark.parametrize("after", [Op.Add, Op.Gelu])
+@pytest.mark.parametrize("t,k,n", [(551, 1481, 2305), (1411, 6162, 2516)])  # slices of 64 x 64 and of 128 x 128 blocks, ragged
+def test_behind_a_gemm_cut_along_k(case, after, t, k, n):
+    case(f"gemm {t, k, n} in slices, {after}")
+    m = graph(1, t, k, n, after, False, "first", 0)
+    rng = np.random.default_rng(13)
+    x, r = (rng.standard_normal(d).astype(np.float32) for d in ((t, k), (t, n)))
+    together, apart = HipSessionBuilder(m).build(), HipSessionBuilder(m).with_strided_views(False).build()
+    assert_bits_equal(together.run([x, r])[0], apart.run([x, r])[0], "the nodes together and apart")
+    assert together.copies_avoided() > apart.copies_avoided()
+
+
 @pytest.mark.parametrize("product", ["MatMul", "Gemm", "Gemm and Reshape"])
 def test_behind_a_residual_that_is_still_owed(case, product):
     """s = a + b stands in front of a LayerNormalization that leaves the sum to its own kernel, which runs behind the product

@@ -10,11 +10,13 @@ from conftest import assert_bits_equal
 
 pytestmark = pytest.mark.gpu
 
-# Sizes around the tiles' edges and k around the steps of 16, 32 and 64 values; in the second row few tiles with a long k
-# (slices), in the third enough tiles for the 64 x 64, 128 x 64 and 128 x 128 blocks, last ones ragged.
+# Sizes around the tiles' edges and k around the steps of 16, 32 and 64 values; in the second row few tiles with a long k (slices of
+# 32 x 32 blocks), in the third enough tiles for the 64 x 64, 128 x 64 and 128 x 128 blocks, last ones ragged, in the fourth slices
+# of 64 x 64 and of 128 x 128 blocks.
 SIZES = [(1, 1, 1), (31, 33, 15), (32, 32, 64), (33, 31, 65), (65, 63, 17), (40, 36, 44),
          (1, 1000, 1024), (77, 768, 3072), (5, 130, 2052), (100, 40, 1031),
-         (1024, 3072, 48), (1025, 3071, 33), (6304, 2300, 20), (6300, 3073, 37)]
+         (1024, 3072, 48), (1025, 3071, 33), (6304, 2300, 20), (6300, 3073, 37), (3300, 3200, 33),
+         (551, 2305, 1481), (1411, 2516, 6162)]
 
 
 def padded(rng, rows, cols, pad, offset):
