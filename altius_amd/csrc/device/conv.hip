@@ -127,7 +127,11 @@ __global__ __launch_bounds__(BLOCK) void conv_depthwise(DepthwiseArgs g) {
     }
 }
 
-// Returns false (nothing launched) for a geometry whose tile does not fit LDS or whose indices do not fit 31 bits.
+// Returns false (nothing launched) for a geometry that products are better for: one whose tile does not fit LDS or whose indices do
+// not fit 31 bits, and one whose blocks read far more than they need or have little to compute (rows or columns of the kernel far
+// apart, kernels of thousands of taps): a tile of [1,1,2500,2000], 2 x 1 with dilation 2000, holds 8004 values for 4 outputs and
+// takes 8.8 ms, against 24 us as a product; [16,256,33,33], 3 x 3, takes 15 us at dilation 1, 77 at 24 (117 as a product) and 216 at
+// 36 (110).  Both sides' estimates are fitted to 68 geometries from 3 x 3 to 64 x 64 taps, dilations up to 2000 and strides up to 128.
 bool launch_depthwise(DeviceCtx &ctx, float *out, const float *x, const float *w, const float *bias, size_t batch, size_t c, size_t ih,
                       size_t iw, size_t oc, size_t oh, size_t ow, size_t kh, size_t kw, size_t sh, size_t sw, size_t dh, size_t dw,
                       size_t pad_t, size_t pad_l) {
@@ -155,7 +159,12 @@ bool launch_depthwise(DeviceCtx &ctx, float *out, const float *x, const float *w
     }
     step = std::min(step, planes);
     const size_t blocks = tiles_x * tiles_y * up(planes, step);
-    if (blocks >= lim) return false;
+    if (blocks * BLOCK > 0xffffffffu) return false;  // a grid ends at 2^32 threads
+    const double tap_rounds = square ? 0.0 : (double)(kh * kw * up(step * ygroups * cols, BLOCK));
+    const double here_us = 3.0 + 0.03 * tap_rounds + (double)blocks * (6e-4 + 6.7e-7 * (double)floats() + 2.6e-5 * tap_rounds);
+    const size_t chunks = up(kh * kw, 16);
+    const double product_us = 3.0 + 0.5 * (double)up(chunks, 8) + 3.6e-4 * (double)(up(oc / c, 16) * up(batch * oh * ow, 16) * c * chunks);
+    if (here_us > 1.25 * product_us) return false;
     DepthwiseArgs g;
     g.x = x, g.w = w, g.bias = bias, g.out = out;
     g.cols = make_fastdiv((uint32_t)cols), g.ygroups = make_fastdiv((uint32_t)ygroups);

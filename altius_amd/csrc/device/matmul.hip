@@ -393,6 +393,7 @@ size_t tail_rounds(size_t rounds) { return rounds == 4 || rounds == 5 ? 6 : roun
 struct Choice {
     int shape = 0;
     uint32_t slices = 1, slice_k = 0;
+    double us = 0.0;
 };
 
 // What a product adds up in which order is decided by the sizes alone, so that a product and the same product with an operand stored
@@ -425,9 +426,14 @@ Choice choose(size_t batch, size_t m, size_t n, size_t k, size_t cus_per_xcd, bo
     if (best.shape == N_SHAPES - 1 && best.slices == 1 && tail) {
         const Shape &large = SHAPES[N_SHAPES - 1], &half = SHAPES[N_SHAPES - 2];
         const size_t blocks = chunk_of(half);
-        if (blocks * 8 * 256 <= 0xffffffffu && cost_us(half, rounds_of(blocks), k) < cost_us(large, tail_rounds(rounds_of(chunk_of(large))), k))
+        const double half_us = cost_us(half, rounds_of(blocks), k);
+        best_us = cost_us(large, tail_rounds(rounds_of(chunk_of(large))), k);
+        if (blocks * 8 * 256 <= 0xffffffffu && half_us < best_us) {
+            best_us = half_us;
             best.shape = N_SHAPES - 2;
+        }
     }
+    best.us = best_us;
     return best;
 }
 

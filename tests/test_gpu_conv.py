@@ -69,6 +69,32 @@ def test_conv2d_kernel_edges(ctx, case, x, w, args):
         assert_bits_equal(ctx.conv2d(xi, wi, b, **args), O.conv2d(xi, wi, b, **args), "vs oracle")
 
 
+@pytest.mark.parametrize("x, w, args", [
+    ((1, 1, 520, 7), (1, 1, 2, 1), dict(dilations=(500, 1))),                       # few outputs to a tile of 8192 values
+    ((2, 3, 33, 33), (3, 1, 3, 3), dict(dilations=(36, 36), pads=(36,) * 4, group=3)),
+    ((2, 3, 40, 41), (3, 1, 3, 3), dict(dilations=(24, 24), pads=(24,) * 4, group=3)),
+    ((1, 2, 70, 70), (2, 1, 64, 64), dict(group=2)),                                # thousands of taps
+    ((1, 2, 1, 5000), (4, 1, 1, 3), dict(dilations=(1, 2048), group=2)),
+    ((3, 2, 64, 64), (2, 1, 16, 16), dict(strides=(16, 16), group=2)),
+])
+def test_depthwise_that_reads_far_apart(ctx, case, x, w, args):
+    case(f"depthwise far apart {x} {w} {args}")
+    args = {**dict(strides=(1, 1), pads=(0, 0, 0, 0), dilations=(1, 1), group=1), **args}
+    xi, wi = RNG.integers(-3, 4, size=x).astype(np.float32), RNG.integers(-3, 4, size=w).astype(np.float32)
+    bias = RNG.integers(-3, 4, size=w[0]).astype(np.float32)
+    for b in (bias, None):
+        assert_bits_equal(ctx.conv2d(xi, wi, b, **args), O.conv2d(xi, wi, b, **args), "vs oracle")
+
+
+def test_depthwise_of_more_tiles_than_a_grid_holds(ctx, case):
+    """A tile of this geometry holds four outputs: 2^24 of them are 2^32 threads."""
+    rows, cols, apart = 2000, 33600, 2000
+    case(f"depthwise [1,1,{rows + apart},{cols}], 2 x 1, dilation {apart}")
+    x = RNG.integers(-3, 4, size=(1, 1, rows + apart, cols)).astype(np.float32)
+    got = ctx.conv2d(x, np.array([2.0, -3.0], np.float32).reshape(1, 1, 2, 1), None, dilations=(apart, 1))
+    assert np.array_equal(got, 2.0 * x[:, :, :rows] - 3.0 * x[:, :, apart:])
+
+
 def test_max_pool(ctx, case):
     case("maxpool")
     x = RNG.standard_normal((2, 5, 33, 31)).astype(np.float32)
