@@ -1,13 +1,19 @@
 // Conv2d on NCHW (the reference unfolds the input and calls sgemm per image and group,
-// crates/session_interpreter/src/conv2d.rs:26-211).  Two routes, by what the shape is bound by:
+// crates/session_interpreter/src/conv2d.rs:26-211).  Three routes:
 //
 //   depthwise   one input channel per group: 2 k^2 flop per output and no reuse across channels, so the convolution is
 //               bound by reading x and writing y once.  conv_depthwise, over tiles in LDS.
-//   the rest    one product per group, W[oc / group, K] times the unfolded input [K, batch * oh * ow] with
+//   in place    one product per group, W[oc / group, K] times the unfolded input [K, batch * oh * ow] with
 //               K = c / group * kh * kw, whose second operand is read from x in place (an element's address is worked out
 //               from its k and its output position; 1 x 1 kernels need no more than k * ih * iw).  The columns of all images
-//               are one axis, so that small images fill whole tiles.  conv_gemm_tiled where the tiles fill the chip,
-//               conv_gemm_small, which cuts K over the wavefronts of a block, where they do not.
+//               are one axis, so that small images fill whole tiles.  conv_gemm_small, which cuts K over the wavefronts of a
+//               block, in tiles of 16 x 16 or 32 x 32, or conv_gemm_tiled.
+//   unfolded    the general fp32 product (matmul.hip), batched over the images, of the input as it lies (1 x 1 kernels) or of
+//               an unfolded copy: its tiles go to LDS without passing registers, k can be cut over blocks, and an element's
+//               address is worked out once instead of once per tile of output channels.  Ahead where K and the output
+//               channels are many.
+//
+// Which one of the last two, and which tile, is decided by what each is estimated to take (conv_route).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -405,6 +411,102 @@ __global__ __launch_bounds__(BLOCK) void conv_gemm_tiled(ConvGemmArgs g) {
     }
 }
 
+// col[image][c][fy][fx][oh][ow] = x[image][c][oh * sh - pad_t + fy * dh][ow * sw - pad_l + fx * dw], zero outside the image
+// (conv2d.rs:82-150, 213-333).  Bound by writing col: 2.0 us per million elements.
+struct UnfoldArgs {
+    FastDiv ow, oh, kw, kh;
+    uint32_t ih, iw, sh, sw, dh, dw, total;
+    int32_t pad_t, pad_l;
+};
+
+__global__ __launch_bounds__(BLOCK) void conv_unfold(float *__restrict__ col, const float *__restrict__ x, UnfoldArgs g) {
+    const uint32_t i = blockIdx.x * BLOCK + threadIdx.x;
+    if (i >= g.total) return;
+    const uint32_t r1 = g.ow.div(i), ox = i - r1 * g.ow.d;
+    const uint32_t r2 = g.oh.div(r1), oy = r1 - r2 * g.oh.d;
+    const uint32_t r3 = g.kw.div(r2), fx = r2 - r3 * g.kw.d;
+    const uint32_t plane = g.kh.div(r3), fy = r3 - plane * g.kh.d;
+    const int yy = (int)(oy * g.sh + fy * g.dh) - g.pad_t, xx = (int)(ox * g.sw + fx * g.dw) - g.pad_l;
+    float v = 0.0f;
+    if (yy >= 0 && yy < (int)g.ih && xx >= 0 && xx < (int)g.iw) v = x[((size_t)plane * g.ih + (uint32_t)yy) * g.iw + (uint32_t)xx];
+    col[i] = v;
+}
+
+// The unfolded copy lives in the context's workspace, of as many images at a time as this holds, or of as many output rows of one
+// image: 1 GiB ([32,2048,28,28] -> 256, 3 x 3: 4010 us in passes of four images, 256 MiB; 3300 in two passes).
+constexpr size_t UNFOLD_FLOATS = (size_t)256 << 20;
+
+enum Route { SMALL_16, SMALL_32, TILED, UNFOLDED };
+
+// What a launch of an in-place kernel takes, in us, over `chunks` of 16 values of k: base + chain * (chunks one wavefront walks)
+// + tiles * (chunk * chunks + tile) for the small ones; for the tiled one rounds * (tile + chunk * chunks), of 256 tiles each, or
+// alone + alone_chunk * chunks where that is one.  The unfolded route takes its own kernel and one product per group.  Fitted to 336
+// geometries (1 x 1 to 16 x 16 taps, 3 to 2048 channels, images of 7 x 7 to 224 x 224, batches of 1 to 64, up to 32 groups), every
+// route timed on each: within 9 % (rms) of the unfolded one, 9 to 15 % of the tiled and 16 to 24 % of the small ones, and the route
+// chosen is 1.3 % behind the best one on average.  (Before, tiles from 512 of them on and no unfolded route: 19 %;
+// [32,1024,14,14] -> 2048, 1 x 1 with stride 2: 260 us, 95 unfolded; [4,320,64,64] -> 320, 3 x 3: 555 and 322.)
+struct SmallCost { double base, chain, chunk, tile; };
+struct TiledCost { double base, tile, chunk, alone, alone_chunk; };
+constexpr SmallCost SMALL_COST[2][2] = {{{2.8, 0.55, 0.28e-3, 0.41e-3}, {2.8, 0.11, 0.27e-3, 0.16e-3}},   // 16 x 16: windows, pointwise
+                                        {{2.9, 1.26, 0.65e-3, 1.10e-3}, {2.9, 0.68, 0.62e-3, 0.66e-3}}};  // 32 x 32
+constexpr TiledCost TILED_COST[2] = {{6.0, 0.5, 1.01, 0.0, 1.82}, {3.6, 1.75, 0.64, 3.4, 0.94}};
+
+// What the unfolded route takes at a time: `images` images, or `rows` output rows of one; none where it cannot be taken.
+struct Pass { size_t images = 0, rows = 0; };
+
+Route conv_route(const DeviceCtx &ctx, size_t batch, size_t m, size_t oh, size_t ow, size_t k, size_t group, Pass pass, bool pointwise, bool vec) {
+    auto up = [](size_t a, size_t b) { return (a + b - 1) / b; };
+    const size_t n = batch * oh * ow, chunks = up(k, 16), waves = std::min<size_t>(8, std::max<size_t>(1, chunks));
+    const TiledCost &t = TILED_COST[pointwise];
+    const size_t rounds = up(up(m, TM) * up(n, TN) * group, 256);
+    Route best = TILED;
+    double best_us = t.base + (rounds > 1 ? (double)rounds * (t.tile + t.chunk * (double)chunks) : t.alone + t.alone_chunk * (double)chunks);
+    for (size_t s = 0; s < 2; s++) {
+        const size_t tiles = up(m, 16 << s) * up(n, 16 << s);
+        if (tiles * 64 * waves > 0xffffffffu) continue;  // a grid ends at 2^32 threads
+        const SmallCost &c = SMALL_COST[s][pointwise];
+        const double us = c.base + c.chain * (double)up(chunks, waves) + (double)(tiles * group) * (c.chunk * (double)chunks + c.tile);
+        if (us < best_us) best_us = us, best = s ? SMALL_32 : SMALL_16;
+    }
+    if (pass.images) {
+        const size_t cols = pass.rows * ow;
+        const double pass_us = (pointwise ? 0.0 : 2.8 + 2.0e-6 * (double)(pass.images * group * k * cols)) +
+                               (double)group * gemm_f32_us(ctx, pass.images, m, cols, k, false, vec);
+        if ((double)(batch * oh) / (double)(pass.images * pass.rows) * pass_us < best_us) best = UNFOLDED;
+    }
+    return best;
+}
+
+int launch_unfolded(DeviceCtx &ctx, float *out, const float *x, const float *w, const float *bias, Pass pass, bool pointwise, size_t batch, size_t c,
+                    size_t ih, size_t iw, size_t oc, size_t oh, size_t ow, size_t kh, size_t kw, size_t sh, size_t sw, size_t dh, size_t dw, size_t pad_t,
+                    size_t pad_l, size_t group) {
+    const size_t ohw = oh * ow, m = oc / group, k = c / group * kh * kw;
+    void *ws = nullptr;
+    if (!pointwise)
+        if (int rc = gemm_workspace(ctx, pass.images * c * kh * kw * pass.rows * ow * sizeof(float), &ws)) return rc;
+    for (size_t b0 = 0; b0 < batch; b0 += pass.images)
+        for (size_t y0 = 0; y0 < oh; y0 += pass.rows) {
+            const size_t images = std::min(pass.images, batch - b0), rows = std::min(pass.rows, oh - y0), cols = rows * ow, total = images * c * kh * kw * cols;
+            const float *src = x + b0 * c * ih * iw;
+            if (!pointwise) {
+                UnfoldArgs g;
+                g.ow = make_fastdiv((uint32_t)ow), g.oh = make_fastdiv((uint32_t)rows), g.kw = make_fastdiv((uint32_t)kw), g.kh = make_fastdiv((uint32_t)kh);
+                g.ih = (uint32_t)ih, g.iw = (uint32_t)iw, g.sh = (uint32_t)sh, g.sw = (uint32_t)sw, g.dh = (uint32_t)dh, g.dw = (uint32_t)dw;
+                g.pad_t = (int32_t)((int64_t)pad_t - (int64_t)(y0 * sh)), g.pad_l = (int32_t)pad_l, g.total = (uint32_t)total;
+                hipLaunchKernelGGL(conv_unfold, dim3((unsigned)((total + BLOCK - 1) / BLOCK)), dim3(BLOCK), 0, ctx.stream, static_cast<float *>(ws), src, g);
+                if (int rc = ctx.check(hipGetLastError(), "conv2d launch")) return rc;
+                src = static_cast<const float *>(ws);
+            }
+            const size_t none[2] = {0, 0}, b_bs[2] = {group * k * cols, 0}, c_bs[2] = {oc * ohw, 0};
+            for (size_t q = 0; q < group; q++) {
+                const int rc = launch_gemm_f32(ctx, out + (b0 * oc + q * m) * ohw + y0 * ow, w + q * m * k, src + q * k * cols, bias ? bias + q * m : nullptr,
+                                               images, 1, m, cols, k, 0, 0, k, cols, ohw, none, b_bs, c_bs, 1, 0, 1.0f, bias ? 1.0f : 0.0f);
+                if (rc) return rc;
+            }
+        }
+    return AHIP_OK;
+}
+
 }  // namespace
 
 int launch_conv2d(DeviceCtx &ctx, float *out, const float *x, const float *w, const float *bias, size_t batch, size_t c, size_t ih, size_t iw,
@@ -430,17 +532,28 @@ int launch_conv2d(DeviceCtx &ctx, float *out, const float *x, const float *w, co
     auto a16 = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
     g.w_vec = k % 4 == 0 && a16(w);
     g.x_vec = pointwise && (ih * iw) % 4 == 0 && a16(x);
-    const size_t cus = ctx.cus_per_xcd ? (size_t)ctx.cus_per_xcd * 8 : 256;
     auto up = [](size_t a, size_t b) { return (a + b - 1) / b; };
     auto grid = [&](size_t bm, size_t bn) {
         g.tiles_n = (uint32_t)up(n, bn);
         return up(m, bm) * up(n, bn);
     };
-    const bool tiled = grid(TM, TN) * group >= 2 * cus, wide = !tiled && grid(32, 32) * group >= 2 * cus;
+    Pass pass;
+    const size_t row = c * kh * kw * ow;  // floats of one output row, unfolded; the product's rows of 2^24 columns are far apart (matmul.hip)
+    if (pointwise) pass.images = batch, pass.rows = oh;
+    else if (row && row * oh <= UNFOLD_FLOATS) pass.images = up(batch, up(batch, UNFOLD_FLOATS / (row * oh))), pass.rows = oh;
+    else if (row && row <= UNFOLD_FLOATS) pass.images = 1, pass.rows = up(oh, up(oh, UNFOLD_FLOATS / row));
+    if (pass.rows * ow > (size_t)1 << 24) pass.images = 0;
+    Route route = conv_route(ctx, batch, m, oh, ow, k, group, pass, pointwise, g.w_vec && (pass.rows * ow) % 4 == 0 && (!pointwise || a16(x)));
+    if (route == UNFOLDED) {
+        const int rc = launch_unfolded(ctx, out, x, w, bias, pass, pointwise, batch, c, ih, iw, oc, oh, ow, kh, kw, sh, sw, dh, dw, pad_t, pad_l, group);
+        if (rc != AHIP_ERR_OOM && rc != AHIP_ERR_UNSUPPORTED) return rc;
+        route = conv_route(ctx, batch, m, oh, ow, k, group, Pass(), pointwise, false);  // no room for the copy
+    }
+    const bool tiled = route == TILED, wide = route == SMALL_32;
     const size_t blocks = tiled ? grid(TM, TN) : wide ? grid(32, 32) : grid(16, 16);
-    if (blocks >= lim) return ctx.fail(AHIP_ERR_UNSUPPORTED, "conv2d: more than 2^31 tiles");
     const size_t waves = std::min<size_t>(8, std::max<size_t>(1, up(k, 16))), lds = waves * (wide ? 1024 : 256) * sizeof(float);
     const dim3 block((unsigned)(tiled ? BLOCK : 64 * waves));
+    if (blocks * block.x > 0xffffffffu) return ctx.fail(AHIP_ERR_UNSUPPORTED, "conv2d: more tiles than a grid holds");
     // Groups lie along the grid's second axis, which ends at 65535.
     for (size_t g0 = 0; g0 < group; g0 += MAX_GRID_Y) {
         const dim3 dim((unsigned)blocks, (unsigned)std::min(group - g0, MAX_GRID_Y));

@@ -178,6 +178,14 @@ int launch_gemm_batch2(DeviceCtx &ctx, float *c, const float *a, const float *b,
                        const size_t a_batch_strides[2], const size_t b_batch_strides[2], const size_t c_batch_strides[2],
                        size_t c0_row_stride, size_t c0_col_stride, float alpha, float beta, const GemmPost *post = nullptr);
 
+// The same, on the fp32 kernels whatever ctx.gemm_algorithm says; and about how long the tiled one takes, in us (k_rows: k is the
+// contiguous axis of both operands, vec: both allow 16-byte loads).
+int launch_gemm_f32(DeviceCtx &ctx, float *c, const float *a, const float *b, const float *c0, size_t batch_outer, size_t batch_inner, size_t m,
+                    size_t n, size_t k, int trans_a, int trans_b, size_t lda, size_t ldb, size_t ldc, const size_t a_batch_strides[2],
+                    const size_t b_batch_strides[2], const size_t c_batch_strides[2], size_t c0_row_stride, size_t c0_col_stride, float alpha,
+                    float beta, const GemmPost *post = nullptr);
+double gemm_f32_us(const DeviceCtx &ctx, size_t batch, size_t m, size_t n, size_t k, bool k_rows, bool vec);
+
 // Many small products at once (matmul_small.hip): one block per matrix.  C = A B, A with unit stride along k.
 bool gemm_small_batched_fits(size_t batch, size_t m, size_t n, size_t k);
 int launch_gemm_small_batched(DeviceCtx &ctx, float *c, const float *a, const float *b, size_t batch_outer, size_t batch_inner, size_t m, size_t n,
@@ -236,7 +244,7 @@ void gemm_release_all(DeviceCtx &ctx);
 // Max pooling over [planes, ih, iw] (movement.hip).
 int launch_maxpool(DeviceCtx &ctx, float *out, const float *x, size_t planes, size_t ih, size_t iw, size_t oh, size_t ow,
                    size_t kh, size_t kw, size_t sh, size_t sw, size_t pad_t, size_t pad_l);
-// Conv2d on NCHW (conv.hip); bias may be null.
+// Conv2d on NCHW (conv.hip); bias may be null.  Uses the GEMM workspace, up to 1 GiB of it.
 int launch_conv2d(DeviceCtx &ctx, float *out, const float *x, const float *w, const float *bias, size_t batch, size_t c, size_t ih, size_t iw,
                   size_t oc, size_t oh, size_t ow, size_t kh, size_t kw, size_t sh, size_t sw, size_t dh, size_t dw, size_t pad_t, size_t pad_l,
                   size_t group);

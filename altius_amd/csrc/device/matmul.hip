@@ -492,16 +492,16 @@ static int launch_gemm_far_rows(DeviceCtx &ctx, int axis, size_t part, float *c,
         int rc;
         if (axis == 2) {
             const bool last = i + w == extent;
-            rc = launch_gemm_batch2(ctx, c, a + (trans_a ? i * lda : i), b + (trans_b ? i : i * ldb), i ? c : c0, 1, 1, m, n, w, trans_a, trans_b, lda, ldb,
-                                    ldc, none, none, none, i ? ldc : c0_rs, i ? 1 : c0_cs, alpha, i ? 1.0f : beta, last ? post : nullptr);
+            rc = launch_gemm_f32(ctx, c, a + (trans_a ? i * lda : i), b + (trans_b ? i : i * ldb), i ? c : c0, 1, 1, m, n, w, trans_a, trans_b, lda, ldb,
+                                 ldc, none, none, none, i ? ldc : c0_rs, i ? 1 : c0_cs, alpha, i ? 1.0f : beta, last ? post : nullptr);
         } else {
             const size_t r = axis == 0 ? i : 0, q = axis == 1 ? i : 0;
             GemmPost p;
             if (post) p = *post;
             if (p.residual) p.residual += r * ldc + q;
-            rc = launch_gemm_batch2(ctx, c + r * ldc + q, a + (trans_a ? r : r * lda), b + (trans_b ? q * ldb : q), c0 ? c0 + r * c0_rs + q * c0_cs : nullptr,
-                                    batch_outer, batch_inner, axis == 0 ? w : m, axis == 1 ? w : n, k, trans_a, trans_b, lda, ldb, ldc, a_bs, b_bs, c_bs,
-                                    c0_rs, c0_cs, alpha, beta, post ? &p : nullptr);
+            rc = launch_gemm_f32(ctx, c + r * ldc + q, a + (trans_a ? r : r * lda), b + (trans_b ? q * ldb : q), c0 ? c0 + r * c0_rs + q * c0_cs : nullptr,
+                                 batch_outer, batch_inner, axis == 0 ? w : m, axis == 1 ? w : n, k, trans_a, trans_b, lda, ldb, ldc, a_bs, b_bs, c_bs,
+                                 c0_rs, c0_cs, alpha, beta, post ? &p : nullptr);
         }
         if (rc) return rc;
     }
@@ -512,6 +512,22 @@ int launch_gemm_batch2(DeviceCtx &ctx, float *c, const float *a, const float *b,
                        size_t batch_inner, size_t m, size_t n, size_t k, int trans_a, int trans_b, size_t lda, size_t ldb, size_t ldc,
                        const size_t a_batch_strides[2], const size_t b_batch_strides[2], const size_t c_batch_strides[2],
                        size_t c0_row_stride, size_t c0_col_stride, float alpha, float beta, const GemmPost *post) {
+    const bool has_post = post && (post->act != 0 || post->residual);
+    if (!has_post && batch_outer * batch_inner == 1 && m && n && c && a && b && gemm_takes_split(ctx, m, n, k))
+        return launch_gemm_split(ctx, c, a, b, c0, m, n, k, trans_a, trans_b, lda, ldb, ldc, c0_row_stride, c0_col_stride, alpha, beta);
+    return launch_gemm_f32(ctx, c, a, b, c0, batch_outer, batch_inner, m, n, k, trans_a, trans_b, lda, ldb, ldc, a_batch_strides, b_batch_strides,
+                           c_batch_strides, c0_row_stride, c0_col_stride, alpha, beta, post);
+}
+
+double gemm_f32_us(const DeviceCtx &ctx, size_t batch, size_t m, size_t n, size_t k, bool k_rows, bool vec) {
+    const size_t cus = ctx.cus_per_xcd ? (size_t)ctx.cus_per_xcd : 32;
+    return choose(batch, m, n, k, cus, ctx.gemm_split_k, vec && !k_rows).us * (vec ? 1.0 : 1.2);
+}
+
+int launch_gemm_f32(DeviceCtx &ctx, float *c, const float *a, const float *b, const float *c0, size_t batch_outer, size_t batch_inner, size_t m,
+                    size_t n, size_t k, int trans_a, int trans_b, size_t lda, size_t ldb, size_t ldc, const size_t a_batch_strides[2],
+                    const size_t b_batch_strides[2], const size_t c_batch_strides[2], size_t c0_row_stride, size_t c0_col_stride, float alpha,
+                    float beta, const GemmPost *post) {
     const size_t batch = batch_outer * batch_inner;
     if (batch == 0 || m == 0 || n == 0) return AHIP_OK;
     if (!c || (k && (!a || !b))) return ctx.fail(AHIP_ERR_ARG, "gemm: null pointer");
@@ -519,8 +535,6 @@ int launch_gemm_batch2(DeviceCtx &ctx, float *c, const float *a, const float *b,
     if (has_post && batch != 1) return ctx.fail(AHIP_ERR_UNSUPPORTED, "gemm: an activation or a residual needs a single batch");
     if (has_post && post->act != 0 && post->act != AHIP_GELU && post->act != AHIP_RELU)
         return ctx.fail(AHIP_ERR_UNSUPPORTED, "gemm: only Gelu and Relu can follow the product in its kernel");
-    if (!has_post && batch == 1 && gemm_takes_split(ctx, m, n, k))
-        return launch_gemm_split(ctx, c, a, b, c0, m, n, k, trans_a, trans_b, lda, ldb, ldc, c0_row_stride, c0_col_stride, alpha, beta);
     const size_t lim = (size_t)1 << 31;
     if (m >= lim || n >= lim || k >= lim || lda >= lim || ldb >= lim || ldc >= lim || m * ldc >= ((size_t)1 << 40))
         return ctx.fail(AHIP_ERR_UNSUPPORTED, "gemm: extent above 2^31");

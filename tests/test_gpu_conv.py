@@ -70,6 +70,70 @@ def test_conv2d_kernel_edges(ctx, case, x, w, args):
 
 
 @pytest.mark.parametrize("x, w, args", [
+    # many channels and values of k: products of the input as it lies (1 x 1) or of an unfolded copy
+    ((1, 700, 12, 12), (128, 700, 3, 3), dict(pads=(1, 1, 1, 1))),                              # k in slices
+    ((3, 257, 19, 23), (301, 257, 3, 3), dict(pads=(1, 0, 1, 2))),
+    ((2, 40, 40, 40), (300, 40, 3, 3), dict(pads=(1, 1, 1, 1), dilations=(2, 2))),
+    ((2, 129, 30, 31), (260, 129, 5, 3), dict(pads=(2, 1, 2, 1), strides=(1, 2))),
+    ((1, 3, 224, 224), (768, 3, 16, 16), dict(strides=(16, 16))),
+    ((3, 250, 33, 31), (270, 125, 3, 3), dict(pads=(1, 1, 1, 1), group=2)),
+    ((8, 256, 28, 28), (130, 256, 1, 1), dict()),
+    ((4, 601, 16, 16), (515, 601, 1, 1), dict()),
+])
+def test_conv2d_unfolded(ctx, case, x, w, args):
+    case(f"conv2d unfolded {x} {w} {args}")
+    args = {**dict(strides=(1, 1), pads=(0, 0, 0, 0), dilations=(1, 1), group=1), **args}
+    xi, wi = RNG.integers(-3, 4, size=x).astype(np.float32), RNG.integers(-3, 4, size=w).astype(np.float32)
+    bias = RNG.integers(-3, 4, size=w[0]).astype(np.float32)
+    for b in (bias, None):
+        assert_bits_equal(ctx.conv2d(xi, wi, b, **args), O.conv2d(xi, wi, b, **args), "vs oracle")
+
+
+@pytest.mark.parametrize("x", [(1, 512, 243, 244), (3, 256, 208, 209)])
+def test_conv2d_unfolded_in_passes(ctx, case, x):
+    """An image whose unfolded copy is more than the workspace's 1 GiB is taken in bands of rows, a batch in groups of images; the
+    last one of either is smaller.  Whole numbers, at the corners of every image, around the bands' seam and at random places."""
+    b, c, h, wd = x
+    oc = 256
+    case(f"conv2d in passes {x}")
+    xi = RNG.integers(-3, 4, size=x).astype(np.float32)
+    wi = RNG.integers(-3, 4, size=(oc, c, 3, 3)).astype(np.float32)
+    bias = RNG.integers(-3, 4, size=oc).astype(np.float32)
+    got = ctx.conv2d(xi, wi, bias, pads=(1, 1, 1, 1))
+    assert got.shape == (b, oc, h, wd)
+    padded = np.pad(xi, ((0, 0), (0, 0), (1, 1), (1, 1)))
+    rows, cols = [0, h // 2 - 1, h // 2, h // 2 + 1, h - 1], [0, 1, wd - 1]
+    at = [(i, y, z) for i in range(b) for y in rows for z in cols]
+    at += list(zip(RNG.integers(0, b, 200), RNG.integers(0, h, 200), RNG.integers(0, wd, 200)))
+    patches = np.stack([padded[i, :, y:y + 3, z:z + 3].reshape(-1) for i, y, z in at]).astype(np.float64)
+    want = patches @ wi.reshape(oc, -1).T.astype(np.float64) + bias
+    assert np.array_equal(np.stack([got[i, :, y, z] for i, y, z in at]), want)
+
+
+def test_unfolded_convolutions_of_a_session_replayed(case):
+    """Two of them share the workspace; the recorded run gives the eager run's bits."""
+    case("session conv2d unfolded, recorded")
+    m = Model(opset_version=13)
+    v = m.new_val_named_and_shaped("x", [2, 96, 20, 22])
+    m.add_input(v)
+    w = [RNG.integers(-2, 3, size=s).astype(np.float32) for s in ((256, 96, 3, 3), (300, 256, 3, 3))]
+    y = v
+    for a in w:
+        out = m.new_val()
+        m.add_node(Op.Conv2d, [y, m.new_initializer(a)], [out], kernel_shape=[3, 3], strides=[1, 1], pads=[1, 1, 1, 1])
+        y = out
+    m.add_output(y)
+    session = HipSessionBuilder(m).with_graph_replay().build()
+    for _ in range(4):
+        x = RNG.integers(-2, 3, size=(2, 96, 20, 22)).astype(np.float32)
+        want = x
+        for a in w:
+            want = O.conv2d(want, a, None, pads=(1, 1, 1, 1))
+        assert_bits_equal(session.run([x])[0], want, "vs oracle")
+    assert session.graph_replays() > 0
+
+
+@pytest.mark.parametrize("x, w, args", [
     ((1, 1, 520, 7), (1, 1, 2, 1), dict(dilations=(500, 1))),                       # few outputs to a tile of 8192 values
     ((2, 3, 33, 33), (3, 1, 3, 3), dict(dilations=(36, 36), pads=(36,) * 4, group=3)),
     ((2, 3, 40, 41), (3, 1, 3, 3), dict(dilations=(24, 24), pads=(24,) * 4, group=3)),
