@@ -585,13 +585,12 @@ int ahip_gemm_unregister_constant(ahip_ctx *ctx, const void *ptr) try {
     return altius::caught_at_boundary("ahip_gemm_unregister_constant");
 }
 
-int ahip_conv2d(ahip_ctx *ctx, float *out, const float *x, const float *w, const float *bias, float *col, size_t batch,
+int ahip_conv2d(ahip_ctx *ctx, float *out, const float *x, const float *w, const float *bias, float * /* col */, size_t batch,
                 size_t c, size_t ih, size_t iw, size_t oc, size_t oh, size_t ow, size_t kh, size_t kw, size_t stride_h,
                 size_t stride_w, size_t dilation_h, size_t dilation_w, size_t pad_top, size_t pad_left, size_t group) try {
     REQUIRE_CTX(ctx, "ahip_conv2d");
     if (!kh || !kw || !stride_h || !stride_w || !dilation_h || !dilation_w)
         return ctx->d.fail(AHIP_ERR_ARG, "ahip_conv2d: kernel, stride and dilation must be positive");
-    if (batch && oc && oh && ow && !col) return ctx->d.fail(AHIP_ERR_ARG, "conv2d: null pointer");
     return altius::launch_conv2d(ctx->d, out, x, w, bias, batch, c, ih, iw, oc, oh, ow, kh, kw, stride_h, stride_w,
                                  dilation_h, dilation_w, pad_top, pad_left, group);
 } catch (...) {

@@ -532,14 +532,13 @@ class Context:
         ow = (iw + pads[1] + pads[3] - dilations[1] * (kw - 1) - 1) // strides[1] + 1
         dx, dw = self.upload(x), self.upload(w)
         db = self.upload(np.asarray(bias, dtype=np.float32)) if bias is not None else None
-        dcol = self.alloc(max(b * c * kh * kw * oh * ow * 4, 4))
         do = self.alloc(max(b * oc * oh * ow * 4, 4))
         try:
-            check(self.L.ahip_conv2d(self.handle, do.ptr, dx.ptr, dw.ptr, db.ptr if db else None, dcol.ptr, b, c, ih, iw, oc, oh, ow,
+            check(self.L.ahip_conv2d(self.handle, do.ptr, dx.ptr, dw.ptr, db.ptr if db else None, None, b, c, ih, iw, oc, oh, ow,
                                      kh, kw, strides[0], strides[1], dilations[0], dilations[1], pads[0], pads[1], group), self.handle)
             return self.download(do, (b, oc, oh, ow))
         finally:
-            for t in (dx, dw, dcol, do) + ((db,) if db else ()):
+            for t in (dx, dw, do) + ((db,) if db else ()):
                 self.free(t)
 
     def max_pool(self, x, kernel, strides, pads=(0, 0, 0, 0)):

@@ -376,9 +376,10 @@ int ahip_xcd_round_robin_holds(int cu_count, const uint32_t *xcc_of_block, size_
 int ahip_gemm_register_constant(ahip_ctx *ctx, const void *ptr, size_t bytes);
 int ahip_gemm_unregister_constant(ahip_ctx *ctx, const void *ptr);
 
-/* Conv2d on NCHW (crates/session_interpreter/src/conv2d.rs:26-211), which unfolds the input into `col`;
- * the kernels here read x in place: `col` must not be NULL, and is neither read nor written.  w is [oc, c/group, kh, kw]; bias ([oc]) may be NULL.  oh / ow are the
- * output extents the caller inferred (shape.rs:38-88).
+/* Conv2d on NCHW (crates/session_interpreter/src/conv2d.rs:26-211), which unfolds the input into `col`:
+ * here the context has room of its own where that is worth while, and `col` is neither read nor written and
+ * may be NULL.  w is [oc, c/group, kh, kw]; bias ([oc]) may be NULL.  oh / ow are the output extents the
+ * caller inferred (shape.rs:38-88).
  * MaxPool (compute_max_pool, session.rs:324-382) over [planes, ih, iw] -> [planes, oh, ow]. */
 int ahip_conv2d(ahip_ctx *ctx, float *out, const float *x, const float *w, const float *bias, float *col, size_t batch,
                 size_t c, size_t ih, size_t iw, size_t oc, size_t oh, size_t ow, size_t kh, size_t kw, size_t stride_h,
