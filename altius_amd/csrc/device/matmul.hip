@@ -587,7 +587,8 @@ int launch_gemm_f32(DeviceCtx &ctx, float *c, const float *a, const float *b, co
     const Choice ch = choose(batch, m, n, k, cus, ctx.gemm_split_k, both && !(a_kc && b_kc));
     const Shape &sh = SHAPES[ch.shape];
     const size_t gy = (m + sh.bm - 1) / sh.bm, gx = (n + sh.bn - 1) / sh.bn, tiles = gx * gy * batch;
-    if (gx * gy >= lim || batch >= lim || tiles >= lim / 16) return ctx.fail(AHIP_ERR_UNSUPPORTED, "gemm: too many tiles");
+    if (gx * gy >= lim || batch >= lim || (tiles + 7) / 8 * 8 * ch.slices * 256 > 0xffffffffu)
+        return ctx.fail(AHIP_ERR_UNSUPPORTED, "gemm: more tiles than a grid holds");
     g.tiles_n = (uint32_t)gx;
     g.tiles_m = (uint32_t)gy;
     g.tiles = (uint32_t)tiles;

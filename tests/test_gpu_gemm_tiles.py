@@ -6,6 +6,7 @@ import ctypes
 import numpy as np
 import pytest
 
+from altius_amd._lib import AltiusHipError
 from conftest import assert_bits_equal
 
 pytestmark = pytest.mark.gpu
@@ -100,6 +101,23 @@ def test_rows_too_far_apart_for_32_bit_offsets(ctx, case, axis):
     finally:
         for d in (da, db, dc0, dc):
             ctx.free(d)
+
+
+def test_more_products_than_a_grid_holds_are_refused(ctx, case):
+    """A block of 256 threads at least for each: 2^24 of them are 2^32 threads, one more than a grid holds.  Eight fewer (one for each XCD) run."""
+    batch = 1 << 24
+    case(f"gemm batch of {batch} [1,1] x [1,1]")
+    x = np.arange(batch, dtype=np.float32)
+    da, dc = ctx.upload(x), ctx.upload(np.zeros(batch, np.float32))
+    try:
+        with pytest.raises(AltiusHipError, match="more tiles than a grid holds"):
+            ctx.gemm_raw(dc.ptr, da.ptr, da.ptr, None, batch, 1, 1, 1, True, False, a_bs=1, b_bs=0, c_bs=1, alpha=2.0)
+        ctx.gemm_raw(dc.ptr, da.ptr, da.ptr + 4, None, batch - 8, 1, 1, 1, True, False, a_bs=1, b_bs=0, c_bs=1, alpha=2.0)
+        got = ctx.download(dc, (batch,))
+        assert np.array_equal(got[:-8], 2.0 * x[:-8]) and not got[-8:].any()
+    finally:
+        ctx.free(da)
+        ctx.free(dc)
 
 
 def test_more_columns_than_a_grid_of_small_tiles_holds(ctx, case):
