@@ -228,8 +228,13 @@ int gemm_workspace(DeviceCtx &ctx, size_t bytes, void **p);
 // counters of such tiles (ctx.gemm_counters, GEMM_COUNTERS of them, zero between launches).
 constexpr size_t GEMM_COUNTERS = 2048;
 int gemm_partials(DeviceCtx &ctx, size_t bytes);
+// How launch_reduce goes about whole rows (reduce.hip), and with it the order in which a row's values are added: a few lanes per
+// row, groups of rows through LDS, a wavefront per row, or blocks.
+enum class RowsBy { Lanes, LdsGroups, Wavefront, Blocks };
+RowsBy reduce_rows_by(const float *in, size_t rows, size_t len);
 // Row sums (optionally times `scale`) or maxima of a [rows, len] matrix through LDS-staged groups of rows (rows.hip): for
-// rows that are short or not whole float4s.  Returns -1 without launching when the shape is not one it is meant for.
+// rows that are short or not whole float4s.  Only for shapes reduce_rows_lds_fits accepts.
+bool reduce_rows_lds_fits(const float *in, size_t rows, size_t len);
 int launch_reduce_rows_lds(DeviceCtx &ctx, bool is_max, float *out, const float *in, size_t rows, size_t len, float scale, bool scaled);
 // Whether launch_gemm would send this single-batch product through launch_gemm_split.
 bool gemm_takes_split(const DeviceCtx &ctx, size_t m, size_t n, size_t k);

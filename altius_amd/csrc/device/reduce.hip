@@ -654,46 +654,45 @@ int claim_partials(DeviceCtx &ctx, const Partials &pt) {
     return AHIP_OK;
 }
 
+constexpr int SUB4_UNROLL = 4;
+// Lanes that reduce_rows_sub4 gives a row of whole float4s.
+int sub4_lanes(size_t red) {
+    const size_t v4 = red / 4;
+    return v4 <= 4 ? 4 : v4 <= 8 ? 8 : v4 <= 16 ? 16 : v4 <= 32 ? 32 : 64;
+}
+size_t sub4_blocks(size_t outer, size_t red) {
+    const size_t per_block = (size_t)(WAVE / sub4_lanes(red)) * SUB4_UNROLL * ROW_WAVES;
+    return (outer + per_block - 1) / per_block;
+}
+
 template <class OP, bool SCALE>
 int reduce_impl(DeviceCtx &ctx, const Partials &pt, float *out, const float *in, size_t outer, size_t red, size_t inner,
                 float scale) {
     hipStream_t s = ctx.stream;
     if (inner == 1) {
-        // Rows of up to 256 elements that are whole float4s: a few lanes per row, straight from memory.
-        if (red % 4 == 0 && red >= 16 && red <= 256 && aligned16(in)) {
-            constexpr int U = 4;
-            const size_t v4 = red / 4;
-            const int sub = v4 <= 4 ? 4 : v4 <= 8 ? 8 : v4 <= 16 ? 16 : v4 <= 32 ? 32 : 64;
-            const size_t rows_per_wave = (size_t)(WAVE / sub) * U;
-            const size_t blocks = (outer + rows_per_wave * ROW_WAVES - 1) / (rows_per_wave * ROW_WAVES);
-            if (blocks <= MAX_GRID_X) {
-                const bool nt = ctx.streaming(outer * red * sizeof(float));
-                const dim3 grid((unsigned)blocks), block(ROW_BLOCK);
+        const RowsBy by = reduce_rows_by(in, outer, red);
+        if (by == RowsBy::Lanes) {
+            constexpr int U = SUB4_UNROLL;
+            const int sub = sub4_lanes(red);
+            const bool nt = ctx.streaming(outer * red * sizeof(float));
+            const dim3 grid((unsigned)sub4_blocks(outer, red)), block(ROW_BLOCK);
 #define ALTIUS_SUB4(SUBV)                                                                                                          \
     do {                                                                                                                           \
         if (nt) hipLaunchKernelGGL((reduce_rows_sub4<OP, SUBV, U, SCALE, true>), grid, block, 0, s, out, in, outer, (uint32_t)red, scale);  \
         else hipLaunchKernelGGL((reduce_rows_sub4<OP, SUBV, U, SCALE, false>), grid, block, 0, s, out, in, outer, (uint32_t)red, scale);    \
     } while (0)
-                switch (sub) {
-                case 4: ALTIUS_SUB4(4); break;
-                case 8: ALTIUS_SUB4(8); break;
-                case 16: ALTIUS_SUB4(16); break;
-                case 32: ALTIUS_SUB4(32); break;
-                default: ALTIUS_SUB4(64); break;
-                }
-#undef ALTIUS_SUB4
-                return ctx.check(hipGetLastError(), "reduce rows (lane groups) launch");
+            switch (sub) {
+            case 4: ALTIUS_SUB4(4); break;
+            case 8: ALTIUS_SUB4(8); break;
+            case 16: ALTIUS_SUB4(16); break;
+            case 32: ALTIUS_SUB4(32); break;
+            default: ALTIUS_SUB4(64); break;
             }
+#undef ALTIUS_SUB4
+            return ctx.check(hipGetLastError(), "reduce rows (lane groups) launch");
         }
-        // Short rows and rows that are not whole 128-byte lines (a wavefront per row would fetch the lines two rows
-        // share twice: 10 % more traffic on rows of 1000): groups of rows staged through LDS, a few lanes per row.
-        if (red <= 1024 && (red % 32 != 0 || red < 256)) {
-            const int rc = launch_reduce_rows_lds(ctx, std::is_same<OP, MaxOp>::value, out, in, outer, red, scale, SCALE);
-            if (rc >= 0) return rc;
-        }
-        // A wavefront per row below 4096 elements, a block of four above (measured over 96 M elements, non-temporal loads
-        // in both: 4096: 84 against 88 % of the HBM peak, 8192: 82 / 88, 16384: 77 / 87; 3072: 86.5 / 85.5).
-        if (red < 4096 || outer >= 65536) {
+        if (by == RowsBy::LdsGroups) return launch_reduce_rows_lds(ctx, std::is_same<OP, MaxOp>::value, out, in, outer, red, scale, SCALE);
+        if (by == RowsBy::Wavefront) {
             if ((outer + ROW_WAVES - 1) / ROW_WAVES > MAX_GRID_X)
                 return ctx.fail(AHIP_ERR_UNSUPPORTED, "reduce: too many rows for one launch");
             rows_wave_launch<OP, SCALE>(s, out, in, outer, red, scale, ctx.streaming(outer * red * sizeof(float)));
@@ -843,6 +842,17 @@ int reduce_with(DeviceCtx &ctx, const Partials &pt, int kind, float *out, const 
 }
 
 }  // namespace
+
+RowsBy reduce_rows_by(const float *in, size_t rows, size_t len) {
+    // Rows of up to 256 elements that are whole float4s: a few lanes per row, straight from memory.
+    if (len % 4 == 0 && len >= 16 && len <= 256 && aligned16(in) && sub4_blocks(rows, len) <= MAX_GRID_X) return RowsBy::Lanes;
+    // Short rows and rows that are not whole 128-byte lines (a wavefront per row would fetch the lines two rows
+    // share twice: 10 % more traffic on rows of 1000): groups of rows staged through LDS, a few lanes per row.
+    if (len <= 1024 && (len % 32 != 0 || len < 256) && reduce_rows_lds_fits(in, rows, len)) return RowsBy::LdsGroups;
+    // A wavefront per row below 4096 elements, a block of four above (measured over 96 M elements, non-temporal loads
+    // in both: 4096: 84 against 88 % of the HBM peak, 8192: 82 / 88, 16384: 77 / 87; 3072: 86.5 / 85.5).
+    return len < 4096 || rows >= 65536 ? RowsBy::Wavefront : RowsBy::Blocks;
+}
 
 int launch_reduce(DeviceCtx &ctx, int kind, float *out, const float *in, size_t outer, size_t red,
                   size_t inner) {

@@ -1500,9 +1500,10 @@ __global__ __launch_bounds__(BLOCK) void norm_chain_rows(float *__restrict__ out
 bool norm_chain_fits(const float *out, const float *in, const float *gamma, const float *beta, size_t rows, size_t len) {
     if (!out || !in || !gamma || !beta || !aligned16(out) || !aligned16(in) || !aligned16(gamma) || !aligned16(beta)) return false;
     // Up to 4096 elements (sixteen float4s per lane: a row still fits the registers), where the reduction takes one of the two kernels
-    // (rows of up to 32 elements and ragged ones of 260 to 1020 are added in orders of their own there).
+    // whose order is followed (the first with rows of up to 32 elements, and groups through LDS, add in orders of their own).
     if (rows == 0 || (rows + WAVES_PER_BLOCK - 1) / WAVES_PER_BLOCK > MAX_GRID || len <= 32 || len >= 4096 || len % 4 != 0) return false;
-    return len <= 256 || len > 1024 || len % 32 == 0 || rows < 64;
+    const RowsBy by = reduce_rows_by(in, rows, len);
+    return by == RowsBy::Lanes || by == RowsBy::Wavefront;
 }
 
 int launch_norm_chain(DeviceCtx &ctx, float *out, const float *in, const float *gamma, const float *beta, size_t rows, size_t len, float eps) {
@@ -1666,16 +1667,23 @@ int launch_layernorm(DeviceCtx &ctx, float *out, const float *in, const float *g
 }
 
 // Row sums / maxima through reduce_rows_lds; -1 (nothing launched) when the shape is not one it is meant for.
+// Read-only: blocks of 512 threads, four to a CU (72-75 % of the HBM peak with 1024 become 83-90 %); two float4 per
+// thread where a line-aligned group of rows fits 16 KiB, four where it takes 32 KiB (197).
+constexpr int REDUCE_LDS_THREADS = LDS_BLOCK / 2;
+inline bool reduce_lds_deep(size_t len) { return lds_block_threads(len) == LDS_BLOCK; }
+inline size_t reduce_lds_group(size_t len) { return softmax_lds_group_rows(len, (size_t)(reduce_lds_deep(len) ? 4 : 2) * REDUCE_LDS_THREADS * 4); }
+
+bool reduce_rows_lds_fits(const float *in, size_t rows, size_t len) {
+    if (len == 0 || len > 1024 || rows < 64 || !aligned16(in)) return false;
+    const size_t g = reduce_lds_group(len);
+    return (g * len) % 4 == 0 && (rows + g - 1) / g <= 0x7FFFFFFFu;  // groups must start 16-byte aligned
+}
+
 int launch_reduce_rows_lds(DeviceCtx &ctx, bool is_max, float *out, const float *in, size_t rows, size_t len, float scale, bool scaled) {
-    if (len == 0 || len > 1024 || rows < 64 || !aligned16(in)) return -1;
-    // Read-only: blocks of 512 threads, four to a CU (72-75 % of the HBM peak with 1024 become 83-90 %); two float4 per
-    // thread where a line-aligned group of rows fits 16 KiB, four where it takes 32 KiB (197).
-    constexpr int RT = LDS_BLOCK / 2;
-    const bool deep = lds_block_threads(len) == LDS_BLOCK;
-    const size_t g = softmax_lds_group_rows(len, (size_t)(deep ? 4 : 2) * RT * 4);
-    if ((g * len) % 4 != 0) return -1;  // groups must start 16-byte aligned
-    const size_t groups = (rows + g - 1) / g;
-    if (groups > 0x7FFFFFFFu) return -1;
+    if (!reduce_rows_lds_fits(in, rows, len)) return ctx.fail(AHIP_ERR_UNSUPPORTED, "reduce: not rows the kernel takes");
+    constexpr int RT = REDUCE_LDS_THREADS;
+    const bool deep = reduce_lds_deep(len);
+    const size_t g = reduce_lds_group(len), groups = (rows + g - 1) / g;
     const bool nt = ctx.streaming(rows * len * sizeof(float));
     const dim3 grid((unsigned)groups);
     const size_t shmem = g * len * sizeof(float);
