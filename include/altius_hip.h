@@ -629,7 +629,8 @@ int ahip_session_builder_with_strided_views(ahip_session_builder *builder, int e
  * product's operand planes (the split of the same values). */
 int ahip_session_builder_with_fused_attention(ahip_session_builder *builder, int enable);
 /* Nodes of the last node-by-node run that were served without their copy (views taken, transposed layouts
- * written in place). */
+ * written in place) or by another node's kernel (what follows a product, the steps of a written-out
+ * LayerNormalization). */
 int ahip_session_copies_avoided(const ahip_session *session, size_t *count);
 /* Lanes the session holds so far (1 until two ahip_session_run calls have overlapped). */
 int ahip_session_lanes(ahip_session *session, size_t *count);

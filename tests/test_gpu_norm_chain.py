@@ -40,8 +40,10 @@ def test_lengths(case, length):
     for rows in (1, 7):
         x = rng.standard_normal((rows, length)).astype(np.float32) * 3 + 1
         g, b = rng.standard_normal(length).astype(np.float32), rng.standard_normal(length).astype(np.float32)
-        (got,) = HipSessionBuilder(chain(x.shape, g, b, 1e-5)).build().run([x])
+        session = HipSessionBuilder(chain(x.shape, g, b, 1e-5)).build()
+        (got,) = session.run([x])
         assert_close(got, nine_steps(x, g, b, 1e-5), what=f"{rows} rows")
+        assert session.copies_avoided() == (8 if length % 4 == 0 and 32 < length < 4096 else 0), "one kernel for the nine steps"
 
 
 @pytest.mark.parametrize("length", [4, 64, 256, 1024, 4096])
@@ -52,8 +54,10 @@ def test_every_rounding_where_the_sums_are_exact(case, length):
     x[..., : length // 2] = 3 - x[..., length // 2:]  # mean 1.5, squares of halves
     x[1, 2] = 2.0                                     # variance 0
     g, b = rng.standard_normal(length).astype(np.float32), rng.standard_normal(length).astype(np.float32)
-    (got,) = HipSessionBuilder(chain(x.shape, g, b, 1e-5)).build().run([x])
+    session = HipSessionBuilder(chain(x.shape, g, b, 1e-5)).build()
+    (got,) = session.run([x])
     assert_bits_equal(got, nine_steps(x, g, b, 1e-5), "result")
+    assert session.copies_avoided() == (8 if 32 < length < 4096 else 0)
 
 
 def test_infinities_and_zero_over_zero(case):
@@ -72,7 +76,9 @@ def test_a_step_that_is_seen_keeps_the_operators(case, see):
     x = rng.integers(0, 4, size=(5, 256)).astype(np.float32)
     g, b = rng.standard_normal(256).astype(np.float32), rng.standard_normal(256).astype(np.float32)
     plain = HipSessionBuilder(chain(x.shape, g, b, 1e-5)).build().run([x])[0]
-    got, step = HipSessionBuilder(chain(x.shape, g, b, 1e-5, see)).build().run([x])
+    session = HipSessionBuilder(chain(x.shape, g, b, 1e-5, see)).build()
+    got, step = session.run([x])
+    assert session.copies_avoided() == 0
     assert_close(got, plain, what="result")
     assert step.size in (5, 5 * 256)
 
@@ -97,7 +103,9 @@ def test_scale_that_the_caller_may_replace_and_other_forms(case):
         var = op(Op.ReduceMean, [op(Op.Pow, [d, const(exponent)])], axes=[axis], keep_dims=True)
         s = op(Op.Sqrt, [op(Op.Add, [const([10.0]), var])])
         m.add_output(op(Op.Add, [const(b), op(Op.Mul, [const(g), op(Op.Div, [d, s])])]))
-        (got,) = HipSessionBuilder(m).build().run([x])
+        session = HipSessionBuilder(m).build()
+        (got,) = session.run([x])
+        assert session.copies_avoided() == 0  # rows of 8 are too short, and the others are no such chain
         y = x.astype(np.float64)
         y = y - y.mean(axis, keepdims=True)
         want = y / np.sqrt((y ** exponent).mean(axis, keepdims=True) + 10.0) * g + b
@@ -111,6 +119,8 @@ def test_bits_of_the_operators_run_one_by_one(case, shape):
     rng = np.random.default_rng(sum(shape))
     x = (rng.standard_normal(shape) * 2 - 1).astype(np.float32)
     g, b = rng.standard_normal(shape[-1]).astype(np.float32), rng.standard_normal(shape[-1]).astype(np.float32)
-    (one,) = HipSessionBuilder(chain(shape, g, b, 1e-5)).build().run([x])
-    (nine,) = HipSessionBuilder(chain(shape, g, b, 1e-5)).with_profiling_enabled(True).build().run([x])
-    assert_bits_equal(one, nine, "one kernel against nine")
+    together, apart = HipSessionBuilder(chain(shape, g, b, 1e-5)).build(), HipSessionBuilder(chain(shape, g, b, 1e-5)).with_profiling_enabled(True).build()
+    assert_bits_equal(together.run([x])[0], apart.run([x])[0], "one kernel against nine")
+    rows, length = int(np.prod(shape[:-1])), shape[-1]
+    grouped = rows >= 64 and 256 < length <= 1024 and length % 32 != 0  # rows that the reduction adds up through LDS
+    assert together.copies_avoided() == (8 if length > 32 and not grouped else 0) and apart.copies_avoided() == 0
