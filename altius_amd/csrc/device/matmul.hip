@@ -387,7 +387,9 @@ double cost_us(const Shape &sh, size_t rounds, size_t k) {
 
 // Three 128 x 128 blocks fit a CU.  Those that run together end together where k is cut, or where an operand of 16-byte loads has its
 // rows along m or n, and the blocks left over then fill the slots of few CUs: a fourth or fifth round takes as long as three more, a
-// seventh as two (4096^3: 1440 us for four rounds, 128 x 64 tiles 1070; with both operands' k contiguous 1025 and 1045).
+// seventh as two (4096^3: 1440 us for four rounds, 128 x 64 tiles 1070; with both operands' k contiguous 1025 and 1045).  An
+// activation behind the product spreads the ends of short blocks: five rounds of up to 1024 values of k stay five then
+// ([6304,768] x [768,3072] with Gelu 265 us, 128 x 64 tiles 271; four rounds, 4096^3: 1480 and 1080).
 size_t tail_rounds(size_t rounds) { return rounds == 4 || rounds == 5 ? 6 : rounds == 7 ? 8 : rounds; }
 
 struct Choice {
@@ -398,8 +400,8 @@ struct Choice {
 
 // What a product adds up in which order is decided by the sizes alone, so that a product and the same product with an operand stored
 // the other way round add up alike (the last two tiles do, as long as k is whole).
-// cut: k may be cut into slices.  tail: an operand of 16-byte loads has its rows along m or n.
-Choice choose(size_t batch, size_t m, size_t n, size_t k, size_t cus_per_xcd, bool cut, bool tail) {
+// cut: k may be cut into slices.  tail: an operand of 16-byte loads has its rows along m or n.  act: an activation follows.
+Choice choose(size_t batch, size_t m, size_t n, size_t k, size_t cus_per_xcd, bool cut, bool tail, bool act) {
     Choice best;
     double best_us = 0.0;
     auto chunk_of = [&](const Shape &sh) { return (((m + sh.bm - 1) / sh.bm) * ((n + sh.bn - 1) / sh.bn) * batch + 7) / 8; };
@@ -425,9 +427,9 @@ Choice choose(size_t batch, size_t m, size_t n, size_t k, size_t cus_per_xcd, bo
     }
     if (best.shape == N_SHAPES - 1 && best.slices == 1 && tail) {
         const Shape &large = SHAPES[N_SHAPES - 1], &half = SHAPES[N_SHAPES - 2];
-        const size_t blocks = chunk_of(half);
+        const size_t blocks = chunk_of(half), rounds = rounds_of(chunk_of(large));
         const double half_us = cost_us(half, rounds_of(blocks), k);
-        best_us = cost_us(large, tail_rounds(rounds_of(chunk_of(large))), k);
+        best_us = cost_us(large, act && rounds == 5 && k <= 1024 ? rounds : tail_rounds(rounds), k);
         if (blocks * 8 * 256 <= 0xffffffffu && half_us < best_us) {
             best_us = half_us;
             best.shape = N_SHAPES - 2;
@@ -521,7 +523,7 @@ int launch_gemm_batch2(DeviceCtx &ctx, float *c, const float *a, const float *b,
 
 double gemm_f32_us(const DeviceCtx &ctx, size_t batch, size_t m, size_t n, size_t k, bool k_rows, bool vec) {
     const size_t cus = ctx.cus_per_xcd ? (size_t)ctx.cus_per_xcd : 32;
-    return choose(batch, m, n, k, cus, ctx.gemm_split_k, vec && !k_rows).us * (vec ? 1.0 : 1.2);
+    return choose(batch, m, n, k, cus, ctx.gemm_split_k, vec && !k_rows, false).us * (vec ? 1.0 : 1.2);
 }
 
 int launch_gemm_f32(DeviceCtx &ctx, float *c, const float *a, const float *b, const float *c0, size_t batch_outer, size_t batch_inner, size_t m,
@@ -584,7 +586,7 @@ int launch_gemm_f32(DeviceCtx &ctx, float *c, const float *a, const float *b, co
         return aligned16(p) && contiguous % 4 == 0 && ld % 4 == 0 && bs[0] % 4 == 0 && bs[1] % 4 == 0;
     };
     const bool both = vec(a, a_kc ? k : m, lda, a_batch_strides) && vec(b, b_kc ? k : n, ldb, b_batch_strides);
-    const Choice ch = choose(batch, m, n, k, cus, ctx.gemm_split_k, both && !(a_kc && b_kc));
+    const Choice ch = choose(batch, m, n, k, cus, ctx.gemm_split_k, both && !(a_kc && b_kc), g.act != 0);
     const Shape &sh = SHAPES[ch.shape];
     const size_t gy = (m + sh.bm - 1) / sh.bm, gx = (n + sh.bn - 1) / sh.bn, tiles = gx * gy * batch;
     if (gx * gy >= lim || batch >= lim || (tiles + 7) / 8 * 8 * ch.slices * 256 > 0xffffffffu)

@@ -68,9 +68,10 @@ def test_behind_a_gemm(case, after, reshape, form):
 
 
 @pytest.mark.parametrize("after", [Op.Add, Op.Gelu])
-@pytest.mark.parametrize("t,k,n", [(551, 1481, 2305), (1411, 6162, 2516)])  # slices of 64 x 64 and of 128 x 128 blocks, ragged
-def test_behind_a_gemm_cut_along_k(case, after, t, k, n):
-    case(f"gemm {t, k, n} in slices, {after}")
+# slices of 64 x 64 and of 128 x 128 blocks, ragged; 128 x 128 blocks behind which an activation follows, 128 x 64 where none does
+@pytest.mark.parametrize("t,k,n", [(551, 1481, 2305), (1411, 6162, 2516), (4301, 100, 4304)])
+def test_behind_a_gemm_of_other_tiles(case, after, t, k, n):
+    case(f"gemm {t, k, n}, {after}")
     m = graph(1, t, k, n, after, False, "first", 0)
     rng = np.random.default_rng(13)
     x, r = (rng.standard_normal(d).astype(np.float32) for d in ((t, k), (t, n)))
