@@ -316,8 +316,7 @@ __global__ __launch_bounds__(512) void conv_gemm_small(ConvGemmArgs g) {
 }
 
 // 64 x 128 tile per block of four wavefronts (32 x 64 each), k in steps of 16 through two LDS buffers; the loads of step
-// t + 1 are in flight during the products of step t.  From two blocks per CU on: [72,16] x [16, 32 * 3136] takes 15 us here.
-// w lies in LDS as [row][k] (pitch 20: the 16-byte reads of 16 rows
+// t + 1 are in flight during the products of step t.  [72,16] x [16, 32 * 3136] takes 15 us here.  w lies in LDS as [row][k] (pitch 20: the 16-byte reads of 16 rows
 // meet all 64 banks), x as [k][column] (pitch 132: the four k of a step are 16 banks apart).
 constexpr int TM = 64, TN = 128, TK = 16, WP = TK + 4, XP = TN + 4;
 
@@ -443,7 +442,7 @@ enum Route { SMALL_16, SMALL_32, TILED, UNFOLDED };
 // alone + alone_chunk * chunks where that is one.  The unfolded route takes its own kernel and one product per group.  Fitted to 336
 // geometries (1 x 1 to 16 x 16 taps, 3 to 2048 channels, images of 7 x 7 to 224 x 224, batches of 1 to 64, up to 32 groups), every
 // route timed on each: within 9 % (rms) of the unfolded one, 9 to 15 % of the tiled and 16 to 24 % of the small ones, and the route
-// chosen is 1.3 % behind the best one on average.  (Before, tiles from 512 of them on and no unfolded route: 19 %;
+// chosen is 1.5 % behind the best one on average.  (Before, tiles from 512 of them on and no unfolded route: 19 %;
 // [32,1024,14,14] -> 2048, 1 x 1 with stride 2: 260 us, 95 unfolded; [4,320,64,64] -> 320, 3 x 3: 555 and 322.)
 struct SmallCost { double base, chain, chunk, tile; };
 struct TiledCost { double base, tile, chunk, alone, alone_chunk; };

@@ -570,9 +570,11 @@ int gemm_workspace(DeviceCtx &ctx, size_t bytes, void **p) {
 }
 
 bool gemm_split_worthwhile(size_t m, size_t n, size_t k) {
-    // Large products whose C fills most of its 256 x 256 tiles.  Products with few rows (one image through a
-    // transformer layer: [197, 768] x [768, 2304]) are faster on the fp32 kernel with k cut into batches: its
-    // tiles are smaller and nothing has to be split into planes first (30 against 49 us for that shape).
+    // Large products whose C fills most of its 256 x 256 tiles.  Products with few rows are faster on the fp32 kernel: its tiles are
+    // smaller and nothing has to be split into planes first (us, fp32 and here, constant B): [197,768] x [768,2304] 13 and 47,
+    // [788,768] x [768,3072] 44 and 54, [3152,768] x [768,2304] 103 and 86, [6304,768] x [768,2304] 192 and 114.  The line was drawn
+    // with an fp32 kernel that took 67 us for [1024,768] x [768,3072]; that one now takes 45 (54 here), and up to about 2000 rows
+    // fp32 is level or ahead.
     if (m < 1024 || n < 256 || k < 128) return false;
     const double useful = (double)m * (double)n / ((double)round_up(m, TM) * (double)round_up(n, TN));
     return useful >= 0.8 && (double)m * (double)n * (double)k >= 2147483648.0;

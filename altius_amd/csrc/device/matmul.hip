@@ -16,12 +16,17 @@
 // a half takes k = 8 i + 4 half + 0 .. 3 in turn, the same for both layouts, so that a product does not depend on them.
 //
 // Measured against 128 x 128 and 128 x 64 tiles staged through registers, cut along k into batches whose sums a second kernel
-// added, with activations and residuals in a pass of their own (us, whole layers' products in sessions):
+// added, with activations and residuals in a pass of their own (us, whole layers' products in sessions but for the last four):
 //   [197,768] x [768,768 / 2304 / 3072]: 17 -> 10, 23 -> 14, 29 -> 20 (latency: 168 to 672 tiles of 32 x 32)
 //   [1024,768] x [768,768]: 27 -> 16;  [1024,768] x [768,3072] with Gelu: 76 -> 50
 //   [6304,768] x [768,2304]: 229 -> 200 (112 Tflop/s);  x [768,3072] with Gelu: 323 -> 269
 //   [197,197] x [197,64], 12 heads: 19 -> 7 (single-value loads: rows of 197 start anywhere)
-// What is left on large shapes is power (2.1 GHz under load, where the rate is quoted for 2.4) and the gaps around barriers.
+//   [50432,768] x [768,768 / 2304 / 3072]: 518 -> 495, 1520 -> 1383, 1970 -> 1784;  [50432,3072] x [3072,768]: 2006 -> 1900
+// Single-value loads are taken for both operands where one of them needs them: [6304,768] x [768,768] 72 us with 16-byte loads, 84
+// with an operand one float off (the earlier kernel, which decided per operand, 91 and 110 to 152).
+// What is left on large shapes is not the clock (2.40 GHz, where the rate is quoted for 2.4) but matrix pipes that are busy 84 % of the
+// cycles at 50432 rows, 71 to 73 % at 6304 and 60 % in [6304,768] x [768,768].  The waits the code has are a step's fragments, all of
+// them read before its first product and right behind a barrier, and a last round of blocks that is partly empty.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
