@@ -118,6 +118,13 @@ int check_device_flags(DeviceCtx &ctx) {
     return ctx.fail(AHIP_ERR_ARG, "Gather: an index is outside the gathered axis");
 }
 
+bool stream_is_recording(const DeviceCtx &ctx) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(ctx.stream, &status) == hipSuccess) return status != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return false;
+}
+
 void destroy_device_ctx(DeviceCtx *ctx) {
     if (hipSetDevice(ctx->device) != hipSuccess) return;
     (void)hipStreamSynchronize(ctx->stream);

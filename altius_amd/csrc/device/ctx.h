@@ -64,6 +64,9 @@ struct DeviceCtx {
     void *gemm_partials = nullptr;
     size_t gemm_partials_bytes = 0;
     int *gemm_counters = nullptr;
+    // The owner drops recorded launches when gemm_ws_generation moves (a session).  Without it, what somebody records on the stream
+    // keeps out of the workspace where another route is there: a later call may move it.
+    bool drops_recordings = false;
     bool gemm_split_k = true;
     int cus_per_xcd = 0;  // compute units / 8, read when the context is created
     // Measured when the context is created (placement.hip): blocks whose ids agree mod 8 run on one XCD, and
@@ -100,6 +103,8 @@ void destroy_device_ctx(DeviceCtx *ctx);
 bool xcd_round_robin_holds(int cu_count, const uint32_t *xcc_of_block, size_t n_blocks);
 // Runs the probe launch on the context's stream (uses the scratch buffer) and sets ctx.xcd_round_robin.
 int probe_xcd_placement(DeviceCtx &ctx, int cu_count);
+// Whether launches on the context's stream are being recorded.
+bool stream_is_recording(const DeviceCtx &ctx);
 // After the stream has been synchronised: reports and clears an error flag raised by a kernel.
 int check_device_flags(DeviceCtx &ctx);
 
@@ -222,7 +227,8 @@ size_t gemm_planes_bytes(size_t rows, size_t k);
 int launch_layernorm_planes(DeviceCtx &ctx, void *planes, float *sum_out, const float *in, const float *in2, const float *gamma,
                             const float *beta, size_t rows, size_t len, float eps);
 bool layernorm_planes_fits(size_t rows, size_t len);
-// The context's grow-only GEMM workspace, at least `bytes` large (stream-ordered use only).
+// The context's grow-only GEMM workspace, at least `bytes` large (stream-ordered use only).  AHIP_ERR_OOM where there is no memory
+// for it, or where it would have to grow while the stream is being recorded; so too gemm_partials.
 int gemm_workspace(DeviceCtx &ctx, size_t bytes, void **p);
 // Room for the partial sums of tiles that a product cuts along k (ctx.gemm_partials, at least `bytes`, grow-only) and the
 // counters of such tiles (ctx.gemm_counters, GEMM_COUNTERS of them, zero between launches).

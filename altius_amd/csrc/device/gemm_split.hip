@@ -526,6 +526,7 @@ const void *cached_planes(DeviceCtx &ctx, const float *src, size_t rows, size_t 
 
 int ensure_workspace(DeviceCtx &ctx, size_t bytes) {
     if (bytes <= ctx.gemm_ws_bytes) return AHIP_OK;
+    if (stream_is_recording(ctx)) return ctx.fail(AHIP_ERR_OOM, "gemm: the workspace cannot grow while the stream is being recorded");
     // Work already queued may still read the old buffer.
     int rc = ctx.check(hipStreamSynchronize(ctx.stream), "hipStreamSynchronize");
     if (rc) return rc;
@@ -547,6 +548,7 @@ int ensure_workspace(DeviceCtx &ctx, size_t bytes) {
 
 int gemm_partials(DeviceCtx &ctx, size_t bytes) {
     if (bytes <= ctx.gemm_partials_bytes) return AHIP_OK;
+    if (stream_is_recording(ctx)) return ctx.fail(AHIP_ERR_OOM, "gemm: the room for partial sums cannot grow while the stream is being recorded");
     int rc = ctx.check(hipStreamSynchronize(ctx.stream), "hipStreamSynchronize");
     if (rc) return rc;
     if (ctx.gemm_partials) (void)hipFree(ctx.gemm_partials);

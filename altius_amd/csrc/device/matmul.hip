@@ -591,7 +591,15 @@ int launch_gemm_f32(DeviceCtx &ctx, float *c, const float *a, const float *b, co
         return aligned16(p) && contiguous % 4 == 0 && ld % 4 == 0 && bs[0] % 4 == 0 && bs[1] % 4 == 0;
     };
     const bool both = vec(a, a_kc ? k : m, lda, a_batch_strides) && vec(b, b_kc ? k : n, ldb, b_batch_strides);
-    const Choice ch = choose(batch, m, n, k, cus, ctx.gemm_split_k, both && !(a_kc && b_kc), g.act != 0);
+    const bool tail = both && !(a_kc && b_kc);
+    Choice ch = choose(batch, m, n, k, cus, ctx.gemm_split_k, tail, g.act != 0);
+    if (ch.slices > 1) {
+        const Shape &cut = SHAPES[ch.shape];
+        const size_t cut_tiles = ((m + cut.bm - 1) / cut.bm * ((n + cut.bn - 1) / cut.bn) + 7) / 8 * 8;
+        const int rc = gemm_partials(ctx, cut_tiles * ch.slices * cut.bm * cut.bn * sizeof(float));
+        if (rc == AHIP_ERR_OOM) ch = choose(batch, m, n, k, cus, false, tail, g.act != 0);  // no room: whole
+        else if (rc) return rc;
+    }
     const Shape &sh = SHAPES[ch.shape];
     const size_t gy = (m + sh.bm - 1) / sh.bm, gx = (n + sh.bn - 1) / sh.bn, tiles = gx * gy * batch;
     if (gx * gy >= lim || batch >= lim || (tiles + 7) / 8 * 8 * ch.slices * 256 > 0xffffffffu)
@@ -610,8 +618,6 @@ int launch_gemm_f32(DeviceCtx &ctx, float *c, const float *a, const float *b, co
     g.slices = ch.slices;
     g.slice_k = ch.slices > 1 ? ch.slice_k : (uint32_t)k;
     if (g.slices > 1) {
-        const int rc = gemm_partials(ctx, (size_t)g.chunk * 8 * g.slices * sh.bm * sh.bn * sizeof(float));
-        if (rc) return rc;
         g.partials = static_cast<float *>(ctx.gemm_partials);
         g.counters = ctx.gemm_counters;
     }

@@ -120,6 +120,7 @@ std::unique_ptr<HipSession> HipSessionBuilder::build(SessionError *err) {
 
     std::string derr;
     int rc = create_device_ctx(device_, nullptr, true, &s->ctx_, &derr);
+    s->ctx_.drops_recordings = true;
     if (rc) {
         fail_code(err, rc, derr);
         return nullptr;

@@ -2,18 +2,68 @@
 input shapes is seen and replayed afterwards.  Every replay must give the bits of the node-by-node
 run, for fresh inputs each time, with other GPU work and synchronisations in between; graphs that
 need the host during a run must keep running node by node."""
+import ctypes
+
 import numpy as np
 import pytest
 
 import oracle as O
 from altius_amd import synth
-from altius_amd._lib import AltiusHipError
+from altius_amd._lib import AltiusHipError, check, lib
 from altius_amd.graph import I64, Model, Op
 from altius_amd.graphs import erf_gelu_chain, layer_norm_chain, single_input_model, squeeze_excite
 from altius_amd.session import HipSessionBuilder
 from conftest import assert_bits_equal
 
 pytestmark = pytest.mark.gpu
+
+
+def test_launches_that_a_caller_records(case):
+    """A convolution and a product on a stream that a program records for itself, without a run beforehand: nothing has to grow while
+    it records, and what it recorded holds after later calls have moved the context's workspace."""
+    torch = pytest.importorskip("torch")
+    case("conv2d and gemm recorded by the caller")
+    stream, handle = torch.cuda.Stream(), ctypes.c_void_p()
+    L = lib()
+    check(L.ahip_init_on_stream(0, stream.cuda_stream, ctypes.byref(handle)))
+    rng = np.random.default_rng(3)
+    ints = lambda *s: torch.from_numpy(rng.integers(-3, 4, size=s).astype(np.float32)).cuda()  # noqa: E731
+
+    def conv(out, x, w):
+        check(L.ahip_conv2d(handle, out.data_ptr(), x.data_ptr(), w.data_ptr(), None, None, x.shape[0], x.shape[1], x.shape[2], x.shape[3],
+                            w.shape[0], x.shape[2], x.shape[3], 3, 3, 1, 1, 1, 1, 1, 1, 1), handle)
+
+    def gemm(out, a, b):
+        (m, k), n = a.shape, b.shape[1]
+        check(L.ahip_gemm(handle, out.data_ptr(), a.data_ptr(), b.data_ptr(), None, 1, m, n, k, 0, 0, k, n, n, 0, 0, 0, 0, 0, 1.0, 0.0), handle)
+
+    try:
+        x, w, y = ints(1, 700, 12, 12), ints(128, 700, 3, 3), torch.zeros(1, 128, 12, 12, device="cuda")
+        a, b, c = ints(77, 3072), ints(3072, 768), torch.zeros(77, 768, device="cuda")
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            conv(y, x, w)
+            gemm(c, a, b)
+        for step in range(3):
+            x.copy_(ints(*x.shape))
+            a.copy_(ints(*a.shape))
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(y.cpu(), torch.nn.functional.conv2d(x.cpu(), w.cpu(), padding=1))
+            assert torch.equal(c.cpu(), a.cpu() @ b.cpu())
+            side = 16 + 8 * step  # larger each time: the workspace and the room for partial sums move
+            rows = 200 + 100 * step
+            held = [torch.empty(1, 256, side, side, device="cuda"), ints(1, 700, side, side), ints(256, 700, 3, 3), torch.empty(rows, 768, device="cuda"),
+                    ints(rows, 3072)]
+            torch.cuda.synchronize()
+            conv(*held[:3])
+            gemm(held[3], held[4], b)
+            torch.cuda.synchronize()
+    finally:
+        torch.cuda.synchronize()
+        L.ahip_destroy(handle)
 
 
 def chain_model(shape, gamma, beta):
