@@ -10,6 +10,7 @@ import pytest
 import oracle as O
 from altius_amd import synth
 from altius_amd._lib import AltiusHipError, check, lib
+from altius_amd.device import Context
 from altius_amd.graph import I64, Model, Op
 from altius_amd.graphs import erf_gelu_chain, layer_norm_chain, single_input_model, squeeze_excite
 from altius_amd.session import HipSessionBuilder
@@ -18,52 +19,75 @@ from conftest import assert_bits_equal
 pytestmark = pytest.mark.gpu
 
 
+def hip_runtime():
+    """The HIP runtime that the library is linked against, for what a program records by itself."""
+    lib()
+    with open("/proc/self/maps") as maps:
+        paths = {line.split()[-1] for line in maps if "libamdhip64" in line}
+    assert len(paths) == 1, paths
+    return ctypes.CDLL(paths.pop())
+
+
 def test_launches_that_a_caller_records(case):
     """A convolution and a product on a stream that a program records for itself, without a run beforehand: nothing has to grow while
     it records, and what it recorded holds after later calls have moved the context's workspace."""
-    torch = pytest.importorskip("torch")
     case("conv2d and gemm recorded by the caller")
-    stream, handle = torch.cuda.Stream(), ctypes.c_void_p()
-    L = lib()
-    check(L.ahip_init_on_stream(0, stream.cuda_stream, ctypes.byref(handle)))
+    L, hip = lib(), hip_runtime()
+    stream, graph, replay, handle = (ctypes.c_void_p() for _ in range(4))
+
+    def ok(rc):
+        assert rc == 0, f"HIP error {rc}"
+
     rng = np.random.default_rng(3)
-    ints = lambda *s: torch.from_numpy(rng.integers(-3, 4, size=s).astype(np.float32)).cuda()  # noqa: E731
+    ints = lambda *s: rng.integers(-3, 4, size=s).astype(np.float32)  # noqa: E731
+    with Context(0) as memory:  # buffers and copies, on a stream of its own that is waited for
+        ok(hip.hipStreamCreate(ctypes.byref(stream)))
+        check(L.ahip_init_on_stream(0, stream, ctypes.byref(handle)))
 
-    def conv(out, x, w):
-        check(L.ahip_conv2d(handle, out.data_ptr(), x.data_ptr(), w.data_ptr(), None, None, x.shape[0], x.shape[1], x.shape[2], x.shape[3],
-                            w.shape[0], x.shape[2], x.shape[3], 3, 3, 1, 1, 1, 1, 1, 1, 1), handle)
+        def conv(out, x, w, shape, channels):
+            b, c, h, wd = shape
+            check(L.ahip_conv2d(handle, out.ptr, x.ptr, w.ptr, None, None, b, c, h, wd, channels, h, wd, 3, 3, 1, 1, 1, 1, 1, 1, 1), handle)
 
-    def gemm(out, a, b):
-        (m, k), n = a.shape, b.shape[1]
-        check(L.ahip_gemm(handle, out.data_ptr(), a.data_ptr(), b.data_ptr(), None, 1, m, n, k, 0, 0, k, n, n, 0, 0, 0, 0, 0, 1.0, 0.0), handle)
+        def gemm(out, a, b, m, n, k):
+            check(L.ahip_gemm(handle, out.ptr, a.ptr, b.ptr, None, 1, m, n, k, 0, 0, k, n, n, 0, 0, 0, 0, 0, 1.0, 0.0), handle)
 
-    try:
-        x, w, y = ints(1, 700, 12, 12), ints(128, 700, 3, 3), torch.zeros(1, 128, 12, 12, device="cuda")
-        a, b, c = ints(77, 3072), ints(3072, 768), torch.zeros(77, 768, device="cuda")
-        torch.cuda.synchronize()
-        graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(graph, stream=stream):
-            conv(y, x, w)
-            gemm(c, a, b)
-        for step in range(3):
-            x.copy_(ints(*x.shape))
-            a.copy_(ints(*a.shape))
-            torch.cuda.synchronize()
-            graph.replay()
-            torch.cuda.synchronize()
-            assert torch.equal(y.cpu(), torch.nn.functional.conv2d(x.cpu(), w.cpu(), padding=1))
-            assert torch.equal(c.cpu(), a.cpu() @ b.cpu())
-            side = 16 + 8 * step  # larger each time: the workspace and the room for partial sums move
-            rows = 200 + 100 * step
-            held = [torch.empty(1, 256, side, side, device="cuda"), ints(1, 700, side, side), ints(256, 700, 3, 3), torch.empty(rows, 768, device="cuda"),
-                    ints(rows, 3072)]
-            torch.cuda.synchronize()
-            conv(*held[:3])
-            gemm(held[3], held[4], b)
-            torch.cuda.synchronize()
-    finally:
-        torch.cuda.synchronize()
-        L.ahip_destroy(handle)
+        def refill(buffer, values):
+            check(L.ahip_h2d_async(memory.handle, buffer.ptr, values.ctypes.data, values.nbytes), memory.handle)
+            memory.sync()
+
+        try:
+            shape, (m, n, k) = (1, 700, 12, 12), (77, 768, 3072)
+            wi, bi = ints(128, 700, 3, 3), ints(k, n)
+            x, w, y = memory.alloc(4 * 700 * 144), memory.upload(wi), memory.alloc(4 * 128 * 144)
+            a, b, c = memory.alloc(4 * m * k), memory.upload(bi), memory.alloc(4 * m * n)
+            ok(hip.hipStreamBeginCapture(stream, 1))  # thread-local mode
+            conv(y, x, w, shape, 128)
+            gemm(c, a, b, m, n, k)
+            ok(hip.hipStreamEndCapture(stream, ctypes.byref(graph)))
+            ok(hip.hipGraphInstantiateWithFlags(ctypes.byref(replay), graph, ctypes.c_ulonglong(0)))
+            for step in range(3):
+                xi, ai = ints(*shape), ints(m, k)
+                refill(x, xi)
+                refill(a, ai)
+                ok(hip.hipGraphLaunch(replay, stream))
+                check(L.ahip_sync(handle), handle)
+                assert_bits_equal(memory.download(y, (1, 128, 12, 12)), O.conv2d(xi, wi, None, pads=(1, 1, 1, 1)), "recorded convolution")
+                assert_bits_equal(memory.download(c, (m, n)), (ai.astype(np.float64) @ bi).astype(np.float32), "recorded product")
+                side, rows = 16 + 8 * step, 200 + 100 * step  # larger each time: the workspace and the room for partial sums move
+                big, out = memory.upload(ints(1, 700, side, side)), memory.alloc(4 * 256 * side * side)
+                weights, tall, sums = memory.upload(ints(256, 700, 3, 3)), memory.upload(ints(rows, k)), memory.alloc(4 * rows * n)
+                conv(out, big, weights, (1, 700, side, side), 256)
+                gemm(sums, tall, b, rows, n, k)
+                check(L.ahip_sync(handle), handle)
+        finally:
+            hip.hipStreamSynchronize(stream)
+            if replay.value:
+                hip.hipGraphExecDestroy(replay)
+            if graph.value:
+                hip.hipGraphDestroy(graph)
+            L.ahip_destroy(handle)
+            hip.hipStreamDestroy(stream)
+
 
 
 def chain_model(shape, gamma, beta):
