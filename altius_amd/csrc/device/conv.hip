@@ -316,8 +316,8 @@ __global__ __launch_bounds__(512) void conv_gemm_small(ConvGemmArgs g) {
 }
 
 // 64 x 128 tile per block of four wavefronts (32 x 64 each), k in steps of 16 through two LDS buffers; the loads of step
-// t + 1 are in flight during the products of step t.  [72,16] x [16, 32 * 3136] takes 15 us here.  w lies in LDS as [row][k] (pitch 20: the 16-byte reads of 16 rows
-// meet all 64 banks), x as [k][column] (pitch 132: the four k of a step are 16 banks apart).
+// t + 1 are in flight during the products of step t.  [72,16] x [16, 32 * 3136] takes 15 us here.  w lies in LDS as [row][k]
+// (pitch 20: the 16-byte reads of 16 rows meet all 64 banks), x as [k][column] (pitch 132: the four k of a step are 16 banks apart).
 constexpr int TM = 64, TN = 128, TK = 16, WP = TK + 4, XP = TN + 4;
 
 template <bool POINTWISE>
@@ -432,7 +432,7 @@ __global__ __launch_bounds__(BLOCK) void conv_unfold(float *__restrict__ col, co
 }
 
 // The unfolded copy lives in the context's workspace, of as many images at a time as this holds, or of as many output rows of one
-// image: 1 GiB ([32,2048,28,28] -> 256, 3 x 3: 4010 us in passes of four images, 256 MiB; 3300 in two passes).
+// image: 1 GiB ([32,2048,28,28] -> 256, 3 x 3: 4010 us in passes of four images, 256 MiB; 3570 in two passes).
 constexpr size_t UNFOLD_FLOATS = (size_t)256 << 20;
 
 enum Route { SMALL_16, SMALL_32, TILED, UNFOLDED };
