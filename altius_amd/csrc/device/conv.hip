@@ -544,9 +544,7 @@ int launch_conv2d(DeviceCtx &ctx, float *out, const float *x, const float *w, co
     if (pass.rows * ow > (size_t)1 << 24) pass.images = 0;
     Route route = conv_route(ctx, batch, m, oh, ow, k, group, pass, pointwise, g.w_vec && (pass.rows * ow) % 4 == 0 && (!pointwise || a16(x)));
     if (route == UNFOLDED) {
-        const bool in_place = !ctx.drops_recordings && stream_is_recording(ctx);
-        const int rc = in_place ? AHIP_ERR_UNSUPPORTED
-                                : launch_unfolded(ctx, out, x, w, bias, pass, pointwise, batch, c, ih, iw, oc, oh, ow, kh, kw, sh, sw, dh, dw, pad_t, pad_l, group);
+        const int rc = launch_unfolded(ctx, out, x, w, bias, pass, pointwise, batch, c, ih, iw, oc, oh, ow, kh, kw, sh, sw, dh, dw, pad_t, pad_l, group);
         if (rc != AHIP_ERR_OOM && rc != AHIP_ERR_UNSUPPORTED) return rc;
         route = conv_route(ctx, batch, m, oh, ow, k, group, Pass(), pointwise, false);  // no room for the copy
     }

@@ -64,9 +64,10 @@ struct DeviceCtx {
     void *gemm_partials = nullptr;
     size_t gemm_partials_bytes = 0;
     int *gemm_counters = nullptr;
-    // The owner drops recorded launches when gemm_ws_generation moves (a session).  Without it, what somebody records on the stream
-    // keeps out of the workspace where another route is there: a later call may move it.
-    bool drops_recordings = false;
+    // The owner drops recorded launches when gemm_ws_generation moves (a session).  Elsewhere, once somebody has recorded launches that
+    // may use these buffers, what the buffers outgrow is kept for them until the context goes.
+    bool drops_recordings = false, recorded_by_caller = false;
+    std::vector<void *> outgrown;
     bool gemm_split_k = true;
     int cus_per_xcd = 0;  // compute units / 8, read when the context is created
     // Measured when the context is created (placement.hip): blocks whose ids agree mod 8 run on one XCD, and

@@ -524,45 +524,38 @@ const void *cached_planes(DeviceCtx &ctx, const float *src, size_t rows, size_t 
     return planes;
 }
 
-int ensure_workspace(DeviceCtx &ctx, size_t bytes) {
-    if (bytes <= ctx.gemm_ws_bytes) return AHIP_OK;
-    if (stream_is_recording(ctx)) return ctx.fail(AHIP_ERR_OOM, "gemm: the workspace cannot grow while the stream is being recorded");
+// Makes one of the context's buffers at least `bytes` large.
+int ensure_room(DeviceCtx &ctx, void **buffer, size_t *have, size_t bytes, const char *what) {
+    const bool recording = !ctx.drops_recordings || bytes > *have ? stream_is_recording(ctx) : false;
+    if (recording && !ctx.drops_recordings) ctx.recorded_by_caller = true;
+    if (bytes <= *have) return AHIP_OK;
+    if (recording) return ctx.fail(AHIP_ERR_OOM, std::string("gemm: the room for ") + what + " cannot grow while the stream is being recorded");
     // Work already queued may still read the old buffer.
-    int rc = ctx.check(hipStreamSynchronize(ctx.stream), "hipStreamSynchronize");
+    const int rc = ctx.check(hipStreamSynchronize(ctx.stream), "hipStreamSynchronize");
     if (rc) return rc;
-    if (ctx.gemm_ws) (void)hipFree(ctx.gemm_ws);
-    ctx.gemm_ws = nullptr;
-    ctx.gemm_ws_bytes = 0;
+    if (*buffer && ctx.recorded_by_caller) ctx.outgrown.push_back(*buffer);
+    else if (*buffer) (void)hipFree(*buffer);
+    *buffer = nullptr;
+    *have = 0;
     ctx.gemm_ws_generation++;
     void *p = nullptr;
     if (hipMalloc(&p, bytes) != hipSuccess) {
         (void)hipGetLastError();
-        return ctx.fail(AHIP_ERR_OOM, "gemm: no memory for the bf16 planes of the operands");
+        return ctx.fail(AHIP_ERR_OOM, std::string("gemm: no memory for ") + what);
     }
-    ctx.gemm_ws = p;
-    ctx.gemm_ws_bytes = bytes;
+    *buffer = p;
+    *have = bytes;
     return AHIP_OK;
+}
+
+int ensure_workspace(DeviceCtx &ctx, size_t bytes) {
+    return ensure_room(ctx, &ctx.gemm_ws, &ctx.gemm_ws_bytes, bytes, "the operands' bf16 planes or an unfolded input");
 }
 
 }  // namespace
 
 int gemm_partials(DeviceCtx &ctx, size_t bytes) {
-    if (bytes <= ctx.gemm_partials_bytes) return AHIP_OK;
-    if (stream_is_recording(ctx)) return ctx.fail(AHIP_ERR_OOM, "gemm: the room for partial sums cannot grow while the stream is being recorded");
-    int rc = ctx.check(hipStreamSynchronize(ctx.stream), "hipStreamSynchronize");
-    if (rc) return rc;
-    if (ctx.gemm_partials) (void)hipFree(ctx.gemm_partials);
-    ctx.gemm_partials = nullptr;
-    ctx.gemm_partials_bytes = 0;
-    ctx.gemm_ws_generation++;
-    void *p = nullptr;
-    if (hipMalloc(&p, bytes) != hipSuccess) {
-        (void)hipGetLastError();
-        return ctx.fail(AHIP_ERR_OOM, "gemm: no memory for the partial sums of tiles cut along k");
-    }
-    ctx.gemm_partials = p;
-    ctx.gemm_partials_bytes = bytes;
-    return AHIP_OK;
+    return ensure_room(ctx, &ctx.gemm_partials, &ctx.gemm_partials_bytes, bytes, "the partial sums of tiles cut along k");
 }
 
 int gemm_workspace(DeviceCtx &ctx, size_t bytes, void **p) {
@@ -752,6 +745,8 @@ void gemm_release_all(DeviceCtx &ctx) {
     if (ctx.gemm_partials) (void)hipFree(ctx.gemm_partials);
     ctx.gemm_partials = nullptr;
     ctx.gemm_partials_bytes = 0;
+    for (void *p : ctx.outgrown) (void)hipFree(p);
+    ctx.outgrown.clear();
 }
 
 }  // namespace altius

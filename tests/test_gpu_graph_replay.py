@@ -28,10 +28,11 @@ def hip_runtime():
     return ctypes.CDLL(paths.pop())
 
 
-def test_launches_that_a_caller_records(case):
-    """A convolution and a product on a stream that a program records for itself, without a run beforehand: nothing has to grow while
-    it records, and what it recorded holds after later calls have moved the context's workspace."""
-    case("conv2d and gemm recorded by the caller")
+@pytest.mark.parametrize("run_first", [False, True])
+def test_launches_that_a_caller_records(case, run_first):
+    """A convolution and a product on a stream that a program records for itself: without a run beforehand nothing has to grow while it
+    records, and what it recorded holds after later calls have outgrown the context's buffers."""
+    case(f"conv2d and gemm recorded by the caller, run first: {run_first}")
     L, hip = lib(), hip_runtime()
     stream, graph, replay, handle = (ctypes.c_void_p() for _ in range(4))
 
@@ -60,6 +61,10 @@ def test_launches_that_a_caller_records(case):
             wi, bi = ints(128, 700, 3, 3), ints(k, n)
             x, w, y = memory.alloc(4 * 700 * 144), memory.upload(wi), memory.alloc(4 * 128 * 144)
             a, b, c = memory.alloc(4 * m * k), memory.upload(bi), memory.alloc(4 * m * n)
+            if run_first:
+                conv(y, x, w, shape, 128)
+                gemm(c, a, b, m, n, k)
+                check(L.ahip_sync(handle), handle)
             ok(hip.hipStreamBeginCapture(stream, 1))  # thread-local mode
             conv(y, x, w, shape, 128)
             gemm(c, a, b, m, n, k)
