@@ -470,7 +470,7 @@ Route conv_route(const DeviceCtx &ctx, size_t batch, size_t m, size_t oh, size_t
     if (pass.images) {
         const size_t cols = pass.rows * ow;
         const double pass_us = (pointwise ? 0.0 : 2.8 + 2.0e-6 * (double)(pass.images * group * k * cols)) +
-                               (double)group * gemm_f32_us(ctx, pass.images, m, cols, k, false, vec);
+                               (double)group * gemm_f32_us(ctx, pass.images, m, cols, k, vec);
         if ((double)(batch * oh) / (double)(pass.images * pass.rows) * pass_us < best_us) best = UNFOLDED;
     }
     return best;

@@ -184,13 +184,13 @@ int launch_gemm_batch2(DeviceCtx &ctx, float *c, const float *a, const float *b,
                        const size_t a_batch_strides[2], const size_t b_batch_strides[2], const size_t c_batch_strides[2],
                        size_t c0_row_stride, size_t c0_col_stride, float alpha, float beta, const GemmPost *post = nullptr);
 
-// The same, on the fp32 kernels whatever ctx.gemm_algorithm says; and about how long the tiled one takes, in us (k_rows: k is the
-// contiguous axis of both operands, vec: both allow 16-byte loads).
+// The same, on the fp32 kernels whatever ctx.gemm_algorithm says; and about how long the tiled one takes, in us (vec: both operands
+// allow 16-byte loads).
 int launch_gemm_f32(DeviceCtx &ctx, float *c, const float *a, const float *b, const float *c0, size_t batch_outer, size_t batch_inner, size_t m,
                     size_t n, size_t k, int trans_a, int trans_b, size_t lda, size_t ldb, size_t ldc, const size_t a_batch_strides[2],
                     const size_t b_batch_strides[2], const size_t c_batch_strides[2], size_t c0_row_stride, size_t c0_col_stride, float alpha,
                     float beta, const GemmPost *post = nullptr);
-double gemm_f32_us(const DeviceCtx &ctx, size_t batch, size_t m, size_t n, size_t k, bool k_rows, bool vec);
+double gemm_f32_us(const DeviceCtx &ctx, size_t batch, size_t m, size_t n, size_t k, bool vec);
 
 // Many small products at once (matmul_small.hip): one block per matrix.  C = A B, A with unit stride along k.
 bool gemm_small_batched_fits(size_t batch, size_t m, size_t n, size_t k);

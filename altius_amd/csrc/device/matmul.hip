@@ -15,21 +15,21 @@
 // TA (TB) neighbouring rows, one for each of its tiles.  The instruction takes two values of k, one per half of the wavefront;
 // a half takes k = 8 i + 4 half + 0 .. 3 in turn, the same for both layouts, so that a product does not depend on them.
 //
-// Measured against 128 x 128 and 128 x 64 tiles staged through registers, cut along k into batches whose sums a second kernel
-// added, with activations and residuals in a pass of their own (us, whole layers' products in sessions but for the last four):
-//   [197,768] x [768,768 / 2304 / 3072]: 17 -> 10, 23 -> 14, 29 -> 20 (latency: 168 to 672 tiles of 32 x 32)
-//   [1024,768] x [768,768]: 27 -> 16;  [1024,768] x [768,3072] with Gelu: 76 -> 50
-//   [6304,768] x [768,2304]: 229 -> 200 (112 Tflop/s);  x [768,3072] with Gelu: 323 -> 269
-//   [197,197] x [197,64], 12 heads: 19 -> 7 (single-value loads: rows of 197 start anywhere)
-//   [50432,768] x [768,768 / 2304 / 3072]: 518 -> 495, 1520 -> 1383, 1970 -> 1784;  [50432,3072] x [3072,768]: 2006 -> 1900
-// Single-value loads are taken for both operands where one of them needs them: [6304,768] x [768,768] 72 us with 16-byte loads, 84
-// with an operand one float off (the earlier kernel, which decided per operand, 91 and 110 to 152).
-// What is left on large shapes is not the clock (2.40 GHz, where the rate is quoted for 2.4) but matrix pipes that are busy 84 % of the
-// cycles at 50432 rows, 71 to 73 % at 6304 and 60 % in [6304,768] x [768,768].  The waits the code has are a step's fragments, all of
-// them read before its first product and right behind a barrier, and a last round of blocks that is partly empty.
+// A step's two halves take turns in registers: while one half's products run, the other's fragments come from LDS, and what else a step
+// does (the next loads and their addresses) stands between the products, where the matrix pipe covers it.  With a step's fragments
+// all read in front of its products and the addresses worked out anew in every step, the pipes were busy 60 to 84 % of the cycles:
+//   [6304,768] x [768,768 / 2304 / 3072]: 72 -> 63 us, 192 -> 184, 258 -> 228;  [6304,3072] x [3072,768]: 262 -> 227
+//   [1024,768] x [768,768 / 3072]: 16.4 -> 14.7, 45 -> 40;  [1024,3072] x [3072,768]: 51 -> 46
+//   [197,768] x [768,768]: 8.6 -> 7.1;  [77,768] x [768,3072]: 12.0 -> 10.2
+//   4096^3: 1061 -> 938 us (147 Tflop/s);  [50432,768] x [768,3072]: 1788 -> 1670 (143)
+// Single-value loads are taken for both operands where one of them needs them.
+// What is left on large shapes: the blocks' first loads and their results (1 us of 12 in a 64 x 64 tile with 768 values of k), and a last
+// round of blocks that is partly empty ([6304,768] x [768,768]: 4.6 rounds take five).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
+#include <utility>
 
 #include "common.h"
 #include "ctx.h"
@@ -42,6 +42,7 @@ namespace {
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void *lds_ptr;
 
 constexpr int BK = 16;  // values of k a wavefront multiplies between two barriers
@@ -62,6 +63,8 @@ struct GemmArgs {
     uint32_t tiles_m, tiles_n, tiles, chunk, group_n;  // tiles: of all batches
     // A tile's k cut into `slices` of slice_k values (whole steps of the block; the last one takes the rest): see the epilogue.
     uint32_t slices, slice_k;
+    // Steps that 32-bit byte offsets reach behind the tile whose first element they count from, for both operands.
+    uint32_t window;
     float *partials;
     int *counters;
     float alpha, beta;
@@ -92,106 +95,97 @@ __device__ __forceinline__ f32x4 load_shared(const f32x4 *p) {
     return __builtin_bit_cast(f32x4, b);
 }
 
-// What a lane holds of T tiles of an operand for BK values of k: at(tile, step).  KC: k is the operand's contiguous axis.
-template <bool KC, int T> struct FragRegs;
-template <> struct FragRegs<true, 1> { f32x4 v[2]; __device__ float at(int, int s) const { return v[s >> 2][s & 3]; } };
-template <> struct FragRegs<true, 2> { f32x4 v[4]; __device__ float at(int t, int s) const { return v[t * 2 + (s >> 2)][s & 3]; } };
-template <> struct FragRegs<false, 1> { float v[8]; __device__ float at(int, int s) const { return v[s]; } };
-template <> struct FragRegs<false, 2> { f32x2 v[8]; __device__ float at(int t, int s) const { return v[s][t]; } };
-
-// A stage's fragments of both operands, read and waited for in one asm statement: the compiler's wait-count pass drains every
-// outstanding memory -> LDS load before an LDS read that it cannot prove independent of them, which would undo the prefetch.
-#define RD_K1(X) "ds_read_b128 %[" X "0], %[p" X "0]\n\tds_read_b128 %[" X "1], %[p" X "1]\n\t"
-#define RD_K2(X) RD_K1(X) "ds_read_b128 %[" X "2], %[p" X "0] offset:2048\n\tds_read_b128 %[" X "3], %[p" X "1] offset:2048\n\t"
-#define RD_M8(X, W) \
-    "ds_read_" W " %[" X "0], %[p" X "0]\n\tds_read_" W " %[" X "1], %[p" X "0] offset:%c[s" X "1]\n\t" \
-    "ds_read_" W " %[" X "2], %[p" X "0] offset:%c[s" X "2]\n\tds_read_" W " %[" X "3], %[p" X "0] offset:%c[s" X "3]\n\t" \
-    "ds_read_" W " %[" X "4], %[p" X "0] offset:%c[s" X "4]\n\tds_read_" W " %[" X "5], %[p" X "0] offset:%c[s" X "5]\n\t" \
-    "ds_read_" W " %[" X "6], %[p" X "0] offset:%c[s" X "6]\n\tds_read_" W " %[" X "7], %[p" X "0] offset:%c[s" X "7]\n\t"
-#define RD_M1(X) RD_M8(X, "b32")
-#define RD_M2(X) RD_M8(X, "b64")
-#define OUT_K1(X, F) [X##0] "=&v"(F.v[0]), [X##1] "=&v"(F.v[1])
-#define OUT_K2(X, F) OUT_K1(X, F), [X##2] "=&v"(F.v[2]), [X##3] "=&v"(F.v[3])
-#define OUT_M1(X, F) OUT_K2(X, F), [X##4] "=&v"(F.v[4]), [X##5] "=&v"(F.v[5]), [X##6] "=&v"(F.v[6]), [X##7] "=&v"(F.v[7])
-#define OUT_M2(X, F) OUT_M1(X, F)
-#define IN_K1(X, P, PITCH) [p##X##0] "v"(P[0]), [p##X##1] "v"(P[1])
-#define IN_K2(X, P, PITCH) IN_K1(X, P, PITCH)
-#define IN_M1(X, P, PITCH)                                                                                                             \
-    [p##X##0] "v"(P[0]), [s##X##1] "i"((PITCH) * 4), [s##X##2] "i"((PITCH) * 8), [s##X##3] "i"((PITCH) * 12), [s##X##4] "i"((PITCH) * 32), \
-        [s##X##5] "i"((PITCH) * 36), [s##X##6] "i"((PITCH) * 40), [s##X##7] "i"((PITCH) * 44)
-#define IN_M2(X, P, PITCH) IN_M1(X, P, PITCH)
-
-template <bool AK, int TA, bool BKC, int TB, int PA, int PB> struct Reader;
-#define READER(AK_, TA_, AKIND, BK_, TB_, BKIND)                                                                                       \
-    template <int PA, int PB> struct Reader<AK_, TA_, BK_, TB_, PA, PB> {                                                              \
-        static __device__ __forceinline__ void read(FragRegs<AK_, TA_> &fa, FragRegs<BK_, TB_> &fb, const uint32_t (&pa)[2], const uint32_t (&pb)[2]) { \
-            asm volatile(RD_##AKIND("a") RD_##BKIND("b") "s_waitcnt lgkmcnt(0)"                                                         \
-                         : OUT_##AKIND(a, fa), OUT_##BKIND(b, fb)                                                                       \
-                         : IN_##AKIND(a, pa, PA), IN_##BKIND(b, pb, PB)                                                                 \
-                         : "memory");                                                                                                   \
-        }                                                                                                                               \
-    };
-READER(true, 1, K1, true, 1, K1)
-READER(true, 1, K1, true, 2, K2)
-READER(true, 2, K2, true, 1, K1)
-READER(true, 2, K2, true, 2, K2)
-READER(true, 1, K1, false, 1, M1)
-READER(true, 1, K1, false, 2, M2)
-READER(true, 2, K2, false, 1, M1)
-READER(true, 2, K2, false, 2, M2)
-READER(false, 1, M1, true, 1, K1)
-READER(false, 1, M1, true, 2, K2)
-READER(false, 2, M2, true, 1, K1)
-READER(false, 2, M2, true, 2, K2)
-READER(false, 1, M1, false, 1, M1)
-READER(false, 1, M1, false, 2, M2)
-READER(false, 2, M2, false, 1, M1)
-READER(false, 2, M2, false, 2, M2)
-
-template <int N> __device__ __forceinline__ void wait_loads_and_barrier() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory"); }
-
-// Copies an operand's tiles to LDS: [WK][W][BK] (KC, pieces exchanged) or [WK][BK][W], VEC floats per lane and instruction.  The
-// operand is addressed as a buffer that ends behind its last element; p walks along k.  A lane whose k lies past the end asks for
-// an offset behind any buffer, and lanes of rows past the edge for zeros or for values that only reach sums nobody stores.
-template <bool KC, int W, int WK, int WAVES, int VEC> struct Loader {
-    static constexpr int PER = 64 * VEC, TILE = W * BK, COUNT = TILE * WK / PER / WAVES;
-    static_assert(COUNT * PER * WAVES == TILE * WK, "whole instructions");
-    uint32_t off[COUNT], kk[COUNT];  // of this lane's pieces: byte offset from p, value of k
-    const float *p;
-    uint64_t left, step;             // floats from p to the operand's end; floats to the next tile
-    __device__ __forceinline__ void init(const float *base, uint64_t floats, uint32_t ld, int wave, int lane) {
-        p = base, left = floats, step = KC ? (uint64_t)(BK * WK) : (uint64_t)(BK * WK) * ld;
+// What a lane holds of T tiles of an operand for four values of k, half a step: at(tile, step).  KC: k is the operand's contiguous axis.
+template <bool KC, int T> struct Frag;
+template <int T> struct Frag<true, T> {
+    f32x4 v[T];
+    __device__ __forceinline__ float at(int t, int s) const { return v[t][s]; }
+    template <int PITCH> __device__ __forceinline__ void read(const float *p) {
 #pragma unroll
-        for (int u = 0; u < COUNT; u++) {
-            const uint32_t f = ((u * WAVES + wave) * 64 + lane) * VEC, sub = f / TILE, q = f % TILE;
-            if (KC) {
-                const uint32_t row = q / BK, piece = (q % BK) / 4, k = sub * BK + ((piece ^ ((row >> 2) & 3)) * 4) + (q & 3);
-                off[u] = (row * ld + k) * 4, kk[u] = k;
-            } else {
-                const uint32_t row = q / W, k = sub * BK + row;
-                off[u] = (k * ld + q % W) * 4, kk[u] = k;
-            }
-        }
+        for (int t = 0; t < T; t++) v[t] = *reinterpret_cast<const f32x4 *>(p + t * (32 * BK));
     }
-    // k_left: values of k from this tile on
-    __device__ __forceinline__ void issue(float *stage, int wave, uint32_t k_left) {
-        const uint32_t bytes = (uint32_t)min(left, (uint64_t)0x3fffffff) * 4u;
-        const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p), 0, (int)bytes, 0x00020000);
+};
+template <> struct Frag<false, 1> {
+    float v[4];
+    __device__ __forceinline__ float at(int, int s) const { return v[s]; }
+    template <int PITCH> __device__ __forceinline__ void read(const float *p) {
 #pragma unroll
-        for (int u = 0; u < COUNT; u++) {
-            const uint32_t o = kk[u] < k_left ? off[u] : 0xffffffffu;
-            if constexpr (VEC == 4) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr)(stage + (u * WAVES + wave) * PER), 16, (int)o, 0, 0, 0);
-            else __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr)(stage + (u * WAVES + wave) * PER), 4, (int)o, 0, 0, 0);
-        }
-        const uint64_t s = min(step, left);
-        p += s;
-        left -= s;
+        for (int s = 0; s < 4; s++) v[s] = p[s * PITCH];
+    }
+};
+template <> struct Frag<false, 2> {
+    f32x2 v[4];
+    __device__ __forceinline__ float at(int t, int s) const { return v[s][t]; }
+    template <int PITCH> __device__ __forceinline__ void read(const float *p) {
+#pragma unroll
+        for (int s = 0; s < 4; s++) v[s] = *reinterpret_cast<const f32x2 *>(p + s * PITCH);
     }
 };
 
+template <int N> __device__ __forceinline__ void wait_loads_and_barrier() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory"); }
+
+// A wavefront's VEC floats per lane from a buffer to LDS, in asm: of loads it knows the compiler waits for all before any LDS read that it
+// cannot prove independent of them, which would undo the prefetch.  Waits are wait_loads_and_barrier's.  (m0 and an SGPR that a vector
+// instruction wrote need one and five cycles before the load reads them.)
+template <int VEC> __device__ __forceinline__ void load_to_lds(i32x4 rsrc, uint32_t off, uint32_t to) {
+    if constexpr (VEC == 4) asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(off), "s"(rsrc), "s"(to) : "memory");
+    else asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dword %0, %1, 0 offen lds" ::"v"(off), "s"(rsrc), "s"(to) : "memory");
+}
+
+// Copies an operand's tiles to LDS: [WK][W][BK] (KC, pieces exchanged) or [WK][BK][W], VEC floats per lane and instruction.  The
+// operand is addressed as a buffer that ends behind its last element.  A lane whose k lies past the end asks for an offset behind any
+// buffer, and lanes of rows past the edge for zeros or for values that only reach sums nobody stores.
+template <bool KC, int W, int WK, int WAVES, int VEC> struct Loader {
+    static constexpr int PER = 64 * VEC, TILE = W * BK, COUNT = TILE * WK / PER / WAVES;
+    static_assert(COUNT * PER * WAVES == TILE * WK, "whole instructions");
+    uint32_t off[COUNT];  // byte offsets of this lane's pieces of the tile to load next
+    uint32_t lo, hi, bytes;  // the buffer: from the first tile that off counts from to the operand's end
+    // A tile that starts at p, floats before the operand's end, with k_left values of k.
+    __device__ __forceinline__ void start(const float *p, uint64_t floats, uint32_t ld, uint32_t k_left, int wave, int lane) {
+        const uint64_t at = (uint64_t)(uintptr_t)p;
+        lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)at);
+        hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(at >> 32) & 0xffff);
+        bytes = (uint32_t)__builtin_amdgcn_readfirstlane((int)((uint32_t)min(floats, (uint64_t)0x3fffffff) * 4u));
+        asm volatile("s_nop 4" ::"s"(lo), "s"(hi), "s"(bytes));
+#pragma unroll
+        for (int u = 0; u < COUNT; u++) {
+            const uint32_t f = ((u * WAVES + wave) * 64 + lane) * VEC, sub = f / TILE, q = f % TILE;
+            uint32_t k, o;
+            if (KC) {
+                const uint32_t row = q / BK, piece = (q % BK) / 4;
+                k = sub * BK + ((piece ^ ((row >> 2) & 3)) * 4) + (q & 3);
+                o = row * ld + k;
+            } else {
+                k = sub * BK + q / W;
+                o = k * ld + q % W;
+            }
+            off[u] = k < k_left ? o * 4 : 0xffffffffu;
+        }
+    }
+    __device__ __forceinline__ void next(uint32_t step_bytes) {
+#pragma unroll
+        for (int u = 0; u < COUNT; u++) off[u] += step_bytes;
+    }
+    __device__ __forceinline__ void nothing() {
+#pragma unroll
+        for (int u = 0; u < COUNT; u++) off[u] = 0xffffffffu;
+    }
+    __device__ __forceinline__ void load(int u, uint32_t stage, int wave) {
+        const i32x4 rsrc = {(int)lo, (int)hi, (int)bytes, 0x00020000};
+        load_to_lds<VEC>(rsrc, off[u], stage + (u * WAVES + wave) * (PER * 4));
+    }
+};
+
+// f(0) .. f(N - 1) with the number known when f is compiled.
+template <class F, int... I> __device__ __forceinline__ void each_of(F f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>()), ...); }
+template <int N, class F> __device__ __forceinline__ void each(F f) { each_of(f, std::make_integer_sequence<int, N>()); }
+
 template <bool AKC, bool BKC, int WM, int WN, int WK, int TA, int TB, int VEC>
 __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_f32_tiles(GemmArgs g) {
-    constexpr int S = 3;  // stages; a fourth is 3 to 10 % slower, it costs a block per CU
+    // Stages, and with them how many blocks a CU holds (48 KB of LDS: three).  A fourth is 3 to 10 % slower for the small tiles, which lose
+    // a block by it.  Of 128 x 128 tiles a CU holds two: three in step end together, and the blocks left then fill the slots of few CUs
+    // (4096^3, four rounds: 1153 us with three, 938 with two; five rounds, [4096,1024] x [1024,5120]: 354 and 304).
+    constexpr int S = TA == 2 ? 4 : 3;
     constexpr int WAVES = WM * WN * WK, THREADS = 64 * WAVES, BM = 32 * WM * TA, BN = 32 * WN * TB, BKT = BK * WK;
     constexpr int STAGE_A = BM * BKT, STAGE = (BM + BN) * BKT;
     constexpr int CP = BN + 4, PASS_ROWS = 32 * WM, SUMS = WK * PASS_ROWS * CP;  // the epilogue's [WK][PASS_ROWS][CP]
@@ -216,8 +210,9 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_f32_tiles(GemmArgs g) 
 
     Loader<AKC, BM, WK, WAVES, VEC> la;
     Loader<BKC, BN, WK, WAVES, VEC> lb;
-    la.init(a, k == 0 ? 0 : AKC ? (uint64_t)(min(g.m - m0, (uint32_t)BM) - 1) * g.lda + k : (uint64_t)(k - 1) * g.lda + (g.m - m0), g.lda, wave, lane);
-    lb.init(b, k == 0 ? 0 : BKC ? (uint64_t)(min(g.n - n0, (uint32_t)BN) - 1) * g.ldb + k : (uint64_t)(k - 1) * g.ldb + (g.n - n0), g.ldb, wave, lane);
+    const uint64_t a_floats = k == 0 ? 0 : AKC ? (uint64_t)(min(g.m - m0, (uint32_t)BM) - 1) * g.lda + k : (uint64_t)(k - 1) * g.lda + (g.m - m0);
+    const uint64_t b_floats = k == 0 ? 0 : BKC ? (uint64_t)(min(g.n - n0, (uint32_t)BN) - 1) * g.ldb + k : (uint64_t)(k - 1) * g.ldb + (g.n - n0);
+    const uint64_t a_step = AKC ? (uint64_t)BKT : (uint64_t)BKT * g.lda, b_step = BKC ? (uint64_t)BKT : (uint64_t)BKT * g.ldb;
     constexpr int LOADS = decltype(la)::COUNT + decltype(lb)::COUNT;
 
     floatx16 acc[TA][TB];
@@ -228,50 +223,102 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_f32_tiles(GemmArgs g) 
 #pragma unroll
             for (int e = 0; e < 16; e++) acc[i][j][e] = 0.0f;
 
-    const uint32_t nk = (k + BKT - 1) / BKT;
-    uint32_t k_left = k;
-    auto issue = [&](uint32_t s) {
-        la.issue(lds + s * STAGE, wave, k_left);
-        lb.issue(lds + s * STAGE + STAGE_A, wave, k_left);
-        k_left -= min(k_left, (uint32_t)BKT);
+    // Where a tile and the one behind it are whole, and 32 bits reach, its addresses are the last tile's and a step (near: up to which
+    // tile).  Per step that is an addition per load; a base, an end and a mask worked out anew each time held the products up by
+    // 300 cycles a step (64 x 64 tiles: 18.8 ns a value of k for a CU's only block, 13.6 now).
+    const uint32_t nk = (k + BKT - 1) / BKT, whole = k / BKT;
+    uint32_t tile_k = 0, near = 0;
+    auto advance_near = [&]() __attribute__((always_inline)) {
+        la.next((uint32_t)a_step * 4);
+        lb.next((uint32_t)b_step * 4);
+        tile_k++;
+    };
+    auto advance_far = [&] __attribute__((always_inline)) {
+        la.start(a + tile_k * a_step, a_floats - tile_k * a_step, g.lda, k - tile_k * BKT, wave, lane);
+        lb.start(b + tile_k * b_step, b_floats - tile_k * b_step, g.ldb, k - tile_k * BKT, wave, lane);
+        near = min(whole, tile_k + 1 + min(g.window, 0x7fffffffu - tile_k));
+        tile_k++;
+    };
+    auto nothing_left = [&] __attribute__((always_inline)) {
+        la.nothing();
+        lb.nothing();
+    };
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr)lds;
+    auto load = [&](auto u, uint32_t stage) __attribute__((always_inline)) {
+        if constexpr (u < la.COUNT) la.load(u, lds0 + stage * (STAGE * 4), wave);
+        else lb.load(u - la.COUNT, lds0 + (stage * STAGE + STAGE_A) * 4, wave);
     };
 #pragma unroll
-    for (int s = 0; s < S - 1; s++) issue(s);
-
-    // Byte addresses of this lane's fragments in stage 0.
-    uint32_t pa[2], pb[2];
-    const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr)lds;
-    if (AKC) {
-        const uint32_t row = wm * (32 * TA) + lr, sw = (row >> 2) & 3;
-        pa[0] = lds0 + ((wk * BM + row) * BK + ((uint32_t)(lk ^ sw) << 2)) * 4, pa[1] = lds0 + ((wk * BM + row) * BK + ((uint32_t)((2 + lk) ^ sw) << 2)) * 4;
-    } else {
-        pa[0] = lds0 + ((wk * BK + 4 * lk) * BM + wm * (32 * TA) + TA * lr) * 4, pa[1] = 0;
-    }
-    if (BKC) {
-        const uint32_t row = wn * (32 * TB) + lr, sw = (row >> 2) & 3;
-        pb[0] = lds0 + (STAGE_A + (wk * BN + row) * BK + ((uint32_t)(lk ^ sw) << 2)) * 4, pb[1] = lds0 + (STAGE_A + (wk * BN + row) * BK + ((uint32_t)((2 + lk) ^ sw) << 2)) * 4;
-    } else {
-        pb[0] = lds0 + (STAGE_A + (wk * BK + 4 * lk) * BN + wn * (32 * TB) + TB * lr) * 4, pb[1] = 0;
+    for (int s = 0; s < S; s++) {
+        if (tile_k < near) advance_near();
+        else if (tile_k < nk) advance_far();
+        else nothing_left();
+        each<LOADS>([&](auto u) __attribute__((always_inline)) { load(u, s); });
     }
 
-    uint32_t cur = 0, put = S - 1;
-    for (uint32_t kt = 0; kt < nk; kt++) {
-        wait_loads_and_barrier<(S - 2) * LOADS>();
-        issue(put);
-        if (++put == S) put = 0;
-        FragRegs<AKC, TA> fa;
-        FragRegs<BKC, TB> fb;
-        const uint32_t so = cur * (STAGE * 4);
-        const uint32_t qa[2] = {pa[0] + so, pa[1] + so}, qb[2] = {pb[0] + so, pb[1] + so};
-        Reader<AKC, TA, BKC, TB, BM, BN>::read(fa, fb, qa, qb);
-        if (++cur == S) cur = 0;
+    // This lane's fragments in stage 0, of either half of a step.
+    const float *pa[2], *pb[2];
 #pragma unroll
-        for (int s = 0; s < 8; s++)
-#pragma unroll
-            for (int i = 0; i < TA; i++)
-#pragma unroll
-                for (int j = 0; j < TB; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa.at(i, s), fb.at(j, s), acc[i][j], 0, 0, 0);
+    for (int h = 0; h < 2; h++) {
+        if (AKC) {
+            const int row = wm * (32 * TA) + lr;
+            pa[h] = lds + (wk * BM + row) * BK + (((2 * h + lk) ^ ((row >> 2) & 3)) << 2);
+        } else {
+            pa[h] = lds + (wk * BK + 8 * h + 4 * lk) * BM + wm * (32 * TA) + TA * lr;
+        }
+        if (BKC) {
+            const int row = wn * (32 * TB) + lr;
+            pb[h] = lds + STAGE_A + (wk * BN + row) * BK + (((2 * h + lk) ^ ((row >> 2) & 3)) << 2);
+        } else {
+            pb[h] = lds + STAGE_A + (wk * BK + 8 * h + 4 * lk) * BN + wn * (32 * TB) + TB * lr;
+        }
     }
+
+    // Half a step's products while the next half's fragments are on their way.
+    Frag<AKC, TA> fa[2];
+    Frag<BKC, TB> fb[2];
+    auto read = [&](int h, uint32_t stage) __attribute__((always_inline)) {
+        fa[h].template read<BM>(pa[h] + stage * STAGE);
+        fb[h].template read<BN>(pb[h] + stage * STAGE);
+    };
+    constexpr int Q = 4 * TA * TB;
+    auto multiply = [&](int h, int q) __attribute__((always_inline)) {
+        const int s = q / (TA * TB), i = q / TB % TA, j = q % TB;
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[h].at(i, s), fb[h].at(j, s), acc[i][j], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    wait_loads_and_barrier<(S - 1) * LOADS>();
+    read(0, 0);
+    uint32_t cur = 0;
+    auto step = [&](auto is_near) __attribute__((always_inline)) {
+        each<Q>([&](auto q) __attribute__((always_inline)) {
+            multiply(0, q);
+            if constexpr (q == 0) read(1, cur);
+            if constexpr (q == 1 && is_near) advance_near();
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        const uint32_t next = cur + 1 == S ? 0 : cur + 1;
+        each<Q>([&](auto q) __attribute__((always_inline)) {
+            constexpr int R = Q > 4 ? 1 : 0;
+            multiply(1, q);
+            if constexpr (q == 0) wait_loads_and_barrier<(S - 2) * LOADS>();  // this stage is read, the next one there
+            if constexpr (q == R) read(0, next);
+            each<LOADS>([&](auto u) __attribute__((always_inline)) {
+                if constexpr (R + 1 + u * (Q - 1 - R) / LOADS == q) load(u, cur);
+            });
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        cur = next;
+    };
+    while (tile_k < nk) {
+        if (tile_k >= near) {
+            advance_far();
+            step(std::false_type());
+        }
+        while (tile_k < near) step(std::true_type());
+    }
+    nothing_left();
+    for (uint32_t kt = min(nk, (uint32_t)S); kt > 0; kt--) step(std::false_type());
     wait_loads_and_barrier<0>();
 
     // Epilogue, TA passes of PASS_ROWS rows: accumulator e of lane l is row 8 (e / 4) + 4 (l / 32) + e % 4, column l % 32 of its
@@ -372,30 +419,19 @@ inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 
 
 // The block tiles, and what a launch of them takes: launch_us + rounds * (block_us + k_us * k / 768), rounds being the blocks that
 // the busiest CU runs (dealt to the XCDs in turn), times `lone` where that is one: a CU's only block has nothing to fill its gaps
-// with.  Where k is cut, 0.8 us more, slice_us for each slice and the partial sums at 2.5 TB/s.  Fitted to 222 products of 1e8 to
-// 5e11 multiplications with every tile (within 3 % rms of the first three's times and, but for tail_rounds, the fourth's) and to 210
-// of up to 2e7 sums with every tile and cut; of those the choice is 0.7 % behind the best one on average.  Per value of C a small
-// tile costs more (each of its operands serves fewer products), but its rounds come in smaller units.
+// with.  Where k is cut, 0.8 us more, slice_us for each slice and the partial sums at 2.5 TB/s.  Fitted to 120 products of 1e8 to
+// 2e11 multiplications with every tile and 70 of up to 1500 tiles of 32 x 32 with every tile and cut (6, 4, 4 and 4 % rms); the choice
+// is 0.4 % behind the best one on average.  Per value of C a small tile costs more (each of its operands serves fewer products), but its
+// rounds come in smaller units.  A k_us of 10.24 per 64 x 64 would be the matrix cores' peak.
 struct Shape {
     uint32_t bm, bn, step;  // step: values of k per barrier
     double launch_us, block_us, k_us, lone, slice_us;
 };
-constexpr Shape SHAPES[] = {{32, 32, 64, 3.0, 0.81, 3.71, 1.29, 0.3},
-                            {64, 64, 32, 3.7, 1.15, 12.7, 1.14, 0.9},
-                            {128, 64, 16, 4.9, 1.18, 24.7, 1.16, 1.8},
-                            {128, 128, 16, 4.9, 2.06, 46.5, 1.12, 4.0}};
+constexpr Shape SHAPES[] = {{32, 32, 64, 2.97, 0.72, 3.18, 1.02, 0.27},
+                            {64, 64, 32, 2.82, 1.06, 11.11, 1.04, 0.83},
+                            {128, 64, 16, 2.81, 1.38, 21.95, 1.04, 1.61},
+                            {128, 128, 16, 2.07, 3.63, 42.81, 1.02, 3.21}};
 constexpr int N_SHAPES = 4;
-
-double cost_us(const Shape &sh, size_t rounds, size_t k) {
-    return sh.launch_us + (double)rounds * (sh.block_us + sh.k_us * (double)k / 768.0) * (rounds == 1 ? sh.lone : 1.0);
-}
-
-// Three 128 x 128 blocks fit a CU.  Those that run together end together where k is cut, or where an operand of 16-byte loads has its
-// rows along m or n, and the blocks left over then fill the slots of few CUs: a fourth or fifth round takes as long as three more, a
-// seventh as two (4096^3: 1440 us for four rounds, 128 x 64 tiles 1070; with both operands' k contiguous 1025 and 1045).  An
-// activation behind the product spreads the ends of short blocks: five rounds of up to 1024 values of k stay five then
-// ([6304,768] x [768,3072] with Gelu 265 us, 128 x 64 tiles 271; four rounds, 4096^3: 1480 and 1080).
-size_t tail_rounds(size_t rounds) { return rounds == 4 || rounds == 5 ? 6 : rounds == 7 ? 8 : rounds; }
 
 struct Choice {
     int shape = 0;
@@ -404,43 +440,24 @@ struct Choice {
 };
 
 // What a product adds up in which order is decided by the sizes alone, so that a product and the same product with an operand stored
-// the other way round add up alike (the last two tiles do, as long as k is whole).
-// cut: k may be cut into slices.  tail: an operand of 16-byte loads has its rows along m or n.  act: an activation follows.
-Choice choose(size_t batch, size_t m, size_t n, size_t k, size_t cus_per_xcd, bool cut, bool tail, bool act) {
+// the other way round add up alike.  cut: k may be cut into slices.
+Choice choose(size_t batch, size_t m, size_t n, size_t k, size_t cus_per_xcd, bool cut) {
     Choice best;
-    double best_us = 0.0;
-    auto chunk_of = [&](const Shape &sh) { return (((m + sh.bm - 1) / sh.bm) * ((n + sh.bn - 1) / sh.bn) * batch + 7) / 8; };
-    auto rounds_of = [&](size_t blocks_per_xcd) { return (blocks_per_xcd + cus_per_xcd - 1) / cus_per_xcd; };
     for (int s = 0; s < N_SHAPES; s++) {
         const Shape &sh = SHAPES[s];
-        const size_t chunk = chunk_of(sh);
+        const size_t chunk = (((m + sh.bm - 1) / sh.bm) * ((n + sh.bn - 1) / sh.bn) * batch + 7) / 8;
         for (uint32_t want = 1; want <= 8; want *= 2) {
             if (want > 1 && (!cut || batch != 1 || k < 128 * (size_t)want || chunk * 8 > GEMM_COUNTERS)) break;
             const size_t slice_k = ((k + want - 1) / want + sh.step - 1) / sh.step * sh.step, slices = slice_k ? (k + slice_k - 1) / slice_k : 1;
             if (want > 1 && slices != want) continue;
             // A grid ends at 2^32 threads: a few rows with 2^29 columns are more blocks of 32 x 32 than that.
             if (s < N_SHAPES - 1 && chunk * 8 * want * 256 > 0xffffffffu) break;
-            size_t rounds = rounds_of(chunk * want);
-            if (want > 1 && s == N_SHAPES - 1) rounds = tail_rounds(rounds);
-            const double us = cost_us(sh, rounds, std::max<size_t>(slice_k, sh.step)) +
-                              (want > 1 ? 0.8 + want * (sh.slice_us + (double)(chunk * 8) * sh.bm * sh.bn * sizeof(float) / 2.5e6) : 0.0);
-            if (best_us == 0.0 || us < best_us) {
-                best_us = us;
-                best.shape = s, best.slices = want, best.slice_k = (uint32_t)slice_k;
-            }
+            const size_t rounds = (chunk * want + cus_per_xcd - 1) / cus_per_xcd;
+            double us = sh.launch_us + (double)rounds * (sh.block_us + sh.k_us * (double)std::max<size_t>(slice_k, sh.step) / 768.0) * (rounds == 1 ? sh.lone : 1.0);
+            if (want > 1) us += 0.8 + want * (sh.slice_us + (double)(chunk * 8) * sh.bm * sh.bn * sizeof(float) / 2.5e6);
+            if (best.us == 0.0 || us < best.us) best = {s, want, (uint32_t)slice_k, us};
         }
     }
-    if (best.shape == N_SHAPES - 1 && best.slices == 1 && tail) {
-        const Shape &large = SHAPES[N_SHAPES - 1], &half = SHAPES[N_SHAPES - 2];
-        const size_t blocks = chunk_of(half), rounds = rounds_of(chunk_of(large));
-        const double half_us = cost_us(half, rounds_of(blocks), k);
-        best_us = cost_us(large, act && rounds == 5 && k <= 1024 ? rounds : tail_rounds(rounds), k);
-        if (blocks * 8 * 256 <= 0xffffffffu && half_us < best_us) {
-            best_us = half_us;
-            best.shape = N_SHAPES - 2;
-        }
-    }
-    best.us = best_us;
     return best;
 }
 
@@ -526,9 +543,9 @@ int launch_gemm_batch2(DeviceCtx &ctx, float *c, const float *a, const float *b,
                            c_batch_strides, c0_row_stride, c0_col_stride, alpha, beta, post);
 }
 
-double gemm_f32_us(const DeviceCtx &ctx, size_t batch, size_t m, size_t n, size_t k, bool k_rows, bool vec) {
+double gemm_f32_us(const DeviceCtx &ctx, size_t batch, size_t m, size_t n, size_t k, bool vec) {
     const size_t cus = ctx.cus_per_xcd ? (size_t)ctx.cus_per_xcd : 32;
-    return choose(batch, m, n, k, cus, ctx.gemm_split_k, vec && !k_rows, false).us * (vec ? 1.0 : 1.2);
+    return choose(batch, m, n, k, cus, ctx.gemm_split_k).us * (vec ? 1.0 : 1.2);
 }
 
 int launch_gemm_f32(DeviceCtx &ctx, float *c, const float *a, const float *b, const float *c0, size_t batch_outer, size_t batch_inner, size_t m,
@@ -591,13 +608,12 @@ int launch_gemm_f32(DeviceCtx &ctx, float *c, const float *a, const float *b, co
         return aligned16(p) && contiguous % 4 == 0 && ld % 4 == 0 && bs[0] % 4 == 0 && bs[1] % 4 == 0;
     };
     const bool both = vec(a, a_kc ? k : m, lda, a_batch_strides) && vec(b, b_kc ? k : n, ldb, b_batch_strides);
-    const bool tail = both && !(a_kc && b_kc);
-    Choice ch = choose(batch, m, n, k, cus, ctx.gemm_split_k, tail, g.act != 0);
+    Choice ch = choose(batch, m, n, k, cus, ctx.gemm_split_k);
     if (ch.slices > 1) {
         const Shape &cut = SHAPES[ch.shape];
         const size_t cut_tiles = ((m + cut.bm - 1) / cut.bm * ((n + cut.bn - 1) / cut.bn) + 7) / 8 * 8;
         const int rc = gemm_partials(ctx, cut_tiles * ch.slices * cut.bm * cut.bn * sizeof(float));
-        if (rc == AHIP_ERR_OOM) ch = choose(batch, m, n, k, cus, false, tail, g.act != 0);  // no room: whole
+        if (rc == AHIP_ERR_OOM) ch = choose(batch, m, n, k, cus, false);  // no room: whole
         else if (rc) return rc;
     }
     const Shape &sh = SHAPES[ch.shape];
@@ -621,6 +637,12 @@ int launch_gemm_f32(DeviceCtx &ctx, float *c, const float *a, const float *b, co
         g.partials = static_cast<float *>(ctx.gemm_partials);
         g.counters = ctx.gemm_counters;
     }
+    auto window = [&](bool kc, size_t rows, size_t ld) {
+        const size_t end = ((size_t)1 << 32) - 64, step = (kc ? (size_t)sh.step : sh.step * ld) * 4;
+        const size_t span = (kc ? (rows - 1) * ld + sh.step : (sh.step - 1) * ld + rows) * 4;
+        return span < end ? std::min<size_t>((end - span) / std::max<size_t>(step, 1), 0x7fffffff) : 0;
+    };
+    g.window = (uint32_t)std::min(window(a_kc, std::min<size_t>(sh.bm, a_kc ? m : sh.bm), lda), window(b_kc, std::min<size_t>(sh.bn, b_kc ? n : sh.bn), ldb));
     if (a_kc && b_kc) launch_tiles<true, true>(ctx, g, ch.shape, both);
     else if (a_kc) launch_tiles<true, false>(ctx, g, ch.shape, both);
     else if (b_kc) launch_tiles<false, true>(ctx, g, ch.shape, both);

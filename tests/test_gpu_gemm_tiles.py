@@ -136,3 +136,51 @@ def test_more_columns_than_a_grid_of_small_tiles_holds(ctx, case):
     finally:
         for d in (da, db, dc):
             ctx.free(d)
+
+
+# The tiles that the sizes above leave out, ragged, and k around as many steps as a block has stages (3 of 64 x 64: 32 values each, of
+# 128 x 64: 16; 4 of 128 x 128: 16): fewer, as many, one more, each with and without a rest.
+TURNS = ([(1646, 132, k) for k in (15, 31, 32, 64, 96, 97, 128, 140)] + [(2300, 1300, k) for k in (16, 32, 48, 50, 64)] +
+         [(325, 3735, 2506), (834, 3482, 700), (9001, 2500, 64), (9001, 2500, 83)])
+
+
+@pytest.mark.parametrize("trans_a", [False, True])
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("pad,offset", [(0, 0), (3, 1)])
+def test_stages_in_turn(ctx, case, trans_a, trans_b, pad, offset):
+    rng = np.random.default_rng(8)
+    for m, n, k in TURNS:
+        case(f"gemm [{m},{k}] x [{k},{n}] trans {trans_a} {trans_b} pad {pad} offset {offset}")
+        a, abuf, lda = padded(rng, *((k, m) if trans_a else (m, k)), pad, offset)
+        b, bbuf, ldb = padded(rng, *((n, k) if trans_b else (k, n)), pad, offset)
+        da, db, dc = ctx.upload(abuf), ctx.upload(bbuf), ctx.alloc(4 * m * n)
+        try:
+            ctx.gemm_raw(dc.ptr, da.ptr + 4 * offset, db.ptr + 4 * offset, None, 1, m, n, k, trans_a, trans_b, lda, ldb, n)
+            want = np.matmul(a.T if trans_a else a, b.T if trans_b else b)  # whole numbers below 2^24: exact in any order
+            assert_bits_equal(ctx.download(dc, (m, n)), want, "product")
+        finally:
+            for x in (da, db, dc):
+                ctx.free(x)
+
+
+def test_more_steps_than_32_bit_offsets_reach(ctx, case):
+    """Rows of k next to each other that take 4.3 GB, in two batches so that k stays whole: the offsets are counted from a later tile again."""
+    block_rows, n, m = 4096, 1028, 3
+    k = 257 * block_rows - 13
+    case(f"gemm [{m},{k}] x [{k},{n}]")
+    rng = np.random.default_rng(9)
+    block = rng.integers(-1, 2, size=(block_rows, n)).astype(np.float32)
+    a = rng.integers(-1, 2, size=(2 * m, k)).astype(np.float32)
+    da, db, dc = ctx.upload(a), ctx.alloc(4 * k * n), ctx.alloc(8 * m * n)
+    try:
+        want = np.zeros((2 * m, n))
+        for r in range(0, k, block_rows):
+            rows = min(block_rows, k - r)
+            assert ctx.L.ahip_h2d_async(ctx.handle, db.ptr + 4 * r * n, block.ctypes.data, 4 * rows * n) == 0
+            want += np.matmul(a[:, r:r + rows], block[:rows])
+        ctx.sync()
+        ctx.gemm_raw(dc.ptr, da.ptr, db.ptr, None, 2, m, n, k, a_bs=m * k, c_bs=m * n)
+        assert_bits_equal(ctx.download(dc, (2 * m, n)), want.astype(np.float32), "product")
+    finally:
+        for x in (da, db, dc):
+            ctx.free(x)
