@@ -112,14 +112,27 @@ int check_device_flags(DeviceCtx &ctx);
 constexpr int MAX_RANK = 8;
 constexpr size_t SCRATCH_FLOATS = 1u << 20;  // 4 MiB
 
+// An operator without a code of its own in the C interface: x * HardSigmoid(x) (hard swish).
+constexpr int ACT_HARD_SWISH = 100;
+
+// What the operators behind the product would do to its result (a `post` of null: nothing), done while it is written, always on
+// the fp32 kernel: C = act(alpha * op(A) op(B) + beta * C0) + residual, act 0, AHIP_GELU, AHIP_RELU, AHIP_HARDSIGMOID or
+// ACT_HARD_SWISH (the last two with alpha and beta), residual null or matrices laid out like C (same pitch, same batch
+// strides).  Each step rounds as its own kernel would.
+struct GemmPost {
+    int act = 0;
+    const float *residual = nullptr;
+    float alpha = 0.0f, beta = 0.0f;
+};
+
 int launch_binary(DeviceCtx &ctx, int op, float *out, const float *a, const float *b, int rank,
                   const int64_t *out_dims, const int64_t *a_strides, const int64_t *b_strides);
 int launch_unary(DeviceCtx &ctx, int op, float *out, const float *in, size_t n, float alpha,
                  float beta);
 // A chain of element-wise steps in one kernel (fused.hip); AHIP_ERR_UNSUPPORTED when the geometry
-// needs the operator-by-operator route.
+// needs the operator-by-operator route.  then (may be null): a hard swish of the chain's result.
 int launch_fused_elemwise(DeviceCtx &ctx, float *out, int rank, const int64_t *out_dims, int n_inputs, const float *const *inputs,
-                          const int64_t *const *input_strides, int n_steps, const ahip_fused_step *steps);
+                          const int64_t *const *input_strides, int n_steps, const ahip_fused_step *steps, const GemmPost *then = nullptr);
 int launch_softmax(DeviceCtx &ctx, float *out, const float *in, size_t rows, size_t len);
 // Softmax of (in [*|/] scale) + mask over the last axis; scale_op 0 none / 1 multiply / 2 divide, mask (may be
 // null) holds rows / rows_per_mask rows of len values.  AHIP_ERR_UNSUPPORTED when the geometry needs separate kernels.
@@ -142,6 +155,8 @@ int reduce_static_setup(int device);
 // A stream that is about to be destroyed (its work has been waited for) no longer owns the fixed array.
 void reduce_static_forget_stream(int device, hipStream_t stream);
 size_t reduce_static_capacity_floats();
+// The sum of every plane divided by its extent (GlobalAveragePool): the division of DIV_BY, in the reduction's kernel.
+int launch_average_pool(DeviceCtx &ctx, float *out, const float *in, size_t planes, size_t area);
 
 
 // Data movement (movement.hip).  Strides are in elements; elem_size in bytes (1, 4 or 8).
@@ -172,13 +187,7 @@ int launch_gemm(DeviceCtx &ctx, float *c, const float *a, const float *b, const 
 // The same with the batch index split in two, z = (z / batch_inner, z % batch_inner), each part with its own
 // stride per operand: operands that are strided views of a larger tensor (the heads of a [b, t, h, d] tensor
 // read in place as b x h matrices of t x d with row pitch h * d) need no copy.
-// post (may be null): what the operators behind the product would do to its result, done while it is written, single
-// batch only and always on the fp32 kernel: C = act(alpha * op(A) op(B) + beta * C0) + residual, act 0 or AHIP_GELU /
-// AHIP_RELU, residual null or a matrix laid out like C (same pitch).  Each step rounds as its own kernel would.
-struct GemmPost {
-    int act = 0;
-    const float *residual = nullptr;
-};
+// post (may be null): GemmPost.
 int launch_gemm_batch2(DeviceCtx &ctx, float *c, const float *a, const float *b, const float *c0, size_t batch_outer,
                        size_t batch_inner, size_t m, size_t n, size_t k, int trans_a, int trans_b, size_t lda, size_t ldb, size_t ldc,
                        const size_t a_batch_strides[2], const size_t b_batch_strides[2], const size_t c_batch_strides[2],
@@ -242,7 +251,7 @@ RowsBy reduce_rows_by(const float *in, size_t rows, size_t len);
 // Row sums (optionally times `scale`) or maxima of a [rows, len] matrix through LDS-staged groups of rows (rows.hip): for
 // rows that are short or not whole float4s.  Only for shapes reduce_rows_lds_fits accepts.
 bool reduce_rows_lds_fits(const float *in, size_t rows, size_t len);
-int launch_reduce_rows_lds(DeviceCtx &ctx, bool is_max, float *out, const float *in, size_t rows, size_t len, float scale, bool scaled);
+int launch_reduce_rows_lds(DeviceCtx &ctx, bool is_max, float *out, const float *in, size_t rows, size_t len, float scale, int scaled);
 // Whether launch_gemm would send this single-batch product through launch_gemm_split.
 bool gemm_takes_split(const DeviceCtx &ctx, size_t m, size_t n, size_t k);
 // Large and tile-filling enough for the split kernel to win (the AHIP_GEMM_AUTO rule).
@@ -256,10 +265,19 @@ void gemm_release_all(DeviceCtx &ctx);
 // Max pooling over [planes, ih, iw] (movement.hip).
 int launch_maxpool(DeviceCtx &ctx, float *out, const float *x, size_t planes, size_t ih, size_t iw, size_t oh, size_t ow,
                    size_t kh, size_t kw, size_t sh, size_t sw, size_t pad_t, size_t pad_l);
+// What the operators behind a convolution would do to its result, done while it is written: BatchNormalization with one value
+// per output channel (mean null: none), then an activation and a residual as GemmPost has them.  Each step rounds as its own kernel
+// would.  launch_conv2d says in `applied` whether it did all of it or (a normalisation in front of a route that has none) nothing.
+struct ConvPost {
+    const float *mean = nullptr, *var = nullptr, *scale = nullptr, *shift = nullptr;
+    float eps = 0.0f;
+    GemmPost then;
+    bool applied = false;
+};
 // Conv2d on NCHW (conv.hip); bias may be null.  Uses the GEMM workspace, up to 1 GiB of it.
 int launch_conv2d(DeviceCtx &ctx, float *out, const float *x, const float *w, const float *bias, size_t batch, size_t c, size_t ih, size_t iw,
                   size_t oc, size_t oh, size_t ow, size_t kh, size_t kw, size_t sh, size_t sw, size_t dh, size_t dw, size_t pad_t, size_t pad_l,
-                  size_t group);
+                  size_t group, ConvPost *post = nullptr);
 
 // Resize on [planes, ih, iw] -> [planes, oh, ow]: nearest, or the reference's bilinear blend (movement.hip).
 int launch_resize(DeviceCtx &ctx, float *out, const float *x, size_t planes, size_t ih, size_t iw, size_t oh, size_t ow,

@@ -47,6 +47,7 @@ constexpr uint32_t ACC = 0xFF;  // operand selector: the previous step's result
 enum Code : uint32_t {
     C_ADD, C_SUB, C_MUL, C_DIV, C_POW, C_POW_SCALAR_EXP,
     C_SQRT, C_ERF, C_GELU, C_SIGMOID, C_HARDSIGMOID, C_RELU, C_TANH, C_LEAKYRELU, C_EXP, C_ROUND, C_CLIP, C_DIV_BY,
+    C_HARD_SWISH,  // x * HardSigmoid(x): what may follow a chain
 };
 
 struct Step {
@@ -89,6 +90,7 @@ __device__ __forceinline__ float apply(uint32_t code, float a, float b, float al
     case C_EXP: return expf(a);
     case C_ROUND: return rintf(a);
     case C_CLIP: return clip_elem(a, alpha, beta);
+    case C_HARD_SWISH: return hard_sigmoid_elem(a, alpha, beta) * a;
     default: return a / alpha;  // C_DIV_BY
     }
 }
@@ -152,6 +154,7 @@ template <int VEC> __device__ __forceinline__ void run_steps(const Program &prog
             ALTIUS_STEP(C_EXP)
             ALTIUS_STEP(C_ROUND)
             ALTIUS_STEP(C_CLIP)
+            ALTIUS_STEP(C_HARD_SWISH)
         default:
 #pragma unroll
             for (int j = 0; j < VEC; j++) file[ACC_SLOT * VEC + j] = apply(C_DIV_BY, a[j], b[j], st.alpha, st.beta);
@@ -228,6 +231,14 @@ using AddAddChain = Chain<3, 3, S<C_ADD, 0, 1>, S<C_ADD, ACC, 2>>;
 using SiluChain = Chain<1, 1, S<C_SIGMOID, 0>, S<C_MUL, ACC, 0>>;
 // x * HardSigmoid(x)  (hard swish)
 using HardSwishChain = Chain<1, 1, S<C_HARDSIGMOID, 0>, S<C_MUL, ACC, 0>>;
+// HardSigmoid(s) * x with one s per plane (squeeze and excite) on (x | s), alone, -> Relu and -> hard swish; on (s, x) in the
+// kernel of one element, which planes of odd extents take.
+using GateChain = Chain<1, 2, S<C_HARDSIGMOID, 1>, S<C_MUL, ACC, 0>>;
+using GateReluChain = Chain<1, 2, S<C_HARDSIGMOID, 1>, S<C_MUL, ACC, 0>, S<C_RELU, ACC>>;
+using GateHardSwishChain = Chain<1, 2, S<C_HARDSIGMOID, 1>, S<C_MUL, ACC, 0>, S<C_HARD_SWISH, ACC>>;
+using OddGateChain = Chain<0, 2, S<C_HARDSIGMOID, 0>, S<C_MUL, ACC, 1>>;
+using OddGateReluChain = Chain<0, 2, S<C_HARDSIGMOID, 0>, S<C_MUL, ACC, 1>, S<C_RELU, ACC>>;
+using OddGateHardSwishChain = Chain<0, 2, S<C_HARDSIGMOID, 0>, S<C_MUL, ACC, 1>, S<C_HARD_SWISH, ACC>>;
 
 // Four consecutive output elements per lane.  The host guarantees that the innermost extent is a
 // multiple of 4 (the four elements share a row), that the operands in slots [0, n_vec) have innermost
@@ -274,6 +285,7 @@ __global__ __launch_bounds__(BLOCK) void fused_elemwise_vec4(float *__restrict__
 }
 
 // One element per lane: any innermost extent, any strides, any alignment.
+template <class CHAIN>
 __global__ __launch_bounds__(BLOCK) void fused_elemwise_scalar(float *__restrict__ out, const Program prog) {
     const uint32_t i = blockIdx.x * BLOCK + threadIdx.x;
     if (i >= prog.total) return;
@@ -296,7 +308,7 @@ __global__ __launch_bounds__(BLOCK) void fused_elemwise_scalar(float *__restrict
         }
     }
     float acc[1] = {0.0f};
-    run_steps<1>(prog, in, acc);
+    CHAIN::template run<1>(prog, in, acc);
     out[i] = acc[0];
 }
 
@@ -313,13 +325,21 @@ template <class CHAIN> bool try_static(hipStream_t s, dim3 grid, bool nt, float 
     return true;
 }
 
+template <class CHAIN> bool try_static_scalar(hipStream_t s, dim3 grid, float *out, const Program &prog) {
+    if (!CHAIN::matches(prog)) return false;
+    hipLaunchKernelGGL(fused_elemwise_scalar<CHAIN>, grid, dim3(BLOCK), 0, s, out, prog);
+    return true;
+}
+
 }  // namespace
 
 int launch_fused_elemwise(DeviceCtx &ctx, float *out, int rank, const int64_t *out_dims, int n_inputs, const float *const *inputs,
-                          const int64_t *const *input_strides, int n_steps, const ahip_fused_step *steps) {
+                          const int64_t *const *input_strides, int n_steps, const ahip_fused_step *steps, const GemmPost *then) {
     if (rank < 0 || rank > MAX_RANK) return ctx.fail(AHIP_ERR_ARG, "fused: rank out of range");
     if (n_inputs < 1 || n_inputs > MAX_IN) return ctx.fail(AHIP_ERR_UNSUPPORTED, "fused: between 1 and 6 operands are supported");
-    if (n_steps < 1 || n_steps > MAX_STEPS) return ctx.fail(AHIP_ERR_UNSUPPORTED, "fused: between 1 and 16 steps are supported");
+    const int then_steps = then ? 1 : 0;
+    if (then && then->act != ACT_HARD_SWISH) return ctx.fail(AHIP_ERR_UNSUPPORTED, "fused: only a hard swish can follow the chain in its kernel");
+    if (n_steps < 1 || n_steps > MAX_STEPS - then_steps) return ctx.fail(AHIP_ERR_UNSUPPORTED, "fused: between 1 and 16 steps are supported");
     if ((rank > 0 && !out_dims) || !inputs || !input_strides || !steps) return ctx.fail(AHIP_ERR_ARG, "fused: null argument");
     size_t total = 1;
     for (int i = 0; i < rank; i++) {
@@ -360,6 +380,10 @@ int launch_fused_elemwise(DeviceCtx &ctx, float *out, int rank, const int64_t *o
             if (!sel(s.rhs, &d.rhs)) return ctx.fail(AHIP_ERR_ARG, "fused: bad operand selector");
             d.code = s.op == AHIP_POW && s.pow_scalar_exponent ? (uint32_t)C_POW_SCALAR_EXP : (uint32_t)(C_ADD + s.op);
         }
+    }
+    if (then) {
+        prog.steps[n_steps] = Step{C_HARD_SWISH, ACC, ACC, then->alpha, then->beta};
+        n_steps++;
     }
     for (int t = n_steps; t < MAX_STEPS; t++) prog.steps[t] = Step{C_ADD, ACC, ACC, 0.0f, 0.0f};
     // a + b and a * b have the bits of b + a and b * a: keep the previous result on the left.
@@ -453,11 +477,15 @@ int launch_fused_elemwise(DeviceCtx &ctx, float *out, int rank, const int64_t *o
                             try_static<NormaliseScaleShiftChain>(s, grid, nt, out, prog) || try_static<MulAddChain>(s, grid, nt, out, prog) ||
                             try_static<AddReluChain>(s, grid, nt, out, prog) || try_static<AddGeluChain>(s, grid, nt, out, prog) ||
                             try_static<AddAddChain>(s, grid, nt, out, prog) || try_static<SiluChain>(s, grid, nt, out, prog) ||
-                            try_static<HardSwishChain>(s, grid, nt, out, prog));
+                            try_static<HardSwishChain>(s, grid, nt, out, prog) || try_static<GateChain>(s, grid, nt, out, prog) ||
+                            try_static<GateReluChain>(s, grid, nt, out, prog) || try_static<GateHardSwishChain>(s, grid, nt, out, prog));
         if (!fixed) launch_vec4<AnyChain>(s, grid, nt, out, prog);
     } else {
         const dim3 grid((unsigned)((total + BLOCK - 1) / BLOCK));
-        hipLaunchKernelGGL(fused_elemwise_scalar, grid, dim3(BLOCK), 0, ctx.stream, out, prog);
+        hipStream_t s = ctx.stream;
+        const bool fixed = ctx.fused_static_chains && (try_static_scalar<OddGateChain>(s, grid, out, prog) || try_static_scalar<OddGateReluChain>(s, grid, out, prog) ||
+                                                       try_static_scalar<OddGateHardSwishChain>(s, grid, out, prog));
+        if (!fixed) hipLaunchKernelGGL(fused_elemwise_scalar<AnyChain>, grid, dim3(BLOCK), 0, s, out, prog);
     }
     return ctx.check(hipGetLastError(), "fused launch");
 }

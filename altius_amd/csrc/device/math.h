@@ -6,6 +6,7 @@
 #pragma once
 
 #include "common.h"
+#include "ctx.h"
 
 namespace altius {
 namespace dev {
@@ -145,6 +146,15 @@ __device__ __forceinline__ float relu_elem(float x) { return x > 0.0f ? x : 0.0f
 
 // Op::LeakyReLU (session.rs:819): alpha * x below zero, x otherwise (NaN and -0.0 pass through).
 __device__ __forceinline__ float leaky_relu_elem(float x, float alpha) { return x < 0.0f ? alpha * x : x; }
+
+// What a product or a convolution applies to a value before storing it (GemmPost::act).
+__device__ __forceinline__ float activation(float v, int act, float alpha, float beta) {
+    if (act == AHIP_GELU) return gelu_elem(v);
+    if (act == AHIP_RELU) return relu_elem(v);
+    if (act == AHIP_HARDSIGMOID) return hard_sigmoid_elem(v, alpha, beta);
+    if (act == ACT_HARD_SWISH) return hard_sigmoid_elem(v, alpha, beta) * v;
+    return v;
+}
 
 // Op::Clip: min(max(x, lo), hi) as ONNX defines it; the reference interpreter has no kernel
 // (session.rs:201).  NaN stays NaN.

@@ -69,13 +69,8 @@ struct GemmArgs {
     int *counters;
     float alpha, beta;
     int act;
+    float act_alpha, act_beta;
 };
-
-__device__ __forceinline__ float activation(float v, int act) {
-    if (act == AHIP_GELU) return dev::gelu_elem(v);
-    if (act == AHIP_RELU) return dev::relu_elem(v);
-    return v;
-}
 
 // Four floats that blocks on any XCD read and write.
 struct Halves {
@@ -323,7 +318,9 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_f32_tiles(GemmArgs g) 
 
     // Epilogue, TA passes of PASS_ROWS rows: accumulator e of lane l is row 8 (e / 4) + 4 (l / 32) + e % 4, column l % 32 of its
     // tile; through LDS the WK sums of an element meet and rows of C are stored 16 bytes per lane.
-    float *c = g.c + (size_t)zo * g.c_bs + (size_t)zi * g.c_bs2;
+    const size_t c_at = (size_t)zo * g.c_bs + (size_t)zi * g.c_bs2;
+    float *c = g.c + c_at;
+    const float *residual = g.residual ? g.residual + c_at : nullptr;
     constexpr int PIECES = PASS_ROWS * BN / 4 / THREADS;  // per thread and pass
     static_assert(PIECES * THREADS * 4 == PASS_ROWS * BN, "whole pieces");
     // A thread's pieces lie in the same columns: a bias row is read once.
@@ -349,18 +346,26 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_f32_tiles(GemmArgs g) 
                 const f32x4 x = {q[0], q[g.c0_cs], q[2 * (size_t)g.c0_cs], q[3 * (size_t)g.c0_cs]};
                 v += g.beta * x;
             }
-            if (g.act) {
+            if (g.act) {  // one look at act for the four
+                auto each4 = [&](auto f) __attribute__((always_inline)) {
 #pragma unroll
-                for (int e = 0; e < 4; e++) v[e] = activation(v[e], g.act);
+                    for (int e = 0; e < 4; e++) v[e] = f(v[e]);
+                };
+                if (g.act == AHIP_GELU) each4([](float x) { return dev::gelu_elem(x); });
+                else if (g.act == AHIP_RELU) each4([](float x) { return dev::relu_elem(x); });
+                else each4([&](float x) {
+                    const float s = dev::hard_sigmoid_elem(x, g.act_alpha, g.act_beta);
+                    return g.act == ACT_HARD_SWISH ? s * x : s;
+                });
             }
-            if (g.residual) v += *reinterpret_cast<const dev::v4f_dword *>(g.residual + at);
+            if (residual) v += *reinterpret_cast<const dev::v4f_dword *>(residual + at);
             *reinterpret_cast<dev::v4f_dword *>(c + at) = v;
         } else {
             for (uint32_t e = 0; e < w; e++) {
                 float x = e == 0 ? v.x : e == 1 ? v.y : v.z;
                 if (g.c0 && !bias) x += g.beta * g.c0[(size_t)row * g.c0_rs + (size_t)(col + e) * g.c0_cs];
-                x = activation(x, g.act);
-                if (g.residual) x += g.residual[at + e];
+                x = dev::activation(x, g.act, g.act_alpha, g.act_beta);
+                if (residual) x += residual[at + e];
                 c[at + e] = x;
             }
         }
@@ -503,9 +508,12 @@ static int launch_gemm_far_rows(DeviceCtx &ctx, int axis, size_t part, float *c,
     if (axis == 2 && batch_outer * batch_inner > 1) {  // C0 of the second part on is C, which has batches of its own
         for (size_t z = 0; z < batch_outer * batch_inner; z++) {
             const size_t zo = z / batch_inner, zi = z % batch_inner;
+            GemmPost p;
+            if (post) p = *post;
+            if (p.residual) p.residual += zo * c_bs[0] + zi * c_bs[1];
             const int rc = launch_gemm_far_rows(ctx, axis, part, c + zo * c_bs[0] + zi * c_bs[1], a + zo * a_bs[0] + zi * a_bs[1],
                                                 b + zo * b_bs[0] + zi * b_bs[1], c0, 1, 1, m, n, k, trans_a, trans_b, lda, ldb, ldc, none, none, none,
-                                                c0_rs, c0_cs, alpha, beta, post);
+                                                c0_rs, c0_cs, alpha, beta, post ? &p : nullptr);
             if (rc) return rc;
         }
         return AHIP_OK;
@@ -556,9 +564,8 @@ int launch_gemm_f32(DeviceCtx &ctx, float *c, const float *a, const float *b, co
     if (batch == 0 || m == 0 || n == 0) return AHIP_OK;
     if (!c || (k && (!a || !b))) return ctx.fail(AHIP_ERR_ARG, "gemm: null pointer");
     const bool has_post = post && (post->act != 0 || post->residual);
-    if (has_post && batch != 1) return ctx.fail(AHIP_ERR_UNSUPPORTED, "gemm: an activation or a residual needs a single batch");
-    if (has_post && post->act != 0 && post->act != AHIP_GELU && post->act != AHIP_RELU)
-        return ctx.fail(AHIP_ERR_UNSUPPORTED, "gemm: only Gelu and Relu can follow the product in its kernel");
+    if (has_post && post->act != 0 && post->act != AHIP_GELU && post->act != AHIP_RELU && post->act != AHIP_HARDSIGMOID && post->act != ACT_HARD_SWISH)
+        return ctx.fail(AHIP_ERR_UNSUPPORTED, "gemm: not an activation that can follow the product in its kernel");
     const size_t lim = (size_t)1 << 31;
     if (m >= lim || n >= lim || k >= lim || lda >= lim || ldb >= lim || ldc >= lim || m * ldc >= ((size_t)1 << 40))
         return ctx.fail(AHIP_ERR_UNSUPPORTED, "gemm: extent above 2^31");
@@ -603,6 +610,7 @@ int launch_gemm_f32(DeviceCtx &ctx, float *c, const float *a, const float *b, co
     g.beta = beta;
     g.act = has_post ? post->act : 0;
     g.residual = has_post ? post->residual : nullptr;
+    g.act_alpha = has_post ? post->alpha : 0.0f, g.act_beta = has_post ? post->beta : 0.0f;
     // 16-byte loads: every piece aligned, and whole inside its row.
     auto vec = [&](const float *p, size_t contiguous, size_t ld, const size_t bs[2]) {
         return aligned16(p) && contiguous % 4 == 0 && ld % 4 == 0 && bs[0] % 4 == 0 && bs[1] % 4 == 0;

@@ -127,8 +127,14 @@ __device__ __forceinline__ float peeled_fold(const float *__restrict__ x, size_t
     return OP::apply(acc, strided_fold<OP, 4, NT>(x, begin + head, end, tid, nthreads));
 }
 
+// What is written of a sum: the sum, times `scale` (a mean, which multiplies by the reciprocal) or divided by it (an average pool).
+enum Scaled { AS_IS, MULTIPLIED, DIVIDED };
+template <int SCALE> __device__ __forceinline__ float scaled(float sum, float scale) {
+    return SCALE == MULTIPLIED ? sum * scale : SCALE == DIVIDED ? sum / scale : sum;
+}
+
 // VEC: 4 = rows of whole float4s on 16-byte boundaries, 0 = rows that start anywhere (peeled_fold), 1 = single elements.
-template <class OP, int VEC, bool SCALE, bool NT>
+template <class OP, int VEC, int SCALE, bool NT>
 __global__ __launch_bounds__(ROW_BLOCK) void reduce_rows_wave(float *__restrict__ out,
                                                               const float *__restrict__ in, size_t outer,
                                                               size_t red, float scale) {
@@ -137,14 +143,14 @@ __global__ __launch_bounds__(ROW_BLOCK) void reduce_rows_wave(float *__restrict_
     if (row >= outer) return;
     float acc = VEC == 0 ? peeled_fold<OP, NT>(in + row * red, 0, red, lane, WAVE) : strided_fold<OP, VEC == 0 ? 1 : VEC, NT>(in + row * red, 0, red, lane, WAVE);
     acc = wave_reduce<OP>(acc);
-    if (lane == 0) out[row] = SCALE ? acc * scale : acc;
+    if (lane == 0) out[row] = scaled<SCALE>(acc, scale);
 }
 
 // Rows of 4 to 256 elements that are whole float4s: SUB = 1 to 64 lanes per row, one 16-byte load per lane, so a
 // wavefront's load is one contiguous piece of the tensor holding 64 / SUB whole rows (lanes past the row's last
 // float4 idle when the float4 count is not a power of two).  Each wavefront takes U such pieces, all loads requested
 // before the first is folded.
-template <class OP, int SUB, int U, bool SCALE, bool NT>
+template <class OP, int SUB, int U, int SCALE, bool NT>
 __global__ __launch_bounds__(ROW_BLOCK) void reduce_rows_sub4(float *__restrict__ out, const float *__restrict__ in, size_t outer,
                                                               uint32_t red, float scale) {
     constexpr int RPP = WAVE / SUB;  // rows per wavefront pass
@@ -165,13 +171,13 @@ __global__ __launch_bounds__(ROW_BLOCK) void reduce_rows_sub4(float *__restrict_
         const size_t row = row0 + (size_t)u * RPP;
         float acc = OP::apply(OP::apply(v[u].x, v[u].y), OP::apply(v[u].z, v[u].w));
         if (SUB > 1) acc = subwave_allreduce<OP, SUB < 4 ? 4 : SUB>(acc);
-        if (s == 0 && row < outer) out[row] = SCALE ? acc * scale : acc;
+        if (s == 0 && row < outer) out[row] = scaled<SCALE>(acc, scale);
     }
 }
 
 // grid = (splits, outer).  Block (s, o) folds chunk s of row o into
 // dst[o * splits + s].
-template <class OP, int VEC, bool SCALE, bool NT = false>
+template <class OP, int VEC, int SCALE, bool NT = false>
 __global__ __launch_bounds__(ROW_BLOCK) void reduce_rows_block(float *__restrict__ dst,
                                                                const float *__restrict__ in, size_t red,
                                                                size_t chunk, float scale) {
@@ -185,7 +191,7 @@ __global__ __launch_bounds__(ROW_BLOCK) void reduce_rows_block(float *__restrict
         acc = VEC == 0 ? peeled_fold<OP, NT>(in + o * red, begin, end, threadIdx.x, ROW_BLOCK)
                        : strided_fold<OP, VEC == 0 ? 1 : VEC, NT>(in + o * red, begin, end, threadIdx.x, ROW_BLOCK);
     acc = block_reduce<OP, ROW_WAVES>(acc, lds);
-    if (threadIdx.x == 0) dst[o * gridDim.x + s] = SCALE ? acc * scale : acc;
+    if (threadIdx.x == 0) dst[o * gridDim.x + s] = scaled<SCALE>(acc, scale);
 }
 
 // ---------------------------------------------------------------------------
@@ -513,7 +519,7 @@ inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 
 constexpr size_t MAX_GRID_X = 0x7FFFFFFFu;
 constexpr size_t MAX_GRID_Y = 65535;
 
-template <class OP, bool SCALE>
+template <class OP, int SCALE>
 void rows_wave_launch(hipStream_t s, float *out, const float *in, size_t outer, size_t red, float scale,
                       bool nt = false) {
     const bool vec4 = (red % 4 == 0) && aligned16(in);
@@ -535,7 +541,7 @@ void rows_wave_launch(hipStream_t s, float *out, const float *in, size_t outer, 
                            in, outer, red, scale);
 }
 
-template <class OP, bool SCALE>
+template <class OP, int SCALE>
 void rows_block_launch(hipStream_t s, float *dst, const float *in, size_t outer, size_t red, size_t splits,
                        size_t chunk, float scale, bool nt = false) {
     // Chunks start 16-byte aligned when the row pitch and the chunk length are multiples of 4.
@@ -665,62 +671,67 @@ size_t sub4_blocks(size_t outer, size_t red) {
     return (outer + per_block - 1) / per_block;
 }
 
+// Trailing axes: [outer, red] -> [outer].
+template <class OP, int SCALE>
+int reduce_rows(DeviceCtx &ctx, const Partials &pt, float *out, const float *in, size_t outer, size_t red, float scale) {
+    hipStream_t s = ctx.stream;
+    const RowsBy by = reduce_rows_by(in, outer, red);
+    if (by == RowsBy::Lanes) {
+        constexpr int U = SUB4_UNROLL;
+        const int sub = sub4_lanes(red);
+        const bool nt = ctx.streaming(outer * red * sizeof(float));
+        const dim3 grid((unsigned)sub4_blocks(outer, red)), block(ROW_BLOCK);
+#define ALTIUS_SUB4(SUBV)                                                                                                          \
+do {                                                                                                                           \
+    if (nt) hipLaunchKernelGGL((reduce_rows_sub4<OP, SUBV, U, SCALE, true>), grid, block, 0, s, out, in, outer, (uint32_t)red, scale);  \
+    else hipLaunchKernelGGL((reduce_rows_sub4<OP, SUBV, U, SCALE, false>), grid, block, 0, s, out, in, outer, (uint32_t)red, scale);    \
+} while (0)
+        switch (sub) {
+        case 4: ALTIUS_SUB4(4); break;
+        case 8: ALTIUS_SUB4(8); break;
+        case 16: ALTIUS_SUB4(16); break;
+        case 32: ALTIUS_SUB4(32); break;
+        default: ALTIUS_SUB4(64); break;
+        }
+#undef ALTIUS_SUB4
+        return ctx.check(hipGetLastError(), "reduce rows (lane groups) launch");
+    }
+    if (by == RowsBy::LdsGroups) return launch_reduce_rows_lds(ctx, std::is_same<OP, MaxOp>::value, out, in, outer, red, scale, SCALE);
+    if (by == RowsBy::Wavefront) {
+        if ((outer + ROW_WAVES - 1) / ROW_WAVES > MAX_GRID_X)
+            return ctx.fail(AHIP_ERR_UNSUPPORTED, "reduce: too many rows for one launch");
+        rows_wave_launch<OP, SCALE>(s, out, in, outer, red, scale, ctx.streaming(outer * red * sizeof(float)));
+        return ctx.check(hipGetLastError(), "reduce rows (wave) launch");
+    }
+    if (outer > MAX_GRID_Y) return ctx.fail(AHIP_ERR_UNSUPPORTED, "reduce: too many rows for one launch");
+    // Aim for a few thousand blocks; every block gets at least 4096 elements.
+    size_t splits = 1;
+    if (outer < 1024) {
+        splits = (4096 + outer - 1) / outer;
+        const size_t max_splits = (red + 4095) / 4096;
+        if (splits > max_splits) splits = max_splits;
+        if (splits < 1) splits = 1;
+    }
+    size_t chunk = (red + splits - 1) / splits;
+    chunk = (chunk + 1023) / 1024 * 1024;
+    splits = (red + chunk - 1) / chunk;
+    const bool nt = ctx.streaming(outer * red * sizeof(float));
+    if (splits == 1) {
+        rows_block_launch<OP, SCALE>(s, out, in, outer, red, 1, chunk, scale, nt);
+        return ctx.check(hipGetLastError(), "reduce rows (block) launch");
+    }
+    if (outer * splits > pt.floats) return partials_too_small(ctx, outer * splits, pt);
+    if (int rc = claim_partials(ctx, pt)) return rc;
+    rows_block_launch<OP, AS_IS>(s, pt.ptr, in, outer, red, splits, chunk, 1.0f, nt);
+    rows_wave_launch<OP, SCALE>(s, out, pt.ptr, outer, splits, scale);
+    return ctx.check(hipGetLastError(), "reduce rows (two-stage) launch");
+}
+
 template <class OP, bool SCALE>
 int reduce_impl(DeviceCtx &ctx, const Partials &pt, float *out, const float *in, size_t outer, size_t red, size_t inner,
                 float scale) {
     hipStream_t s = ctx.stream;
-    if (inner == 1) {
-        const RowsBy by = reduce_rows_by(in, outer, red);
-        if (by == RowsBy::Lanes) {
-            constexpr int U = SUB4_UNROLL;
-            const int sub = sub4_lanes(red);
-            const bool nt = ctx.streaming(outer * red * sizeof(float));
-            const dim3 grid((unsigned)sub4_blocks(outer, red)), block(ROW_BLOCK);
-#define ALTIUS_SUB4(SUBV)                                                                                                          \
-    do {                                                                                                                           \
-        if (nt) hipLaunchKernelGGL((reduce_rows_sub4<OP, SUBV, U, SCALE, true>), grid, block, 0, s, out, in, outer, (uint32_t)red, scale);  \
-        else hipLaunchKernelGGL((reduce_rows_sub4<OP, SUBV, U, SCALE, false>), grid, block, 0, s, out, in, outer, (uint32_t)red, scale);    \
-    } while (0)
-            switch (sub) {
-            case 4: ALTIUS_SUB4(4); break;
-            case 8: ALTIUS_SUB4(8); break;
-            case 16: ALTIUS_SUB4(16); break;
-            case 32: ALTIUS_SUB4(32); break;
-            default: ALTIUS_SUB4(64); break;
-            }
-#undef ALTIUS_SUB4
-            return ctx.check(hipGetLastError(), "reduce rows (lane groups) launch");
-        }
-        if (by == RowsBy::LdsGroups) return launch_reduce_rows_lds(ctx, std::is_same<OP, MaxOp>::value, out, in, outer, red, scale, SCALE);
-        if (by == RowsBy::Wavefront) {
-            if ((outer + ROW_WAVES - 1) / ROW_WAVES > MAX_GRID_X)
-                return ctx.fail(AHIP_ERR_UNSUPPORTED, "reduce: too many rows for one launch");
-            rows_wave_launch<OP, SCALE>(s, out, in, outer, red, scale, ctx.streaming(outer * red * sizeof(float)));
-            return ctx.check(hipGetLastError(), "reduce rows (wave) launch");
-        }
-        if (outer > MAX_GRID_Y) return ctx.fail(AHIP_ERR_UNSUPPORTED, "reduce: too many rows for one launch");
-        // Aim for a few thousand blocks; every block gets at least 4096 elements.
-        size_t splits = 1;
-        if (outer < 1024) {
-            splits = (4096 + outer - 1) / outer;
-            const size_t max_splits = (red + 4095) / 4096;
-            if (splits > max_splits) splits = max_splits;
-            if (splits < 1) splits = 1;
-        }
-        size_t chunk = (red + splits - 1) / splits;
-        chunk = (chunk + 1023) / 1024 * 1024;
-        splits = (red + chunk - 1) / chunk;
-        const bool nt = ctx.streaming(outer * red * sizeof(float));
-        if (splits == 1) {
-            rows_block_launch<OP, SCALE>(s, out, in, outer, red, 1, chunk, scale, nt);
-            return ctx.check(hipGetLastError(), "reduce rows (block) launch");
-        }
-        if (outer * splits > pt.floats) return partials_too_small(ctx, outer * splits, pt);
-        if (int rc = claim_partials(ctx, pt)) return rc;
-        rows_block_launch<OP, false>(s, pt.ptr, in, outer, red, splits, chunk, 1.0f, nt);
-        rows_wave_launch<OP, SCALE>(s, out, pt.ptr, outer, splits, scale);
-        return ctx.check(hipGetLastError(), "reduce rows (two-stage) launch");
-    }
+    if (inner == 1) return reduce_rows<OP, SCALE ? MULTIPLIED : AS_IS>(ctx, pt, out, in, outer, red, scale);
 
     // inner > 1
     if (red >= ((size_t)1 << 32) || inner >= ((size_t)1 << 31))
@@ -857,6 +868,13 @@ RowsBy reduce_rows_by(const float *in, size_t rows, size_t len) {
 int launch_reduce(DeviceCtx &ctx, int kind, float *out, const float *in, size_t outer, size_t red,
                   size_t inner) {
     return reduce_with(ctx, Partials{ctx.scratch, ctx.scratch_floats, false}, kind, out, in, outer, red, inner);
+}
+
+int launch_average_pool(DeviceCtx &ctx, float *out, const float *in, size_t planes, size_t area) {
+    if (planes == 0) return AHIP_OK;
+    if (area == 0) return ctx.fail(AHIP_ERR_ARG, "average pool: empty plane");
+    if (!out || !in) return ctx.fail(AHIP_ERR_ARG, "average pool: null tensor pointer");
+    return reduce_rows<SumOp, DIVIDED>(ctx, Partials{ctx.scratch, ctx.scratch_floats, false}, out, in, planes, area, (float)area);
 }
 
 int reduce_static_setup(int device) {

@@ -429,7 +429,8 @@ __global__ __launch_bounds__(BT, 8) void layernorm_lds(float *__restrict__ out, 
 // wavefront per row would leave most lanes idle and read 4 bytes per lane.  Same staging as softmax_lds: a
 // line-aligned group of rows goes to LDS with 16-byte loads, then SUB lanes fold each row and lane 0 of the group
 // writes out[row] (times `scale` for a mean).
-template <int BT, int ST, class OP, int SUB, bool SCALE, bool NT>
+// SCALE: 1 times `scale` (a mean), 2 divided by it (an average pool).
+template <int BT, int ST, class OP, int SUB, int SCALE, bool NT>
 __global__ __launch_bounds__(BT) void reduce_rows_lds(float *__restrict__ out, const float *__restrict__ in, size_t rows,
                                                              int len, int group_rows, float scale) {
     extern __shared__ __align__(16) float lds[];
@@ -472,7 +473,7 @@ __global__ __launch_bounds__(BT) void reduce_rows_lds(float *__restrict__ out, c
         float acc = OP::identity();
         for (int k = s; k < len; k += SUB) acc = OP::apply(acc, row[k]);
         acc = subwave_allreduce<OP, SUB>(acc);
-        if (s == 0 && r0 + rr < nrows) out[row0 + r] = SCALE ? acc * scale : acc;
+        if (s == 0 && r0 + rr < nrows) out[row0 + r] = SCALE == 1 ? acc * scale : SCALE == 2 ? acc / scale : acc;
     }
 }
 
@@ -1679,7 +1680,7 @@ bool reduce_rows_lds_fits(const float *in, size_t rows, size_t len) {
     return (g * len) % 4 == 0 && (rows + g - 1) / g <= 0x7FFFFFFFu;  // groups must start 16-byte aligned
 }
 
-int launch_reduce_rows_lds(DeviceCtx &ctx, bool is_max, float *out, const float *in, size_t rows, size_t len, float scale, bool scaled) {
+int launch_reduce_rows_lds(DeviceCtx &ctx, bool is_max, float *out, const float *in, size_t rows, size_t len, float scale, int scaled) {
     if (!reduce_rows_lds_fits(in, rows, len)) return ctx.fail(AHIP_ERR_UNSUPPORTED, "reduce: not rows the kernel takes");
     constexpr int RT = REDUCE_LDS_THREADS;
     const bool deep = reduce_lds_deep(len);
@@ -1697,9 +1698,10 @@ int launch_reduce_rows_lds(DeviceCtx &ctx, bool is_max, float *out, const float 
     } while (0)
 #define ALTIUS_RED_SUB(SUB)                                   \
     do {                                                      \
-        if (is_max) ALTIUS_RED(MaxOp, SUB, false);            \
-        else if (scaled) ALTIUS_RED(SumOp, SUB, true);        \
-        else ALTIUS_RED(SumOp, SUB, false);                   \
+        if (is_max) ALTIUS_RED(MaxOp, SUB, 0);                \
+        else if (scaled == 2) ALTIUS_RED(SumOp, SUB, 2);      \
+        else if (scaled) ALTIUS_RED(SumOp, SUB, 1);           \
+        else ALTIUS_RED(SumOp, SUB, 0);                       \
     } while (0)
     if (len <= 64 && len % 8 != 0) ALTIUS_RED_SUB(4);
     else if (len <= 128) ALTIUS_RED_SUB(8);

@@ -298,7 +298,7 @@ bool HipSession::run(const std::vector<Tensor> &inputs, std::vector<Tensor> *out
     std::map<ValueId, DeviceTensor> values;
     copies_avoided_ = 0;
     pending_attn_.clear();
-    absorbed_add_.clear();
+    absorbed_.clear();
     passed_over_.clear();
     std::vector<hipEvent_t> events;
     // Nothing may still read a block when it goes back to the pool for another run, and input
@@ -402,7 +402,7 @@ bool HipSession::run_device(const std::vector<DeviceTensor> &inputs, std::vector
     std::map<ValueId, DeviceTensor> values;
     copies_avoided_ = 0;
     pending_attn_.clear();
-    absorbed_add_.clear();
+    absorbed_.clear();
     passed_over_.clear();
     for (size_t i = 0; i < g.inputs.size(); i++) {
         if (!inputs[i].ptr && inputs[i].nbytes())
@@ -477,7 +477,7 @@ bool HipSession::try_capture(const std::string &key, const std::vector<Tensor> &
     std::map<ValueId, DeviceTensor> values;
     copies_avoided_ = 0;
     pending_attn_.clear();
-    absorbed_add_.clear();
+    absorbed_.clear();
     passed_over_.clear();
     for (size_t i = 0; i < g.inputs.size(); i++) {
         DeviceTensor d;
@@ -687,16 +687,16 @@ bool HipSession::run_node(NodeId id, std::map<ValueId, DeviceTensor> &values, Se
     std::vector<DeviceTensor> outs;
     values_ = &values;
 
-    auto absorbed = absorbed_add_.find(id);
-    if (absorbed != absorbed_add_.end() && absorbed->second < in.size() && in[absorbed->second]) {
-        // The MatMul that produced one operand has added the other one already.
+    auto absorbed = absorbed_.find(id);
+    if (absorbed != absorbed_.end() && absorbed->second < in.size() && in[absorbed->second]) {
+        // The product or convolution that made one operand has added the other one, or normalised its result, already.
         DeviceTensor o = *in[absorbed->second];
-        absorbed_add_.erase(absorbed);
+        absorbed_.erase(absorbed);
         o.dims = shapes[0].dims;
         copies_avoided_++;
         outs.push_back(std::move(o));
-    } else if ((op.kind == OpKind::Gelu || op.kind == OpKind::ReLU) && in[0] && in[0]->applied_op == (op.kind == OpKind::Gelu ? AHIP_GELU : AHIP_RELU)) {
-        // The MatMul that produced the operand has applied this activation already.
+    } else if (in.size() == 1 && in[0] && in[0]->applied_op >= 0 && !is_alias_op(op.kind)) {
+        // The node that made the operand has applied this activation, its only reader, already.
         DeviceTensor o = *in[0];
         o.dims = shapes[0].dims;
         o.applied_op = -1;
@@ -969,9 +969,13 @@ bool HipSession::run_fused_elemwise(const Node &node, const Op &op, const std::v
         }
         std::vector<int64_t> dims;
         for (auto x : out.dims.as_vec()) dims.push_back((int64_t)x);
+        GemmPost then;
+        if (auto cp = chain_post_.find(current_node_); cp != chain_post_.end() && steps.size() < AHIP_FUSED_MAX_STEPS)
+            then.act = cp->second.act, then.alpha = cp->second.alpha, then.beta = cp->second.beta;
         const int rc = launch_fused_elemwise(ctx_, static_cast<float *>(out.ptr), (int)dims.size(), dims.data(), (int)ptrs.size(), ptrs.data(),
-                                             stride_ptrs.data(), (int)steps.size(), steps.data());
+                                             stride_ptrs.data(), (int)steps.size(), steps.data(), then.act ? &then : nullptr);
         if (rc == AHIP_OK) {
+            if (then.act) out.applied_op = then.act;
             outs->push_back(std::move(out));
             return true;
         }
@@ -1017,6 +1021,7 @@ bool HipSession::run_fused_elemwise(const Node &node, const Op &op, const std::v
 GemmPost HipSession::gemm_post(const MatMulPost &mp, const FixedDimensions &product) const {
     GemmPost post;
     post.act = mp.act;
+    post.alpha = mp.alpha, post.beta = mp.beta;
     if (!mp.has_add || !values_) return post;
     const FixedDimensions *dims = &product;
     if (mp.reshaped) {  // the shape under which the Add reads the product
@@ -1297,8 +1302,7 @@ bool HipSession::run_device_op(const Node &node, const Op &op, const std::vector
         const FixedDimensions &d = in[0]->dims;
         const size_t planes = d[0] * d[1], area = d[2] * d[3];
         if (area == 0) return fail(err, SessionError::Shape, "GlobalAveragePool: empty plane");
-        rc = launch_reduce(ctx_, AHIP_REDUCE_SUM, o, f(in[0]), planes, area, 1);
-        if (!rc) rc = launch_unary(ctx_, AHIP_DIV_BY, o, o, planes, (float)area, 0);
+        rc = launch_average_pool(ctx_, o, f(in[0]), planes, area);
         break;
     }
     case OpKind::BatchNormalization: {
@@ -1445,9 +1449,30 @@ bool HipSession::run_device_op(const Node &node, const Op &op, const std::vector
             if (in[2]->elem_ty != TensorElemType::F32 || in[2]->dims.total_elems() != w[0]) return fail(err, SessionError::Shape, "Conv2d: bias must hold one f32 per output channel");
             bias = f(in[2]);
         }
+        ConvPost post;
+        auto mp = matmul_post_.find(current_node_);
+        if (mp != matmul_post_.end()) {
+            bool norm_ok = true;
+            if (mp->second.has_norm) {
+                const Node &bn = model_.graph.nodes[mp->second.norm];
+                const float *p[5] = {};
+                for (size_t k = 1; k < 5; k++) {
+                    auto it = inits_.find(bn.inputs[k]);
+                    if (it != inits_.end() && it->second.elem_ty == TensorElemType::F32 && it->second.dims.total_elems() == w[0]) p[k] = f(&it->second);
+                    norm_ok = norm_ok && p[k];
+                }
+                if (norm_ok) post.scale = p[1], post.shift = p[2], post.mean = p[3], post.var = p[4], post.eps = bn.op.epsilon;
+            }
+            if (norm_ok) post.then = gemm_post(mp->second, out.dims);
+        }
         rc = launch_conv2d(ctx_, o, f(in[0]), f(in[1]), bias, x[0], x[1], x[2], x[3], w[0], out.dims[2], out.dims[3], w[2], w[3],
                            (size_t)op.strides[0], (size_t)op.strides[1], (size_t)op.dilations[0], (size_t)op.dilations[1],
-                           (size_t)op.padding[0], (size_t)op.padding[1], group);
+                           (size_t)op.padding[0], (size_t)op.padding[1], group, &post);
+        if (!rc && post.applied) {
+            if (post.mean) absorbed_[mp->second.norm] = 0;
+            if (post.then.act) out.applied_op = post.then.act;
+            if (post.then.residual) absorbed_[mp->second.add_node] = mp->second.add_input;
+        }
         break;
     }
     case OpKind::MaxPool: {  // compute_max_pool (session.rs:324-382)
@@ -1553,7 +1578,7 @@ bool HipSession::run_device_op(const Node &node, const Op &op, const std::vector
                     rc = launch_gemm_batch2(ctx_, o, f(in[0]), f(in[1]), bias, 1, 1, batch * m, n, k, 0, tb, A.ld, B.ld, n, none, none, none, 0, 1, 1.0f,
                                             beta, &post);
                     if (!rc && post.act) out.applied_op = post.act;
-                    if (!rc && post.residual) absorbed_add_[mp->second.add_node] = mp->second.add_input;
+                    if (!rc && post.residual) absorbed_[mp->second.add_node] = mp->second.add_input;
                     break;
                 }
             }
@@ -1638,7 +1663,7 @@ bool HipSession::run_device_op(const Node &node, const Op &op, const std::vector
                 rc = launch_gemm_batch2(ctx_, o, f(in[0]), f(in[1]), c0, 1, 1, m, n, k, op.trans_a, op.trans_b, a[1], b[1], n, none, none, none, rs, cs,
                                         op.alpha, c0 ? op.beta : 0.0f, &post);
                 if (!rc && post.act) out.applied_op = post.act;
-                if (!rc && post.residual) absorbed_add_[mp->second.add_node] = mp->second.add_input;
+                if (!rc && post.residual) absorbed_[mp->second.add_node] = mp->second.add_input;
                 break;
             }
         }

@@ -102,8 +102,8 @@ struct DeviceTensor {
     // An activation (AHIP_GELU / AHIP_RELU) that has not been applied yet: the tensor holds the
     // activation's input, and its one reader, a MatMul, applies it while splitting the operand.
     int pending_op = -1;
-    // An activation (AHIP_GELU / AHIP_RELU) that the MatMul which produced the tensor has already applied while
-    // writing it: the activation node that follows passes the tensor on.
+    // An activation (AHIP_* or ACT_HARD_SWISH) that the node which produced the tensor has already applied while writing it:
+    // the activation node that follows, its only reader, passes the tensor on.
     int applied_op = -1;
     // The block does not hold fp32 values but the tensor's three bf16 planes, laid out as the first operand of the
     // tall bf16 product that is its only reader; the LayerNormalization that produced the tensor wrote them instead
@@ -259,11 +259,14 @@ private:
     std::map<NodeId, AttentionPlan> attn_head_;                  // first MatMul of a fusable attention -> the rest
     std::set<NodeId> attn_softmax_, attn_tail_;
     std::map<ValueId, PendingAttention> pending_attn_;
-    // What follows a MatMul or a Gemm whose result has one reader and can be done while the product is written (fp32 kernel):
-    // a Gelu / Relu node, or an Add of a tensor of the result's shape (a residual connection); a Gemm's may stand behind the
-    // Reshape that gives it back the axes exporters fold for it.
+    // What follows a MatMul, a Gemm or a Conv2d whose result has one reader and can be done while the result is written (fp32
+    // kernel): an activation, or an Add of a tensor of the result's shape (a residual connection); a Gemm's may stand behind the
+    // Reshape that gives it back the axes exporters fold for it, a Conv2d's behind its BatchNormalization.
     struct MatMulPost {
-        int act = 0;            // AHIP_GELU / AHIP_RELU, 0: none
+        int act = 0;            // AHIP_GELU / AHIP_RELU / AHIP_HARDSIGMOID / ACT_HARD_SWISH, 0: none
+        float alpha = 0.0f, beta = 0.0f;
+        bool has_norm = false;
+        NodeId norm = 0;
         bool has_add = false;
         NodeId add_node = 0;
         size_t add_input = 0;   // which input of the Add is the product
@@ -274,7 +277,10 @@ private:
     // What of a plan can be done for a product of this shape now: nothing, an activation, or a residual of the same shape.
     GemmPost gemm_post(const MatMulPost &mp, const FixedDimensions &product) const;
     std::map<NodeId, MatMulPost> matmul_post_;
-    std::map<NodeId, size_t> absorbed_add_;                     // Add nodes whose sum a MatMul wrote in this run -> input holding it
+    // Element-wise chains whose one reader is a hard swish that their kernel can do.
+    std::map<NodeId, MatMulPost> chain_post_;
+    // Add and BatchNormalization nodes whose result a product or a convolution wrote in this run -> input holding it
+    std::map<NodeId, size_t> absorbed_;
     const std::map<ValueId, DeviceTensor> *values_ = nullptr;   // the running call's values, for run_device_op
     std::set<NodeId> deferred_unary_;                           // Gelu / Relu nodes folded into the MatMul that reads them
     // LayerNormalization -> MatMul(weights) with a single reader: where the product takes the bf16 route the

@@ -284,15 +284,15 @@ void HipSession::plan_views(bool fused_attention) {
         }
         return true;
     };
-    // Product -> Gelu / Relu, or product -> Add(residual): done by the product's own kernel when it is the fp32 one.
-    // v: the product as that node reads it.
+    // Product or convolution -> activation, or -> Add(residual): done by its own kernel when that is an fp32 one.
+    // v: the result as that node reads it.
     auto plan_post = [&](NodeId id, ValueId v, MatMulPost mp) {
         auto it = users.find(v);
         if (it == users.end() || it->second.size() != 1 || is_output(v)) return;
         const NodeId uid = *it->second.begin();
         const Node &u = g.nodes[uid];
-        if ((u.op.kind == OpKind::Gelu || u.op.kind == OpKind::ReLU) && u.inputs.size() == 1 && u.outputs.size() == 1) {
-            mp.act = u.op.kind == OpKind::Gelu ? AHIP_GELU : AHIP_RELU;
+        if (const int act = u.inputs.size() == 1 && u.outputs.size() == 1 ? activation_of(u.op, &mp.alpha, &mp.beta) : 0) {
+            mp.act = act;
             matmul_post_[id] = mp;
         } else if (u.op.kind == OpKind::Add && u.inputs.size() == 2 && u.outputs.size() == 1 && u.inputs[0] != u.inputs[1]) {
             mp.has_add = true;
@@ -340,6 +340,31 @@ void HipSession::plan_views(bool fused_attention) {
                 const Node &add = g.nodes[par->second];
                 if (add.op.kind == OpKind::Add && add.inputs.size() == 2 && add.outputs.size() == 1 && add.inputs[0] != add.inputs[1])
                     add_into_ln_[par->second] = id;
+            }
+        } else if (n.op.kind == OpKind::Conv2d && n.outputs.size() == 1 && !is_output(n.outputs[0])) {
+            MatMulPost mp;
+            ValueId v = n.outputs[0];
+            auto it = users.find(v);
+            if (it == users.end() || it->second.size() != 1) continue;
+            const Node &bn = g.nodes[*it->second.begin()];
+            if (bn.op.kind == OpKind::BatchNormalization && !bn.op.training_mode && bn.inputs.size() == 5 && bn.inputs[0] == v && bn.outputs.size() == 1) {
+                bool constant = true;  // its four parameters are weights
+                for (size_t k = 1; k < 5; k++) constant = constant && bn.inputs[k] != v && g.inits.count(bn.inputs[k]);
+                if (constant) {
+                    mp.has_norm = true;
+                    mp.norm = *it->second.begin();
+                    matmul_post_[id] = mp;
+                    v = bn.outputs[0];
+                }
+            }
+            plan_post(id, v, mp);
+        } else if (n.op.kind == OpKind::FusedElemwise && n.outputs.size() == 1 && !is_output(n.outputs[0])) {
+            auto it = users.find(n.outputs[0]);
+            if (it == users.end() || it->second.size() != 1) continue;
+            MatMulPost mp;
+            if (is_hard_swish(g.nodes[*it->second.begin()].op, &mp.alpha, &mp.beta)) {
+                mp.act = ACT_HARD_SWISH;
+                chain_post_[id] = mp;
             }
         } else if (n.op.kind == OpKind::Gemm && n.outputs.size() == 1) {
             auto it = users.find(n.outputs[0]);

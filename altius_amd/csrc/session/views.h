@@ -37,6 +37,29 @@ inline bool is_alias_op(OpKind k) {
 // Operators that read a strided view in place (or pass it on as another view).
 inline bool reads_views(OpKind k) { return is_alias_op(k) || k == OpKind::MatMul || k == OpKind::Transpose || k == OpKind::Split; }
 
+// x * HardSigmoid(x) fused into one node (hard swish); fills the HardSigmoid's attributes.
+inline bool is_hard_swish(const Op &op, float *alpha, float *beta) {
+    if (op.kind != OpKind::FusedElemwise || !op.fused || op.fused->input_map.size() != 1 || op.fused->chain.size() != 2) return false;
+    const FusedElemwise::Step &s = op.fused->chain[0], &m = op.fused->chain[1];
+    const size_t x = op.fused->input_map[0];
+    if (s.op.kind != OpKind::HardSigmoid || s.inputs.size() != 1 || s.inputs[0] != x || s.outputs.size() != 1 || s.outputs[0] == x) return false;
+    if (m.op.kind != OpKind::Mul || m.inputs.size() != 2) return false;
+    if (!((m.inputs[0] == x && m.inputs[1] == s.outputs[0]) || (m.inputs[1] == x && m.inputs[0] == s.outputs[0]))) return false;
+    *alpha = s.op.alpha, *beta = s.op.beta;
+    return true;
+}
+
+// The activation that a node applies to its one input, as GemmPost::act names it; 0: none that a product or a convolution can do.
+inline int activation_of(const Op &op, float *alpha, float *beta) {
+    switch (op.kind) {
+    case OpKind::Gelu: return AHIP_GELU;
+    case OpKind::ReLU: return AHIP_RELU;
+    case OpKind::HardSigmoid: *alpha = op.alpha, *beta = op.beta; return AHIP_HARDSIGMOID;
+    case OpKind::FusedElemwise: return is_hard_swish(op, alpha, beta) ? ACT_HARD_SWISH : 0;
+    default: return 0;
+    }
+}
+
 inline std::vector<int64_t> dense_strides(const FixedDimensions &dims) {
     std::vector<int64_t> s(dims.len());
     int64_t acc = 1;
