@@ -21,6 +21,9 @@
 // this one takes 450 us (3072 heads of 197 x 64): its staging, products and stores could only add up.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <cmath>
+
 #include "common.h"
 #include "ctx.h"
 #include "math.h"
@@ -539,7 +542,265 @@ __global__ __launch_bounds__(64 * SW, 1) void attention_keysplit_d64(AttnArgs g)
 
 inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
+// ---- the operators' own arithmetic, one kernel --------------------------------------------------------------------------------
+// MatMul -> [one scale] -> [Where] -> Softmax -> MatMul with the bits of the operators run apart: every product is the same MFMA with
+// the same values of k, in chains that add up as the tiles of matmul.hip do (WK of them, each taking 16 values of k in turn, met in
+// order at the end; which tile the product alone would take decides WK), and a row's sum runs as softmax_lds runs it: SUB lanes, each
+// over every SUB th element, met by the same exchanges.  What is gone are the launches between the operators and the scores' way
+// through memory.
+//
+// A block of eight wavefronts owns 32 queries of one head.  S^T = K Q^T, a tile of 32 keys per wavefront and turn; the scores go to
+// LDS ([32][pitch], zeros behind the last key), where the Softmax works on them in place; O = P V reads them back, a wavefront per chain
+// and 32 columns of V, which it reads from memory, and the chains meet in LDS.
+//
+// Calls of a few hundred heads and less are bound by one block's chain of loads and products; us a layer with the operators' kernels and
+// with this one: ROWS_FIGURES.
+struct RowsArgs {
+    const float *q, *k, *v, *mask;
+    const uint8_t *cond;
+    float *o;
+    uint32_t tq, tk, ldq, ldk, ldv, ldo, batch_inner, qtiles, blocks, pitch;
+    uint64_t q_bs[2], k_bs[2], v_bs[2], o_bs[2];
+    // The Where's condition and the mask are broadcast over the scores: strides of outer batch, inner batch, query and key.
+    uint64_t cond_bs[2], mask_bs[2];
+    uint32_t cond_q, cond_k, mask_q, mask_k;
+    int scale_op, softmax_op;  // 0 none, 1 multiply, 2 divide: in front of the Where, and of the mask
+    float scale, softmax_scale, fill;
+};
+
+constexpr size_t ROWS_MAX_KEYS = 448;
+constexpr int RW = 8;                          // wavefronts
+constexpr int ROWS_MEET = 4 * 2 * 16 * 64;     // floats: the chains of O, [WK][column half][element][lane]
+
+// A row of scores in LDS, SUB lanes wide: Softmax in place.
+template <int SUB> __device__ __forceinline__ void softmax_rows(float *scores, uint32_t pitch, int len, int tid) {
+    constexpr int NCH = 16;  // SUB is chosen so that this many chunks reach the row's end
+    const int s = tid % SUB;
+    for (int r = tid / SUB; r < 32; r += 64 * RW / SUB) {
+        float *row = scores + r * pitch + s;
+        const float nan = __builtin_nanf("");
+        float x[NCH], mx = nan;
+#pragma unroll
+        for (int k = 0; k < NCH; k++) {
+            x[k] = s + SUB * k < len ? row[SUB * k] : nan;
+            mx = dev::nanmax(x[k], mx);
+        }
+        mx = dev::subwave_allreduce<dev::MaxOp, SUB>(mx);
+        float sum = 0.0f;
+#pragma unroll
+        for (int k = 0; k < NCH; k++) {
+            x[k] = dev::softmax_exp(x[k], mx);
+            sum += s + SUB * k < len ? x[k] : 0.0f;
+        }
+        sum = dev::subwave_allreduce<dev::SumOp, SUB>(sum);
+        const float recip = 1.0f / sum;
+#pragma unroll
+        for (int k = 0; k < NCH; k++)
+            if (s + SUB * k < len) row[SUB * k] = x[k] * recip;
+    }
+}
+
+template <int WKQ, int WKP>
+__global__ __launch_bounds__(64 * RW, 2) void attention_rows_d64(RowsArgs g, int sub) {
+    extern __shared__ __align__(16) float scores[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 31, lk = lane >> 5;
+    // The blocks of a head, which read the same keys and values, run on one XCD.
+    const uint32_t piece = dev::piece_of_block(blockIdx.x, g.blocks), z = piece / g.qtiles, q0 = (piece - z * g.qtiles) * 32;
+    const uint32_t zo = z / g.batch_inner, zi = z - zo * g.batch_inner;
+    const float *q = g.q + zo * g.q_bs[0] + zi * g.q_bs[1], *k = g.k + zo * g.k_bs[0] + zi * g.k_bs[1], *v = g.v + zo * g.v_bs[0] + zi * g.v_bs[1];
+    float *o = g.o + zo * g.o_bs[0] + zi * g.o_bs[1];
+    // The operands as buffers that end behind their last row: a row behind it is zeros, without a test, and an address is one addition.
+    auto buffer = [](const float *p, uint32_t rows, uint32_t ld) __attribute__((always_inline)) {
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p), 0, (int)(((rows - 1) * ld + 64) * 4u), 0x00020000);
+    };
+    auto load4 = [](__amdgpu_buffer_rsrc_t b, uint32_t at) __attribute__((always_inline)) {
+        return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(b, at, 0, 0));
+    };
+    const __amdgpu_buffer_rsrc_t qb = buffer(q, g.tq, g.ldq), kb = buffer(k, g.tk, g.ldk), vb = buffer(v, g.tk, g.ldv);
+
+    // A half of the wavefront takes d = 8 i + 4 lk + 0 .. 3 in turn.
+    const uint32_t query = min(q0 + lr, g.tq - 1), q_at = (query * g.ldq + 4 * lk) * 4;
+    f32x4 qf[8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) qf[i] = load4(qb, q_at + 32 * i);
+    const uint8_t *cond = g.cond ? g.cond + zo * g.cond_bs[0] + zi * g.cond_bs[1] + (size_t)query * g.cond_q : nullptr;
+    const float *mask = g.mask ? g.mask + zo * g.mask_bs[0] + zi * g.mask_bs[1] + (size_t)query * g.mask_q : nullptr;
+    const uint32_t key_tiles = (g.tk + 31) / 32;
+    for (uint32_t t = wave; t < key_tiles; t += RW) {
+        f32x4 kf[8];
+        const uint32_t k_at = ((32 * t + lr) * g.ldk + 4 * lk) * 4;
+#pragma unroll
+        for (int i = 0; i < 8; i++) kf[i] = load4(kb, k_at + 32 * i);
+        floatx16 chain[WKQ];
+#pragma unroll
+        for (int w = 0; w < WKQ; w++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) chain[w][e] = 0.0f;
+        // Chain w takes d = 16 w .. 16 w + 15 of every 16 WKQ.
+#pragma unroll
+        for (int turn = 0; turn < 4 / WKQ; turn++)
+#pragma unroll
+            for (int i = 0; i < 2; i++)
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+#pragma unroll
+                    for (int w = 0; w < WKQ; w++) {
+                        const int at = 2 * (turn * WKQ + w) + i;
+                        chain[w] = __builtin_amdgcn_mfma_f32_32x32x2f32(kf[at][e], qf[at][e], chain[w], 0, 0, 0);
+                    }
+        floatx16 st = chain[0];
+#pragma unroll
+        for (int w = 1; w < WKQ; w++) st += chain[w];
+        // Element e is the score of query lr with key 32 t + 8 (e / 4) + 4 lk + e % 4.
+        const uint32_t key0 = 32 * t + 4 * lk;
+        auto each = [&](auto f) __attribute__((always_inline)) {
+#pragma unroll
+            for (int e = 0; e < 16; e++) st[e] = f(st[e], key0 + 8 * (e >> 2) + (e & 3));
+        };
+        auto scaled = [&](int op, float by) __attribute__((always_inline)) {
+            if (op == 1) each([&](float x, uint32_t) { return x * by; });
+            else if (op == 2) each([&](float x, uint32_t) { return x / by; });
+        };
+        scaled(g.scale_op, g.scale);
+        if (cond) each([&](float x, uint32_t key) { return cond[(size_t)min(key, g.tk - 1) * g.cond_k] ? x : g.fill; });
+        scaled(g.softmax_op, g.softmax_scale);
+        if (mask) each([&](float x, uint32_t key) { return x + mask[(size_t)min(key, g.tk - 1) * g.mask_k]; });
+        each([&](float x, uint32_t key) { return key < g.tk ? x : 0.0f; });
+#pragma unroll
+        for (int e4 = 0; e4 < 4; e4++)
+            *reinterpret_cast<f32x4 *>(&scores[lr * g.pitch + key0 + 8 * e4]) = f32x4{st[4 * e4], st[4 * e4 + 1], st[4 * e4 + 2], st[4 * e4 + 3]};
+    }
+    // Zeros up to the last whole turn of the chains of O.
+    const uint32_t steps = (g.tk + 16 * WKP - 1) / (16 * WKP);
+    if (tid < 32)
+        for (uint32_t key = key_tiles * 32; key < steps * 16 * WKP; key++) scores[tid * g.pitch + key] = 0.0f;
+
+    // The first values are on their way while the Softmax runs.
+    const int part = wave % WKP, half = wave / WKP;  // the chain, and the columns of V; further wavefronts have none
+    const bool busy = half < 2;
+    const uint32_t v_row = g.ldv * 4, v_at = ((16 * part + 4 * lk) * g.ldv + 32 * (half & 1) + lr) * 4, v_step = 16 * WKP * v_row;
+    float vf[2][8];
+    auto values = [&](float (&to)[8], uint32_t step) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                to[4 * i + e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(vb, v_at + step * v_step + (8 * i + e) * v_row, 0, 0));
+    };
+    if (busy) values(vf[0], 0);
+    __syncthreads();
+    switch (sub) {
+    case 4: softmax_rows<4>(scores, g.pitch, (int)g.tk, tid); break;
+    case 8: softmax_rows<8>(scores, g.pitch, (int)g.tk, tid); break;
+    case 16: softmax_rows<16>(scores, g.pitch, (int)g.tk, tid); break;
+    default: softmax_rows<32>(scores, g.pitch, (int)g.tk, tid); break;
+    }
+    __syncthreads();
+
+    floatx16 acc;
+#pragma unroll
+    for (int e = 0; e < 16; e++) acc[e] = 0.0f;
+    if (busy) {
+        auto multiply = [&](const float (&x)[8], uint32_t step) __attribute__((always_inline)) {
+            const float *row = scores + lr * g.pitch + 16 * (WKP * step + part) + 4 * lk;
+            const f32x4 p0 = *reinterpret_cast<const f32x4 *>(row), p1 = *reinterpret_cast<const f32x4 *>(row + 8);
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(p0[e], x[e], acc, 0, 0, 0);
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(p1[e], x[4 + e], acc, 0, 0, 0);
+        };
+        for (uint32_t step = 0; step < steps; step += 2) {  // values behind the last step are zeros that nobody multiplies
+            values(vf[1], step + 1);
+            multiply(vf[0], step);
+            values(vf[0], step + 2);
+            if (step + 1 < steps) multiply(vf[1], step + 1);
+        }
+    }
+    __syncthreads();  // the probabilities are read: the chains meet where they were
+    if (busy) {
+#pragma unroll
+        for (int e = 0; e < 16; e++) scores[((part * 2 + half) * 16 + e) * 64 + lane] = acc[e];
+    }
+    __syncthreads();
+    // Element e of lane l is query 8 (e / 4) + 4 (l / 32) + e % 4, column l % 32 of its half.
+    const int h = wave >> 2;
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        const int e = 4 * (wave & 3) + u;
+        float x = scores[(h * 16 + e) * 64 + lane];
+#pragma unroll
+        for (int w = 1; w < WKP; w++) x += scores[((w * 2 + h) * 16 + e) * 64 + lane];
+        const uint32_t row = q0 + 8 * (e >> 2) + 4 * lk + (e & 3);
+        if (row < g.tq) o[(size_t)row * g.ldo + 32 * h + lr] = x;
+    }
+}
+
 }  // namespace
+
+// The operators' order of sums, where this kernel has it: both products on the tiles of matmul.hip, uncut, and the rows through
+// softmax_lds.
+static bool rows_order(const DeviceCtx &ctx, size_t batch, size_t tq, size_t tk, int *qk, int *pv, int *lanes) {
+    *qk = gemm_f32_chains(ctx, batch, tq, tk, D), *pv = gemm_f32_chains(ctx, batch, tq, D, tk), *lanes = softmax_lds_lanes(tk);
+    return *qk && *pv && *lanes && *lanes <= 32;
+}
+
+bool attention_rows_fits(const DeviceCtx &ctx, size_t batch, size_t tq, size_t tk) {
+    const size_t lim = (size_t)1 << 31;
+    int qk, pv, lanes;
+    return batch > 1 && tq > 0 && tk > 0 && tk <= ROWS_MAX_KEYS && tq < lim && batch < lim && batch * ((tq + 31) / 32) < lim / 64 &&
+           rows_order(ctx, batch, tq, tk, &qk, &pv, &lanes);
+}
+
+int launch_attention_rows(DeviceCtx &ctx, const AttentionRows &a) {
+    const size_t batch = a.batch_outer * a.batch_inner;
+    if (batch == 0 || a.tq == 0) return AHIP_OK;
+    if (!a.q || !a.k || !a.v || !a.o) return ctx.fail(AHIP_ERR_ARG, "attention: null pointer");
+    const size_t lim = (size_t)1 << 31;
+    int qk = 0, pv = 0, lanes = 0;
+    if (!attention_rows_fits(ctx, batch, a.tq, a.tk) || !rows_order(ctx, batch, a.tq, a.tk, &qk, &pv, &lanes) || a.ldo >= lim || a.cond_strides[2] >= lim ||
+        a.cond_strides[3] >= lim || a.mask_strides[2] >= lim || a.mask_strides[3] >= lim)
+        return ctx.fail(AHIP_ERR_UNSUPPORTED, "attention: a shape that the operators' kernels are left with");
+    // A head's operand is addressed with 32-bit byte offsets, to 192 rows behind its last one.
+    const size_t reach = (size_t)1 << 29;
+    if ((a.tq + 192) * a.ldq >= reach || (a.tk + 192) * a.ldk >= reach || (a.tk + 192) * a.ldv >= reach || a.ldq < 64 || a.ldk < 64 || a.ldv < 64)
+        return ctx.fail(AHIP_ERR_UNSUPPORTED, "attention: a head's rows lie too far apart");
+    RowsArgs g;
+    g.q = a.q, g.k = a.k, g.v = a.v, g.o = a.o, g.mask = a.mask, g.cond = a.cond;
+    g.tq = (uint32_t)a.tq, g.tk = (uint32_t)a.tk;
+    g.ldq = (uint32_t)a.ldq, g.ldk = (uint32_t)a.ldk, g.ldv = (uint32_t)a.ldv, g.ldo = (uint32_t)a.ldo;
+    g.batch_inner = (uint32_t)a.batch_inner;
+    for (int i = 0; i < 2; i++) {
+        g.q_bs[i] = a.q_bs[i], g.k_bs[i] = a.k_bs[i], g.v_bs[i] = a.v_bs[i], g.o_bs[i] = a.o_bs[i];
+        g.cond_bs[i] = a.cond_strides[i], g.mask_bs[i] = a.mask_strides[i];
+    }
+    g.cond_q = (uint32_t)a.cond_strides[2], g.cond_k = (uint32_t)a.cond_strides[3];
+    g.mask_q = (uint32_t)a.mask_strides[2], g.mask_k = (uint32_t)a.mask_strides[3];
+    // Dividing by a power of two is multiplying by its reciprocal, to the bit.
+    auto factor = [](int *op, float *by) {
+        int e;
+        if (*op == 2 && std::fabs(std::frexp(*by, &e)) == 0.5f && e > -100 && e < 100) *op = 1, *by = 1.0f / *by;
+    };
+    g.scale_op = a.scale_op, g.scale = a.scale, g.softmax_op = a.softmax_op, g.softmax_scale = a.softmax_scale, g.fill = a.fill;
+    factor(&g.scale_op, &g.scale), factor(&g.softmax_op, &g.softmax_scale);
+    g.qtiles = (uint32_t)((a.tq + 31) / 32);
+    g.blocks = (uint32_t)(batch * g.qtiles);
+    g.pitch = (uint32_t)((a.tk + 63) / 64 * 64 + 4);  // rows start four banks apart
+    const size_t shmem = std::max<size_t>(32 * g.pitch, ROWS_MEET) * sizeof(float);
+#define ROWS(Q, P) hipLaunchKernelGGL((attention_rows_d64<Q, P>), dim3(g.blocks), dim3(64 * RW), shmem, ctx.stream, g, lanes)
+    switch (10 * qk + pv) {
+    case 44: ROWS(4, 4); break;
+    case 42: ROWS(4, 2); break;
+    case 41: ROWS(4, 1); break;
+    case 24: ROWS(2, 4); break;
+    case 22: ROWS(2, 2); break;
+    case 21: ROWS(2, 1); break;
+    case 14: ROWS(1, 4); break;
+    case 12: ROWS(1, 2); break;
+    default: ROWS(1, 1); break;
+    }
+#undef ROWS
+    return ctx.check(hipGetLastError(), "attention (rows) launch");
+}
 
 // Whether launch_attention would run the kernel that can write O as operand planes: enough (batch, head) pairs for full
 // blocks on a context whose products may take the bf16 route.

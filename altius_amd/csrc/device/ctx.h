@@ -134,6 +134,8 @@ int launch_unary(DeviceCtx &ctx, int op, float *out, const float *in, size_t n, 
 int launch_fused_elemwise(DeviceCtx &ctx, float *out, int rank, const int64_t *out_dims, int n_inputs, const float *const *inputs,
                           const int64_t *const *input_strides, int n_steps, const ahip_fused_step *steps, const GemmPost *then = nullptr);
 int launch_softmax(DeviceCtx &ctx, float *out, const float *in, size_t rows, size_t len);
+// Lanes that add up a row of `len` values where it goes through LDS (lane s takes s, s + lanes, ...); 0: it does not (aligned tensors).
+int softmax_lds_lanes(size_t len);
 // Softmax of (in [*|/] scale) + mask over the last axis; scale_op 0 none / 1 multiply / 2 divide, mask (may be
 // null) holds rows / rows_per_mask rows of len values.  AHIP_ERR_UNSUPPORTED when the geometry needs separate kernels.
 int launch_softmax_prologue(DeviceCtx &ctx, float *out, const float *in, size_t rows, size_t len, int scale_op, float scale,
@@ -200,12 +202,30 @@ int launch_gemm_f32(DeviceCtx &ctx, float *c, const float *a, const float *b, co
                     const size_t b_batch_strides[2], const size_t c_batch_strides[2], size_t c0_row_stride, size_t c0_col_stride, float alpha,
                     float beta, const GemmPost *post = nullptr);
 double gemm_f32_us(const DeviceCtx &ctx, size_t batch, size_t m, size_t n, size_t k, bool vec);
+// How many chains of sums over k, 16 values each in turn, meet in an element of that product (1, 2 or 4); 0: it is no product of whole
+// tiles (many small matrices, or k cut into slices).
+int gemm_f32_chains(const DeviceCtx &ctx, size_t batch, size_t m, size_t n, size_t k);
 
 // Many small products at once (matmul_small.hip): one block per matrix.  C = A B, A with unit stride along k.
 bool gemm_small_batched_fits(size_t batch, size_t m, size_t n, size_t k);
 int launch_gemm_small_batched(DeviceCtx &ctx, float *c, const float *a, const float *b, size_t batch_outer, size_t batch_inner, size_t m, size_t n,
                               size_t k, int trans_b, size_t lda, size_t ldb, size_t ldc, const size_t a_bs[2], const size_t b_bs[2],
                               const size_t c_bs[2]);
+
+// O = Softmax(softmax_scale(Where(cond, scale(Q K^T), fill)) + mask) V per batch of fp32 matrices with 64 columns, with the bits of
+// the operators run apart (attention.hip).  Batches as in launch_gemm_batch2; cond and mask (either may
+// be null) with the strides of outer batch, inner batch, query and key; scales 0 none / 1 multiply / 2 divide.
+struct AttentionRows {
+    const float *q = nullptr, *k = nullptr, *v = nullptr, *mask = nullptr;
+    const uint8_t *cond = nullptr;
+    float *o = nullptr;
+    size_t batch_outer = 1, batch_inner = 1, tq = 0, tk = 0, ldq = 0, ldk = 0, ldv = 0, ldo = 0;
+    size_t q_bs[2] = {}, k_bs[2] = {}, v_bs[2] = {}, o_bs[2] = {}, cond_strides[4] = {}, mask_strides[4] = {};
+    int scale_op = 0, softmax_op = 0;
+    float scale = 1.0f, softmax_scale = 1.0f, fill = 0.0f;
+};
+bool attention_rows_fits(const DeviceCtx &ctx, size_t batch, size_t tq, size_t tk);
+int launch_attention_rows(DeviceCtx &ctx, const AttentionRows &a);
 
 // O = Softmax(scale(Q K^T) + mask) V per batch, scores kept in registers (attention.hip).  Q [tq, d], K [tk, d], V [tk, d],
 // O [tq, d] with row pitches ld*; batches as in launch_gemm_batch2; scale_op 0 none / 1 multiply / 2 divide; mask (may be

@@ -556,6 +556,12 @@ double gemm_f32_us(const DeviceCtx &ctx, size_t batch, size_t m, size_t n, size_
     return choose(batch, m, n, k, cus, ctx.gemm_split_k).us * (vec ? 1.0 : 1.2);
 }
 
+int gemm_f32_chains(const DeviceCtx &ctx, size_t batch, size_t m, size_t n, size_t k) {
+    if (gemm_small_batched_fits(batch, m, n, k)) return 0;
+    const Choice ch = choose(batch, m, n, k, ctx.cus_per_xcd ? (size_t)ctx.cus_per_xcd : 32, ctx.gemm_split_k);
+    return ch.slices > 1 ? 0 : (int)(SHAPES[ch.shape].step / BK);
+}
+
 int launch_gemm_f32(DeviceCtx &ctx, float *c, const float *a, const float *b, const float *c0, size_t batch_outer, size_t batch_inner, size_t m,
                     size_t n, size_t k, int trans_a, int trans_b, size_t lda, size_t ldb, size_t ldc, const size_t a_batch_strides[2],
                     const size_t b_batch_strides[2], const size_t c_batch_strides[2], size_t c0_row_stride, size_t c0_col_stride, float alpha,

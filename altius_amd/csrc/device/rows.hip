@@ -1384,6 +1384,9 @@ inline int lds_block_threads(size_t len, size_t rows = ~(size_t)0) {
         }                                                                                                           \
     }
 
+// The lanes per row of these layouts.
+constexpr int lds_lanes(size_t len) { return len <= 64 && len % 8 != 0 ? 4 : len <= 128 ? 8 : len <= 256 ? 16 : len <= 512 ? 32 : 64; }
+
 bool softmax_lds_launch(hipStream_t s, float *out, const float *in, size_t rows, size_t len, bool nt,
                         const SoftmaxPrologue *pro = nullptr) {
     static_assert(4 * 1024 <= LDS_GROUP_FLOATS, "four rows of the longest supported length must fit");
@@ -1526,6 +1529,8 @@ int launch_norm_chain(DeviceCtx &ctx, float *out, const float *in, const float *
 
 // Threads of the streaming kernels' block: two float4 per thread and pass up to 8192 elements, then the widest block.
 inline int stream_block_threads(size_t len) { return len <= 2048 ? 256 : len <= 4096 ? 512 : 1024; }
+
+int softmax_lds_lanes(size_t len) { return len && len <= MAX_WAVE_ROW && !wave_row_fits(len) ? lds_lanes(len) : 0; }
 
 int launch_softmax(DeviceCtx &ctx, float *out, const float *in, size_t rows, size_t len) {
     if (rows == 0 || len == 0) return AHIP_OK;

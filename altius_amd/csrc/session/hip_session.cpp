@@ -117,6 +117,7 @@ std::unique_ptr<HipSession> HipSessionBuilder::build(SessionError *err) {
     s->plan_ = create_execution_plan(s->model_);
     if (strided_views_) s->plan_views(fused_attention_);
     if (strided_views_ && !enable_profiling_) s->plan_norm_chains();  // a profile names every node
+    if (strided_views_ && !enable_profiling_) s->plan_attention_rows();
 
     std::string derr;
     int rc = create_device_ctx(device_, nullptr, true, &s->ctx_, &derr);
@@ -300,6 +301,7 @@ bool HipSession::run(const std::vector<Tensor> &inputs, std::vector<Tensor> *out
     pending_attn_.clear();
     absorbed_.clear();
     passed_over_.clear();
+    attention_held_.clear(), attention_operands_.clear();
     std::vector<hipEvent_t> events;
     // Nothing may still read a block when it goes back to the pool for another run, and input
     // tensors must outlive their uploads: every exit path synchronises first.
@@ -404,6 +406,7 @@ bool HipSession::run_device(const std::vector<DeviceTensor> &inputs, std::vector
     pending_attn_.clear();
     absorbed_.clear();
     passed_over_.clear();
+    attention_held_.clear(), attention_operands_.clear();
     for (size_t i = 0; i < g.inputs.size(); i++) {
         if (!inputs[i].ptr && inputs[i].nbytes())
             return fail(err, SessionError::Argument, "run_device: input " + std::to_string(i) + " has no device pointer");
@@ -479,6 +482,7 @@ bool HipSession::try_capture(const std::string &key, const std::vector<Tensor> &
     pending_attn_.clear();
     absorbed_.clear();
     passed_over_.clear();
+    attention_held_.clear(), attention_operands_.clear();
     for (size_t i = 0; i < g.inputs.size(); i++) {
         DeviceTensor d;
         if (!allocate(TypedFixedShape{inputs[i].dims(), inputs[i].elem_ty()}, &d, err)) return false;
@@ -601,6 +605,12 @@ bool HipSession::replay(CapturedRun &run, const std::vector<Tensor> &inputs, std
 bool HipSession::run_node(NodeId id, std::map<ValueId, DeviceTensor> &values, SessionError *err) {
     if (passed_over_.count(id)) return true;
     const Node &node = model_.graph.nodes[id];
+    if (auto held = attention_held_.find(id); held != attention_held_.end()) {
+        const NodeId head = held->second;
+        for (ValueId v : node.inputs)
+            if (auto it = values.find(v); it != values.end()) attention_operands_[head][v] = it->second;
+        return attention_rows_.at(head).rest.back() != id || finish_attention_rows(head, id, values, err);
+    }
     auto opname = [&]() { return std::string(node.op.name()); };  // for messages only
 
     // Inputs: run-time values first, then initializers.  An input whose value is never produced
@@ -648,6 +658,12 @@ bool HipSession::run_node(NodeId id, std::map<ValueId, DeviceTensor> &values, Se
         bool done = false;
         if (!run_norm_chain(id, *in[0], values, &done, err)) return false;
         if (done) return true;
+    }
+
+    if (auto rows = attention_rows_.find(id); rows != attention_rows_.end() && !attention_apart_ && attention_rows_takes(id, in)) {
+        for (size_t i = 0; i < in.size(); i++) attention_operands_[id][node.inputs[i]] = *in[i];
+        for (NodeId n : rows->second.rest) attention_held_[n] = id;
+        return true;
     }
 
     // Output shapes: inferred at build time if possible, else now (session.rs:149-158).  Operands

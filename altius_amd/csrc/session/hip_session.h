@@ -304,10 +304,29 @@ private:
         float eps = 0.0f;
     };
     std::map<NodeId, NormChainPlan> norm_chains_;
-    std::set<NodeId> passed_over_;  // nodes of this run that a norm chain's kernel has done
+    std::set<NodeId> passed_over_;  // nodes of this run that the kernel of a norm chain or an attention has done
     void plan_norm_chains();
     // Runs the chain that starts at node `id` if its operands allow it; *done tells.
     bool run_norm_chain(NodeId id, const DeviceTensor &x, std::map<ValueId, DeviceTensor> &values, bool *done, SessionError *err);
+    // MatMul -> [Mul / Div by one value] -> [Where(cond, ., one value)] -> [Add of a mask] -> Softmax [with its scale and mask] -> MatMul,
+    // by the first MatMul: its nodes leave their operands in `attention_operands_` and run nothing, until the last one's kernel does it all or,
+    // where an operand turns out not to be one that it takes, runs them apart after all.
+    struct AttentionRowsPlan {
+        std::vector<NodeId> rest;  // the nodes behind the first, the last MatMul at the end
+        int scale_op = 0, softmax_op = 0;
+        float scale = 1.0f, softmax_scale = 1.0f, fill = 0.0f;
+        bool has_where = false, has_mask = false;
+        ValueId cond = 0, mask = 0;
+    };
+    std::map<NodeId, AttentionRowsPlan> attention_rows_;
+    void plan_attention_rows();
+    std::map<NodeId, NodeId> attention_held_;  // nodes of this run that a first MatMul has left to their kernel -> that MatMul
+    std::map<NodeId, std::map<ValueId, DeviceTensor>> attention_operands_;  // by that MatMul: what its nodes read
+    bool attention_apart_ = false;
+    bool attention_rows_takes(NodeId id, const std::vector<DeviceTensor *> &in) const;
+    // The last node, `tail`, of the chain that starts at node `id`.
+    bool finish_attention_rows(NodeId id, NodeId tail, std::map<ValueId, DeviceTensor> &values, SessionError *err);
+    bool run_attention_rows(NodeId id, std::map<ValueId, DeviceTensor> &values, bool *done, SessionError *err);
     // Runs a deferred Add into the tensor's block.
     bool flush_add(DeviceTensor *t, SessionError *err);
     std::set<NodeId> lazy_views_;                               // Split / Transpose nodes whose outputs are views

@@ -559,4 +559,214 @@ bool HipSession::run_norm_chain(NodeId id, const DeviceTensor &x, std::map<Value
     return true;
 }
 
+void HipSession::plan_attention_rows() {
+    const auto users = model_.get_value_users();
+    const Graph &g = model_.graph;
+    auto listed = [](const std::vector<ValueId> &l, ValueId v) { return std::find(l.begin(), l.end(), v) != l.end(); };
+    // One f32 value that nothing can stand in for.
+    auto scalar = [&](ValueId v, float *value) {
+        auto it = g.inits.find(v);
+        if (it == g.inits.end() || listed(g.inputs, v) || it->second.elem_ty() != TensorElemType::F32 || it->second.dims().total_elems() != 1 ||
+            !it->second.has_data())
+            return false;
+        *value = it->second.data_f32()[0];
+        return true;
+    };
+    // The only reader of v, which is no output of the graph and read once.
+    auto reader = [&](ValueId v, NodeId *id) -> const Node * {
+        auto it = users.find(v);
+        if (it == users.end() || it->second.size() != 1 || listed(g.outputs, v)) return nullptr;
+        const Node &n = g.nodes[*id = *it->second.begin()];
+        return n.outputs.size() == 1 && std::count(n.inputs.begin(), n.inputs.end(), v) == 1 ? &n : nullptr;
+    };
+    for (const NodeExecutionPlan &step : plan_) {
+        const Node &head = g.nodes[step.node_id];
+        if (head.op.kind != OpKind::MatMul || head.inputs.size() != 2 || head.outputs.size() != 1 || attn_head_.count(step.node_id)) continue;
+        auto scores = inferred_.find(step.node_id);
+        if (scores == inferred_.end() || scores->second.second.empty()) continue;
+        const FixedDimensions &dims = scores->second.second[0].dims;
+        if (dims.len() < 2) continue;
+        auto same_shape = [&](NodeId id) {
+            auto it = inferred_.find(id);
+            return it != inferred_.end() && !it->second.second.empty() && it->second.second[0].dims == dims;
+        };
+        AttentionRowsPlan p;
+        ValueId v = head.outputs[0];
+        NodeId id = 0;
+        const Node *n = reader(v, &id);
+        if (n && (n->op.kind == OpKind::Div || n->op.kind == OpKind::Mul) && n->inputs.size() == 2 && same_shape(id)) {
+            const bool first = n->inputs[0] == v;
+            if (!(first || n->op.kind == OpKind::Mul) || !scalar(n->inputs[first ? 1 : 0], &p.scale)) continue;
+            p.scale_op = n->op.kind == OpKind::Mul ? 1 : 2;
+            p.rest.push_back(id);
+            v = n->outputs[0];
+            n = reader(v, &id);
+        }
+        if (n && n->op.kind == OpKind::Where && n->inputs.size() == 3 && n->inputs[1] == v && same_shape(id)) {
+            if (!scalar(n->inputs[2], &p.fill)) continue;
+            p.has_where = true;
+            p.cond = n->inputs[0];
+            p.rest.push_back(id);
+            v = n->outputs[0];
+            n = reader(v, &id);
+        }
+        bool added = false;  // a mask that the Softmax has not absorbed
+        if (n && n->op.kind == OpKind::Add && n->inputs.size() == 2 && same_shape(id)) {
+            added = true;
+            p.mask = n->inputs[n->inputs[0] == v ? 1 : 0];
+            p.rest.push_back(id);
+            v = n->outputs[0];
+            n = reader(v, &id);
+        }
+        if (!n || n->op.kind != OpKind::Softmax || n->inputs.empty() || n->inputs[0] != v || !same_shape(id)) continue;
+        if (added && (n->op.prologue_scale || n->op.prologue_mask)) continue;
+        if (n->op.axis != -1 && n->op.axis != (int64_t)dims.len() - 1) continue;
+        p.softmax_op = n->op.prologue_scale, p.has_mask = n->op.prologue_mask;
+        if (n->inputs.size() != 1u + (p.softmax_op ? 1 : 0) + (p.has_mask ? 1 : 0)) continue;
+        if (p.softmax_op && !scalar(n->inputs[1], &p.softmax_scale)) continue;
+        if (p.has_mask) p.mask = n->inputs.back();
+        p.has_mask = p.has_mask || added;
+        p.rest.push_back(id);
+        v = n->outputs[0];
+        n = reader(v, &id);
+        if (!n || n->op.kind != OpKind::MatMul || n->inputs.size() != 2 || n->inputs[0] != v || n->op.trans_a) continue;
+        auto result = inferred_.find(id);
+        if (result == inferred_.end() || result->second.second.empty()) continue;
+        p.rest.push_back(id);
+        attention_rows_[step.node_id] = std::move(p);
+    }
+}
+
+namespace {
+// An operand whose values are there, as fp32 (or as conditions).
+bool readable(const DeviceTensor *t, TensorElemType ty) {
+    return t && t->ptr && t->elem_ty == ty && t->pending_op < 0 && t->applied_op < 0 && !t->planes && !t->owes_add() && t->dims.len() >= 2;
+}
+}  // namespace
+
+bool HipSession::attention_rows_takes(NodeId id, const std::vector<DeviceTensor *> &in) const {
+    const FixedDimensions &sd = inferred_.at(id).second[0].dims, &od = inferred_.at(attention_rows_.at(id).rest.back()).second[0].dims;
+    if (in.size() != 2 || !readable(in[0], TensorElemType::F32) || !readable(in[1], TensorElemType::F32) || od.len() != sd.len()) return false;
+    const size_t rank = sd.len();
+    size_t batch = 1, axes = 0;
+    for (size_t i = 0; i + 2 < rank; i++) {
+        if (od[i] != sd[i]) return false;
+        batch *= sd[i];
+        axes += sd[i] != 1;
+    }
+    const bool wide = (inferred_.at(id).first.trans_a ? in[0]->dims[in[0]->dims.len() - 2] : in[0]->dims[in[0]->dims.len() - 1]) == 64;
+    if (!wide || axes > 2 || od[rank - 2] != sd[rank - 2] || od[rank - 1] != 64) return false;
+    return attention_rows_fits(ctx_, batch, sd[rank - 2], sd[rank - 1]);
+}
+
+bool HipSession::finish_attention_rows(NodeId id, NodeId tail, std::map<ValueId, DeviceTensor> &values, SessionError *err) {
+    const AttentionRowsPlan &p = attention_rows_.at(id);
+    for (NodeId n : p.rest) attention_held_.erase(n);
+    bool done = false;
+    if (!run_attention_rows(id, values, &done, err)) return false;
+    if (!done) {
+        // What they read may have been let go in the meantime.
+        std::vector<ValueId> again;
+        for (auto &kv : attention_operands_[id])
+            if (values.emplace(kv.first, kv.second).second) again.push_back(kv.first);
+        attention_apart_ = true;
+        bool ok = run_node(id, values, err);
+        for (NodeId n : p.rest) ok = ok && run_node(n, values, err);
+        attention_apart_ = false;
+        if (!ok) return false;
+        for (ValueId v : again) values.erase(v);
+        values.erase(model_.graph.nodes[id].outputs[0]);
+        for (NodeId n : p.rest)
+            if (n != tail) values.erase(model_.graph.nodes[n].outputs[0]);
+    }
+    attention_operands_.erase(id);
+    return true;
+}
+
+bool HipSession::run_attention_rows(NodeId id, std::map<ValueId, DeviceTensor> &values, bool *done, SessionError *err) {
+    const AttentionRowsPlan &p = attention_rows_.at(id);
+    const Node &head = model_.graph.nodes[id], &tail = model_.graph.nodes[p.rest.back()];
+    const Op &head_op = inferred_.at(id).first, &tail_op = inferred_.at(p.rest.back()).first;
+    const FixedDimensions &sd = inferred_.at(id).second[0].dims, &od = inferred_.at(p.rest.back()).second[0].dims;
+    const size_t rank = sd.len(), tq = sd[rank - 2], tk = sd[rank - 1];
+    std::vector<size_t> bd;
+    size_t batch = 1;
+    for (size_t i = 0; i + 2 < rank; i++) {
+        batch *= sd[i];
+        if (sd[i] != 1) bd.push_back(sd[i]);
+    }
+    std::map<ValueId, DeviceTensor> &operands = attention_operands_[id];
+    auto value = [&](ValueId v) -> DeviceTensor * {
+        auto it = operands.find(v);
+        if (it != operands.end()) return &it->second;
+        auto ii = inits_.find(v);
+        return ii != inits_.end() ? &ii->second : nullptr;
+    };
+    DeviceTensor *in[2] = {value(head.inputs[0]), value(head.inputs[1])};
+    DeviceTensor *vt = value(tail.inputs[1]), *ct = p.has_where ? value(p.cond) : nullptr, *mt = p.has_mask ? value(p.mask) : nullptr;
+    if (!in[0] || !in[1] || !readable(vt, TensorElemType::F32)) return true;
+    auto over = [&](const DeviceTensor *t, TensorElemType ty) { return t && t->ptr && t->elem_ty == ty && t->pending_op < 0 && t->applied_op < 0 && !t->planes && !t->owes_add() && t->strides.empty(); };
+    if ((p.has_where && !over(ct, TensorElemType::Bool)) || (p.has_mask && !over(mt, TensorElemType::F32))) return true;
+    MatOperand Q, K, V;
+    if (!describe_operand(in[0], &Q, err) || !describe_operand(in[1], &K, err) || !describe_operand(vt, &V, err)) return false;
+    // Q [tq, 64], K [tk, 64] and V [tk, 64] as stored rows.
+    const bool q_rows = head_op.trans_a == Q.stored_transposed, k_rows = head_op.trans_b != K.stored_transposed, v_rows = tail_op.trans_b == V.stored_transposed;
+    auto extent = [](const MatOperand &o, size_t r) { return (o.stored_transposed ? o.cols : o.rows) == r && (o.stored_transposed ? o.rows : o.cols) == 64; };
+    if (!q_rows || !k_rows || !v_rows || !extent(Q, tq) || !extent(K, tk) || !extent(V, tk)) return true;
+    if (Q.batch != batch || (K.batch != batch && K.batch != 1) || (V.batch != batch && V.batch != 1)) return true;
+    std::vector<int64_t> qs, ks, vs;
+    if (!operand_batch_strides(bd, Q.bdims, Q.bstr, in[0]->strides.empty(), tq * 64, Q.batch, &qs) ||
+        !operand_batch_strides(bd, K.bdims, K.bstr, in[1]->strides.empty(), tk * 64, K.batch, &ks) ||
+        !operand_batch_strides(bd, V.bdims, V.bstr, vt->strides.empty(), tk * 64, V.batch, &vs))
+        return true;
+    AttentionRows a;
+    auto two = [&](const std::vector<int64_t> &s, size_t out2[2]) {
+        out2[0] = s.size() > 0 ? (size_t)s[0] : 0;
+        out2[1] = s.size() > 1 ? (size_t)s[1] : 0;
+    };
+    two(qs, a.q_bs), two(ks, a.k_bs), two(vs, a.v_bs);
+    // A condition or mask over the scores: strides of the batch axes, the query and the key.
+    auto over_scores = [&](const DeviceTensor *t, size_t out4[4]) {
+        auto st = t->dims.strides_for_broadcasting_to(sd);
+        if (!st || st->len() != rank) return false;
+        std::vector<int64_t> b;
+        for (size_t i = 0; i + 2 < rank; i++)
+            if (sd[i] != 1) b.push_back((int64_t)(*st)[i]);
+        two(b, out4);
+        out4[2] = (*st)[rank - 2], out4[3] = (*st)[rank - 1];
+        return true;
+    };
+    if ((ct && !over_scores(ct, a.cond_strides)) || (mt && !over_scores(mt, a.mask_strides))) return true;
+
+    DeviceTensor out;
+    if (!allocate({od, TensorElemType::F32}, &out, err)) return false;
+    // Dense, or the layout of the Transpose behind the last product.
+    std::vector<int64_t> c_str = dense_strides(od);
+    auto pv = matmul_out_perm_.find(p.rest.back());
+    if (pv != matmul_out_perm_.end() && pv->second.size() == rank) {
+        FixedDimensions td = od;
+        for (size_t i = 0; i < rank; i++) td[i] = od[(size_t)pv->second[i]];
+        const std::vector<int64_t> ts = dense_strides(td);
+        for (size_t i = 0; i < rank; i++) c_str[(size_t)pv->second[i]] = ts[i];
+        if (!is_dense(od, c_str)) out.strides = c_str;
+    }
+    std::vector<int64_t> os;
+    for (size_t i = 0; i + 2 < rank; i++)
+        if (od[i] != 1) os.push_back(c_str[i]);
+    two(os, a.o_bs);
+    auto f = [](const DeviceTensor *t) { return static_cast<const float *>(t->ptr); };
+    a.q = f(in[0]), a.k = f(in[1]), a.v = f(vt), a.o = static_cast<float *>(out.ptr);
+    a.mask = mt ? f(mt) : nullptr, a.cond = ct ? static_cast<const uint8_t *>(ct->ptr) : nullptr;
+    a.batch_outer = bd.size() > 0 ? bd[0] : 1, a.batch_inner = bd.size() > 1 ? bd[1] : 1;
+    a.tq = tq, a.tk = tk, a.ldq = Q.ld, a.ldk = K.ld, a.ldv = V.ld, a.ldo = tq > 1 ? (size_t)c_str[rank - 2] : 64;
+    a.scale_op = p.scale_op, a.scale = p.scale, a.softmax_op = p.softmax_op, a.softmax_scale = p.softmax_scale, a.fill = p.fill;
+    const int rc = launch_attention_rows(ctx_, a);
+    if (rc == AHIP_ERR_UNSUPPORTED) return true;
+    if (rc) return fail_code(err, rc, ctx_.last_error);
+    values[tail.outputs[0]] = std::move(out);
+    copies_avoided_ += p.rest.size();
+    *done = true;
+    return true;
+}
+
 }  // namespace altius
