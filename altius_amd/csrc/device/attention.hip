@@ -553,8 +553,10 @@ inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 
 // LDS ([32][pitch], zeros behind the last key), where the Softmax works on them in place; O = P V reads them back, a wavefront per chain
 // and 32 columns of V, which it reads from memory, and the chains meet in LDS.
 //
-// Calls of a few hundred heads and less are bound by one block's chain of loads and products; us a layer with the operators' kernels and
-// with this one: ROWS_FIGURES.
+// Calls of up to a hundred heads are bound by one block's chain of loads and products, larger ones by the matrix cores and the
+// exponentials.  us with the operators' kernels (back to back, scale and mask in the Softmax) and with this one: 12 heads of 12, 77, 197
+// and 257 queries and keys 11.0 -> 6.8, 13.4 -> 8.6, 16.7 -> 10.8, 20.2 -> 13.7; 96 of 128 and 197 23.0 -> 12.7, 36.1 -> 28.1;
+// 384 of 257 165 -> 124; 192 of 400, the least that was found, 147 -> 146.
 struct RowsArgs {
     const float *q, *k, *v, *mask;
     const uint8_t *cond;
@@ -738,7 +740,8 @@ __global__ __launch_bounds__(64 * RW, 2) void attention_rows_d64(RowsArgs g, int
 }  // namespace
 
 // The operators' order of sums, where this kernel has it: both products on the tiles of matmul.hip, uncut, and the rows through
-// softmax_lds.
+// softmax_lds.  (From 128 heads of up to 208 keys on the products are matmul_small.hip's, which take as long as this kernel would:
+// 384 heads of 197 96 us.)
 static bool rows_order(const DeviceCtx &ctx, size_t batch, size_t tq, size_t tk, int *qk, int *pv, int *lanes) {
     *qk = gemm_f32_chains(ctx, batch, tq, tk, D), *pv = gemm_f32_chains(ctx, batch, tq, D, tk), *lanes = softmax_lds_lanes(tk);
     return *qk && *pv && *lanes && *lanes <= 32;
