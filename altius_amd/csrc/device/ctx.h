@@ -246,9 +246,11 @@ bool attention_writes_planes(const DeviceCtx &ctx, size_t batch_outer, size_t ba
 // a_op: 0, or AHIP_GELU / AHIP_RELU applied to A's values while they are split (C = alpha f(A) B + beta C0).
 // a_planes (may be null): the first operand already as planes, as launch_layernorm_planes writes them (then a, lda
 // and a_op are not used): rows = m, k = k, gemm_planes_bytes(m, k) bytes.
+// c_planes (may be null): AHIP_GELU or AHIP_RELU (c_op) of the result as the planes of a [m, n] first operand instead of C (c and ldc are
+// not used; C0 is null or a bias row), bit for bit what a_op of the product that reads it would make of C.
 int launch_gemm_split(DeviceCtx &ctx, float *c, const float *a, const float *b, const float *c0, size_t m, size_t n, size_t k,
                       int trans_a, int trans_b, size_t lda, size_t ldb, size_t ldc, size_t c0_row_stride, size_t c0_col_stride,
-                      float alpha, float beta, int a_op = 0, const void *a_planes = nullptr);
+                      float alpha, float beta, int a_op = 0, const void *a_planes = nullptr, int c_op = 0, void *c_planes = nullptr);
 size_t gemm_planes_bytes(size_t rows, size_t k);
 // LayerNormalization over rows of `len` elements written as the planes of the first operand of a product on the
 // bf16 route (rows = rows, k = len; gemm_planes_bytes(rows, len) bytes) instead of fp32 values: the planes that

@@ -207,6 +207,8 @@ struct SplitGemmArgs {
     int *misplaced;  // raised when the slices of a tile did not all run on one XCD
     int c_vec;    // 16-byte stores into C are aligned
     int c_stream;  // C is large: write it with non-temporal stores
+    u32x4 *c_planes;  // f(C) as the planes of the next product's first operand instead of C: k groups of them, mp rows
+    uint32_t c_kgs;
 };
 
 typedef __attribute__((address_space(3))) void *lds_ptr;
@@ -269,7 +271,8 @@ __device__ __forceinline__ void slot_barrier(bool loads_left_in_flight) {
     else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
-__global__ __launch_bounds__(THREADS, 1) void gemm_bf16x3(SplitGemmArgs g) {
+// POST: 0, or the AHIP_* activation f behind which the result leaves as operand planes (c_planes).
+template <int POST> __global__ __launch_bounds__(THREADS, 1) void gemm_bf16x3(SplitGemmArgs g) {
     __shared__ Stage S[3];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1, lr = lane & 31, lk = lane >> 5;
@@ -395,6 +398,13 @@ __global__ __launch_bounds__(THREADS, 1) void gemm_bf16x3(SplitGemmArgs g) {
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
     constexpr int EP = 132;
     float *stage = reinterpret_cast<float *>(&S[0]) + wave * (32 * EP);
+    // For planes: beta times the bias row, behind the wavefronts' regions.
+    float *tile_bias = reinterpret_cast<float *>(&S[0]) + 8 * (32 * EP);
+    static_assert(sizeof(S) >= (8 * 32 * EP + TN) * sizeof(float), "the bias row fits behind the staged rows");
+    if constexpr (POST != 0) {
+        if (tid < TN) tile_bias[tid] = g.c0 && n0 + tid < g.n ? g.beta * g.c0[(size_t)(n0 + tid) * g.c0_cs] : 0.0f;
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    }
     // A bias row (c0_rs == 0) is the same for every row of the tile: read it once, ahead of the stores.
     const uint32_t gcol = n0 + wn * 128 + lr * 4;
     const bool row_bias = g.c0 && g.c0_rs == 0;
@@ -413,6 +423,40 @@ __global__ __launch_bounds__(THREADS, 1) void gemm_bf16x3(SplitGemmArgs g) {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        if constexpr (POST != 0) {
+            // What the reader of C would have done with it: the activation, and the split into planes.  Half a wavefront takes 32 rows of
+            // one k group, 512 contiguous bytes of each plane; rows and columns behind C's last are zeros, as the split writes them.
+            // [25216, 768] x [768, 3072] with Gelu 526 us and 160 for its split before, 625 here: the activation and
+            // the split are 46 vector instructions a value, which nothing hides (a CU holds one block).  The bias from memory in
+            // each turn, one turn at a time, took 650.
+            const uint32_t grow = m0 + wm * 64 + i * 32 + lr;
+#pragma unroll 2
+            for (int q = 0; q < 8; q++) {
+                const uint32_t kgl = 2 * q + lk, col = n0 + wn * 128 + kgl * 8, kg = col / 8;
+                const f32x4 lo = *reinterpret_cast<const f32x4 *>(stage + lr * EP + kgl * 8), hi = *reinterpret_cast<const f32x4 *>(stage + lr * EP + kgl * 8 + 4);
+                const f32x4 blo = *reinterpret_cast<const f32x4 *>(tile_bias + wn * 128 + kgl * 8), bhi = *reinterpret_cast<const f32x4 *>(tile_bias + wn * 128 + kgl * 8 + 4);
+                float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+                const float add[8] = {blo.x, blo.y, blo.z, blo.w, bhi.x, bhi.y, bhi.z, bhi.w};
+                uint32_t h[3][4];
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    v[e] = g.alpha * v[e];
+                    if (g.c0) v[e] += add[e];
+                    v[e] = grow < g.m && col + e < g.n ? pre<POST>(v[e]) : 0.0f;
+                }
+#pragma unroll
+                for (int j = 0; j < 4; j++) split3_pair(v[2 * j], v[2 * j + 1], h[0][j], h[1][j], h[2][j]);
+                if (kg < g.c_kgs) {
+#pragma unroll
+                    for (int p = 0; p < 3; p++) {
+                        u32x4 *dst = g.c_planes + ((size_t)p * g.c_kgs + kg) * g.mp + grow;
+                        const u32x4 o = {h[p][0], h[p][1], h[p][2], h[p][3]};
+                        if (g.c_stream) __builtin_nontemporal_store(o, dst);
+                        else *dst = o;
+                    }
+                }
+            }
+        } else {
 #pragma unroll 4
         for (int q = 0; q < 16; q++) {
             const int row = 2 * q + lk;
@@ -440,6 +484,7 @@ __global__ __launch_bounds__(THREADS, 1) void gemm_bf16x3(SplitGemmArgs g) {
                 for (int e = 0; e < 4; e++)
                     if (gcol + e < g.n) dst[e] = v[e];
             }
+        }
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -577,12 +622,15 @@ bool gemm_split_worthwhile(size_t m, size_t n, size_t k) {
 
 int launch_gemm_split(DeviceCtx &ctx, float *c, const float *a, const float *b, const float *c0, size_t m, size_t n, size_t k,
                       int trans_a, int trans_b, size_t lda, size_t ldb, size_t ldc, size_t c0_row_stride, size_t c0_col_stride,
-                      float alpha, float beta, int a_op, const void *a_planes) {
+                      float alpha, float beta, int a_op, const void *a_planes, int c_op, void *c_planes) {
     if (a_op != 0 && a_op != AHIP_GELU && a_op != AHIP_RELU)
         return ctx.fail(AHIP_ERR_UNSUPPORTED, "gemm (bf16 x 3): only Gelu and Relu can be folded into the operand split");
     if (a_planes && (a_op || trans_a)) return ctx.fail(AHIP_ERR_ARG, "gemm (bf16 x 3): planes of the first operand come as they are");
+    if (c_planes && (c_op != AHIP_GELU && c_op != AHIP_RELU))
+        return ctx.fail(AHIP_ERR_UNSUPPORTED, "gemm (bf16 x 3): only Gelu and Relu can stand between a product and its result's planes");
+    if (c_planes && c0 && beta != 0.0f && c0_row_stride != 0) return ctx.fail(AHIP_ERR_UNSUPPORTED, "gemm (bf16 x 3): only a bias row can be added in front of planes");
     if (m == 0 || n == 0) return AHIP_OK;
-    if (!c || (!a && !a_planes) || !b || k == 0) return ctx.fail(AHIP_ERR_ARG, "gemm (bf16 x 3): null pointer or k = 0");
+    if ((!c && !c_planes) || (!a && !a_planes) || !b || k == 0) return ctx.fail(AHIP_ERR_ARG, "gemm (bf16 x 3): null pointer or k = 0");
     const size_t lim = (size_t)1 << 31;
     if (m >= lim - 256 || n >= lim - 256 || k >= lim - 16 || lda >= lim || ldb >= lim || ldc >= lim || c0_row_stride >= lim ||
         c0_col_stride >= lim)
@@ -660,8 +708,12 @@ int launch_gemm_split(DeviceCtx &ctx, float *c, const float *a, const float *b, 
     }
     const uint32_t slots = g.full + (g.chunk - g.full) * g.sf;
     g.c_vec = aligned16(c) && ldc % 4 == 0;
-    g.c_stream = ctx.streaming(m * n * sizeof(float));
-    hipLaunchKernelGGL(gemm_bf16x3, dim3(slots * 8), dim3(THREADS), 0, ctx.stream, g);
+    g.c_planes = static_cast<u32x4 *>(c_planes);
+    g.c_kgs = (uint32_t)plane_dims(m, n).kgs;
+    g.c_stream = ctx.streaming(c_planes ? plane_dims(m, n).bytes : m * n * sizeof(float));
+    if (!c_planes) hipLaunchKernelGGL(gemm_bf16x3<0>, dim3(slots * 8), dim3(THREADS), 0, ctx.stream, g);
+    else if (c_op == AHIP_GELU) hipLaunchKernelGGL(gemm_bf16x3<AHIP_GELU>, dim3(slots * 8), dim3(THREADS), 0, ctx.stream, g);
+    else hipLaunchKernelGGL(gemm_bf16x3<AHIP_RELU>, dim3(slots * 8), dim3(THREADS), 0, ctx.stream, g);
     return ctx.check(hipGetLastError(), "gemm (bf16 x 3) launch");
 }
 

@@ -712,7 +712,7 @@ bool HipSession::run_node(NodeId id, std::map<ValueId, DeviceTensor> &values, Se
         copies_avoided_++;
         outs.push_back(std::move(o));
     } else if (in.size() == 1 && in[0] && in[0]->applied_op >= 0 && !is_alias_op(op.kind)) {
-        // The node that made the operand has applied this activation, its only reader, already.
+        // The node that made the operand has applied this activation, its only reader, already (and may have left it as planes).
         DeviceTensor o = *in[0];
         o.dims = shapes[0].dims;
         o.applied_op = -1;
@@ -1533,8 +1533,11 @@ bool HipSession::run_device_op(const Node &node, const Op &op, const std::vector
                     return fail(err, SessionError::Shape, "MatMul: the absorbed bias must hold one f32 value per output column");
                 bias_p = f(in[2]);
             }
+            void *c_planes = nullptr;
+            int c_op = 0;
+            if (!act_planes_for(rows, nn, kk, &out, &c_planes, &c_op, err)) return false;
             rc = launch_gemm_split(ctx_, o, nullptr, f(in[1]), bias_p, rows, nn, kk, 0, op.trans_b ? 1 : 0, kk, op.trans_b ? kk : nn, nn, 0, 1, 1.0f,
-                                   bias_p ? 1.0f : 0.0f, 0, in[0]->ptr);
+                                   bias_p ? 1.0f : 0.0f, 0, in[0]->ptr, c_op, c_planes);
             break;
         }
         // The activation the first operand still owes is folded into the bf16 route's operand split when this
@@ -1598,7 +1601,11 @@ bool HipSession::run_device_op(const Node &node, const Op &op, const std::vector
                     break;
                 }
             }
-            if (a_op) rc = launch_gemm_split(ctx_, o, f(in[0]), f(in[1]), bias, batch * m, n, k, 0, tb, A.ld, B.ld, n, 0, 1, 1.0f, beta, a_op);
+            void *c_planes = nullptr;
+            int c_op = 0;
+            if (!act_planes_for(batch * m, n, k, &out, &c_planes, &c_op, err)) return false;
+            if (a_op || c_planes)
+                rc = launch_gemm_split(ctx_, o, f(in[0]), f(in[1]), bias, batch * m, n, k, 0, tb, A.ld, B.ld, n, 0, 1, 1.0f, beta, a_op, nullptr, c_op, c_planes);
             else rc = launch_gemm(ctx_, o, f(in[0]), f(in[1]), bias, 1, batch * m, n, k, 0, tb, A.ld, B.ld, n, 0, 0, 0, 0, 1, 1.0f, beta);
             break;
         }

@@ -295,6 +295,15 @@ private:
     // writes that last product's operand planes; the two nodes between pass them on.
     std::map<NodeId, PlanesPlan> attn_planes_;
     std::set<NodeId> planes_pass_;
+    // Product with a weight matrix -> Gelu / Relu -> product with a weight matrix, nobody else between them: where both take the bf16 route
+    // the first writes the activation's values as the second's operand planes, and the activation passes them on.
+    struct ActPlanesPlan {
+        PlanesPlan next;
+        int act = 0;
+    };
+    std::map<NodeId, ActPlanesPlan> act_planes_;
+    // The block that product `current_node_`, [m, k] x [k, n], writes such planes to (null: it writes none), made part of `out`.
+    bool act_planes_for(size_t m, size_t n, size_t k, DeviceTensor *out, void **planes, int *act, SessionError *err);
     std::map<NodeId, NodeId> add_into_ln_;  // Add nodes (a residual connection) -> the planes-writing LayerNormalization that reads the sum
     // A LayerNormalization written out as nine operators whose intermediate results nobody else reads, by its first node: one
     // kernel computes the last node's result when the first one is due, and the nodes between are passed over.

@@ -318,7 +318,27 @@ void HipSession::plan_views(bool fused_attention) {
             if (mm.op.kind != OpKind::MatMul || mm.inputs.size() < 2 || mm.inputs[0] != n.outputs[0]) continue;
             bool elsewhere = false;
             for (size_t i = 1; i < mm.inputs.size(); i++) elsewhere = elsewhere || mm.inputs[i] == n.outputs[0];
-            if (!elsewhere) deferred_unary_.insert(id);
+            if (elsewhere) continue;
+            deferred_unary_.insert(id);
+            auto par = parents.find(n.inputs[0]);
+            if (par == parents.end() || is_output(n.inputs[0])) continue;
+            const Node &first = g.nodes[par->second];
+            auto fu = users.find(n.inputs[0]);
+            auto weights = [&](const Node &p) {
+                auto w = p.inputs.size() > 1 ? g.inits.find(p.inputs[1]) : g.inits.end();
+                return w != g.inits.end() && w->second.dims().len() == 2 && w->second.elem_ty() == TensorElemType::F32 ? &w->second : nullptr;
+            };
+            const Tensor *w = weights(mm);
+            if (first.op.kind != OpKind::MatMul || first.outputs.size() != 1 || first.op.trans_a || mm.op.trans_a || fu == users.end() || fu->second.size() != 1 ||
+                !weights(first) || !w)
+                continue;
+            ActPlanesPlan ap;
+            ap.next.consumer = *it->second.begin();
+            ap.next.next_n = mm.op.trans_b ? w->dims()[0] : w->dims()[1];
+            ap.act = n.op.kind == OpKind::Gelu ? AHIP_GELU : AHIP_RELU;
+            act_planes_[par->second] = ap;
+            planes_consumer_.insert(ap.next.consumer);
+            planes_pass_.insert(id);
         } else if (n.op.kind == OpKind::LayerNormalization && n.outputs.size() == 1 && n.inputs.size() == 3 && !is_output(n.outputs[0])) {
             // LayerNormalization read only by a product with a weight matrix: it can write that product's operand planes.
             auto it = users.find(n.outputs[0]);
@@ -466,6 +486,23 @@ void HipSession::plan_views(bool fused_attention) {
         planes_pass_.insert(tr);
         planes_pass_.insert(rs);
     }
+}
+
+bool HipSession::act_planes_for(size_t m, size_t n, size_t k, DeviceTensor *out, void **planes, int *act, SessionError *err) {
+    *planes = nullptr;
+    auto ap = act_planes_.find(current_node_);
+    // The second product reads [m, n]; it is given planes only if it would have split its operand itself.
+    if (ap == act_planes_.end() || matmul_out_perm_.count(ap->second.next.consumer) || !gemm_takes_split(ctx_, m, n, k) ||
+        !gemm_takes_split(ctx_, m, ap->second.next.next_n, n))
+        return true;
+    DeviceTensor t;
+    if (!allocate_bytes(gemm_planes_bytes(m, n), &t, err)) return false;
+    out->block = t.block;  // the fp32 block goes back to the pool unused
+    out->ptr = *planes = t.ptr;
+    out->planes = true;
+    out->planes_rows = m, out->planes_k = n;
+    out->applied_op = *act = ap->second.act;
+    return true;
 }
 
 void HipSession::plan_norm_chains() {
@@ -764,7 +801,6 @@ bool HipSession::run_attention_rows(NodeId id, std::map<ValueId, DeviceTensor> &
     if (rc == AHIP_ERR_UNSUPPORTED) return true;
     if (rc) return fail_code(err, rc, ctx_.last_error);
     values[tail.outputs[0]] = std::move(out);
-    copies_avoided_ += p.rest.size();
     *done = true;
     return true;
 }

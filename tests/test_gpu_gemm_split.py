@@ -8,6 +8,8 @@ import pytest
 
 import oracle as O
 from altius_amd import device as D
+from altius_amd.graph import Model, Op
+from altius_amd.session import HipSessionBuilder
 from conftest import assert_bits_equal
 
 pytestmark = pytest.mark.gpu
@@ -229,3 +231,32 @@ def test_auto_takes_the_split_kernel_at_model_size(ctx, case):
     err = np.abs(got[rows].astype(np.float64) - (exact + bias)) / (scale + np.abs(bias))
     assert err.max() <= (k + 3) * 2.0 ** -24
     assert np.sqrt((err ** 2).mean()) < 1e-7
+
+
+# one tile and ragged tiles, columns that end inside a k group, inside a tile and on its edge, k cut into slices, fewer rows than a tile
+@pytest.mark.parametrize("m,k,n,after", [(1, 16, 8, 8), (37, 24, 100, 40), (256, 64, 256, 256), (300, 1000, 259, 33), (513, 768, 1300, 96), (700, 4096, 264, 64)])
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("act", [Op.Gelu, Op.ReLU])
+def test_activation_written_as_planes(case, m, k, n, after, bias, act):
+    """Product -> activation -> product: the first writes the second's operand planes, with the bits of the nodes run apart."""
+    case(f"[{m},{k}] x [{k},{n}], {act}, x [{n},{after}], bias {bias}")
+    rng = np.random.default_rng(m + n)
+    normal = lambda *s: rng.standard_normal(s).astype(np.float32)  # noqa: E731
+    g = Model(opset_version=13)
+    x = g.new_val_named_and_shaped("x", [m, k])
+    g.add_input(x)
+    h, u, y = g.new_val(), g.new_val(), g.new_val()
+    g.add_node(Op.MatMul, [x, g.new_initializer(normal(k, n) / np.float32(np.sqrt(k)))], [h])
+    if bias:
+        g.add_node(Op.Add, [h, g.new_initializer(normal(n))], [b := g.new_val()])
+        h = b
+    g.add_node(act, [h], [u])
+    g.add_node(Op.MatMul, [u, g.new_initializer(normal(n, after))], [y])
+    g.add_output(y)
+    g.fuse_matmul_bias()
+    feed = 2 * normal(m, k)
+    feed.flat[0], feed.flat[-1] = np.float32(3e38), np.float32(1e-42)
+    build = lambda views: HipSessionBuilder(g).with_gemm_algorithm(D.GEMM_BF16X3).with_strided_views(views).build()  # noqa: E731
+    together, apart = build(True), build(False)
+    for _ in range(2):
+        assert_bits_equal(together.run([feed])[0], apart.run([feed])[0], "planes from the product and from the split")
