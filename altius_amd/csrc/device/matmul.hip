@@ -24,7 +24,7 @@
 //   4096^3: 1061 -> 938 us (147 Tflop/s);  [50432,768] x [768,3072]: 1788 -> 1670 (143)
 // Single-value loads are taken for both operands where one of them needs them.
 // What is left on large shapes: the blocks' first loads and their results (1 us of 12 in a 64 x 64 tile with 768 values of k), and a last
-// round of blocks that is partly empty ([6304,768] x [768,768]: 4.6 rounds take five).
+// round of blocks that is partly empty where a cut costs as much as it gives ([6304,768] x [768,768]: 4.6 rounds take five, cut 64 us).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -61,8 +61,9 @@ struct GemmArgs {
     // that the blocks it runs together share panels.  Within that order tiles go by groups of group_n tile columns, each group
     // walked row of tiles by row of tiles, so that those blocks cover few columns of B (they stay in its L2) and many rows of A.
     uint32_t tiles_m, tiles_n, tiles, chunk, group_n;  // tiles: of all batches
-    // A tile's k cut into `slices` of slice_k values (whole steps of the block; the last one takes the rest): see the epilogue.
-    uint32_t slices, slice_k;
+    // Of each XCD's run the first `full` tiles are whole; of the others k is cut into `slices` of slice_k values (whole steps of the
+    // block; the last one takes the rest): see the epilogue.
+    uint32_t full, slices, slice_k;
     // Steps that 32-bit byte offsets reach behind the tile whose first element they count from, for both operands.
     uint32_t window;
     float *partials;
@@ -189,17 +190,19 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_f32_tiles(GemmArgs g) 
     const int wk = wave / (WM * WN), wmn = wave % (WM * WN), wm = wmn / WN, wn = wmn % WN;
     const int lr = lane & 31, lk = lane >> 5;
 
-    // block id -> (slice, tile): an XCD gets a run of consecutive tiles, the slices of a tile next to each other in it
+    // block id -> (slice, tile): an XCD gets a run of consecutive tiles, the cut ones behind the whole ones, a tile's slices next to each other
     const uint32_t xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
-    const uint32_t in_run = local / g.slices, slice = local - in_run * g.slices;
+    const bool cut = local >= g.full;
+    const uint32_t cut_tile = cut ? (local - g.full) / g.slices : 0, slice = cut ? local - g.full - cut_tile * g.slices : 0;
+    const uint32_t in_run = cut ? g.full + cut_tile : local;
     const uint32_t tile = xcd * g.chunk + in_run;
-    if (tile >= g.tiles) return;
+    if (in_run >= g.chunk || tile >= g.tiles) return;
     const uint32_t per_batch = g.tiles_m * g.tiles_n, z = tile / per_batch, t = tile - z * per_batch;
     const uint32_t per_group = g.tiles_m * g.group_n, grp = t / per_group, r = t - grp * per_group;
     const uint32_t width = min(g.group_n, g.tiles_n - grp * g.group_n);
     const uint32_t m0 = (r / width) * BM, n0 = (grp * g.group_n + r % width) * BN;
     const uint32_t zo = z / g.batch_inner, zi = z - zo * g.batch_inner;
-    const uint32_t k0 = slice * g.slice_k, k = min(g.slice_k, g.k - k0);
+    const uint32_t k0 = slice * g.slice_k, k = cut ? min(g.slice_k, g.k - k0) : g.k;
     const float *a = g.a + (size_t)zo * g.a_bs + (size_t)zi * g.a_bs2 + (AKC ? (size_t)m0 * g.lda + k0 : (size_t)k0 * g.lda + m0);
     const float *b = g.b + (size_t)zo * g.b_bs + (size_t)zi * g.b_bs2 + (BKC ? (size_t)n0 * g.ldb + k0 : (size_t)k0 * g.ldb + n0);
 
@@ -370,7 +373,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_f32_tiles(GemmArgs g) 
             }
         }
     };
-    const uint32_t idx = xcd * g.chunk + in_run;
+    const uint32_t idx = xcd * (g.chunk - g.full) + cut_tile;
     f32x4 *parts = reinterpret_cast<f32x4 *>(g.partials) + (size_t)idx * g.slices * (BM * BN / 4) + tid;
 #pragma unroll
     for (int i = 0; i < TA; i++) {
@@ -390,7 +393,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_f32_tiles(GemmArgs g) 
             for (int w = 1; w < WK; w++) v += *reinterpret_cast<const f32x4 *>(s + w * (PASS_ROWS * CP));
             return v;
         };
-        if (g.slices > 1) {
+        if (cut) {
 #pragma unroll
             for (int u = 0; u < PIECES; u++) store_shared(parts + (size_t)slice * (BM * BN / 4) + (i * PIECES + u) * THREADS, sum_at(u));
         } else if (g.act) {  // one copy of the activation's code: unrolled, it slowed every launch down
@@ -401,7 +404,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_f32_tiles(GemmArgs g) 
             for (int u = 0; u < PIECES; u++) finish(sum_at(u), i, u);
         }
     }
-    if (g.slices == 1) return;
+    if (!cut) return;
 
     // A tile cut along k: the block that arrives last adds the slices' sums up in slice order, so the result does not depend on who
     // was last.  The sums pass by the L2s (agent-scope accesses), so it does not matter on which XCD a slice ran; vmcnt(0) says
@@ -424,7 +427,10 @@ inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 
 
 // The block tiles, and what a launch of them takes: launch_us + rounds * (block_us + k_us * k / 768), rounds being the blocks that
 // the busiest CU runs (dealt to the XCDs in turn), times `lone` where that is one: a CU's only block has nothing to fill its gaps
-// with.  Where k is cut, 0.8 us more, slice_us for each slice and the partial sums at 2.5 TB/s.  Fitted to 120 products of 1e8 to
+// with.  The tiles of a last round that is partly empty may be cut along k, so that it takes a part of a round: 0.8 us more, slice_us for
+// each slice and the partial sums at 2.5 TB/s ([3152,3072] x [3072,768] 137 -> 116 us, [1536,1536] x [1536,1536] 65 -> 56,
+// [2500,1000] x [1000,2000] 100 -> 79, against every tile cut alike or none; [197 and 77,3072] x [3072,768] in three slices, which only
+// powers of two did not allow, 16.9 -> 16.0 and 11.7 -> 10.1; on nine sizes the choice is 0 to 4 % behind the best tile and cut).  Fitted to 120 products of 1e8 to
 // 2e11 multiplications with every tile and 70 of up to 1500 tiles of 32 x 32 with every tile and cut (6, 4, 4 and 4 % rms); the choice
 // is 0.4 % behind the best one on average.  Per value of C a small tile costs more (each of its operands serves fewer products), but its
 // rounds come in smaller units.  A k_us of 10.24 per 64 x 64 would be the matrix cores' peak.
@@ -440,7 +446,7 @@ constexpr int N_SHAPES = 4;
 
 struct Choice {
     int shape = 0;
-    uint32_t slices = 1, slice_k = 0;
+    uint32_t full = 0, slices = 1, slice_k = 0;  // full: whole tiles of an XCD's run where others are cut
     double us = 0.0;
 };
 
@@ -451,23 +457,25 @@ Choice choose(size_t batch, size_t m, size_t n, size_t k, size_t cus_per_xcd, bo
     for (int s = 0; s < N_SHAPES; s++) {
         const Shape &sh = SHAPES[s];
         const size_t chunk = (((m + sh.bm - 1) / sh.bm) * ((n + sh.bn - 1) / sh.bn) * batch + 7) / 8;
-        for (uint32_t want = 1; want <= 8; want *= 2) {
-            if (want > 1 && (!cut || batch != 1 || k < 128 * (size_t)want || chunk * 8 > GEMM_COUNTERS)) break;
+        const size_t rem = chunk % cus_per_xcd, whole = chunk / cus_per_xcd;  // tiles of a last round that is partly empty; rounds before it
+        auto round_us = [&](size_t values) { return sh.block_us + sh.k_us * (double)std::max<size_t>(values, sh.step) / 768.0; };
+        for (uint32_t want = 1; want <= 8; want++) {
+            if (want > 1 && (!cut || batch != 1 || k < 128 * (size_t)want || rem == 0 || rem * 8 > GEMM_COUNTERS)) break;
             const size_t slice_k = ((k + want - 1) / want + sh.step - 1) / sh.step * sh.step, slices = slice_k ? (k + slice_k - 1) / slice_k : 1;
             if (want > 1 && slices != want) continue;
             // A grid ends at 2^32 threads: a few rows with 2^29 columns are more blocks of 32 x 32 than that.
-            if (s < N_SHAPES - 1 && chunk * 8 * want * 256 > 0xffffffffu) break;
-            const size_t rounds = (chunk * want + cus_per_xcd - 1) / cus_per_xcd;
-            double us = sh.launch_us + (double)rounds * (sh.block_us + sh.k_us * (double)std::max<size_t>(slice_k, sh.step) / 768.0) * (rounds == 1 ? sh.lone : 1.0);
-            if (want > 1) us += 0.8 + want * (sh.slice_us + (double)(chunk * 8) * sh.bm * sh.bn * sizeof(float) / 2.5e6);
-            if (best.us == 0.0 || us < best.us) best = {s, want, (uint32_t)slice_k, us};
+            if (s < N_SHAPES - 1 && (chunk + rem * (want - 1)) * 8 * 256 > 0xffffffffu) break;
+            const size_t last = want == 1 ? rem != 0 : (rem * want + cus_per_xcd - 1) / cus_per_xcd;
+            double us = sh.launch_us + ((double)whole * round_us(k) + (double)last * round_us(want == 1 ? k : slice_k)) * (whole + last == 1 ? sh.lone : 1.0);
+            if (want > 1) us += 0.8 + want * (sh.slice_us + (double)(rem * 8) * sh.bm * sh.bn * sizeof(float) / 2.5e6);
+            if (best.us == 0.0 || us < best.us) best = {s, (uint32_t)(whole * cus_per_xcd), want, (uint32_t)slice_k, us};
         }
     }
     return best;
 }
 
 template <bool AKC, bool BKC> void launch_tiles(const DeviceCtx &ctx, const GemmArgs &g, int shape, bool vec) {
-    const dim3 grid(g.chunk * 8 * g.slices), block(256);
+    const dim3 grid((g.full + (g.chunk - g.full) * g.slices) * 8), block(256);
 #define TILES(...)                                                                                                                      \
     do {                                                                                                                                \
         if (vec) hipLaunchKernelGGL((gemm_f32_tiles<AKC, BKC, __VA_ARGS__, 4>), grid, block, 0, ctx.stream, g);                         \
@@ -625,7 +633,7 @@ int launch_gemm_f32(DeviceCtx &ctx, float *c, const float *a, const float *b, co
     Choice ch = choose(batch, m, n, k, cus, ctx.gemm_split_k);
     if (ch.slices > 1) {
         const Shape &cut = SHAPES[ch.shape];
-        const size_t cut_tiles = ((m + cut.bm - 1) / cut.bm * ((n + cut.bn - 1) / cut.bn) + 7) / 8 * 8;
+        const size_t cut_tiles = ((m + cut.bm - 1) / cut.bm * ((n + cut.bn - 1) / cut.bn) + 7) / 8 * 8 - 8 * (size_t)ch.full;
         const int rc = gemm_partials(ctx, cut_tiles * ch.slices * cut.bm * cut.bn * sizeof(float));
         if (rc == AHIP_ERR_OOM) ch = choose(batch, m, n, k, cus, false);  // no room: whole
         else if (rc) return rc;
@@ -646,6 +654,7 @@ int launch_gemm_f32(DeviceCtx &ctx, float *c, const float *a, const float *b, co
         g.group_n = (uint32_t)((gx + groups - 1) / groups);
     }
     g.slices = ch.slices;
+    g.full = ch.slices > 1 ? ch.full : g.chunk;
     g.slice_k = ch.slices > 1 ? ch.slice_k : (uint32_t)k;
     if (g.slices > 1) {
         g.partials = static_cast<float *>(ctx.gemm_partials);

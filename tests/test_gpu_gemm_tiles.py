@@ -184,3 +184,24 @@ def test_more_steps_than_32_bit_offsets_reach(ctx, case):
     finally:
         for x in (da, db, dc):
             ctx.free(x)
+
+
+# whole rounds of tiles and a last one that is cut along k, in two to eight slices and for every tile, ragged; then sizes that are one cut round
+@pytest.mark.parametrize("m,n,k", [(1536, 1536, 1536), (2500, 2000, 1000), (2499, 1999, 1001), (3152, 768, 3072), (1100, 1000, 4100), (4200, 2100, 2050), (9000, 300, 1030),
+                                   (197, 768, 3072), (77, 768, 3072), (300, 200, 1100)])
+@pytest.mark.parametrize("trans_b", [False, True])
+def test_last_round_cut_along_k(ctx, case, m, n, k, trans_b):
+    case(f"gemm [{m},{k}] x [{k},{n}] trans_b {trans_b}")
+    rng = np.random.default_rng(m)
+    a, b = (rng.integers(-3, 4, size=s).astype(np.float32) for s in ((m, k), (n, k) if trans_b else (k, n)))
+    res = rng.integers(-3, 4, size=(m, n)).astype(np.float32)
+    da, db, dr, dc = ctx.upload(a), ctx.upload(b), ctx.upload(res), ctx.upload(np.full((m, n), 7.0, np.float32))
+    # float32 products of integers below 2^24 are exact in any order, BLAS's too
+    want = np.matmul(a, b.T if trans_b else b)
+    try:
+        for _ in range(3):
+            ctx.gemm_raw(dc.ptr, da.ptr, db.ptr, dr.ptr, 1, m, n, k, trans_b=trans_b, c0_rs=n, c0_cs=1, alpha=1.0, beta=1.0)
+            assert_bits_equal(ctx.download(dc, (m, n)), want + res, "product and residual")
+    finally:
+        for x in (da, db, dr, dc):
+            ctx.free(x)
