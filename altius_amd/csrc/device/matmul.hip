@@ -71,6 +71,8 @@ struct GemmArgs {
     float alpha, beta;
     int act;
     float act_alpha, act_beta;
+    // The blocks of a CU all start together, and go out of step by priorities: one's first loads and results beside another's products.
+    int apart;
 };
 
 // Four floats that blocks on any XCD read and write.
@@ -187,6 +189,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_f32_tiles(GemmArgs g) 
     constexpr int CP = BN + 4, PASS_ROWS = 32 * WM, SUMS = WK * PASS_ROWS * CP;  // the epilogue's [WK][PASS_ROWS][CP]
     __shared__ __align__(16) float lds[S * STAGE > SUMS ? S * STAGE : SUMS];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if (WK == 4 && g.apart) __builtin_amdgcn_s_setprio(3);
     const int wk = wave / (WM * WN), wmn = wave % (WM * WN), wm = wmn / WN, wn = wmn % WN;
     const int lr = lane & 31, lk = lane >> 5;
 
@@ -285,6 +288,12 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_f32_tiles(GemmArgs g) 
         acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[h].at(i, s), fb[h].at(j, s), acc[i][j], 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
     };
+    if (WK == 4 && g.apart) {
+        const uint32_t turn = (blockIdx.x >> 8) % 3;
+        if (turn == 0) __builtin_amdgcn_s_setprio(0);
+        else if (turn == 1) __builtin_amdgcn_s_setprio(1);
+        else __builtin_amdgcn_s_setprio(2);
+    }
     wait_loads_and_barrier<(S - 1) * LOADS>();
     read(0, 0);
     uint32_t cur = 0;
@@ -319,6 +328,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_f32_tiles(GemmArgs g) 
     for (uint32_t kt = min(nk, (uint32_t)S); kt > 0; kt--) step(std::false_type());
     wait_loads_and_barrier<0>();
 
+    if (WK == 4 && g.apart) __builtin_amdgcn_s_setprio(3);
     // Epilogue, TA passes of PASS_ROWS rows: accumulator e of lane l is row 8 (e / 4) + 4 (l / 32) + e % 4, column l % 32 of its
     // tile; through LDS the WK sums of an element meet and rows of C are stored 16 bytes per lane.
     const size_t c_at = (size_t)zo * g.c_bs + (size_t)zi * g.c_bs2;
@@ -656,6 +666,10 @@ int launch_gemm_f32(DeviceCtx &ctx, float *c, const float *a, const float *b, co
     g.slices = ch.slices;
     g.full = ch.slices > 1 ? ch.full : g.chunk;
     g.slice_k = ch.slices > 1 ? ch.slice_k : (uint32_t)k;
+    // Up to the three blocks of 32 x 32 that a CU holds ([197,768] x [768,2304 / 3072] 10.4 -> 10.15 us, 13.6 -> 13.25, [1024,768] x [768,768]
+    // 13.9 -> 13.5, [1024,3072] x [3072,768] 42.8 -> 41.8; of 4713 tiles the later ones starve, 82 -> 87, cut ones gain nothing, and
+    // 64 x 64 tiles lose 7 % of three rounds and more).
+    g.apart = ch.slices == 1 && g.chunk <= 3 * cus;
     if (g.slices > 1) {
         g.partials = static_cast<float *>(ctx.gemm_partials);
         g.counters = ctx.gemm_counters;
