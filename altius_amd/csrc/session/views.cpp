@@ -750,7 +750,8 @@ bool HipSession::run_attention_rows(NodeId id, std::map<ValueId, DeviceTensor> &
     const bool q_rows = head_op.trans_a == Q.stored_transposed, k_rows = head_op.trans_b != K.stored_transposed, v_rows = tail_op.trans_b == V.stored_transposed;
     auto extent = [](const MatOperand &o, size_t r) { return (o.stored_transposed ? o.cols : o.rows) == r && (o.stored_transposed ? o.rows : o.cols) == 64; };
     if (!q_rows || !k_rows || !v_rows || !extent(Q, tq) || !extent(K, tk) || !extent(V, tk)) return true;
-    if (Q.batch != batch || (K.batch != batch && K.batch != 1) || (V.batch != batch && V.batch != 1)) return true;
+    // (Keys or values that all heads share make one tall product of the heads' rows, which may add up in another order.)
+    if (Q.batch != batch || K.batch != batch || V.batch != batch) return true;
     std::vector<int64_t> qs, ks, vs;
     if (!operand_batch_strides(bd, Q.bdims, Q.bstr, in[0]->strides.empty(), tq * 64, Q.batch, &qs) ||
         !operand_batch_strides(bd, K.bdims, K.bstr, in[1]->strides.empty(), tk * 64, K.batch, &ks) ||

@@ -115,6 +115,31 @@ def test_rows_without_a_finite_score(case):
     assert_bits_equal(got, want, "one kernel and the nodes apart")
 
 
+@pytest.mark.parametrize("shared", ["keys", "values", "both"])
+@pytest.mark.parametrize("heads,t", [(12, 77), (40, 200), (3, 50)])
+def test_heads_that_share_keys_or_values(case, shared, heads, t):
+    """One [t, 64] matrix for all heads: its product is one of all heads' rows, and the nodes run apart after they were held."""
+    case(f"{heads} heads of {t} share {shared}")
+    m = Model(opset_version=13)
+    one, own = [64, t], [1, heads, 64, t]
+    shapes = [[1, heads, t, 64], own if shared == "values" else one, [1, heads, t, 64] if shared == "keys" else [t, 64]]
+    q, k, v = (m.new_val_named_and_shaped(n, s) for n, s in zip("qkv", shapes))
+    for x in (q, k, v):
+        m.add_input(x)
+    s, s2, p, v2, o = (m.new_val() for _ in range(5))
+    m.add_node(Op.MatMul, [q, k], [s])
+    m.add_node(Op.Div, [s, m.new_initializer(np.array(8.0, np.float32))], [s2])
+    m.add_node(Op.Softmax, [s2], [p], axis=-1)
+    m.add_node(Op.Mul, [v, m.new_initializer(np.array(1.0, np.float32))], [v2])
+    m.add_node(Op.MatMul, [p, v2], [o])
+    m.add_output(o)
+    rng = np.random.default_rng(t)
+    x = [rng.standard_normal(d).astype(np.float32) for d in shapes]
+    together, apart = HipSessionBuilder(m).build(), HipSessionBuilder(m).with_strided_views(False).build()
+    for _ in range(2):
+        assert_bits_equal(together.run(x)[0], apart.run(x)[0], "held and run apart, and apart")
+
+
 @pytest.mark.parametrize("tq,tk", [(77, 77), (197, 197), (40, 447)])
 def test_no_scores_in_memory(case, tq, tk):
     """Where the probabilities are asked for the nodes run apart, which takes blocks for the scores and for them."""
