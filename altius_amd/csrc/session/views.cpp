@@ -368,8 +368,10 @@ void HipSession::plan_views(bool fused_attention) {
             if (it == users.end() || it->second.size() != 1) continue;
             const Node &bn = g.nodes[*it->second.begin()];
             if (bn.op.kind == OpKind::BatchNormalization && !bn.op.training_mode && bn.inputs.size() == 5 && bn.inputs[0] == v && bn.outputs.size() == 1) {
-                bool constant = true;  // its four parameters are weights
-                for (size_t k = 1; k < 5; k++) constant = constant && bn.inputs[k] != v && g.inits.count(bn.inputs[k]);
+                bool constant = true;  // its four parameters are weights that no input of the graph can stand in for
+                for (size_t k = 1; k < 5; k++)
+                    constant = constant && bn.inputs[k] != v && g.inits.count(bn.inputs[k]) &&
+                               std::find(g.inputs.begin(), g.inputs.end(), bn.inputs[k]) == g.inputs.end();
                 if (constant) {
                     mp.has_norm = true;
                     mp.norm = *it->second.begin();

@@ -85,6 +85,26 @@ def test_behind_a_convolution(case, geometry, after):
         assert together.copies_avoided() == 1
 
 
+def test_norm_whose_scale_an_input_replaces(case):
+    """An initializer that is an input of the graph too: the run's value counts."""
+    case("conv, BatchNormalization with a scale that is an input")
+    m = Model(opset_version=13)
+    x = m.new_val_named_and_shaped("x", [1, 3, 9, 9])
+    m.add_input(x)
+    rng = np.random.default_rng(2)
+    const = lambda *s: m.new_initializer(rng.random(s).astype(np.float32) + np.float32(0.5))  # noqa: E731
+    c, y, scale = m.new_val(), m.new_val(), const(5)
+    m.add_input(scale)
+    m.add_node(Op.Conv2d, [x, const(5, 3, 3, 3)], [c], kernel_shape=[3, 3], pads=[1] * 4)
+    m.add_node(Op.BatchNormalization, [c, scale, const(5), const(5), const(5)], [y], epsilon=1e-5)
+    m.add_output(y)
+    feed = [rng.standard_normal((1, 3, 9, 9)).astype(np.float32), np.arange(5, dtype=np.float32)]
+    together, apart = HipSessionBuilder(m).build(), HipSessionBuilder(m).with_strided_views(False).build()
+    got = together.run(feed)[0]
+    assert_bits_equal(got, apart.run(feed)[0], "the nodes together and apart")
+    assert np.ptp(got[0, 0]) == 0.0  # scaled by the input's zero
+
+
 # planes below and above every kernel that row sums take, rows that start anywhere, few planes that are cut into parts
 @pytest.mark.parametrize("planes,side", [(3, 1), (5, 2), (70, 4), (40, 7), (3, 14), (9, 16), (12, 28), (6, 33), (4, 56), (3, 64), (2, 113), (1, 301)])
 def test_average_pool(case, ctx, planes, side):
