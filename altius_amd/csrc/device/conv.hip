@@ -589,9 +589,13 @@ int launch_conv2d(DeviceCtx &ctx, float *out, const float *x, const float *w, co
     if (pass.rows * ow > (size_t)1 << 24) pass.images = 0;
     Route route = conv_route(ctx, batch, m, oh, ow, k, group, pass, pointwise, g.w_vec && (pass.rows * ow) % 4 == 0 && (!pointwise || a16(x)));
     if (route == UNFOLDED) {
+        // Without a bias the products of many small images are one launch of matmul_small.hip's kernel, which has no epilogue and adds up in
+        // another order than the tiles that have one: what stands behind such a convolution stays with its own node.  (Where images are taken
+        // in passes, the first pass has the most of them.)
+        const bool takes_post = conv_post && !post.mean && (bias || !gemm_small_batched_fits(pass.images, m, pass.rows * ow, k));
         const int rc = launch_unfolded(ctx, out, x, w, bias, pass, pointwise, batch, c, ih, iw, oc, oh, ow, kh, kw, sh, sw, dh, dw, pad_t, pad_l, group,
-                                       post.mean ? GemmPost() : conv_post ? conv_post->then : GemmPost());
-        if (!rc && conv_post) conv_post->applied = !post.mean;
+                                       takes_post ? conv_post->then : GemmPost());
+        if (!rc && conv_post) conv_post->applied = takes_post;
         if (rc != AHIP_ERR_OOM && rc != AHIP_ERR_UNSUPPORTED) return rc;
         route = conv_route(ctx, batch, m, oh, ow, k, group, Pass(), pointwise, false);  // no room for the copy
     }

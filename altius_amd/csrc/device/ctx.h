@@ -289,7 +289,8 @@ int launch_maxpool(DeviceCtx &ctx, float *out, const float *x, size_t planes, si
                    size_t kh, size_t kw, size_t sh, size_t sw, size_t pad_t, size_t pad_l);
 // What the operators behind a convolution would do to its result, done while it is written: BatchNormalization with one value
 // per output channel (mean null: none), then an activation and a residual as GemmPost has them.  Each step rounds as its own kernel
-// would.  launch_conv2d says in `applied` whether it did all of it or (a normalisation in front of a route that has none) nothing.
+// would.  launch_conv2d says in `applied` whether it did all of it or (a normalisation in front of a route that has none, a product of
+// many small images, which has no epilogue) nothing.
 struct ConvPost {
     const float *mean = nullptr, *var = nullptr, *scale = nullptr, *shift = nullptr;
     float eps = 0.0f;

@@ -85,6 +85,20 @@ def test_behind_a_convolution(case, geometry, after):
         assert together.copies_avoided() == 1
 
 
+# From 128 images on a product of small ones without a bias is the kernel of many small matrices, in one chunk of k and in several.
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("after", ["relu", "hard_swish", "add"])
+@pytest.mark.parametrize("geometry", [(128, 64, 14, 192, 1, 1, 1), (128, 1024, 7, 192, 1, 1, 1), (144, 64, 14, 200, 1, 1, 1), (127, 64, 14, 192, 1, 1, 1)])
+def test_behind_products_of_many_images(case, geometry, after, bias):
+    case(f"conv {geometry}, {after}, bias {bias}")
+    m, x_dims, r_dims = graph(*geometry, after, bias=bias)
+    rng = np.random.default_rng(6)
+    x, r = (3 * rng.standard_normal(d).astype(np.float32) for d in (x_dims, r_dims))
+    together, apart = HipSessionBuilder(m).build(), HipSessionBuilder(m).with_strided_views(False).build()
+    assert_bits_equal(together.run([x, r])[0], apart.run([x, r])[0], "the nodes together and apart")
+    assert together.copies_avoided() == (1 if bias or geometry[0] < 128 else 0)
+
+
 def test_norm_whose_scale_an_input_replaces(case):
     """An initializer that is an input of the graph too: the run's value counts."""
     case("conv, BatchNormalization with a scale that is an input")
