@@ -137,7 +137,7 @@ template <bool KC, int W, int WK, int WAVES, int VEC> struct Loader {
     static constexpr int PER = 64 * VEC, TILE = W * BK, COUNT = TILE * WK / PER / WAVES;
     static_assert(COUNT * PER * WAVES == TILE * WK, "whole instructions");
     uint32_t off[COUNT];  // byte offsets of this lane's pieces of the tile to load next
-    uint32_t lo, hi, bytes;  // the buffer: from the first tile that off counts from to the operand's end
+    uint32_t lo = 0, hi = 0, bytes = 0;  // the buffer: from the first tile that off counts from to the operand's end; empty where there is none (k = 0)
     // A tile that starts at p, floats before the operand's end, with k_left values of k.
     __device__ __forceinline__ void start(const float *p, uint64_t floats, uint32_t ld, uint32_t k_left, int wave, int lane) {
         const uint64_t at = (uint64_t)(uintptr_t)p;

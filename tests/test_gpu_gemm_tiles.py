@@ -205,3 +205,21 @@ def test_last_round_cut_along_k(ctx, case, m, n, k, trans_b):
     finally:
         for x in (da, db, dr, dc):
             ctx.free(x)
+
+
+@pytest.mark.parametrize("trans_a", [False, True])
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("m,n", [(1, 1), (33, 70), (1646, 132), (1025, 3071), (6300, 3073)])
+def test_sums_of_nothing(ctx, case, m, n, trans_a, trans_b):
+    """k = 0: no operand is read (there is none), and the result is beta C0, or zeros."""
+    case(f"gemm [{m},0] x [0,{n}] trans {trans_a} {trans_b}")
+    c0 = np.random.default_rng(m).integers(-9, 10, size=(m, n)).astype(np.float32)
+    d0, dc = ctx.upload(c0), ctx.upload(np.full((m, n), 7.0, np.float32))
+    try:
+        ctx.gemm_raw(dc.ptr, None, None, d0.ptr, 1, m, n, 0, trans_a, trans_b, m if trans_a else 1, 1 if trans_b else n, n, c0_rs=n, c0_cs=1, alpha=3.0, beta=2.0)
+        assert_bits_equal(ctx.download(dc, (m, n)), 2.0 * c0, "C0")
+        ctx.gemm_raw(dc.ptr, None, None, None, 1, m, n, 0, trans_a, trans_b, m if trans_a else 1, 1 if trans_b else n, n)
+        assert_bits_equal(ctx.download(dc, (m, n)), np.zeros((m, n), np.float32), "zeros")
+    finally:
+        ctx.free(d0)
+        ctx.free(dc)
