@@ -124,11 +124,15 @@ template <int N> __device__ __forceinline__ void wait_loads_and_barrier() { asm 
 
 // A wavefront's VEC floats per lane from a buffer to LDS, in asm: of loads it knows the compiler waits for all before any LDS read that it
 // cannot prove independent of them, which would undo the prefetch.  Waits are wait_loads_and_barrier's.  (m0 and an SGPR that a vector
-// instruction wrote need one and five cycles before the load reads them.)
+// instruction wrote need one and five cycles before the load reads them.  The compiler warns of any clobber that names m0, which it
+// reserves; named, it does not take a value of its own in m0 to last across the asm.)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 template <int VEC> __device__ __forceinline__ void load_to_lds(i32x4 rsrc, uint32_t off, uint32_t to) {
-    if constexpr (VEC == 4) asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(off), "s"(rsrc), "s"(to) : "memory");
-    else asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dword %0, %1, 0 offen lds" ::"v"(off), "s"(rsrc), "s"(to) : "memory");
+    if constexpr (VEC == 4) asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds" ::"v"(off), "s"(rsrc), "s"(to) : "m0", "memory");
+    else asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dword %0, %1, 0 offen lds" ::"v"(off), "s"(rsrc), "s"(to) : "m0", "memory");
 }
+#pragma clang diagnostic pop
 
 // Copies an operand's tiles to LDS: [WK][W][BK] (KC, pieces exchanged) or [WK][BK][W], VEC floats per lane and instruction.  The
 // operand is addressed as a buffer that ends behind its last element.  A lane whose k lies past the end asks for an offset behind any
