@@ -177,6 +177,13 @@ HipSession::~HipSession() {
     }
 }
 
+HipSession::RunNotes::~RunNotes() {
+    s->pending_attn_.clear();
+    s->absorbed_.clear();
+    s->passed_over_.clear();
+    s->attention_held_.clear(), s->attention_operands_.clear();
+}
+
 bool HipSession::allocate(const TypedFixedShape &shape, DeviceTensor *out, SessionError *err) {
     out->dims = shape.dims;
     out->elem_ty = shape.elem_ty;
@@ -296,12 +303,9 @@ bool HipSession::run(const std::vector<Tensor> &inputs, std::vector<Tensor> *out
         eager_runs_[key]++;
     }
 
+    const RunNotes notes(this);
     std::map<ValueId, DeviceTensor> values;
     copies_avoided_ = 0;
-    pending_attn_.clear();
-    absorbed_.clear();
-    passed_over_.clear();
-    attention_held_.clear(), attention_operands_.clear();
     std::vector<hipEvent_t> events;
     // Nothing may still read a block when it goes back to the pool for another run, and input
     // tensors must outlive their uploads: every exit path synchronises first.
@@ -401,12 +405,9 @@ bool HipSession::run_device(const std::vector<DeviceTensor> &inputs, std::vector
                         std::to_string(g.inputs.size()));
     if (hipSetDevice(ctx_.device) != hipSuccess) return fail(err, SessionError::Hip, "hipSetDevice failed");
 
+    const RunNotes notes(this);
     std::map<ValueId, DeviceTensor> values;
     copies_avoided_ = 0;
-    pending_attn_.clear();
-    absorbed_.clear();
-    passed_over_.clear();
-    attention_held_.clear(), attention_operands_.clear();
     for (size_t i = 0; i < g.inputs.size(); i++) {
         if (!inputs[i].ptr && inputs[i].nbytes())
             return fail(err, SessionError::Argument, "run_device: input " + std::to_string(i) + " has no device pointer");
@@ -477,12 +478,9 @@ void HipSession::drop_graphs() {
 bool HipSession::try_capture(const std::string &key, const std::vector<Tensor> &inputs, SessionError *err) {
     const Graph &g = model_.graph;
     CapturedRun run;
+    const RunNotes notes(this);
     std::map<ValueId, DeviceTensor> values;
     copies_avoided_ = 0;
-    pending_attn_.clear();
-    absorbed_.clear();
-    passed_over_.clear();
-    attention_held_.clear(), attention_operands_.clear();
     for (size_t i = 0; i < g.inputs.size(); i++) {
         DeviceTensor d;
         if (!allocate(TypedFixedShape{inputs[i].dims(), inputs[i].elem_ty()}, &d, err)) return false;
@@ -535,7 +533,6 @@ bool HipSession::try_capture(const std::string &key, const std::vector<Tensor> &
         // plan freed them (and were reused inside the recording, which stream order allows); take every one of
         // them out of the pool for as long as the graph lives.
         values.clear();
-        pending_attn_.clear();
         std::sort(capture_allocs_.begin(), capture_allocs_.end());
         capture_allocs_.erase(std::unique(capture_allocs_.begin(), capture_allocs_.end()), capture_allocs_.end());
         for (const auto &a : capture_allocs_)

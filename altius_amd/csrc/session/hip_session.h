@@ -228,6 +228,13 @@ private:
     bool try_defer_attention(const Node &node, const Op &op, const std::vector<DeviceTensor *> &in,
                              const std::vector<TypedFixedShape> &shapes, std::vector<DeviceTensor> *outs, SessionError *err);
     bool run_attention_tail(const Op &op, const std::vector<DeviceTensor *> &in, DeviceTensor *out, SessionError *err);
+    // What nodes have left for the ones behind them is gone when a run ends, also when it fails in between: the blocks go back to the pool
+    // and do not outlive it.
+    struct RunNotes {
+        HipSession *s;
+        explicit RunNotes(HipSession *session) : s(session) {}
+        ~RunNotes();
+    };
     // Runs the activation a tensor still owes (pending_op) into a new buffer.
     bool apply_pending(DeviceTensor *t, SessionError *err);
 

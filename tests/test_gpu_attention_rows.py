@@ -1,14 +1,17 @@
 """Attention as one kernel: the bits of its nodes run apart, in every form of scale, condition and mask, at the edges of its tiles and
 for every order of sums that the products alone would have; and apart after all where an operand is not one that the kernel takes."""
+import ctypes
+
 import numpy as np
 import pytest
 
+from altius_amd._lib import AltiusHipError
 from altius_amd.graph import Model, Op
 from altius_amd.session import HipSessionBuilder
 from conftest import assert_bits_equal
+from test_gpu_graph_replay import hip_runtime
 
 pytestmark = pytest.mark.gpu
-
 
 
 def attention(b, h, tq, tk, d=64, scale="div", cond=None, mask=(1, 1, 1, "k"), value_late=False, k_form="transposed", seen=False, rewritten=True):
@@ -151,6 +154,41 @@ def test_no_scores_in_memory(case, tq, tk):
         session.run([np.zeros(dims, np.float32) for dims in shapes.values()])
         allocations.append(session.device_allocations())
     assert allocations[0] < allocations[1]
+
+
+@pytest.mark.parametrize("fused", [False, True])
+def test_a_run_that_fails_between_the_products(case, fused):
+    """The values' product, due when the first product's nodes already hold their operands, broadcasts in a way that is refused: the run
+    raises, and the session gives all its memory back when it goes."""
+    case(f"attention whose values cannot be computed, one-kernel attention allowed: {fused}")
+    tq, tk = 1 << 16, 50
+    m = Model(opset_version=13)
+    shapes = [[2, 3, tq, 64], [2, 3, 64, tk], [2, 1, tk, 8], [1, 3, 8, 64]]
+    q, k, a, b = (m.new_val_named_and_shaped(n, s) for n, s in zip("qkab", shapes))
+    for x in (q, k, a, b):
+        m.add_input(x)
+    s, p, v, o = (m.new_val() for _ in range(4))
+    m.add_node(Op.MatMul, [q, k], [s])
+    m.add_node(Op.Softmax, [s], [p], axis=-1)
+    m.add_node(Op.MatMul, [a, b], [v])
+    m.add_node(Op.MatMul, [p, v], [o])
+    m.add_output(o)
+    hip = hip_runtime()
+
+    def free_bytes():
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+
+    x = [np.zeros(d, np.float32) for d in shapes]
+    before = []
+    for _ in range(3):
+        session = HipSessionBuilder(m).with_fused_attention(fused).build()
+        before.append(free_bytes())
+        with pytest.raises(AltiusHipError, match="broadcast against each other partially"):
+            session.run(x)
+        session.close()
+    assert before[0] - before[2] < x[0].nbytes // 2, "device memory that a failed run kept"
 
 
 def test_replayed(case):
