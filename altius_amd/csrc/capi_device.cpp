@@ -506,6 +506,13 @@ int ahip_gemm(ahip_ctx *ctx, float *c, const float *a, const float *b, const flo
     return altius::caught_at_boundary("ahip_gemm");
 }
 
+int ahip_gemm_f32_grid(size_t batch, size_t m, size_t n, size_t k, size_t *blocks, int *slices) try {
+    if (!blocks || !slices || !batch || !m || !n) return AHIP_ERR_ARG;
+    return altius::gemm_f32_grid(altius::DeviceCtx(), batch, m, n, k, blocks, slices);
+} catch (...) {
+    return altius::caught_at_boundary("ahip_gemm_f32_grid");
+}
+
 int ahip_gemm_batch2(ahip_ctx *ctx, float *c, const float *a, const float *b, const float *c0, size_t batch_outer,
                      size_t batch_inner, size_t m, size_t n, size_t k, int trans_a, int trans_b, size_t lda, size_t ldb,
                      size_t ldc, const size_t a_batch_strides[2], const size_t b_batch_strides[2],

@@ -205,6 +205,9 @@ double gemm_f32_us(const DeviceCtx &ctx, size_t batch, size_t m, size_t n, size_
 // How many chains of sums over k, 16 values each in turn, meet in an element of that product (1, 2 or 4); 0: it is no product of whole
 // tiles (many small matrices, or k cut into slices).
 int gemm_f32_chains(const DeviceCtx &ctx, size_t batch, size_t m, size_t n, size_t k);
+// The tiles' launch for that product, and into how many slices those of its last round are cut along k; AHIP_ERR_UNSUPPORTED: more tiles
+// than a grid holds.
+int gemm_f32_grid(const DeviceCtx &ctx, size_t batch, size_t m, size_t n, size_t k, size_t *blocks, int *slices);
 
 // Many small products at once (matmul_small.hip): one block per matrix.  C = A B, A with unit stride along k.
 bool gemm_small_batched_fits(size_t batch, size_t m, size_t n, size_t k);

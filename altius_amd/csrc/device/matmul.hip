@@ -478,7 +478,7 @@ Choice choose(size_t batch, size_t m, size_t n, size_t k, size_t cus_per_xcd, bo
             const size_t slice_k = ((k + want - 1) / want + sh.step - 1) / sh.step * sh.step, slices = slice_k ? (k + slice_k - 1) / slice_k : 1;
             if (want > 1 && slices != want) continue;
             // A grid ends at 2^32 threads: a few rows with 2^29 columns are more blocks of 32 x 32 than that.
-            if (s < N_SHAPES - 1 && (chunk + rem * (want - 1)) * 8 * 256 > 0xffffffffu) break;
+            if ((s < N_SHAPES - 1 || want > 1) && (chunk + rem * (want - 1)) * 8 * 256 > 0xffffffffu) break;
             const size_t last = want == 1 ? rem != 0 : (rem * want + cus_per_xcd - 1) / cus_per_xcd;
             double us = sh.launch_us + ((double)whole * round_us(k) + (double)last * round_us(want == 1 ? k : slice_k)) * (whole + last == 1 ? sh.lone : 1.0);
             if (want > 1) us += 0.8 + want * (sh.slice_us + (double)(rem * 8) * sh.bm * sh.bn * sizeof(float) / 2.5e6);
@@ -487,6 +487,21 @@ Choice choose(size_t batch, size_t m, size_t n, size_t k, size_t cus_per_xcd, bo
     }
     return best;
 }
+
+// A product's grid: of each XCD's run of tiles those that are whole, and the slices of the others.
+struct Grid {
+    size_t gx = 0, gy = 0, tiles = 0, chunk = 0, full = 0, blocks = 0;
+    Grid(const Choice &ch, size_t batch, size_t m, size_t n) {
+        const Shape &sh = SHAPES[ch.shape];
+        gy = (m + sh.bm - 1) / sh.bm, gx = (n + sh.bn - 1) / sh.bn, tiles = gx * gy * batch, chunk = (tiles + 7) / 8;
+        full = ch.slices > 1 ? ch.full : chunk;
+        blocks = (full + (chunk - full) * ch.slices) * 8;
+    }
+    bool fits(size_t batch) const {
+        const size_t lim = (size_t)1 << 31;
+        return gx * gy < lim && batch < lim && tiles < ((size_t)1 << 32) && blocks * 256 <= 0xffffffffu;
+    }
+};
 
 template <bool AKC, bool BKC> void launch_tiles(const DeviceCtx &ctx, const GemmArgs &g, int shape, bool vec) {
     const dim3 grid((g.full + (g.chunk - g.full) * g.slices) * 8), block(256);
@@ -584,6 +599,13 @@ int gemm_f32_chains(const DeviceCtx &ctx, size_t batch, size_t m, size_t n, size
     return ch.slices > 1 ? 0 : (int)(SHAPES[ch.shape].step / BK);
 }
 
+int gemm_f32_grid(const DeviceCtx &ctx, size_t batch, size_t m, size_t n, size_t k, size_t *blocks, int *slices) {
+    const Choice ch = choose(batch, m, n, k, ctx.cus_per_xcd ? (size_t)ctx.cus_per_xcd : 32, ctx.gemm_split_k);
+    const Grid grid(ch, batch, m, n);
+    *blocks = grid.blocks, *slices = (int)ch.slices;
+    return grid.fits(batch) ? AHIP_OK : AHIP_ERR_UNSUPPORTED;
+}
+
 int launch_gemm_f32(DeviceCtx &ctx, float *c, const float *a, const float *b, const float *c0, size_t batch_outer, size_t batch_inner, size_t m,
                     size_t n, size_t k, int trans_a, int trans_b, size_t lda, size_t ldb, size_t ldc, const size_t a_batch_strides[2],
                     const size_t b_batch_strides[2], const size_t c_batch_strides[2], size_t c0_row_stride, size_t c0_col_stride, float alpha,
@@ -647,28 +669,27 @@ int launch_gemm_f32(DeviceCtx &ctx, float *c, const float *a, const float *b, co
     Choice ch = choose(batch, m, n, k, cus, ctx.gemm_split_k);
     if (ch.slices > 1) {
         const Shape &cut = SHAPES[ch.shape];
-        const size_t cut_tiles = ((m + cut.bm - 1) / cut.bm * ((n + cut.bn - 1) / cut.bn) + 7) / 8 * 8 - 8 * (size_t)ch.full;
-        const int rc = gemm_partials(ctx, cut_tiles * ch.slices * cut.bm * cut.bn * sizeof(float));
+        const Grid grid(ch, batch, m, n);
+        const int rc = gemm_partials(ctx, (grid.chunk - grid.full) * 8 * ch.slices * cut.bm * cut.bn * sizeof(float));
         if (rc == AHIP_ERR_OOM) ch = choose(batch, m, n, k, cus, false);  // no room: whole
         else if (rc) return rc;
     }
     const Shape &sh = SHAPES[ch.shape];
-    const size_t gy = (m + sh.bm - 1) / sh.bm, gx = (n + sh.bn - 1) / sh.bn, tiles = gx * gy * batch;
-    if (gx * gy >= lim || batch >= lim || (tiles + 7) / 8 * 8 * ch.slices * 256 > 0xffffffffu)
-        return ctx.fail(AHIP_ERR_UNSUPPORTED, "gemm: more tiles than a grid holds");
-    g.tiles_n = (uint32_t)gx;
-    g.tiles_m = (uint32_t)gy;
-    g.tiles = (uint32_t)tiles;
-    g.chunk = (uint32_t)((tiles + 7) / 8);
+    const Grid grid(ch, batch, m, n);
+    if (!grid.fits(batch)) return ctx.fail(AHIP_ERR_UNSUPPORTED, "gemm: more tiles than a grid holds");
+    g.tiles_n = (uint32_t)grid.gx;
+    g.tiles_m = (uint32_t)grid.gy;
+    g.tiles = (uint32_t)grid.tiles;
+    g.chunk = (uint32_t)grid.chunk;
     {
         // Groups of about 768 columns (measured on [50432,768]x[768,2304..3072] and 4096^3 .. 8192^3: widths of
         // 6 to 16 tile columns are within 1 % of each other and up to 3 % ahead of whole rows of tiles; a single
         // column is 3-6 % behind), all groups equally wide.
-        const size_t group = 768 / sh.bn, groups = (gx + group - 1) / group;
-        g.group_n = (uint32_t)((gx + groups - 1) / groups);
+        const size_t group = 768 / sh.bn, groups = (grid.gx + group - 1) / group;
+        g.group_n = (uint32_t)((grid.gx + groups - 1) / groups);
     }
     g.slices = ch.slices;
-    g.full = ch.slices > 1 ? ch.full : g.chunk;
+    g.full = (uint32_t)grid.full;
     g.slice_k = ch.slices > 1 ? ch.slice_k : (uint32_t)k;
     // Up to the three blocks of 32 x 32 that a CU holds ([197,768] x [768,2304 / 3072] 10.4 -> 10.15 us, 13.6 -> 13.25, [1024,768] x [768,768]
     // 13.9 -> 13.5, [1024,3072] x [3072,768] 42.8 -> 41.8; of 4713 tiles the later ones starve, 82 -> 87, cut ones gain nothing, and

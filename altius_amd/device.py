@@ -26,6 +26,13 @@ def xcd_round_robin_holds(cu_count, xcc_of_block):
     return bool(_lib.lib().ahip_xcd_round_robin_holds(int(cu_count), ids.ctypes.data_as(ctypes.POINTER(ctypes.c_uint32)), ids.size))
 
 
+def gemm_f32_grid(batch, m, n, k):
+    """(blocks, slices) of the fp32 kernel's launch for a product of this size (host only); raises where a grid does not hold its tiles."""
+    blocks, slices = ctypes.c_size_t(), ctypes.c_int()
+    check(_lib.lib().ahip_gemm_f32_grid(batch, m, n, k, ctypes.byref(blocks), ctypes.byref(slices)))
+    return blocks.value, slices.value
+
+
 def broadcast_shape(a_dims, b_dims):
     """fixed_dim::broadcast through the C ABI; raises AltiusHipError(Shape) if incompatible."""
     L = _lib.lib()

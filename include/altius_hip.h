@@ -275,6 +275,11 @@ int ahip_gemm(ahip_ctx *ctx, float *c, const float *a, const float *b, const flo
               size_t b_batch_stride, size_t c_batch_stride, size_t c0_row_stride, size_t c0_col_stride, float alpha,
               float beta);
 
+/* The launch that ahip_gemm makes on the fp32 kernel's tiles for a product of this size (no GPU needed): how many blocks of 256 threads,
+ * and into how many slices the tiles of a last, partly empty round are cut along k (1: none is cut).  AHIP_ERR_UNSUPPORTED: more
+ * tiles than a grid holds, which ahip_gemm refuses.  No counterpart in the reference. */
+int ahip_gemm_f32_grid(size_t batch, size_t m, size_t n, size_t k, size_t *blocks, int *slices);
+
 /* ahip_gemm with the batch index split in two: batch z = (z / batch_inner, z % batch_inner), and operand X of
  * that batch starts at x + (z / batch_inner) * x_batch_strides[0] + (z % batch_inner) * x_batch_strides[1]
  * (elements; 0 shares).  Lets a product read or write the heads of a [b, t, h, d] tensor in place (b x h

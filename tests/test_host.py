@@ -37,6 +37,24 @@ def test_no_cpu_fallback_when_library_is_missing(monkeypatch, tmp_path):
         _lib.lib()
 
 
+@pytest.mark.parametrize("batch,m,n,k", [(1, 187840, 187840, 4096), (1, 187841, 187840, 4096), (1, 187840, 187713, 4097), (1, 262000, 131000, 2048),
+                                         (1, 520000, 520000, 1024), (1, 528000, 520000, 1024), (1, 1, 1 << 29, 1024), (1, 100, 1 << 30, 4096), (1 << 20, 64, 64, 64)])
+def test_products_whose_blocks_a_grid_holds_are_taken(batch, m, n, k):
+    """A grid ends at 2^32 threads.  Of a product whose last round of tiles is cut along k only that round's blocks are more than its tiles:
+    the cut never makes a grid too large, whatever the slices times all tiles would be."""
+    blocks, slices = D.gemm_f32_grid(batch, m, n, k)
+    assert blocks * 256 <= 0xFFFFFFFF and 1 <= slices <= 8
+    largest = -(-m // 128) * -(-n // 128) * batch  # tiles of 128 x 128, the fewest there can be
+    assert blocks >= largest
+
+
+def test_a_product_of_more_tiles_than_a_grid_holds_is_refused():
+    for size in [(1, 530000, 530000, 1024), (1, 1 << 20, 1 << 20, 4096), (1 << 24, 1, 1, 1)]:
+        with pytest.raises(AltiusHipError):
+            D.gemm_f32_grid(*size)
+    assert D.gemm_f32_grid((1 << 24) - 8, 1, 1, 1) == ((1 << 24) - 8, 1)
+
+
 def test_in_kernel_k_cut_is_allowed_only_on_a_round_robin_placement():
     """The bf16 GEMM combines the slices of a tile inside one XCD's L2 only if the probe launch showed blocks 0..7
     on eight different XCDs, every block i where block i % 8 ran, and a CU count that is a multiple of eight;
