@@ -87,6 +87,7 @@ def _declare(L):
     f("ahip_cast", [c_void_p, c_void_p, c_void_p, c_int, c_int, c_size_t])
     f("ahip_batchnorm", [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_size_t, c_size_t, c_size_t,
                          c_float])
+    f("ahip_attention_rows_fits", [c_size_t] * 3)
     f("ahip_gemm_f32_grid", [c_size_t] * 4 + [P(c_size_t), P(c_int)])
     f("ahip_gemm", [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p] + [c_size_t] * 4 + [c_int, c_int] + [c_size_t] * 8
       + [c_float, c_float])

@@ -513,6 +513,12 @@ int ahip_gemm_f32_grid(size_t batch, size_t m, size_t n, size_t k, size_t *block
     return altius::caught_at_boundary("ahip_gemm_f32_grid");
 }
 
+int ahip_attention_rows_fits(size_t batch, size_t tq, size_t tk) try {
+    return altius::attention_rows_fits(altius::DeviceCtx(), batch, tq, tk) ? 1 : 0;
+} catch (...) {
+    return altius::caught_at_boundary("ahip_attention_rows_fits");
+}
+
 int ahip_gemm_batch2(ahip_ctx *ctx, float *c, const float *a, const float *b, const float *c0, size_t batch_outer,
                      size_t batch_inner, size_t m, size_t n, size_t k, int trans_a, int trans_b, size_t lda, size_t ldb,
                      size_t ldc, const size_t a_batch_strides[2], const size_t b_batch_strides[2],

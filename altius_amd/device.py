@@ -33,6 +33,11 @@ def gemm_f32_grid(batch, m, n, k):
     return blocks.value, slices.value
 
 
+def attention_rows_fits(batch, tq, tk):
+    """Whether a session runs attention over that many heads, queries and keys (64 columns) as one kernel (host only)."""
+    return bool(_lib.lib().ahip_attention_rows_fits(batch, tq, tk))
+
+
 def broadcast_shape(a_dims, b_dims):
     """fixed_dim::broadcast through the C ABI; raises AltiusHipError(Shape) if incompatible."""
     L = _lib.lib()

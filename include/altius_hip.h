@@ -280,6 +280,10 @@ int ahip_gemm(ahip_ctx *ctx, float *c, const float *a, const float *b, const flo
  * tiles than a grid holds, which ahip_gemm refuses.  No counterpart in the reference. */
 int ahip_gemm_f32_grid(size_t batch, size_t m, size_t n, size_t k, size_t *blocks, int *slices);
 
+/* 1: a session on the fp32 kernels runs MatMul -> scale, condition, mask -> Softmax -> MatMul over this many heads of tq queries, tk keys
+ * and 64 columns as one kernel with the operators' bits; 0: as its nodes (no GPU needed).  No counterpart in the reference. */
+int ahip_attention_rows_fits(size_t batch, size_t tq, size_t tk);
+
 /* ahip_gemm with the batch index split in two: batch z = (z / batch_inner, z % batch_inner), and operand X of
  * that batch starts at x + (z / batch_inner) * x_batch_strides[0] + (z % batch_inner) * x_batch_strides[1]
  * (elements; 0 shares).  Lets a product read or write the heads of a [b, t, h, d] tensor in place (b x h

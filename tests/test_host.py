@@ -48,6 +48,13 @@ def test_products_whose_blocks_a_grid_holds_are_taken(batch, m, n, k):
     assert blocks >= largest
 
 
+def test_attention_of_more_blocks_than_a_grid_holds_runs_as_its_nodes():
+    """A block of 512 threads for 32 queries of a head: 2^23 of them are 2^32 threads, one more than a grid holds."""
+    assert D.attention_rows_fits(12, 197, 197) and D.attention_rows_fits(12, 77, 77)
+    assert D.attention_rows_fits(32, (1 << 23) - 32, 16) and not D.attention_rows_fits(32, (1 << 23) - 31, 16)
+    assert not D.attention_rows_fits(32, (1 << 30), 16)
+
+
 def test_a_product_of_more_tiles_than_a_grid_holds_is_refused():
     for size in [(1, 530000, 530000, 1024), (1, 1 << 20, 1 << 20, 4096), (1 << 24, 1, 1, 1)]:
         with pytest.raises(AltiusHipError):
