@@ -265,6 +265,12 @@ void HipSession::plan_views(bool fused_attention) {
     const auto parents = model_.get_value_parents();
     const Graph &g = model_.graph;
     auto is_output = [&](ValueId v) { return std::find(g.outputs.begin(), g.outputs.end(), v) != g.outputs.end(); };
+    // The [k, n] f32 weights of a product, which no input of the graph can stand in for.
+    auto weight_matrix = [&](const Node &product) -> const Tensor * {
+        auto w = product.inputs.size() > 1 ? g.inits.find(product.inputs[1]) : g.inits.end();
+        if (w == g.inits.end() || std::find(g.inputs.begin(), g.inputs.end(), product.inputs[1]) != g.inputs.end()) return nullptr;
+        return w->second.dims().len() == 2 && w->second.elem_ty() == TensorElemType::F32 ? &w->second : nullptr;
+    };
     std::function<bool(ValueId, int)> view_ok = [&](ValueId v, int depth) -> bool {
         if (depth > 8 || is_output(v)) return false;
         auto it = users.find(v);
@@ -324,13 +330,9 @@ void HipSession::plan_views(bool fused_attention) {
             if (par == parents.end() || is_output(n.inputs[0])) continue;
             const Node &first = g.nodes[par->second];
             auto fu = users.find(n.inputs[0]);
-            auto weights = [&](const Node &p) {
-                auto w = p.inputs.size() > 1 ? g.inits.find(p.inputs[1]) : g.inits.end();
-                return w != g.inits.end() && w->second.dims().len() == 2 && w->second.elem_ty() == TensorElemType::F32 ? &w->second : nullptr;
-            };
-            const Tensor *w = weights(mm);
+            const Tensor *w = weight_matrix(mm);
             if (first.op.kind != OpKind::MatMul || first.outputs.size() != 1 || first.op.trans_a || mm.op.trans_a || fu == users.end() || fu->second.size() != 1 ||
-                !weights(first) || !w)
+                !weight_matrix(first) || !w)
                 continue;
             ActPlanesPlan ap;
             ap.next.consumer = *it->second.begin();
@@ -347,11 +349,11 @@ void HipSession::plan_views(bool fused_attention) {
             if (mm.op.kind != OpKind::MatMul || mm.inputs.size() < 2 || mm.inputs[0] != n.outputs[0] || mm.op.trans_a) continue;
             bool elsewhere = false;
             for (size_t i = 1; i < mm.inputs.size(); i++) elsewhere = elsewhere || mm.inputs[i] == n.outputs[0];
-            auto w = g.inits.find(mm.inputs[1]);
-            if (elsewhere || w == g.inits.end() || w->second.dims().len() != 2 || w->second.elem_ty() != TensorElemType::F32) continue;
+            const Tensor *w = weight_matrix(mm);
+            if (elsewhere || !w) continue;
             PlanesPlan pp;
             pp.consumer = *it->second.begin();
-            pp.next_n = mm.op.trans_b ? w->second.dims()[0] : w->second.dims()[1];
+            pp.next_n = mm.op.trans_b ? w->dims()[0] : w->dims()[1];
             planes_out_[id] = pp;
             planes_consumer_.insert(pp.consumer);
             // The residual Add in front of it (two tensors of one shape) can leave its sum to this kernel.
@@ -466,8 +468,8 @@ void HipSession::plan_views(bool fused_attention) {
             continue;
         bool elsewhere = false;
         for (size_t i = 1; i < m.inputs.size(); i++) elsewhere = elsewhere || m.inputs[i] == m.inputs[0];
-        auto w = g.inits.find(m.inputs[1]);
-        if (elsewhere || w == g.inits.end() || w->second.dims().len() != 2 || w->second.elem_ty() != TensorElemType::F32) continue;
+        const Tensor *w = weight_matrix(m);
+        if (elsewhere || !w) continue;
         // The planes are laid out for [b * t, h * 64] x weights [h * 64, n]: the attention's result must be [b, h, t, 64],
         // the Reshape must merge exactly the heads into the last axis (any other valid reshape, [b, t * h, 64] say, would
         // read the planes with another geometry), and the weights must have h * 64 rows.  Shapes that are not known
@@ -479,10 +481,10 @@ void HipSession::plan_views(bool fused_attention) {
         const size_t merged = ad[1] * 64, rows = ad[0] * ad[2];
         size_t lead = 1;
         for (size_t i = 0; i + 1 < rd.len(); i++) lead *= rd[i];
-        if (rd[rd.len() - 1] != merged || lead != rows || (m.op.trans_b ? w->second.dims()[1] : w->second.dims()[0]) != merged) continue;
+        if (rd[rd.len() - 1] != merged || lead != rows || (m.op.trans_b ? w->dims()[1] : w->dims()[0]) != merged) continue;
         PlanesPlan pp;
         pp.consumer = mm;
-        pp.next_n = m.op.trans_b ? w->second.dims()[0] : w->second.dims()[1];
+        pp.next_n = m.op.trans_b ? w->dims()[0] : w->dims()[1];
         attn_planes_[tid] = pp;
         planes_consumer_.insert(mm);
         planes_pass_.insert(tr);

@@ -260,3 +260,30 @@ def test_activation_written_as_planes(case, m, k, n, after, bias, act):
     together, apart = build(True), build(False)
     for _ in range(2):
         assert_bits_equal(together.run([feed])[0], apart.run([feed])[0], "planes from the product and from the split")
+
+
+@pytest.mark.parametrize("front", ["gelu", "norm"])
+def test_planes_only_for_weights_that_no_input_replaces(case, front):
+    """The second product's weights are an input of the graph too, and a run brings a stack of two in their place: its first operand has to
+    come as values."""
+    case(f"{front} -> weights that an input replaces")
+    rng = np.random.default_rng(4)
+    normal = lambda *s: rng.standard_normal(s).astype(np.float32)  # noqa: E731
+    m, k, n = 70, 256, 40
+    g = Model(opset_version=17)
+    x, w = g.new_val(), g.new_initializer(normal(k, n))
+    g.add_input(x)
+    g.add_input(w)
+    h, u, y = g.new_val(), g.new_val(), g.new_val()
+    if front == "gelu":
+        g.add_node(Op.MatMul, [x, g.new_initializer(normal(k, k) / np.float32(16))], [h])
+        g.add_node(Op.Gelu, [h], [u])
+    else:
+        g.add_node(Op.LayerNormalization, [x, g.new_initializer(normal(k)), g.new_initializer(normal(k))], [u], axis=-1, epsilon=1e-5)
+    g.add_node(Op.MatMul, [u, w], [y])
+    g.add_output(y)
+    feed = [normal(m, k), normal(2, k, n)]
+    together, apart = (HipSessionBuilder(g).with_gemm_algorithm(D.GEMM_BF16X3).with_strided_views(v).build() for v in (True, False))
+    got = together.run(feed)[0]
+    assert got.shape == (2, m, n)
+    assert_bits_equal(got, apart.run(feed)[0], "the nodes together and apart")
