@@ -1113,7 +1113,9 @@ bool HipSession::run_device_op(const Node &node, const Op &op, const std::vector
     }
 
     DeviceTensor out;
-    if (!allocate(shapes[0], &out, err)) return false;
+    // A product that leaves planes instead of its values needs no block for them (take_act_planes gives it the planes').
+    if (op.kind == OpKind::MatMul && act_planes_due(op, in)) out.dims = shapes[0].dims, out.elem_ty = shapes[0].elem_ty;
+    else if (!allocate(shapes[0], &out, err)) return false;
     float *o = static_cast<float *>(out.ptr);
     const size_t n_out = out.dims.total_elems();
     int rc = AHIP_OK;
@@ -1532,7 +1534,7 @@ bool HipSession::run_device_op(const Node &node, const Op &op, const std::vector
             }
             void *c_planes = nullptr;
             int c_op = 0;
-            if (!act_planes_for(rows, nn, kk, &out, &c_planes, &c_op, err)) return false;
+            if (!out.ptr && !take_act_planes(rows, nn, &out, &c_planes, &c_op, err)) return false;
             rc = launch_gemm_split(ctx_, o, nullptr, f(in[1]), bias_p, rows, nn, kk, 0, op.trans_b ? 1 : 0, kk, op.trans_b ? kk : nn, nn, 0, 1, 1.0f,
                                    bias_p ? 1.0f : 0.0f, 0, in[0]->ptr, c_op, c_planes);
             break;
@@ -1600,13 +1602,14 @@ bool HipSession::run_device_op(const Node &node, const Op &op, const std::vector
             }
             void *c_planes = nullptr;
             int c_op = 0;
-            if (!act_planes_for(batch * m, n, k, &out, &c_planes, &c_op, err)) return false;
+            if (!out.ptr && !take_act_planes(batch * m, n, &out, &c_planes, &c_op, err)) return false;
             if (a_op || c_planes)
                 rc = launch_gemm_split(ctx_, o, f(in[0]), f(in[1]), bias, batch * m, n, k, 0, tb, A.ld, B.ld, n, 0, 1, 1.0f, beta, a_op, nullptr, c_op, c_planes);
             else rc = launch_gemm(ctx_, o, f(in[0]), f(in[1]), bias, 1, batch * m, n, k, 0, tb, A.ld, B.ld, n, 0, 0, 0, 0, 1, 1.0f, beta);
             break;
         }
         if (a_op) return fail(err, SessionError::Message, "MatMul: an activation was left pending on a product that cannot fold it");
+        if (!out.ptr) return fail(err, SessionError::Message, "internal: a product without a block for its values");
         if (out.dims.len() < 2) return fail(err, SessionError::Shape, "MatMul: result of rank < 2");
         if (!((A.batch == batch || A.batch == 1) && (B.batch == batch || B.batch == 1)))
             return fail(err, SessionError::Message, "MatMul: batch axes that broadcast against each other partially are not supported");

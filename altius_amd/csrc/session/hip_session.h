@@ -309,8 +309,9 @@ private:
         int act = 0;
     };
     std::map<NodeId, ActPlanesPlan> act_planes_;
-    // The block that product `current_node_`, [m, k] x [k, n], writes such planes to (null: it writes none), made part of `out`.
-    bool act_planes_for(size_t m, size_t n, size_t k, DeviceTensor *out, void **planes, int *act, SessionError *err);
+    // Whether product `current_node_` writes such planes in this run, and the block that it writes them to, made `out`'s.
+    bool act_planes_due(const Op &op, const std::vector<DeviceTensor *> &in) const;
+    bool take_act_planes(size_t m, size_t n, DeviceTensor *out, void **planes, int *act, SessionError *err);
     std::map<NodeId, NodeId> add_into_ln_;  // Add nodes (a residual connection) -> the planes-writing LayerNormalization that reads the sum
     // A LayerNormalization written out as nine operators whose intermediate results nobody else reads, by its first node: one
     // kernel computes the last node's result when the first one is due, and the nodes between are passed over.

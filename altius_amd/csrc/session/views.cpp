@@ -492,20 +492,24 @@ void HipSession::plan_views(bool fused_attention) {
     }
 }
 
-bool HipSession::act_planes_for(size_t m, size_t n, size_t k, DeviceTensor *out, void **planes, int *act, SessionError *err) {
-    *planes = nullptr;
+bool HipSession::act_planes_due(const Op &op, const std::vector<DeviceTensor *> &in) const {
     auto ap = act_planes_.find(current_node_);
+    if (ap == act_planes_.end() || in.size() < 2 || !in[0] || !in[1] || !in[0]->strides.empty() || !in[1]->strides.empty() || in[0]->pending_op == PENDING_ATTENTION ||
+        in[0]->elem_ty != TensorElemType::F32 || in[1]->elem_ty != TensorElemType::F32 || in[0]->dims.len() < 2 || in[1]->dims.len() != 2 || op.trans_a ||
+        matmul_out_perm_.count(current_node_) || matmul_out_perm_.count(ap->second.next.consumer))
+        return false;
+    const FixedDimensions &ad = in[0]->dims, &wd = in[1]->dims;
+    const size_t k = ad[ad.len() - 1], m = k ? ad.total_elems() / k : 0, n = op.trans_b ? wd[0] : wd[1];
     // The second product reads [m, n]; it is given planes only if it would have split its operand itself.
-    if (ap == act_planes_.end() || matmul_out_perm_.count(ap->second.next.consumer) || !gemm_takes_split(ctx_, m, n, k) ||
-        !gemm_takes_split(ctx_, m, ap->second.next.next_n, n))
-        return true;
-    DeviceTensor t;
-    if (!allocate_bytes(gemm_planes_bytes(m, n), &t, err)) return false;
-    out->block = t.block;  // the fp32 block goes back to the pool unused
-    out->ptr = *planes = t.ptr;
+    return m && n && (op.trans_b ? wd[1] : wd[0]) == k && gemm_takes_split(ctx_, m, n, k) && gemm_takes_split(ctx_, m, ap->second.next.next_n, n);
+}
+
+bool HipSession::take_act_planes(size_t m, size_t n, DeviceTensor *out, void **planes, int *act, SessionError *err) {
+    if (!allocate_bytes(gemm_planes_bytes(m, n), out, err)) return false;
+    *planes = out->ptr;
     out->planes = true;
     out->planes_rows = m, out->planes_k = n;
-    out->applied_op = *act = ap->second.act;
+    out->applied_op = *act = act_planes_.at(current_node_).act;
     return true;
 }
 

@@ -287,3 +287,21 @@ def test_planes_only_for_weights_that_no_input_replaces(case, front):
     got = together.run(feed)[0]
     assert got.shape == (2, m, n)
     assert_bits_equal(got, apart.run(feed)[0], "the nodes together and apart")
+
+
+def test_no_block_for_values_that_leave_as_planes(case):
+    """Blocks of a session: two weights, the input, the planes and the result; none for the values between the products."""
+    case("[1024,256] x [256,512], Gelu, x [512,256]: blocks")
+    rng = np.random.default_rng(9)
+    g = Model(opset_version=13)
+    x = g.new_val_named_and_shaped("x", [1024, 256])
+    g.add_input(x)
+    h, u, y = g.new_val(), g.new_val(), g.new_val()
+    g.add_node(Op.MatMul, [x, g.new_initializer(rng.standard_normal((256, 512)).astype(np.float32))], [h])
+    g.add_node(Op.Gelu, [h], [u])
+    g.add_node(Op.MatMul, [u, g.new_initializer(rng.standard_normal((512, 256)).astype(np.float32))], [y])
+    g.add_output(y)
+    session = HipSessionBuilder(g).with_gemm_algorithm(D.GEMM_BF16X3).build()
+    for _ in range(2):
+        session.run([rng.standard_normal((1024, 256)).astype(np.float32)])
+        assert session.device_allocations() == 5
