@@ -207,6 +207,7 @@ def _declare_graph(L):
     f("ahip_session_builder_with_gemm_algorithm", [c_void_p, c_int])
     f("ahip_session_builder_with_fused_attention", [c_void_p, c_int])
     f("ahip_session_builder_with_strided_views", [c_void_p, c_int])
+    f("ahip_session_fused_kernels", [c_void_p, c_int, P(c_size_t)])
     f("ahip_session_copies_avoided", [c_void_p, P(c_size_t)])
     f("ahip_session_lanes", [c_void_p, P(c_size_t)])
     f("ahip_session_graph_replays", [c_void_p, P(c_size_t)])

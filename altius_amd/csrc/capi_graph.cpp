@@ -762,6 +762,16 @@ int ahip_session_copies_avoided(const ahip_session *session, size_t *count) try 
     return altius::caught_at_boundary("ahip_session_copies_avoided");
 }
 
+int ahip_session_fused_kernels(const ahip_session *session, int which, size_t *count) try {
+    if (!session || !count) return fail(AHIP_ERR_ARG, "ahip_session_fused_kernels: null argument");
+    if (which != AHIP_FUSED_ATTENTION && which != AHIP_FUSED_ACTIVATION_PLANES) return fail(AHIP_ERR_ARG, "ahip_session_fused_kernels: unknown kernel");
+    const auto lane = last_lane_idle(session);
+    *count = which == AHIP_FUSED_ATTENTION ? lane->attentions() : lane->activation_planes();
+    return AHIP_OK;
+} catch (...) {
+    return altius::caught_at_boundary("ahip_session_fused_kernels");
+}
+
 int ahip_session_graph_replays(const ahip_session *session, size_t *count) try {
     if (!session || !count) return fail(AHIP_ERR_ARG, "ahip_session_graph_replays: null argument");
     *count = last_lane_idle(session)->graph_replays();

@@ -750,7 +750,7 @@ static bool rows_order(const DeviceCtx &ctx, size_t batch, size_t tq, size_t tk,
 bool attention_rows_fits(const DeviceCtx &ctx, size_t batch, size_t tq, size_t tk) {
     const size_t lim = (size_t)1 << 31, most = 0xffffffffu / (64 * RW);  // a grid ends at 2^32 threads
     int qk, pv, lanes;
-    return batch > 1 && tq > 0 && tk > 0 && tk <= ROWS_MAX_KEYS && tq < lim && batch < lim && batch * ((tq + 31) / 32) <= most &&
+    return batch > 1 && tq > 0 && tk > 1 && tk <= ROWS_MAX_KEYS && tq < lim && batch < lim && batch * ((tq + 31) / 32) <= most &&
            rows_order(ctx, batch, tq, tk, &qk, &pv, &lanes);
 }
 

@@ -305,7 +305,7 @@ bool HipSession::run(const std::vector<Tensor> &inputs, std::vector<Tensor> *out
 
     const RunNotes notes(this);
     std::map<ValueId, DeviceTensor> values;
-    copies_avoided_ = 0;
+    copies_avoided_ = 0, attentions_ = 0, activation_planes_ = 0;
     std::vector<hipEvent_t> events;
     // Nothing may still read a block when it goes back to the pool for another run, and input
     // tensors must outlive their uploads: every exit path synchronises first.
@@ -407,7 +407,7 @@ bool HipSession::run_device(const std::vector<DeviceTensor> &inputs, std::vector
 
     const RunNotes notes(this);
     std::map<ValueId, DeviceTensor> values;
-    copies_avoided_ = 0;
+    copies_avoided_ = 0, attentions_ = 0, activation_planes_ = 0;
     for (size_t i = 0; i < g.inputs.size(); i++) {
         if (!inputs[i].ptr && inputs[i].nbytes())
             return fail(err, SessionError::Argument, "run_device: input " + std::to_string(i) + " has no device pointer");
@@ -480,7 +480,7 @@ bool HipSession::try_capture(const std::string &key, const std::vector<Tensor> &
     CapturedRun run;
     const RunNotes notes(this);
     std::map<ValueId, DeviceTensor> values;
-    copies_avoided_ = 0;
+    copies_avoided_ = 0, attentions_ = 0, activation_planes_ = 0;
     for (size_t i = 0; i < g.inputs.size(); i++) {
         DeviceTensor d;
         if (!allocate(TypedFixedShape{inputs[i].dims(), inputs[i].elem_ty()}, &d, err)) return false;

@@ -150,6 +150,10 @@ public:
     size_t device_allocations() const { return pool_->device_allocations(); }
     // Nodes of the last node-by-node run that produced a view or wrote a following Transpose's layout.
     size_t copies_avoided() const { return copies_avoided_; }
+    // Kernels of the last node-by-node run that did an attention's nodes (attention_rows_), and products that left as operand planes
+    // with the activation behind them done (act_planes_).
+    size_t attentions() const { return attentions_; }
+    size_t activation_planes() const { return activation_planes_; }
     // Runs served by replaying a captured HIP graph since the session was built.
     size_t graph_replays() const { return graph_replays_; }
     const std::vector<NodeExecutionPlan> &execution_plan() const { return plan_; }
@@ -261,7 +265,7 @@ private:
     std::map<std::string, int> eager_runs_;  // per input signature: eager runs so far (the pool is warm after one)
     size_t graph_replays_ = 0;
     uint64_t seen_ws_generation_ = 0;  // recorded launches hold the GEMM workspace's address: graphs are dropped when it moves
-    size_t copies_avoided_ = 0;
+    size_t copies_avoided_ = 0, attentions_ = 0, activation_planes_ = 0;
     NodeId current_node_ = 0;  // the node run_device_op is working on
     std::map<NodeId, AttentionPlan> attn_head_;                  // first MatMul of a fusable attention -> the rest
     std::set<NodeId> attn_softmax_, attn_tail_;

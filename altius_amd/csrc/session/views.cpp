@@ -510,6 +510,7 @@ bool HipSession::take_act_planes(size_t m, size_t n, DeviceTensor *out, void **p
     out->planes = true;
     out->planes_rows = m, out->planes_k = n;
     out->applied_op = *act = act_planes_.at(current_node_).act;
+    activation_planes_++;
     return true;
 }
 
@@ -810,6 +811,7 @@ bool HipSession::run_attention_rows(NodeId id, std::map<ValueId, DeviceTensor> &
     if (rc == AHIP_ERR_UNSUPPORTED) return true;
     if (rc) return fail_code(err, rc, ctx_.last_error);
     values[tail.outputs[0]] = std::move(out);
+    attentions_++;
     *done = true;
     return true;
 }

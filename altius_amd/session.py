@@ -133,6 +133,19 @@ class HipSession:
         check(self.L.ahip_session_copies_avoided(self.handle, ctypes.byref(c)))
         return c.value
 
+    def fused_attentions(self):
+        """Attentions of the last node-by-node run whose nodes ran as one kernel with their own bits."""
+        return self._fused_kernels(0)
+
+    def fused_activation_planes(self):
+        """Products of that run that wrote the activation behind them as the next product's operand planes."""
+        return self._fused_kernels(1)
+
+    def _fused_kernels(self, which):
+        c = ctypes.c_size_t()
+        check(self.L.ahip_session_fused_kernels(self.handle, which, ctypes.byref(c)))
+        return c.value
+
     def lanes(self):
         """Streams (each with a buffer pool and a copy of the initializers) the session holds so far: 1 until two
         run() calls have overlapped."""

@@ -641,6 +641,12 @@ int ahip_session_builder_with_fused_attention(ahip_session_builder *builder, int
  * written in place) or by another node's kernel (what follows a product, the steps of a written-out
  * LayerNormalization). */
 int ahip_session_copies_avoided(const ahip_session *session, size_t *count);
+/* Kernels of the last node-by-node run that did the work of several nodes, which ahip_session_copies_avoided does not count as such:
+ * AHIP_FUSED_ATTENTION, one for MatMul -> scale, condition, mask -> Softmax -> MatMul with the bits of those nodes run apart;
+ * AHIP_FUSED_ACTIVATION_PLANES, a product on the bf16 route that left as the next product's operand planes with the Gelu or Relu
+ * between them done.  No counterpart in the reference. */
+enum { AHIP_FUSED_ATTENTION = 0, AHIP_FUSED_ACTIVATION_PLANES = 1 };
+int ahip_session_fused_kernels(const ahip_session *session, int which, size_t *count);
 /* Lanes the session holds so far (1 until two ahip_session_run calls have overlapped). */
 int ahip_session_lanes(ahip_session *session, size_t *count);
 /* build(): shape inference (AHIP_ERR_SHAPE on failure), execution plan, device context,

@@ -5,6 +5,7 @@ import ctypes
 import numpy as np
 import pytest
 
+from altius_amd import device as D
 from altius_amd._lib import AltiusHipError
 from altius_amd.graph import Model, Op
 from altius_amd.session import HipSessionBuilder
@@ -60,7 +61,16 @@ def attention(b, h, tq, tk, d=64, scale="div", cond=None, mask=(1, 1, 1, "k"), v
     return m, shapes
 
 
-def check(case, b, h, tq, tk, **form):
+def has_kernel(heads, tq, tk):
+    """More than one head, two to 448 keys (a single key's matrix reads as a column), and the operators' sums in an order that the kernel
+    has: not the Softmax of rows that whole wavefronts take (whole 128-byte lines that fill three quarters of their loads), not the
+    products of many small matrices."""
+    whole_wavefronts = tk % 32 == 0 and 4 * tk >= 3 * (-(-tk // 256) * 256)
+    small_matrices = heads >= 128 and tq <= 208
+    return heads > 1 and 1 < tk <= 448 and not whole_wavefronts and not small_matrices
+
+
+def check(case, b, h, tq, tk, taken=True, **form):
     case(f"attention b {b} h {h} tq {tq} tk {tk} {form}")
     m, shapes = attention(b, h, tq, tk, **form)
     rng = np.random.default_rng(tq + tk)
@@ -72,12 +82,15 @@ def check(case, b, h, tq, tk, **form):
         got, ops = together.run(list(x.values())), apart.run(list(x.values()))
         for g, o in zip(got, ops):
             assert_bits_equal(g, o, "one kernel and the nodes apart")
+        assert apart.fused_attentions() == 0
+        assert together.fused_attentions() == (1 if taken and has_kernel(b * h, tq, tk) else 0)
 
 
 # edges of tiles of 32 queries and keys, of turns of 16, 32 and 64 keys and of the lanes of a row; one key, as many as LDS holds and more
 @pytest.mark.parametrize("tq,tk", [(1, 1), (1, 65), (5, 16), (16, 17), (17, 63), (33, 64), (77, 77), (31, 128), (48, 129), (64, 192), (15, 193), (197, 197),
                                    (20, 256), (257, 257), (16, 321), (40, 447), (40, 449), (7, 600)])
 def test_sizes(case, tq, tk):
+    assert D.attention_rows_fits(6, tq, tk) == has_kernel(6, tq, tk)
     check(case, 2, 3, tq, tk)
 
 
@@ -98,7 +111,7 @@ def test_forms(case, scale, cond, mask):
 @pytest.mark.parametrize("form", [dict(mask=None), dict(mask=None, scale="power"), dict(value_late=True), dict(k_form="twice"), dict(seen=True), dict(rewritten=False), dict(d=32), dict(d=128)])
 @pytest.mark.parametrize("b,h", [(1, 1), (1, 4), (3, 1), (5, 2)])
 def test_operands_and_readers(case, b, h, form):
-    check(case, b, h, 50, 70, **form)
+    check(case, b, h, 50, 70, taken=not form.get("seen") and form.get("d", 64) == 64, **form)
 
 
 def test_rows_without_a_finite_score(case):
@@ -116,6 +129,7 @@ def test_rows_without_a_finite_score(case):
     together, apart = HipSessionBuilder(m).build(), HipSessionBuilder(m).with_strided_views(False).build()
     got, want = together.run(list(x.values()))[0], apart.run(list(x.values()))[0]
     assert_bits_equal(got, want, "one kernel and the nodes apart")
+    assert together.fused_attentions() == 1
 
 
 @pytest.mark.parametrize("shared", ["keys", "values", "both"])
@@ -141,6 +155,7 @@ def test_heads_that_share_keys_or_values(case, shared, heads, t):
     together, apart = HipSessionBuilder(m).build(), HipSessionBuilder(m).with_strided_views(False).build()
     for _ in range(2):
         assert_bits_equal(together.run(x)[0], apart.run(x)[0], "held and run apart, and apart")
+        assert together.fused_attentions() == 0
 
 
 @pytest.mark.parametrize("tq,tk", [(77, 77), (197, 197), (40, 447)])
@@ -200,4 +215,5 @@ def test_replayed(case):
         rng = np.random.default_rng(seed)
         x = [rng.standard_normal(dims).astype(np.float32) for dims in shapes.values()]
         assert_bits_equal(session.run(x)[0], eager.run(x)[0], "recorded and not")
+        assert session.fused_attentions() == eager.fused_attentions() == 1
     assert session.graph_replays() > 0

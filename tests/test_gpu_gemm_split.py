@@ -260,6 +260,7 @@ def test_activation_written_as_planes(case, m, k, n, after, bias, act):
     together, apart = build(True), build(False)
     for _ in range(2):
         assert_bits_equal(together.run([feed])[0], apart.run([feed])[0], "planes from the product and from the split")
+        assert together.fused_activation_planes() == 1 and apart.fused_activation_planes() == 0
 
 
 @pytest.mark.parametrize("front", ["gelu", "norm"])
@@ -287,6 +288,7 @@ def test_planes_only_for_weights_that_no_input_replaces(case, front):
     got = together.run(feed)[0]
     assert got.shape == (2, m, n)
     assert_bits_equal(got, apart.run(feed)[0], "the nodes together and apart")
+    assert together.fused_activation_planes() == 0
 
 
 def test_no_block_for_values_that_leave_as_planes(case):
