@@ -39,6 +39,7 @@ struct Post {
     const float *mean = nullptr, *var = nullptr, *scale = nullptr, *shift = nullptr, *residual = nullptr;
     float eps = 0.0f, alpha = 0.0f, beta = 0.0f;
     int act = 0;
+    bool any() const { return mean || act || residual; }
     // ch: output channel, at: where the value goes in the output
     __device__ __forceinline__ float operator()(float v, uint32_t ch, size_t at) const {
         if (mean) v = ((v - mean[ch]) / sqrtf(var[ch] + eps)) * scale[ch] + shift[ch];
@@ -75,7 +76,7 @@ struct DepthwiseArgs {
 // that an input row it has read serves up to K of them: 8 K instead of 4 K^2 LDS reads for K = 5, RY = 4.
 // K = 0: any kernel, stride and dilation, RY = 1.  The taps are added in row-major order in every variant.
 // [32,240,14,14], 5 x 5: 9.4 us; one product launch per channel took 1.3 ms (240 launches of 5.4 us).
-template <int K, int SH, int RY>
+template <int K, int SH, int RY, bool POST>
 __global__ __launch_bounds__(BLOCK) void conv_depthwise(DepthwiseArgs g) {
     extern __shared__ float lds[];
     const int tid = threadIdx.x;
@@ -155,7 +156,11 @@ __global__ __launch_bounds__(BLOCK) void conv_depthwise(DepthwiseArgs g) {
         const size_t at = ((size_t)pl * g.oh + y) * g.ow + x;
 #pragma unroll
         for (int k = 0; k < RY; k++)
-            if (y + k < g.oh) g.out[at + (size_t)k * g.ow] = g.post(g.bias ? acc[k] + bias : acc[k], ch, at + (size_t)k * g.ow);
+            if (y + k < g.oh) {
+                const float v = g.bias ? acc[k] + bias : acc[k];
+                const size_t here = at + (size_t)k * g.ow;
+                g.out[here] = POST ? g.post(v, ch, here) : v;
+            }
     }
 }
 
@@ -210,7 +215,11 @@ bool launch_depthwise(DeviceCtx &ctx, float *out, const float *x, const float *w
     g.post = post;
     const dim3 grid((unsigned)blocks);
     const size_t lds = floats() * sizeof(float);
-#define DEPTHWISE(K, SH, RY) hipLaunchKernelGGL((conv_depthwise<K, SH, RY>), grid, dim3(BLOCK), lds, ctx.stream, g)
+#define DEPTHWISE(K, SH, RY)                                                                                                      \
+    do {                                                                                                                           \
+        if (post.any()) hipLaunchKernelGGL((conv_depthwise<K, SH, RY, true>), grid, dim3(BLOCK), lds, ctx.stream, g);              \
+        else hipLaunchKernelGGL((conv_depthwise<K, SH, RY, false>), grid, dim3(BLOCK), lds, ctx.stream, g);                        \
+    } while (0)
     if (!square) DEPTHWISE(0, 1, 1);
     else if (ry == 1 && kh == 3) DEPTHWISE(3, 1, 1);
     else if (ry == 1) DEPTHWISE(5, 1, 1);
@@ -288,7 +297,7 @@ __device__ __forceinline__ floatx4 weights4(const float *row, uint32_t k0, uint3
 // (Requesting the next chunk ahead of the products was measured: equal for one tile, 9.1 -> 11.5 us for 2 x 2.)
 // The k of an MFMA may be any four as long as both operands agree: lane q of four takes k0 + 4 q + j in step j, so that
 // a lane's share of w is one 16-byte load per four steps.
-template <bool POINTWISE, int MT, int NT>
+template <bool POINTWISE, int MT, int NT, bool POST>
 __global__ __launch_bounds__(512) void conv_gemm_small(ConvGemmArgs g) {
     extern __shared__ float lds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = blockDim.x >> 6;
@@ -340,7 +349,7 @@ __global__ __launch_bounds__(512) void conv_gemm_small(ConvGemmArgs g) {
         const uint32_t ch = grp * g.m + mm;
         if (g.bias) v += g.bias[ch];
         const size_t at = out_offset(g, ch, n);
-        g.out[at] = g.post(v, ch, at);
+        g.out[at] = POST ? g.post(v, ch, at) : v;
     }
 }
 
@@ -349,7 +358,7 @@ __global__ __launch_bounds__(512) void conv_gemm_small(ConvGemmArgs g) {
 // (pitch 20: the 16-byte reads of 16 rows meet all 64 banks), x as [k][column] (pitch 132: the four k of a step are 16 banks apart).
 constexpr int TM = 64, TN = 128, TK = 16, WP = TK + 4, XP = TN + 4;
 
-template <bool POINTWISE>
+template <bool POINTWISE, bool POST>
 __global__ __launch_bounds__(BLOCK) void conv_gemm_tiled(ConvGemmArgs g) {
     __shared__ __align__(16) float ws[2][TM * WP];
     __shared__ __align__(16) float xs[2][TK * XP];
@@ -437,7 +446,8 @@ __global__ __launch_bounds__(BLOCK) void conv_gemm_tiled(ConvGemmArgs g) {
                 if (mm >= g.m) continue;
                 const uint32_t ch = grp * g.m + mm;
                 const size_t at = first + (size_t)mm * g.ohw.d;
-                g.out[at] = g.post(g.bias ? acc[i][j][e] + g.bias[ch] : acc[i][j][e], ch, at);
+                const float v = g.bias ? acc[i][j][e] + g.bias[ch] : acc[i][j][e];
+                g.out[at] = POST ? g.post(v, ch, at) : v;
             }
     }
 }
@@ -609,12 +619,18 @@ int launch_conv2d(DeviceCtx &ctx, float *out, const float *x, const float *w, co
         const dim3 dim((unsigned)blocks, (unsigned)std::min(group - g0, MAX_GRID_Y));
         g.x = x + g0 * cg * ih * iw, g.w = w + g0 * m * k, g.bias = bias ? bias + g0 * m : nullptr, g.out = out + g0 * m * oh * ow;
         g.post = post.behind(g0 * m, g0 * m * oh * ow);
-        if (tiled && pointwise) hipLaunchKernelGGL((conv_gemm_tiled<true>), dim, block, 0, ctx.stream, g);
-        else if (tiled) hipLaunchKernelGGL((conv_gemm_tiled<false>), dim, block, 0, ctx.stream, g);
-        else if (pointwise && wide) hipLaunchKernelGGL((conv_gemm_small<true, 2, 2>), dim, block, lds, ctx.stream, g);
-        else if (pointwise) hipLaunchKernelGGL((conv_gemm_small<true, 1, 1>), dim, block, lds, ctx.stream, g);
-        else if (wide) hipLaunchKernelGGL((conv_gemm_small<false, 2, 2>), dim, block, lds, ctx.stream, g);
-        else hipLaunchKernelGGL((conv_gemm_small<false, 1, 1>), dim, block, lds, ctx.stream, g);
+#define PRODUCT(KERNEL, ...)                                                                                        \
+    do {                                                                                                             \
+        if (post.any()) hipLaunchKernelGGL((KERNEL<__VA_ARGS__, true>), dim, block, tiled ? 0 : lds, ctx.stream, g); \
+        else hipLaunchKernelGGL((KERNEL<__VA_ARGS__, false>), dim, block, tiled ? 0 : lds, ctx.stream, g);           \
+    } while (0)
+        if (tiled && pointwise) PRODUCT(conv_gemm_tiled, true);
+        else if (tiled) PRODUCT(conv_gemm_tiled, false);
+        else if (pointwise && wide) PRODUCT(conv_gemm_small, true, 2, 2);
+        else if (pointwise) PRODUCT(conv_gemm_small, true, 1, 1);
+        else if (wide) PRODUCT(conv_gemm_small, false, 2, 2);
+        else PRODUCT(conv_gemm_small, false, 1, 1);
+#undef PRODUCT
     }
     return launched();
 }
