@@ -253,8 +253,13 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_f32_tiles(GemmArgs g) 
         if constexpr (u < la.COUNT) la.load(u, lds0 + stage * (STAGE * 4), wave);
         else lb.load(u - la.COUNT, lds0 + (stage * STAGE + STAGE_A) * 4, wave);
     };
+    // Behind the last tile 16-byte loads go on, for nothing: the waits and the steps stay as they are ([1872,3024] x [3024,2256] 202 us,
+    // 209 without those loads).  Single-value loads are four times as many, and end (96 of [148,32] x [32,2821], one step each: 98 us
+    // with the others', 77 without).
+    constexpr bool TO_THE_END = VEC == 4;
 #pragma unroll
     for (int s = 0; s < S; s++) {
+        if (!TO_THE_END && tile_k >= nk) break;
         if (tile_k < near) advance_near();
         else if (tile_k < nk) advance_far();
         else nothing_left();
@@ -298,10 +303,19 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_f32_tiles(GemmArgs g) 
         else if (turn == 1) __builtin_amdgcn_s_setprio(1);
         else __builtin_amdgcn_s_setprio(2);
     }
-    wait_loads_and_barrier<(S - 1) * LOADS>();
+    // Waits until at most `behind` stages, whose loads are the last ones, are on their way.
+    auto wait_behind = [&](uint32_t behind) __attribute__((always_inline)) {
+        if (behind >= S - 1) wait_loads_and_barrier<(S - 1) * LOADS>();
+        else if (S > 3 && behind == 2) wait_loads_and_barrier<2 * LOADS>();
+        else if (behind == 1) wait_loads_and_barrier<LOADS>();
+        else wait_loads_and_barrier<0>();
+    };
+    if (TO_THE_END) wait_loads_and_barrier<(S - 1) * LOADS>();
+    else wait_behind(max(nk, 1u) - 1);
     read(0, 0);
     uint32_t cur = 0;
-    auto step = [&](auto is_near) __attribute__((always_inline)) {
+    // left: 0, or where the loads have ended how many steps there are from this one on.
+    auto step = [&](auto is_near, uint32_t left) __attribute__((always_inline)) {
         each<Q>([&](auto q) __attribute__((always_inline)) {
             multiply(0, q);
             if constexpr (q == 0) read(1, cur);
@@ -312,11 +326,15 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_f32_tiles(GemmArgs g) 
         each<Q>([&](auto q) __attribute__((always_inline)) {
             constexpr int R = Q > 4 ? 1 : 0;
             multiply(1, q);
-            if constexpr (q == 0) wait_loads_and_barrier<(S - 2) * LOADS>();  // this stage is read, the next one there
+            if constexpr (q == 0) {  // this stage is read, the next one there
+                if (left) wait_behind(max(left, 2u) - 2);
+                else wait_loads_and_barrier<(S - 2) * LOADS>();
+            }
             if constexpr (q == R) read(0, next);
-            each<LOADS>([&](auto u) __attribute__((always_inline)) {
-                if constexpr (R + 1 + u * (Q - 1 - R) / LOADS == q) load(u, cur);
-            });
+            if (!left)
+                each<LOADS>([&](auto u) __attribute__((always_inline)) {
+                    if constexpr (R + 1 + u * (Q - 1 - R) / LOADS == q) load(u, cur);
+                });
             __builtin_amdgcn_sched_barrier(0);
         });
         cur = next;
@@ -324,12 +342,12 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_f32_tiles(GemmArgs g) 
     while (tile_k < nk) {
         if (tile_k >= near) {
             advance_far();
-            step(std::false_type());
+            step(std::false_type(), 0);
         }
-        while (tile_k < near) step(std::true_type());
+        while (tile_k < near) step(std::true_type(), 0);
     }
-    nothing_left();
-    for (uint32_t kt = min(nk, (uint32_t)S); kt > 0; kt--) step(std::false_type());
+    if (TO_THE_END) nothing_left();
+    for (uint32_t left = min(nk, (uint32_t)S); left > 0; left--) step(std::false_type(), TO_THE_END ? 0 : left);
     wait_loads_and_barrier<0>();
 
     if (WK == 4 && g.apart) __builtin_amdgcn_s_setprio(3);
