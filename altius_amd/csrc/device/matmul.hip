@@ -606,9 +606,14 @@ int launch_gemm_batch2(DeviceCtx &ctx, float *c, const float *a, const float *b,
                            c_batch_strides, c0_row_stride, c0_col_stride, alpha, beta, post);
 }
 
+// What choose() reckons is fitted to larger products with 16-byte loads; a convolution's, which decide between this and a kernel that reads
+// x in place, take longer: 0.4 to 1.2 us of 4 to 7 ([144,48] x [48,196], 30 images, 5.7 reckoned and 6.8 measured), with single-value loads
+// and a bias per row 1.3 and 2.6 us and 15 % ([576,96] x [96,49], 44 images: 7.1 and 10.8).  Without that, products were taken for images
+// that the in-place kernels do in 5.9 and 9.3 us.
 double gemm_f32_us(const DeviceCtx &ctx, size_t batch, size_t m, size_t n, size_t k, bool vec) {
     const size_t cus = ctx.cus_per_xcd ? (size_t)ctx.cus_per_xcd : 32;
-    return choose(batch, m, n, k, cus, ctx.gemm_split_k).us * (vec ? 1.0 : 1.2);
+    const Choice ch = choose(batch, m, n, k, cus, ctx.gemm_split_k);
+    return vec ? ch.us + (ch.shape ? 1.2 : 0.4) : 1.15 * ch.us + (ch.shape ? 2.6 : 1.3);
 }
 
 int gemm_f32_chains(const DeviceCtx &ctx, size_t batch, size_t m, size_t n, size_t k) {

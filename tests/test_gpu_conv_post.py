@@ -86,6 +86,21 @@ def test_behind_a_convolution(case, geometry, after):
         assert together.copies_avoided() == (0 if "norm" in after and geometry in GEOMETRIES[-2:] else len(after.split()))
 
 
+# Pointwise convolutions whose products would take longer than the kernels that read x in place (those do a normalisation along), and
+# some whose products are faster.
+@pytest.mark.parametrize("geometry,in_place", [((30, 48, 14, 144, 1, 1, 1), True), ((31, 40, 15, 240, 1, 1, 1), True), ((44, 96, 7, 576, 1, 1, 1), True),
+                                               ((8, 40, 16, 240, 1, 1, 1), True), ((29, 144, 14, 48, 1, 1, 1), True), ((44, 138, 11, 89, 1, 1, 1), True),
+                                               ((41, 576, 6, 96, 1, 1, 1), False), ((7, 383, 42, 421, 1, 1, 1), False)])
+def test_small_images_are_read_in_place(case, geometry, in_place):
+    case(f"conv {geometry}, norm")
+    m, x_dims, r_dims = graph(*geometry, "norm", bias=True)
+    rng = np.random.default_rng(8)
+    x, r = (3 * rng.standard_normal(d).astype(np.float32) for d in (x_dims, r_dims))
+    together, apart = HipSessionBuilder(m).build(), HipSessionBuilder(m).with_strided_views(False).build()
+    assert_bits_equal(together.run([x, r])[0], apart.run([x, r])[0], "the nodes together and apart")
+    assert together.copies_avoided() == (1 if in_place else 0)
+
+
 # From 128 images on a product of small ones without a bias is the kernel of many small matrices, in one chunk of k and in several.
 @pytest.mark.parametrize("bias", [False, True])
 @pytest.mark.parametrize("after", ["relu", "hard_swish", "add"])
