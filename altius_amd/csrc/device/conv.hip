@@ -34,7 +34,8 @@ constexpr size_t DW_LDS_FLOATS = 8192;  // 32 KB: five blocks to a CU
 // What follows the convolution in the graph (ConvPost), done to a value before it is stored.  A pass of its own over the result costs 2
 // to 4 us of launch on one image and 3 to 10 us on 32 of 224 x 224; here it costs 0 to 2 (the stem's square root and division 8).  A
 // classifier of that size, 36 convolutions: with the average pool's division and the gates' hard swish in their kernels too 122 launches
-// became 73, 662 us 501 on 32 images and 502 365 on one.
+// became 73, 662 us 486 on 32 images and 502 365 on one.  The kernels' POST is false where nothing follows: with the code for it in
+// them, and nothing to do, they were 5 to 15 % slower (depthwise [59,80,65,65], 1 x 1: 102 and 119 us).
 struct Post {
     const float *mean = nullptr, *var = nullptr, *scale = nullptr, *shift = nullptr, *residual = nullptr;
     float eps = 0.0f, alpha = 0.0f, beta = 0.0f;

@@ -458,33 +458,33 @@ template <int POST> __global__ __launch_bounds__(THREADS, 1) void gemm_bf16x3(Sp
             }
         } else {
 #pragma unroll 4
-        for (int q = 0; q < 16; q++) {
-            const int row = 2 * q + lk;
-            const f32x4 t = *reinterpret_cast<const f32x4 *>(stage + row * EP + lr * 4);
-            const uint32_t grow = m0 + wm * 64 + i * 32 + row;
-            if (grow >= g.m || gcol >= g.n) continue;
-            float v[4] = {g.alpha * t.x, g.alpha * t.y, g.alpha * t.z, g.alpha * t.w};
-            const bool whole = gcol + 3 < g.n;
-            if (row_bias) {
+            for (int q = 0; q < 16; q++) {
+                const int row = 2 * q + lk;
+                const f32x4 t = *reinterpret_cast<const f32x4 *>(stage + row * EP + lr * 4);
+                const uint32_t grow = m0 + wm * 64 + i * 32 + row;
+                if (grow >= g.m || gcol >= g.n) continue;
+                float v[4] = {g.alpha * t.x, g.alpha * t.y, g.alpha * t.z, g.alpha * t.w};
+                const bool whole = gcol + 3 < g.n;
+                if (row_bias) {
 #pragma unroll
-                for (int e = 0; e < 4; e++) v[e] += g.beta * bias[e];
-            } else if (g.c0) {
-                const float *c0 = g.c0 + (size_t)grow * g.c0_rs + (size_t)gcol * g.c0_cs;
+                    for (int e = 0; e < 4; e++) v[e] += g.beta * bias[e];
+                } else if (g.c0) {
+                    const float *c0 = g.c0 + (size_t)grow * g.c0_rs + (size_t)gcol * g.c0_cs;
 #pragma unroll
-                for (int e = 0; e < 4; e++)
-                    if (gcol + e < g.n) v[e] += g.beta * c0[(size_t)e * g.c0_cs];
+                    for (int e = 0; e < 4; e++)
+                        if (gcol + e < g.n) v[e] += g.beta * c0[(size_t)e * g.c0_cs];
+                }
+                float *dst = g.c + (size_t)grow * g.ldc + gcol;
+                if (whole && g.c_vec) {
+                    const f32x4 o = {v[0], v[1], v[2], v[3]};
+                    if (g.c_stream) __builtin_nontemporal_store(o, reinterpret_cast<f32x4 *>(dst));
+                    else *reinterpret_cast<f32x4 *>(dst) = o;
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        if (gcol + e < g.n) dst[e] = v[e];
+                }
             }
-            float *dst = g.c + (size_t)grow * g.ldc + gcol;
-            if (whole && g.c_vec) {
-                const f32x4 o = {v[0], v[1], v[2], v[3]};
-                if (g.c_stream) __builtin_nontemporal_store(o, reinterpret_cast<f32x4 *>(dst));
-                else *reinterpret_cast<f32x4 *>(dst) = o;
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; e++)
-                    if (gcol + e < g.n) dst[e] = v[e];
-            }
-        }
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();

@@ -9,7 +9,7 @@
 // time is a chain of loads that WK cuts, large tiles where the chip is full and traffic per operation counts.
 //
 // Operand tiles go from memory to LDS directly (buffer loads, which read zeros behind an operand's end and wherever k is past
-// its end), S - 1 tiles ahead, with one barrier per tile.  Nothing is transposed on the way: an operand whose k is the
+// its end), up to S tiles ahead, with one barrier per tile.  Nothing is transposed on the way: an operand whose k is the
 // contiguous axis lies in LDS as [row][16], its 16-byte pieces exchanged by piece ^= (row / 4) % 4 so that a column of pieces
 // covers the banks, and a lane reads four values of k at once; one whose rows are contiguous lies as [k][row], and a lane reads
 // TA (TB) neighbouring rows, one for each of its tiles.  The instruction takes two values of k, one per half of the wavefront;
@@ -21,7 +21,7 @@
 //   [6304,768] x [768,768 / 2304 / 3072]: 72 -> 63 us, 192 -> 184, 258 -> 228;  [6304,3072] x [3072,768]: 262 -> 227
 //   [1024,768] x [768,768 / 3072]: 16.4 -> 14.7, 45 -> 40;  [1024,3072] x [3072,768]: 51 -> 46
 //   [197,768] x [768,768]: 8.6 -> 7.1;  [77,768] x [768,3072]: 12.0 -> 10.2
-//   4096^3: 1061 -> 938 us (147 Tflop/s);  [50432,768] x [768,3072]: 1788 -> 1670 (143)
+//   4096^3: 1061 -> 938 us (147 Tflop/s; 145 on another day's card);  [50432,768] x [768,3072]: 1788 -> 1670 (143)
 // Single-value loads are taken for both operands where one of them needs them.
 // What is left on large shapes: the blocks' first loads and their results (1 us of 12 in a 64 x 64 tile with 768 values of k), and a last
 // round of blocks that is partly empty where a cut costs as much as it gives ([6304,768] x [768,768]: 4.6 rounds take five, cut 64 us).
@@ -72,6 +72,8 @@ struct GemmArgs {
     int act;
     float act_alpha, act_beta;
     // The blocks of a CU all start together, and go out of step by priorities: one's first loads and results beside another's products.
+    // (Of 256 blocks dealt in turn each of the part's 256 CUs gets one, the next 256 are its second: with fewer CUs the priorities
+    // would not differ where they should, and the results would be the same.)
     int apart;
 };
 
@@ -482,8 +484,9 @@ struct Choice {
     double us = 0.0;
 };
 
-// What a product adds up in which order is decided by the sizes alone, so that a product and the same product with an operand stored
-// the other way round add up alike.  cut: k may be cut into slices.
+// What a product adds up in which order is decided by the sizes alone, and by where a value lies in C: the values of a last round's
+// tiles add up in slices, the others in one piece, so that equal rows of A need not give equal bits.  A product and the same product with
+// an operand stored the other way round add up alike.  cut: k may be cut into slices.
 Choice choose(size_t batch, size_t m, size_t n, size_t k, size_t cus_per_xcd, bool cut) {
     Choice best;
     for (int s = 0; s < N_SHAPES; s++) {

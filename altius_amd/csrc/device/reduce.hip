@@ -681,11 +681,11 @@ int reduce_rows(DeviceCtx &ctx, const Partials &pt, float *out, const float *in,
         const int sub = sub4_lanes(red);
         const bool nt = ctx.streaming(outer * red * sizeof(float));
         const dim3 grid((unsigned)sub4_blocks(outer, red)), block(ROW_BLOCK);
-#define ALTIUS_SUB4(SUBV)                                                                                                          \
-do {                                                                                                                           \
-    if (nt) hipLaunchKernelGGL((reduce_rows_sub4<OP, SUBV, U, SCALE, true>), grid, block, 0, s, out, in, outer, (uint32_t)red, scale);  \
-    else hipLaunchKernelGGL((reduce_rows_sub4<OP, SUBV, U, SCALE, false>), grid, block, 0, s, out, in, outer, (uint32_t)red, scale);    \
-} while (0)
+#define ALTIUS_SUB4(SUBV)                                                                                                                   \
+    do {                                                                                                                                    \
+        if (nt) hipLaunchKernelGGL((reduce_rows_sub4<OP, SUBV, U, SCALE, true>), grid, block, 0, s, out, in, outer, (uint32_t)red, scale);  \
+        else hipLaunchKernelGGL((reduce_rows_sub4<OP, SUBV, U, SCALE, false>), grid, block, 0, s, out, in, outer, (uint32_t)red, scale);    \
+    } while (0)
         switch (sub) {
         case 4: ALTIUS_SUB4(4); break;
         case 8: ALTIUS_SUB4(8); break;
