@@ -28,6 +28,14 @@ struct PackedOperand {
     size_t bytes;
 };
 
+// A weight matrix [k, n] (k_contig: stored [n, k]) and its planes for the products that read it (device memory, owned).
+struct PackedWeights {
+    const float *b;
+    size_t n, k, ld;
+    bool k_contig;
+    void *planes;
+};
+
 // The streaming threshold of a session's context (see DeviceCtx::nt_threshold_bytes).
 constexpr size_t SESSION_NT_THRESHOLD_BYTES = (size_t)128 << 20;
 
@@ -78,6 +86,7 @@ struct DeviceCtx {
     bool gemm_in_kernel_k_cut = true;
     std::vector<ConstantBuffer> gemm_constants;
     std::vector<PackedOperand> gemm_packed;
+    std::vector<PackedWeights> gemm_weights;
     std::string last_error;
 
     bool streaming(size_t bytes) const { return bytes >= nt_threshold_bytes; }
@@ -200,7 +209,13 @@ int launch_gemm_batch2(DeviceCtx &ctx, float *c, const float *a, const float *b,
 int launch_gemm_f32(DeviceCtx &ctx, float *c, const float *a, const float *b, const float *c0, size_t batch_outer, size_t batch_inner, size_t m,
                     size_t n, size_t k, int trans_a, int trans_b, size_t lda, size_t ldb, size_t ldc, const size_t a_batch_strides[2],
                     const size_t b_batch_strides[2], const size_t c_batch_strides[2], size_t c0_row_stride, size_t c0_col_stride, float alpha,
-                    float beta, const GemmPost *post = nullptr);
+                    float beta, const GemmPost *post = nullptr, const void *planes = nullptr);
+// planes: the second operand's as gemm_packed_weights has them (one batch, op(A) = A).
+// Makes planes of a weight matrix, which is not written to or freed while the context lasts: a product with as many rows as gemm_takes_planes
+// wants then runs on the bf16 matrix cores, every value as the exact sum of three bf16 numbers (gemm_planes.h).  AHIP_ERR_OOM: none made.
+int gemm_pack_weights(DeviceCtx &ctx, const float *b, size_t n, size_t k, size_t ld, bool k_contig);
+const void *gemm_packed_weights(const DeviceCtx &ctx, const float *b, size_t n, size_t k, size_t ld, bool k_contig);
+bool gemm_takes_planes(const DeviceCtx &ctx, size_t m, size_t n, size_t k);
 double gemm_f32_us(const DeviceCtx &ctx, size_t batch, size_t m, size_t n, size_t k, bool vec);
 // How many chains of sums over k, 16 values each in turn, meet in an element of that product (1, 2 or 4); 0: it is no product of whole
 // tiles (many small matrices, or k cut into slices).

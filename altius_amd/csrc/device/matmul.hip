@@ -15,6 +15,9 @@
 // TA (TB) neighbouring rows, one for each of its tiles.  The instruction takes two values of k, one per half of the wavefront;
 // a half takes k = 8 i + 4 half + 0 .. 3 in turn, the same for both layouts, so that a product does not depend on them.
 //
+// Products with a weight matrix of which planes are kept run their sums on the bf16 matrix cores instead (gemm_planes.h), in the same tiles'
+// epilogue.
+//
 // A step's two halves take turns in registers: while one half's products run, the other's fragments come from LDS, and what else a step
 // does (the next loads and their addresses) stands between the products, where the matrix pipe covers it.  With a step's fragments
 // all read in front of its products and the addresses worked out anew in every step, the pipes were busy 60 to 84 % of the cycles:
@@ -33,6 +36,7 @@
 
 #include "common.h"
 #include "ctx.h"
+#include "gemm_planes.h"
 #include "math.h"
 
 namespace altius {
@@ -43,6 +47,7 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void *lds_ptr;
 
 constexpr int BK = 16;  // values of k a wavefront multiplies between two barriers
@@ -71,6 +76,10 @@ struct GemmArgs {
     float alpha, beta;
     int act;
     float act_alpha, act_beta;
+    // The second operand's planes where it has some, [n32s][k16s] sets (gemm_planes.h); b is the same operand as it lies in memory, b_kc: along k.
+    const char *planes;
+    uint32_t n32s, k16s;
+    int b_kc;
     // The blocks of a CU all start together, and go out of step by priorities: one's first loads and results beside another's products.
     // (Of 256 blocks dealt in turn each of the part's 256 CUs gets one, the next 256 are its second: with fewer CUs the priorities
     // would not differ where they should, and the results would be the same.)
@@ -180,12 +189,13 @@ template <bool KC, int W, int WK, int WAVES, int VEC> struct Loader {
     }
 };
 
-// f(0) .. f(N - 1) with the number known when f is compiled.
-template <class F, int... I> __device__ __forceinline__ void each_of(F f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>()), ...); }
-template <int N, class F> __device__ __forceinline__ void each(F f) { each_of(f, std::make_integer_sequence<int, N>()); }
+template <class X> struct PlaneRoom { static constexpr int FLOATS = X::LDS_BYTES / 4; };
+template <> struct PlaneRoom<void> { static constexpr int FLOATS = 0; };
 
-template <bool AKC, bool BKC, int WM, int WN, int WK, int TA, int TB, int VEC>
-__global__ __launch_bounds__(64 * WM * WN * WK) void gemm_f32_tiles(GemmArgs g) {
+template <bool AKC, bool BKC, int WM, int WN, int WK, int TA, int TB, int VEC, class X = void>
+__global__ __launch_bounds__(64 * WM * WN * WK, std::is_void<X>::value ? 1 : 2) void gemm_f32_tiles(GemmArgs g) {
+    constexpr bool PLANES = !std::is_void<X>::value;
+    static_assert(!PLANES || (AKC && BKC), "weights in planes: the first operand's k is contiguous, and a lane's columns are 32 apart");
     // Stages, and with them how many blocks a CU holds (48 KB of LDS: three).  A fourth is 3 to 10 % slower for the small tiles, which lose
     // a block by it.  Of 128 x 128 tiles a CU holds two: three in step end together, and the blocks left then fill the slots of few CUs
     // (4096^3, four rounds: 1153 us with three, 938 with two; five rounds, [4096,1024] x [1024,5120]: 354 and 304).
@@ -193,7 +203,8 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_f32_tiles(GemmArgs g) 
     constexpr int WAVES = WM * WN * WK, THREADS = 64 * WAVES, BM = 32 * WM * TA, BN = 32 * WN * TB, BKT = BK * WK;
     constexpr int STAGE_A = BM * BKT, STAGE = (BM + BN) * BKT;
     constexpr int CP = BN + 4, PASS_ROWS = 32 * WM, SUMS = WK * PASS_ROWS * CP;  // the epilogue's [WK][PASS_ROWS][CP]
-    __shared__ __align__(16) float lds[S * STAGE > SUMS ? S * STAGE : SUMS];
+    constexpr int ROOM = PLANES ? PlaneRoom<X>::FLOATS : S * STAGE;
+    __shared__ __align__(16) float lds[ROOM > SUMS ? ROOM : SUMS];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     if (WK == 4 && g.apart) __builtin_amdgcn_s_setprio(3);
     const int wk = wave / (WM * WN), wmn = wave % (WM * WN), wm = wmn / WN, wn = wmn % WN;
@@ -213,145 +224,193 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void gemm_f32_tiles(GemmArgs g) 
     const uint32_t zo = z / g.batch_inner, zi = z - zo * g.batch_inner;
     const uint32_t k0 = slice * g.slice_k, k = cut ? min(g.slice_k, g.k - k0) : g.k;
     const float *a = g.a + (size_t)zo * g.a_bs + (size_t)zi * g.a_bs2 + (AKC ? (size_t)m0 * g.lda + k0 : (size_t)k0 * g.lda + m0);
-    const float *b = g.b + (size_t)zo * g.b_bs + (size_t)zi * g.b_bs2 + (BKC ? (size_t)n0 * g.ldb + k0 : (size_t)k0 * g.ldb + n0);
-
-    Loader<AKC, BM, WK, WAVES, VEC> la;
-    Loader<BKC, BN, WK, WAVES, VEC> lb;
-    const uint64_t a_floats = k == 0 ? 0 : AKC ? (uint64_t)(min(g.m - m0, (uint32_t)BM) - 1) * g.lda + k : (uint64_t)(k - 1) * g.lda + (g.m - m0);
-    const uint64_t b_floats = k == 0 ? 0 : BKC ? (uint64_t)(min(g.n - n0, (uint32_t)BN) - 1) * g.ldb + k : (uint64_t)(k - 1) * g.ldb + (g.n - n0);
-    const uint64_t a_step = AKC ? (uint64_t)BKT : (uint64_t)BKT * g.lda, b_step = BKC ? (uint64_t)BKT : (uint64_t)BKT * g.ldb;
-    constexpr int LOADS = decltype(la)::COUNT + decltype(lb)::COUNT;
+    const float *b = g.b + (size_t)zo * g.b_bs + (size_t)zi * g.b_bs2 + ((PLANES ? g.b_kc != 0 : BKC) ? (size_t)n0 * g.ldb + k0 : (size_t)k0 * g.ldb + n0);
 
     floatx16 acc[TA][TB];
+    if constexpr (PLANES) {
+        X x;
+        x.start(a, g.lda, min(g.m - m0, (uint32_t)BM), k, g.planes + ((uint64_t)(n0 / 32) * g.k16s + k0 / BK) * planes::SET, g.n32s - n0 / 32, g.k16s,
+                g.k16s - k0 / BK, lds, tid, wm, wn, wk);
+        x.run(acc);
+        // Where a sum is not finite an operand may have been infinite (inf - inf in the planes), or beyond 2^103, or the sum beyond 2^79: the
+        // wavefront's sums over its values of k once more on the fp32 matrix cores, which have fp32 arithmetic's result for every value.
+        bool lost = false;
 #pragma unroll
-    for (int i = 0; i < TA; i++)
+        for (int i = 0; i < TA; i++)
 #pragma unroll
-        for (int j = 0; j < TB; j++)
+            for (int j = 0; j < TB; j++)
 #pragma unroll
-            for (int e = 0; e < 16; e++) acc[i][j][e] = 0.0f;
-
-    // Where a tile and the one behind it are whole, and 32 bits reach, its addresses are the last tile's and a step (near: up to which
-    // tile).  Per step that is an addition per load; a base, an end and a mask worked out anew each time held the products up by
-    // 300 cycles a step (64 x 64 tiles: 18.8 ns a value of k for a CU's only block, 13.6 now).
-    const uint32_t nk = (k + BKT - 1) / BKT, whole = k / BKT;
-    uint32_t tile_k = 0, near = 0;
-    auto advance_near = [&]() __attribute__((always_inline)) {
-        la.next((uint32_t)a_step * 4);
-        lb.next((uint32_t)b_step * 4);
-        tile_k++;
-    };
-    auto advance_far = [&] __attribute__((always_inline)) {
-        la.start(a + tile_k * a_step, a_floats - tile_k * a_step, g.lda, k - tile_k * BKT, wave, lane);
-        lb.start(b + tile_k * b_step, b_floats - tile_k * b_step, g.ldb, k - tile_k * BKT, wave, lane);
-        near = min(whole, tile_k + 1 + min(g.window, 0x7fffffffu - tile_k));
-        tile_k++;
-    };
-    auto nothing_left = [&] __attribute__((always_inline)) {
-        la.nothing();
-        lb.nothing();
-    };
-    const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr)lds;
-    auto load = [&](auto u, uint32_t stage) __attribute__((always_inline)) {
-        if constexpr (u < la.COUNT) la.load(u, lds0 + stage * (STAGE * 4), wave);
-        else lb.load(u - la.COUNT, lds0 + (stage * STAGE + STAGE_A) * 4, wave);
-    };
-    // Behind the last tile 16-byte loads go on, for nothing: the waits and the steps stay as they are ([1872,3024] x [3024,2256] 202 us,
-    // 209 without those loads).  Single-value loads are four times as many, and end (96 of [148,32] x [32,2821], one step each: 98 us
-    // with the others', 77 without).
-    constexpr bool TO_THE_END = VEC == 4;
+                for (int e = 0; e < 16; e++) lost |= !(__builtin_fabsf(acc[i][j][e]) < __builtin_inff());
+        if (__builtin_expect(__any(lost), 0)) {
 #pragma unroll
-    for (int s = 0; s < S; s++) {
-        if (!TO_THE_END && tile_k >= nk) break;
-        if (tile_k < near) advance_near();
-        else if (tile_k < nk) advance_far();
-        else nothing_left();
-        each<LOADS>([&](auto u) __attribute__((always_inline)) { load(u, s); });
-    }
-
-    // This lane's fragments in stage 0, of either half of a step.
-    const float *pa[2], *pb[2];
+            for (int i = 0; i < TA; i++)
 #pragma unroll
-    for (int h = 0; h < 2; h++) {
-        if (AKC) {
-            const int row = wm * (32 * TA) + lr;
-            pa[h] = lds + (wk * BM + row) * BK + (((2 * h + lk) ^ ((row >> 2) & 3)) << 2);
+                for (int j = 0; j < TB; j++)
+#pragma unroll
+                    for (int e = 0; e < 16; e++) acc[i][j][e] = 0.0f;
+            const uint32_t row0 = wm * (32 * TA) + lr, col0 = wn * (32 * TB) + lr;
+#pragma unroll 1
+            for (uint32_t set = wk; set / 4 * 64 < k; set += WK)
+#pragma unroll 1
+                for (uint32_t s = 0; s < 8; s++) {
+                    const uint32_t kk = planes::k_of(set, lk, s);
+                    float va[TA], vb[TB];
+#pragma unroll
+                    for (int i = 0; i < TA; i++) va[i] = m0 + row0 + 32 * i < g.m && kk < k ? a[(size_t)(row0 + 32 * i) * g.lda + kk] : 0.0f;
+#pragma unroll
+                    for (int j = 0; j < TB; j++)
+                        vb[j] = n0 + col0 + 32 * j < g.n && kk < k ? b[g.b_kc ? (size_t)(col0 + 32 * j) * g.ldb + kk : (size_t)kk * g.ldb + col0 + 32 * j] : 0.0f;
+#pragma unroll
+                    for (int i = 0; i < TA; i++)
+#pragma unroll
+                        for (int j = 0; j < TB; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(va[i], vb[j], acc[i][j], 0, 0, 0);
+                }
         } else {
-            pa[h] = lds + (wk * BK + 8 * h + 4 * lk) * BM + wm * (32 * TA) + TA * lr;
+#pragma unroll
+            for (int i = 0; i < TA; i++)
+#pragma unroll
+                for (int j = 0; j < TB; j++)
+#pragma unroll
+                    for (int e = 0; e < 16; e++) acc[i][j][e] *= planes::UNSCALE;
         }
-        if (BKC) {
-            const int row = wn * (32 * TB) + lr;
-            pb[h] = lds + STAGE_A + (wk * BN + row) * BK + (((2 * h + lk) ^ ((row >> 2) & 3)) << 2);
-        } else {
-            pb[h] = lds + STAGE_A + (wk * BK + 8 * h + 4 * lk) * BN + wn * (32 * TB) + TB * lr;
-        }
-    }
+    } else {
+        Loader<AKC, BM, WK, WAVES, VEC> la;
+        Loader<BKC, BN, WK, WAVES, VEC> lb;
+        const uint64_t a_floats = k == 0 ? 0 : AKC ? (uint64_t)(min(g.m - m0, (uint32_t)BM) - 1) * g.lda + k : (uint64_t)(k - 1) * g.lda + (g.m - m0);
+        const uint64_t b_floats = k == 0 ? 0 : BKC ? (uint64_t)(min(g.n - n0, (uint32_t)BN) - 1) * g.ldb + k : (uint64_t)(k - 1) * g.ldb + (g.n - n0);
+        const uint64_t a_step = AKC ? (uint64_t)BKT : (uint64_t)BKT * g.lda, b_step = BKC ? (uint64_t)BKT : (uint64_t)BKT * g.ldb;
+        constexpr int LOADS = decltype(la)::COUNT + decltype(lb)::COUNT;
 
-    // Half a step's products while the next half's fragments are on their way.
-    Frag<AKC, TA> fa[2];
-    Frag<BKC, TB> fb[2];
-    auto read = [&](int h, uint32_t stage) __attribute__((always_inline)) {
-        fa[h].template read<BM>(pa[h] + stage * STAGE);
-        fb[h].template read<BN>(pb[h] + stage * STAGE);
-    };
-    constexpr int Q = 4 * TA * TB;
-    auto multiply = [&](int h, int q) __attribute__((always_inline)) {
-        const int s = q / (TA * TB), i = q / TB % TA, j = q % TB;
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[h].at(i, s), fb[h].at(j, s), acc[i][j], 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    if (WK == 4 && g.apart) {
-        const uint32_t turn = (blockIdx.x >> 8) % 3;
-        if (turn == 0) __builtin_amdgcn_s_setprio(0);
-        else if (turn == 1) __builtin_amdgcn_s_setprio(1);
-        else __builtin_amdgcn_s_setprio(2);
-    }
-    // Waits until at most `behind` stages, whose loads are the last ones, are on their way.
-    auto wait_behind = [&](uint32_t behind) __attribute__((always_inline)) {
-        if (behind >= S - 1) wait_loads_and_barrier<(S - 1) * LOADS>();
-        else if (S > 3 && behind == 2) wait_loads_and_barrier<2 * LOADS>();
-        else if (behind == 1) wait_loads_and_barrier<LOADS>();
-        else wait_loads_and_barrier<0>();
-    };
-    if (TO_THE_END) wait_loads_and_barrier<(S - 1) * LOADS>();
-    else wait_behind(max(nk, 1u) - 1);
-    read(0, 0);
-    uint32_t cur = 0;
-    // left: 0, or where the loads have ended how many steps there are from this one on.
-    auto step = [&](auto is_near, uint32_t left) __attribute__((always_inline)) {
-        each<Q>([&](auto q) __attribute__((always_inline)) {
-            multiply(0, q);
-            if constexpr (q == 0) read(1, cur);
-            if constexpr (q == 1 && is_near) advance_near();
-            __builtin_amdgcn_sched_barrier(0);
-        });
-        const uint32_t next = cur + 1 == S ? 0 : cur + 1;
-        each<Q>([&](auto q) __attribute__((always_inline)) {
-            constexpr int R = Q > 4 ? 1 : 0;
-            multiply(1, q);
-            if constexpr (q == 0) {  // this stage is read, the next one there
-                if (left) wait_behind(max(left, 2u) - 2);
-                else wait_loads_and_barrier<(S - 2) * LOADS>();
+#pragma unroll
+        for (int i = 0; i < TA; i++)
+#pragma unroll
+            for (int j = 0; j < TB; j++)
+#pragma unroll
+                for (int e = 0; e < 16; e++) acc[i][j][e] = 0.0f;
+
+        // Where a tile and the one behind it are whole, and 32 bits reach, its addresses are the last tile's and a step (near: up to which
+        // tile).  Per step that is an addition per load; a base, an end and a mask worked out anew each time held the products up by
+        // 300 cycles a step (64 x 64 tiles: 18.8 ns a value of k for a CU's only block, 13.6 now).
+        const uint32_t nk = (k + BKT - 1) / BKT, whole = k / BKT;
+        uint32_t tile_k = 0, near = 0;
+        auto advance_near = [&]() __attribute__((always_inline)) {
+            la.next((uint32_t)a_step * 4);
+            lb.next((uint32_t)b_step * 4);
+            tile_k++;
+        };
+        auto advance_far = [&] __attribute__((always_inline)) {
+            la.start(a + tile_k * a_step, a_floats - tile_k * a_step, g.lda, k - tile_k * BKT, wave, lane);
+            lb.start(b + tile_k * b_step, b_floats - tile_k * b_step, g.ldb, k - tile_k * BKT, wave, lane);
+            near = min(whole, tile_k + 1 + min(g.window, 0x7fffffffu - tile_k));
+            tile_k++;
+        };
+        auto nothing_left = [&] __attribute__((always_inline)) {
+            la.nothing();
+            lb.nothing();
+        };
+        const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_ptr)lds;
+        auto load = [&](auto u, uint32_t stage) __attribute__((always_inline)) {
+            if constexpr (u < la.COUNT) la.load(u, lds0 + stage * (STAGE * 4), wave);
+            else lb.load(u - la.COUNT, lds0 + (stage * STAGE + STAGE_A) * 4, wave);
+        };
+        // Behind the last tile 16-byte loads go on, for nothing: the waits and the steps stay as they are ([1872,3024] x [3024,2256] 202 us,
+        // 209 without those loads).  Single-value loads are four times as many, and end (96 of [148,32] x [32,2821], one step each: 98 us
+        // with the others', 77 without).
+        constexpr bool TO_THE_END = VEC == 4;
+#pragma unroll
+        for (int s = 0; s < S; s++) {
+            if (!TO_THE_END && tile_k >= nk) break;
+            if (tile_k < near) advance_near();
+            else if (tile_k < nk) advance_far();
+            else nothing_left();
+            each<LOADS>([&](auto u) __attribute__((always_inline)) { load(u, s); });
+        }
+
+        // This lane's fragments in stage 0, of either half of a step.
+        const float *pa[2], *pb[2];
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            if (AKC) {
+                const int row = wm * (32 * TA) + lr;
+                pa[h] = lds + (wk * BM + row) * BK + (((2 * h + lk) ^ ((row >> 2) & 3)) << 2);
+            } else {
+                pa[h] = lds + (wk * BK + 8 * h + 4 * lk) * BM + wm * (32 * TA) + TA * lr;
             }
-            if constexpr (q == R) read(0, next);
-            if (!left)
-                each<LOADS>([&](auto u) __attribute__((always_inline)) {
-                    if constexpr (R + 1 + u * (Q - 1 - R) / LOADS == q) load(u, cur);
-                });
-            __builtin_amdgcn_sched_barrier(0);
-        });
-        cur = next;
-    };
-    while (tile_k < nk) {
-        if (tile_k >= near) {
-            advance_far();
-            step(std::false_type(), 0);
+            if (BKC) {
+                const int row = wn * (32 * TB) + lr;
+                pb[h] = lds + STAGE_A + (wk * BN + row) * BK + (((2 * h + lk) ^ ((row >> 2) & 3)) << 2);
+            } else {
+                pb[h] = lds + STAGE_A + (wk * BK + 8 * h + 4 * lk) * BN + wn * (32 * TB) + TB * lr;
+            }
         }
-        while (tile_k < near) step(std::true_type(), 0);
-    }
-    if (TO_THE_END) nothing_left();
-    for (uint32_t left = min(nk, (uint32_t)S); left > 0; left--) step(std::false_type(), TO_THE_END ? 0 : left);
-    wait_loads_and_barrier<0>();
 
+        // Half a step's products while the next half's fragments are on their way.
+        Frag<AKC, TA> fa[2];
+        Frag<BKC, TB> fb[2];
+        auto read = [&](int h, uint32_t stage) __attribute__((always_inline)) {
+            fa[h].template read<BM>(pa[h] + stage * STAGE);
+            fb[h].template read<BN>(pb[h] + stage * STAGE);
+        };
+        constexpr int Q = 4 * TA * TB;
+        auto multiply = [&](int h, int q) __attribute__((always_inline)) {
+            const int s = q / (TA * TB), i = q / TB % TA, j = q % TB;
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[h].at(i, s), fb[h].at(j, s), acc[i][j], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        if (WK == 4 && g.apart) {
+            const uint32_t turn = (blockIdx.x >> 8) % 3;
+            if (turn == 0) __builtin_amdgcn_s_setprio(0);
+            else if (turn == 1) __builtin_amdgcn_s_setprio(1);
+            else __builtin_amdgcn_s_setprio(2);
+        }
+        // Waits until at most `behind` stages, whose loads are the last ones, are on their way.
+        auto wait_behind = [&](uint32_t behind) __attribute__((always_inline)) {
+            if (behind >= S - 1) wait_loads_and_barrier<(S - 1) * LOADS>();
+            else if (S > 3 && behind == 2) wait_loads_and_barrier<2 * LOADS>();
+            else if (behind == 1) wait_loads_and_barrier<LOADS>();
+            else wait_loads_and_barrier<0>();
+        };
+        if (TO_THE_END) wait_loads_and_barrier<(S - 1) * LOADS>();
+        else wait_behind(max(nk, 1u) - 1);
+        read(0, 0);
+        uint32_t cur = 0;
+        // left: 0, or where the loads have ended how many steps there are from this one on.
+        auto step = [&](auto is_near, uint32_t left) __attribute__((always_inline)) {
+            each<Q>([&](auto q) __attribute__((always_inline)) {
+                multiply(0, q);
+                if constexpr (q == 0) read(1, cur);
+                if constexpr (q == 1 && is_near) advance_near();
+                __builtin_amdgcn_sched_barrier(0);
+            });
+            const uint32_t next = cur + 1 == S ? 0 : cur + 1;
+            each<Q>([&](auto q) __attribute__((always_inline)) {
+                constexpr int R = Q > 4 ? 1 : 0;
+                multiply(1, q);
+                if constexpr (q == 0) {  // this stage is read, the next one there
+                    if (left) wait_behind(max(left, 2u) - 2);
+                    else wait_loads_and_barrier<(S - 2) * LOADS>();
+                }
+                if constexpr (q == R) read(0, next);
+                if (!left)
+                    each<LOADS>([&](auto u) __attribute__((always_inline)) {
+                        if constexpr (R + 1 + u * (Q - 1 - R) / LOADS == q) load(u, cur);
+                    });
+                __builtin_amdgcn_sched_barrier(0);
+            });
+            cur = next;
+        };
+        while (tile_k < nk) {
+            if (tile_k >= near) {
+                advance_far();
+                step(std::false_type(), 0);
+            }
+            while (tile_k < near) step(std::true_type(), 0);
+        }
+        if (TO_THE_END) nothing_left();
+        for (uint32_t left = min(nk, (uint32_t)S); left > 0; left--) step(std::false_type(), TO_THE_END ? 0 : left);
+        wait_loads_and_barrier<0>();
+
+    }
     if (WK == 4 && g.apart) __builtin_amdgcn_s_setprio(3);
     // Epilogue, TA passes of PASS_ROWS rows: accumulator e of lane l is row 8 (e / 4) + 4 (l / 32) + e % 4, column l % 32 of its
     // tile; through LDS the WK sums of an element meet and rows of C are stored 16 bytes per lane.
@@ -469,14 +528,22 @@ inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 
 // is 0.4 % behind the best one on average.  Per value of C a small tile costs more (each of its operands serves fewer products), but its
 // rounds come in smaller units.  A k_us of 10.24 per 64 x 64 would be the matrix cores' peak.
 struct Shape {
-    uint32_t bm, bn, step;  // step: values of k per barrier
+    uint32_t bm, bn, step, threads;  // step: values of k that a cut counts in
     double launch_us, block_us, k_us, lone, slice_us;
 };
-constexpr Shape SHAPES[] = {{32, 32, 64, 2.97, 0.72, 3.18, 1.02, 0.27},
-                            {64, 64, 32, 2.82, 1.06, 11.11, 1.04, 0.83},
-                            {128, 64, 16, 2.81, 1.38, 21.95, 1.04, 1.61},
-                            {128, 128, 16, 2.07, 3.63, 42.81, 1.02, 3.21}};
+constexpr Shape SHAPES[] = {{32, 32, 64, 256, 2.97, 0.72, 3.18, 1.02, 0.27},
+                            {64, 64, 32, 256, 2.82, 1.06, 11.11, 1.04, 0.83},
+                            {128, 64, 16, 256, 2.81, 1.38, 21.95, 1.04, 1.61},
+                            {128, 128, 16, 256, 2.07, 3.63, 42.81, 1.02, 3.21}};
 constexpr int N_SHAPES = 4;
+// The same with a weight matrix's planes for the second operand: 64 x 64, 64 x 128 and 128 x 128 with eight wavefronts, of which a CU holds
+// one block, and 128 x 128 with four, of which it holds two.  Fitted to 96 products of 256 to 12608 rows and 192 to 3072 values of k with
+// every tile, and 898 of them with the last round cut (7 and 6 % rms); the choice is 0.8 % behind the best one on average.
+constexpr Shape PLANE_SHAPES[] = {{64, 64, 64, 512, 1.18, 4.18, 7.38, 0.92, 0.59},
+                                  {64, 128, 64, 512, 1.0, 6.32, 12.38, 0.89, 0.85},
+                                  {128, 128, 64, 512, 1.0, 7.07, 24.52, 0.86, 1.5},
+                                  {128, 128, 64, 256, 1.0, 4.14, 26.38, 1.3, 2.9}};
+constexpr int N_PLANE_SHAPES = 4;
 
 struct Choice {
     int shape = 0;
@@ -487,10 +554,14 @@ struct Choice {
 // What a product adds up in which order is decided by the sizes alone, and by where a value lies in C: the values of a last round's
 // tiles add up in slices, the others in one piece, so that equal rows of A need not give equal bits.  A product and the same product with
 // an operand stored the other way round add up alike.  cut: k may be cut into slices.
-Choice choose(size_t batch, size_t m, size_t n, size_t k, size_t cus_per_xcd, bool cut) {
+// planes: of the tiles for weights as planes.
+Choice choose(size_t batch, size_t m, size_t n, size_t k, size_t cus_per_xcd, bool cut, bool planes = false) {
     Choice best;
-    for (int s = 0; s < N_SHAPES; s++) {
-        const Shape &sh = SHAPES[s];
+    const Shape *shapes = planes ? PLANE_SHAPES : SHAPES;
+    const int n_shapes = planes ? N_PLANE_SHAPES : N_SHAPES;
+    if (planes) k = (k + 63) / 64 * 64;
+    for (int s = 0; s < n_shapes; s++) {
+        const Shape &sh = shapes[s];
         const size_t chunk = (((m + sh.bm - 1) / sh.bm) * ((n + sh.bn - 1) / sh.bn) * batch + 7) / 8;
         const size_t rem = chunk % cus_per_xcd, whole = chunk / cus_per_xcd;  // tiles of a last round that is partly empty; rounds before it
         auto round_us = [&](size_t values) { return sh.block_us + sh.k_us * (double)std::max<size_t>(values, sh.step) / 768.0; };
@@ -499,7 +570,7 @@ Choice choose(size_t batch, size_t m, size_t n, size_t k, size_t cus_per_xcd, bo
             const size_t slice_k = ((k + want - 1) / want + sh.step - 1) / sh.step * sh.step, slices = slice_k ? (k + slice_k - 1) / slice_k : 1;
             if (want > 1 && slices != want) continue;
             // A grid ends at 2^32 threads: a few rows with 2^29 columns are more blocks of 32 x 32 than that.
-            if ((s < N_SHAPES - 1 || want > 1) && (chunk + rem * (want - 1)) * 8 * 256 > 0xffffffffu) break;
+            if ((s < n_shapes - 1 || want > 1) && (chunk + rem * (want - 1)) * 8 * sh.threads > 0xffffffffu) break;
             const size_t last = want == 1 ? rem != 0 : (rem * want + cus_per_xcd - 1) / cus_per_xcd;
             double us = sh.launch_us + ((double)whole * round_us(k) + (double)last * round_us(want == 1 ? k : slice_k)) * (whole + last == 1 ? sh.lone : 1.0);
             if (want > 1) us += 0.8 + want * (sh.slice_us + (double)(rem * 8) * sh.bm * sh.bn * sizeof(float) / 2.5e6);
@@ -511,16 +582,17 @@ Choice choose(size_t batch, size_t m, size_t n, size_t k, size_t cus_per_xcd, bo
 
 // A product's grid: of each XCD's run of tiles those that are whole, and the slices of the others.
 struct Grid {
-    size_t gx = 0, gy = 0, tiles = 0, chunk = 0, full = 0, blocks = 0;
-    Grid(const Choice &ch, size_t batch, size_t m, size_t n) {
-        const Shape &sh = SHAPES[ch.shape];
+    size_t gx = 0, gy = 0, tiles = 0, chunk = 0, full = 0, blocks = 0, threads = 256;
+    Grid(const Choice &ch, size_t batch, size_t m, size_t n, bool planes = false) {
+        const Shape &sh = planes ? PLANE_SHAPES[ch.shape] : SHAPES[ch.shape];
+        threads = sh.threads;
         gy = (m + sh.bm - 1) / sh.bm, gx = (n + sh.bn - 1) / sh.bn, tiles = gx * gy * batch, chunk = (tiles + 7) / 8;
         full = ch.slices > 1 ? ch.full : chunk;
         blocks = (full + (chunk - full) * ch.slices) * 8;
     }
     bool fits(size_t batch) const {
         const size_t lim = (size_t)1 << 31;
-        return gx * gy < lim && batch < lim && tiles < ((size_t)1 << 32) && blocks * 256 <= 0xffffffffu;
+        return gx * gy < lim && batch < lim && tiles < ((size_t)1 << 32) && blocks * threads <= 0xffffffffu;
     }
 };
 
@@ -540,9 +612,89 @@ template <bool AKC, bool BKC> void launch_tiles(const DeviceCtx &ctx, const Gemm
 #undef TILES
 }
 
+void launch_plane_tiles(const DeviceCtx &ctx, const GemmArgs &g, int shape, bool vec) {
+    const dim3 grid((g.full + (g.chunk - g.full) * g.slices) * 8), block(PLANE_SHAPES[shape].threads);
+#define TILES(WM, WN, WK, TA, TB, NB, NA)                                                                                               \
+    do {                                                                                                                                \
+        if (vec) hipLaunchKernelGGL((gemm_f32_tiles<true, true, WM, WN, WK, TA, TB, 4, planes::Tile<WM, WN, WK, TA, TB, 4, NB, NA>>),   \
+                                    grid, block, 0, ctx.stream, g);                                                                     \
+        else hipLaunchKernelGGL((gemm_f32_tiles<true, true, WM, WN, WK, TA, TB, 1, planes::Tile<WM, WN, WK, TA, TB, 1, NB, NA>>),       \
+                                grid, block, 0, ctx.stream, g);                                                                         \
+    } while (0)
+    switch (shape) {
+    case 0: TILES(1, 2, 4, 2, 1, 2, 2); break;
+    case 1: TILES(1, 2, 4, 2, 2, 2, 1); break;
+    case 2: TILES(2, 2, 2, 2, 2, 2, 1); break;
+    default: TILES(2, 2, 1, 2, 2, 2, 1); break;
+    }
+#undef TILES
+}
+
+// A weight matrix as planes: a wavefront per set, eight values a lane.  Element (k, n) is b[k * s_k + n * s_n].
+__global__ __launch_bounds__(256) void pack_planes(const float *__restrict__ b, u32x4 *__restrict__ out, uint32_t n, uint32_t k, size_t s_k, size_t s_n,
+                                                   uint32_t n32s, uint32_t k16s) {
+    const uint64_t set = (uint64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (set >= (uint64_t)n32s * k16s) return;
+    const uint32_t lane = threadIdx.x & 63, col = (uint32_t)(set / k16s) * 32 + (lane & 31), j = (uint32_t)(set % k16s);
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+        const uint32_t kk = planes::k_of(j, lane >> 5, e);
+        v[e] = col < n && kk < k ? b[(size_t)kk * s_k + (size_t)col * s_n] : 0.0f;
+    }
+    planes::Split4 s[2];
+    each<8>([&](auto p) {
+        s[0].part<p>(f32x4{v[0], v[1], v[2], v[3]});
+        s[1].part<p>(f32x4{v[4], v[5], v[6], v[7]});
+    });
+    each<3>([&](auto p) { out[set * (planes::SET / 16) + p * 64 + lane] = __builtin_shufflevector(s[0].q<p>(), s[1].q<p>(), 0, 1, 2, 3); });
+}
+
 constexpr size_t TILE_SPAN = (size_t)1 << 30;  // floats from a tile's first element to its last: byte offsets are 32 bits
 
 }  // namespace
+
+namespace {
+size_t weight_k16s(size_t k) { return (k + 63) / 64 * 4; }
+// A tile's rows of the first operand lie within 31-bit byte offsets, and a set's within 32 bits of its column's first.
+bool planes_reach(size_t lda, size_t k) { return k > 0 && k <= ((size_t)1 << 20) && 127 * lda + k < ((size_t)1 << 29); }
+}
+
+// Planes where they are reckoned 5 % faster, about what the estimates are off by: from a few hundred rows on ([1024,768] x [768,768 / 3072]
+// 13.7 -> 12.0 us, 39.8 -> 32.5, [1024,3072] x [3072,768] 42.3 -> 36.4; [6304,768] x [768,768 / 2304 / 3072] 62 -> 51, 171 -> 128,
+// 225 -> 166, [6304,3072] x [3072,768] 223 -> 158; [12608,768] x [768,3072] 450 -> 315).  With fewer, a block's start and end and the 6 bytes a
+// weight takes instead of 4 outweigh the products ([256,768] x [768,768] 6.8 and 10.1, [512,384] x [384,384] 5.4 and 8.0).
+bool gemm_takes_planes(const DeviceCtx &ctx, size_t m, size_t n, size_t k) {
+    if (gemm_takes_split(ctx, m, n, k) || m < 64 || n < 64 || k < 64 || m >= ((size_t)1 << 31) || n >= ((size_t)1 << 31)) return false;
+    const size_t cus = ctx.cus_per_xcd ? (size_t)ctx.cus_per_xcd : 32;
+    const Choice ch = choose(1, m, n, k, cus, ctx.gemm_split_k, true);
+    return ch.us < 0.95 * choose(1, m, n, k, cus, ctx.gemm_split_k).us && Grid(ch, 1, m, n, true).fits(1);
+}
+
+int gemm_pack_weights(DeviceCtx &ctx, const float *b, size_t n, size_t k, size_t ld, bool k_contig) {
+    if (gemm_packed_weights(ctx, b, n, k, ld, k_contig)) return AHIP_OK;
+    const size_t n32s = (n + 31) / 32, k16s = weight_k16s(k);
+    void *planes = nullptr;
+    if (hipMalloc(&planes, n32s * k16s * planes::SET) != hipSuccess) {
+        (void)hipGetLastError();
+        return ctx.fail(AHIP_ERR_OOM, "gemm: no memory for the planes of a weight matrix");
+    }
+    hipLaunchKernelGGL(pack_planes, dim3((unsigned)((n32s * k16s + 3) / 4)), dim3(256), 0, ctx.stream, b, static_cast<u32x4 *>(planes), (uint32_t)n,
+                       (uint32_t)k, k_contig ? (size_t)1 : ld, k_contig ? ld : (size_t)1, (uint32_t)n32s, (uint32_t)k16s);
+    const int rc = ctx.check(hipGetLastError(), "pack_planes launch");
+    if (rc) {
+        (void)hipFree(planes);
+        return rc;
+    }
+    ctx.gemm_weights.push_back(PackedWeights{b, n, k, ld, k_contig, planes});
+    return AHIP_OK;
+}
+
+const void *gemm_packed_weights(const DeviceCtx &ctx, const float *b, size_t n, size_t k, size_t ld, bool k_contig) {
+    for (const PackedWeights &w : ctx.gemm_weights)
+        if (w.b == b && w.n == n && w.k == k && w.ld == ld && w.k_contig == k_contig) return w.planes;
+    return nullptr;
+}
 
 bool gemm_takes_split(const DeviceCtx &ctx, size_t m, size_t n, size_t k) {
     return k > 0 && (ctx.gemm_algorithm == AHIP_GEMM_BF16X3 || (ctx.gemm_algorithm == AHIP_GEMM_AUTO && gemm_split_worthwhile(m, n, k)));
@@ -605,8 +757,11 @@ int launch_gemm_batch2(DeviceCtx &ctx, float *c, const float *a, const float *b,
     const bool has_post = post && (post->act != 0 || post->residual);
     if (!has_post && batch_outer * batch_inner == 1 && m && n && c && a && b && gemm_takes_split(ctx, m, n, k))
         return launch_gemm_split(ctx, c, a, b, c0, m, n, k, trans_a, trans_b, lda, ldb, ldc, c0_row_stride, c0_col_stride, alpha, beta);
+    const void *planes = nullptr;
+    if (batch_outer * batch_inner == 1 && !trans_a && !ctx.gemm_weights.empty() && gemm_takes_planes(ctx, m, n, k) && planes_reach(lda, k))
+        planes = gemm_packed_weights(ctx, b, n, k, ldb, trans_b != 0);
     return launch_gemm_f32(ctx, c, a, b, c0, batch_outer, batch_inner, m, n, k, trans_a, trans_b, lda, ldb, ldc, a_batch_strides, b_batch_strides,
-                           c_batch_strides, c0_row_stride, c0_col_stride, alpha, beta, post);
+                           c_batch_strides, c0_row_stride, c0_col_stride, alpha, beta, post, planes);
 }
 
 // What choose() reckons is fitted to larger products with 16-byte loads; a convolution's, which decide between this and a kernel that reads
@@ -635,7 +790,7 @@ int gemm_f32_grid(const DeviceCtx &ctx, size_t batch, size_t m, size_t n, size_t
 int launch_gemm_f32(DeviceCtx &ctx, float *c, const float *a, const float *b, const float *c0, size_t batch_outer, size_t batch_inner, size_t m,
                     size_t n, size_t k, int trans_a, int trans_b, size_t lda, size_t ldb, size_t ldc, const size_t a_batch_strides[2],
                     const size_t b_batch_strides[2], const size_t c_batch_strides[2], size_t c0_row_stride, size_t c0_col_stride, float alpha,
-                    float beta, const GemmPost *post) {
+                    float beta, const GemmPost *post, const void *planes) {
     const size_t batch = batch_outer * batch_inner;
     if (batch == 0 || m == 0 || n == 0) return AHIP_OK;
     if (!c || (k && (!a || !b))) return ctx.fail(AHIP_ERR_ARG, "gemm: null pointer");
@@ -648,7 +803,7 @@ int launch_gemm_f32(DeviceCtx &ctx, float *c, const float *a, const float *b, co
     // Hundreds of small matrices (attention's two products per head): one block per matrix.
     // (its fetchers address a head's operand with 32-bit byte offsets: 2^29 floats per head at most)
     const size_t a_extent = (m - 1) * lda + k, b_extent = trans_b ? (n - 1) * ldb + k : (k ? k - 1 : 0) * ldb + n;
-    if (!has_post && !trans_a && alpha == 1.0f && (!c0 || beta == 0.0f) && gemm_small_batched_fits(batch, m, n, k) &&
+    if (!planes && !has_post && !trans_a && alpha == 1.0f && (!c0 || beta == 0.0f) && gemm_small_batched_fits(batch, m, n, k) &&
         a_extent < ((size_t)1 << 29) && b_extent < ((size_t)1 << 29))
         return launch_gemm_small_batched(ctx, c, a, b, batch_outer, batch_inner, m, n, k, trans_b, lda, ldb, ldc, a_batch_strides, b_batch_strides,
                                          c_batch_strides);
@@ -691,17 +846,18 @@ int launch_gemm_f32(DeviceCtx &ctx, float *c, const float *a, const float *b, co
     auto vec = [&](const float *p, size_t contiguous, size_t ld, const size_t bs[2]) {
         return aligned16(p) && contiguous % 4 == 0 && ld % 4 == 0 && bs[0] % 4 == 0 && bs[1] % 4 == 0;
     };
-    const bool both = vec(a, a_kc ? k : m, lda, a_batch_strides) && vec(b, b_kc ? k : n, ldb, b_batch_strides);
-    Choice ch = choose(batch, m, n, k, cus, ctx.gemm_split_k);
+    const bool both = vec(a, a_kc ? k : m, lda, a_batch_strides) && (planes || vec(b, b_kc ? k : n, ldb, b_batch_strides));
+    const Shape *shapes = planes ? PLANE_SHAPES : SHAPES;
+    Choice ch = choose(batch, m, n, k, cus, ctx.gemm_split_k, planes);
     if (ch.slices > 1) {
-        const Shape &cut = SHAPES[ch.shape];
-        const Grid grid(ch, batch, m, n);
+        const Shape &cut = shapes[ch.shape];
+        const Grid grid(ch, batch, m, n, planes);
         const int rc = gemm_partials(ctx, (grid.chunk - grid.full) * 8 * ch.slices * cut.bm * cut.bn * sizeof(float));
-        if (rc == AHIP_ERR_OOM) ch = choose(batch, m, n, k, cus, false);  // no room: whole
+        if (rc == AHIP_ERR_OOM) ch = choose(batch, m, n, k, cus, false, planes);  // no room: whole
         else if (rc) return rc;
     }
-    const Shape &sh = SHAPES[ch.shape];
-    const Grid grid(ch, batch, m, n);
+    const Shape &sh = shapes[ch.shape];
+    const Grid grid(ch, batch, m, n, planes);
     if (!grid.fits(batch)) return ctx.fail(AHIP_ERR_UNSUPPORTED, "gemm: more tiles than a grid holds");
     g.tiles_n = (uint32_t)grid.gx;
     g.tiles_m = (uint32_t)grid.gy;
@@ -731,7 +887,13 @@ int launch_gemm_f32(DeviceCtx &ctx, float *c, const float *a, const float *b, co
         return span < end ? std::min<size_t>((end - span) / std::max<size_t>(step, 1), 0x7fffffff) : 0;
     };
     g.window = (uint32_t)std::min(window(a_kc, std::min<size_t>(sh.bm, a_kc ? m : sh.bm), lda), window(b_kc, std::min<size_t>(sh.bn, b_kc ? n : sh.bn), ldb));
-    if (a_kc && b_kc) launch_tiles<true, true>(ctx, g, ch.shape, both);
+    if (planes) {
+        g.window = (uint32_t)window(true, std::min<size_t>(sh.bm, m), lda);
+        g.planes = static_cast<const char *>(planes);
+        g.n32s = (uint32_t)((n + 31) / 32), g.k16s = (uint32_t)weight_k16s(k);
+        g.b_kc = b_kc;
+        launch_plane_tiles(ctx, g, ch.shape, both);
+    } else if (a_kc && b_kc) launch_tiles<true, true>(ctx, g, ch.shape, both);
     else if (a_kc) launch_tiles<true, false>(ctx, g, ch.shape, both);
     else if (b_kc) launch_tiles<false, true>(ctx, g, ch.shape, both);
     else launch_tiles<false, false>(ctx, g, ch.shape, both);

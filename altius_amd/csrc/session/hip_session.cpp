@@ -154,7 +154,8 @@ std::unique_ptr<HipSession> HipSessionBuilder::build(SessionError *err) {
         if (t.elem_ty() == TensorElemType::F32 && d.ptr && d.nbytes()) gemm_register_constant(s->ctx_, d.ptr, d.nbytes());
         s->inits_[kv.first] = std::move(d);
     }
-    rc = s->ctx_.check(hipStreamSynchronize(s->ctx_.stream), "hipStreamSynchronize(build)");
+    rc = s->pack_weights();
+    if (!rc) rc = s->ctx_.check(hipStreamSynchronize(s->ctx_.stream), "hipStreamSynchronize(build)");
     if (rc) {
         fail_code(err, rc, s->ctx_.last_error);
         return nullptr;
@@ -163,6 +164,36 @@ std::unique_ptr<HipSession> HipSessionBuilder::build(SessionError *err) {
 }
 
 // ---- HipSession -------------------------------------------------------------------------
+
+// Planes of the weights whose products take them (gemm_takes_planes), where their shapes were inferred.  Where there is no room for them the
+// products read the weights as they are.
+int HipSession::pack_weights() {
+    for (const NodeExecutionPlan &step : plan_) {
+        const Node &node = model_.graph.nodes[step.node_id];
+        if ((node.op.kind != OpKind::MatMul && node.op.kind != OpKind::Gemm) || node.op.trans_a || node.inputs.size() < 2) continue;
+        auto w = inits_.find(node.inputs[1]);
+        auto shape = inferred_.find(step.node_id);
+        if (w == inits_.end() || shape == inferred_.end() || w->second.elem_ty != TensorElemType::F32 || !w->second.ptr || w->second.dims.len() != 2) continue;
+        const FixedDimensions &wd = w->second.dims, &od = shape->second.second[0].dims;
+        const size_t k = node.op.trans_b ? wd[1] : wd[0], n = node.op.trans_b ? wd[0] : wd[1];
+        size_t rows = 1;
+        for (size_t i = 0; i + 1 < od.len(); i++) rows *= od[i];
+        if (!gemm_takes_planes(ctx_, rows, n, k)) continue;
+        const int rc = gemm_pack_weights(ctx_, static_cast<const float *>(w->second.ptr), n, k, wd[1], node.op.trans_b);
+        if (rc == AHIP_ERR_OOM) return AHIP_OK;
+        if (rc) return rc;
+    }
+    return AHIP_OK;
+}
+
+bool HipSession::matmul_by_planes(const Op &op, const std::vector<DeviceTensor *> &in) const {
+    if (ctx_.gemm_weights.empty() || op.trans_a || in[1]->dims.len() != 2 || !in[1]->strides.empty() || in[0]->dims.len() < 2) return false;
+    const FixedDimensions &ad = in[0]->dims, &wd = in[1]->dims;
+    size_t rows = 1;
+    for (size_t i = 0; i + 1 < ad.len(); i++) rows *= ad[i];
+    const size_t k = ad[ad.len() - 1], n = op.trans_b ? wd[0] : wd[1];
+    return gemm_packed_weights(ctx_, static_cast<const float *>(in[1]->ptr), n, k, wd[1], op.trans_b) && gemm_takes_planes(ctx_, rows, n, k);
+}
 
 HipSession::~HipSession() {
     if (pool_) {
@@ -1555,6 +1586,10 @@ bool HipSession::run_device_op(const Node &node, const Op &op, const std::vector
                 return false;
             }
         }
+        // A product with weights kept as planes takes its first operand as one tall matrix, whichever way it is handed on: other tiles would
+        // add up in another order.
+        const bool by_planes = matmul_by_planes(op, in);
+        if (by_planes && !in[0]->strides.empty() && !rows_at_one_pitch(*in[0]) && !materialize(in[0], err)) return false;
         MatOperand A, B;
         if (!describe_operand(in[0], &A, err) || !describe_operand(in[1], &B, err)) return false;
         // trans_a / trans_b (fuse_transpose_matmul): the logical operand is the transpose of the tensor.
@@ -1577,14 +1612,14 @@ bool HipSession::run_device_op(const Node &node, const Op &op, const std::vector
         // transposed shape, and this node's value is a view of it.
         std::vector<int64_t> c_str = dense_strides(out.dims);
         auto pv = matmul_out_perm_.find(current_node_);
-        if (pv != matmul_out_perm_.end() && pv->second.size() == out.dims.len()) {
+        if (!by_planes && pv != matmul_out_perm_.end() && pv->second.size() == out.dims.len()) {
             FixedDimensions td = out.dims;
             for (size_t i = 0; i < td.len(); i++) td[i] = out.dims[(size_t)pv->second[i]];
             const std::vector<int64_t> ts = dense_strides(td);
             for (size_t i = 0; i < td.len(); i++) c_str[(size_t)pv->second[i]] = ts[i];
             if (!is_dense(out.dims, c_str)) out.strides = c_str;
         }
-        const bool plain = in[0]->strides.empty() && in[1]->strides.empty() && out.strides.empty();
+        const bool plain = (in[0]->strides.empty() || by_planes) && in[1]->strides.empty() && out.strides.empty();
         if (plain && B.batch == 1 && A.batch == batch && !ta) {
             // [.., m, k] x [k, n]: one tall sgemm, as the reference does (session.rs:653-660)
             // On the fp32 kernel, the activation or the residual Add behind the product is done as it is written.

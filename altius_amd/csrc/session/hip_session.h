@@ -209,6 +209,12 @@ private:
         std::vector<size_t> bdims;
         std::vector<int64_t> bstr;
     };
+    // Whether the tensor's rows follow each other at one pitch whatever axes they are counted by: one tall matrix.
+    static bool rows_at_one_pitch(const DeviceTensor &t);
+    // Planes for the weights of products that take them; at build, behind the initializers' upload.
+    int pack_weights();
+    // Whether this MatMul's second operand is such a weight matrix, and the product takes its planes.
+    bool matmul_by_planes(const Op &op, const std::vector<DeviceTensor *> &in) const;
     // Fills *o; a view the GEMM's addressing cannot express is replaced by a dense copy first.
     bool describe_operand(DeviceTensor *t, MatOperand *o, SessionError *err);
     // MatMul -> Softmax -> MatMul as one kernel (plan_views finds the triples): the first MatMul leaves a

@@ -54,6 +54,15 @@ bool HipSession::apply_pending(DeviceTensor *t, SessionError *err) {
     return true;
 }
 
+bool HipSession::rows_at_one_pitch(const DeviceTensor &t) {
+    const size_t r = t.dims.len();
+    const std::vector<int64_t> st = strides_of(t);
+    if (r < 2 || t.dims[r - 2] < 2 || st[r - 1] != 1 || st[r - 2] < (int64_t)t.dims[r - 1]) return false;
+    for (size_t i = 0; i + 2 < r; i++)
+        if (t.dims[i] != 1 && st[i] != st[i + 1] * (int64_t)t.dims[i + 1]) return false;
+    return true;
+}
+
 bool HipSession::describe_operand(DeviceTensor *t, MatOperand *o, SessionError *err) {
     for (int attempt = 0; attempt < 2; attempt++) {
         const size_t r = t->dims.len();

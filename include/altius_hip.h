@@ -620,7 +620,12 @@ int ahip_session_builder_with_device_timing(ahip_session_builder *builder, int e
  * default keeps the reference's semantics for every operand value (compute_mat_mul, session.rs:621-684: an
  * infinite operand gives +-inf); AUTO and BF16X3 are the faster route a caller opts into, where an infinite
  * operand gives NaN.  The session declares its float initializers constant to the GEMM, so the bf16 planes
- * of a weight are made on its first use and kept until the session is freed. */
+ * of a weight are made on its first use and kept until the session is freed.
+ * On the default too a product of some hundred rows and more whose second operand is an initializer runs on the bf16 matrix
+ * cores where that is reckoned faster: six products of the exact three-way split, the small ones summed apart, and what does not
+ * come out finite computed again on the fp32 matrix cores, so that every operand value has fp32 arithmetic's result; against
+ * float64 it is 0.3 to 0.6 times as far off as the fp32 kernel.  Such a weight's planes (1.5 times its size) are made when the
+ * session is built; without room for them the product reads the weight as it is. */
 int ahip_session_builder_with_gemm_algorithm(ahip_session_builder *builder, int algorithm);
 /* Not in the reference, whose Split and Transpose always copy (session.rs:1179-1278, 1488-1548): with enable
  * != 0 (the default) a Split or Transpose whose result only MatMuls read, possibly through reshapes and further

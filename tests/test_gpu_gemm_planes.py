@@ -1,0 +1,114 @@
+"""Products of a session with weights kept as bf16 planes (csrc/device/gemm_planes.h) at the edges of their tiles, against float64: no
+further off than the fp32 kernel, and fp32 arithmetic's result for infinite, NaN, huge and denormal operand values."""
+import numpy as np
+import pytest
+
+from altius_amd import device as D
+from altius_amd.graph import Model, Op
+from altius_amd.session import HipSessionBuilder
+
+pytestmark = pytest.mark.gpu
+
+
+def product(rows, k, n, w, gemm=None, views=True):
+    """x [rows, k] times the weights; gemm: (trans_b, bias) of a Gemm instead of a MatMul."""
+    m = Model(opset_version=13)
+    x, y = m.new_val_named_and_shaped("x", [rows, k]), m.new_val()
+    m.add_input(x)
+    if gemm is None:
+        m.add_node(Op.MatMul, [x, m.new_initializer(w)], [y])
+    else:
+        m.add_node(Op.Gemm, [x, m.new_initializer(np.ascontiguousarray(w.T) if gemm[0] else w), m.new_initializer(gemm[1])], [y], trans_b=gemm[0])
+    m.add_output(y)
+    return HipSessionBuilder(m).with_strided_views(views).build()
+
+
+def fp32_kernel(a, w):
+    with D.Context(0) as ctx:
+        return ctx.matmul(a, w)
+
+
+# Rows at the edges of 64- and 128-row tiles and one past them; values of k that are no whole groups of 64, no whole float4s, and long enough
+# to be cut; columns that are no whole 32, 64 or 128.
+SIZES = [(1024, 768, 768), (1025, 768, 3072), (1089, 3072, 772), (4095, 772, 770), (3153, 770, 1537), (6304, 768, 768), (2049, 3076, 801), (8200, 381, 1000)]
+
+
+@pytest.mark.parametrize("rows,k,n", SIZES)
+def test_as_close_as_the_fp32_kernel(case, rows, k, n):
+    case(f"[{rows},{k}] x [{k},{n}]")
+    rng = np.random.default_rng(rows + k)
+    a = rng.standard_normal((rows, k)).astype(np.float32)
+    w = (rng.standard_normal((k, n)) * 0.05).astype(np.float32)
+    session = product(rows, k, n, w)
+    (got,) = session.run([a])
+    (again,) = session.run([a])
+    assert np.array_equal(got, again)
+    some = np.unique(np.concatenate([np.arange(0, rows, 37), [rows - 1]]))
+    want = a[some].astype(np.float64) @ w.astype(np.float64)
+    plain = fp32_kernel(a, w)
+    assert not np.array_equal(got, plain), "these sizes are meant to take the planes"
+    off, off32 = np.linalg.norm(got[some] - want), np.linalg.norm(plain[some] - want)
+    assert off <= off32
+    # Three dropped terms below 2^-25 of a product each; at most a chain of k / 16 + 1 additions to the larger sums and five times as many to
+    # the ones 2^-8 of them, each off by 2^-23 of what they add to; eight sums that meet behind them.
+    bound = (3 * 2.0**-25 + (k / 16 + 1 + 8) * (1 + 5 * 2.0**-8) * 2.0**-23) * (np.abs(a[some]).astype(np.float64) @ np.abs(w).astype(np.float64))
+    assert (np.abs(got[some] - want) <= bound).all()
+
+
+@pytest.mark.parametrize("trans_b", [False, True])
+def test_gemm_with_bias(case, trans_b):
+    case(f"Gemm, trans_b {trans_b}")
+    rng = np.random.default_rng(3)
+    a, w, b = (rng.standard_normal(s).astype(np.float32) for s in ((1100, 768), (768, 1500), (1500,)))
+    (got,) = product(1100, 768, 1500, w, gemm=(trans_b, b)).run([a])
+    (plain,) = product(1100, 768, 1500, w).run([a])
+    assert np.array_equal(got, plain + b)
+
+
+@pytest.mark.parametrize("rows,k,n", [(1100, 768, 1500), (1025, 771, 3070), (1089, 3072, 772)])
+def test_every_operand_value(case, rows, k, n):
+    case(f"infinite, NaN, huge and denormal operands, [{rows},{k}] x [{k},{n}]")
+    rng = np.random.default_rng(5)
+    a = rng.standard_normal((rows, k)).astype(np.float32)
+    w = (rng.standard_normal((k, n)) * 0.05).astype(np.float32)
+    a[3, 17], a[700, k - 1], a[rows - 1, 0], a[65, 40] = np.inf, -np.inf, np.inf, np.nan
+    a[129, :] = 0
+    a[129, 5], a[200, 9] = 3e38, -2e36
+    a[300] *= np.float32(1e-38)
+    a[301] *= np.float32(2.0**-100)
+    w[:, 7] *= np.float32(2.0**-20)
+    (got,) = product(rows, k, n, w).run([a])
+    with np.errstate(over="ignore", invalid="ignore"):
+        want = a.astype(np.float64) @ w.astype(np.float64)
+        magnitude = np.abs(a).astype(np.float64) @ np.abs(w).astype(np.float64)
+        want32 = want.astype(np.float32)
+    assert np.array_equal(np.isnan(got), np.isnan(want32))
+    infinite = np.isinf(want32)
+    assert infinite[[3, 700, rows - 1]].all() and np.array_equal(got[infinite], want32[infinite])
+    finite = np.isfinite(want32)
+    # fp32 arithmetic: k roundings, each of 2^-24 or, below the smallest normal number, of a whole denormal.
+    assert (np.abs(got[finite] - want[finite]) <= k * (2.0**-24 * magnitude + 2.0**-149)[finite]).all()
+    assert not np.array_equal(got[finite], fp32_kernel(a, w)[finite]), "these sizes are meant to take the planes"
+    assert not np.isfinite(product(rows, k, n, np.full_like(w, np.inf)).run([np.ones_like(a)])[0]).any()
+
+
+def test_a_view_has_the_bits_of_its_copy(case):
+    """Half of a Split's columns, read in place or copied first."""
+    case("a strided view of the first operand")
+    rng = np.random.default_rng(6)
+    x, w = rng.standard_normal((4, 300, 1536)).astype(np.float32), (rng.standard_normal((768, 768)) * 0.05).astype(np.float32)
+
+    def build(views):
+        m = Model(opset_version=13)
+        v = m.new_val_named_and_shaped("x", list(x.shape))
+        m.add_input(v)
+        left, right, y = (m.new_val() for _ in range(3))
+        m.add_node(Op.Split, [v, m.new_initializer(np.array([768, 768], np.int64))], [left, right], axis=2)
+        m.add_node(Op.MatMul, [right, m.new_initializer(w)], [y])
+        m.add_output(y)
+        m.add_output(left)
+        return HipSessionBuilder(m).with_strided_views(views).build()
+
+    in_place, copied = build(True).run([x])[0], build(False).run([x])[0]
+    assert np.array_equal(in_place, copied)
+    assert np.array_equal(in_place.reshape(1200, 768), product(1200, 768, 768, w).run([np.ascontiguousarray(x[..., 768:]).reshape(1200, 768)])[0])
