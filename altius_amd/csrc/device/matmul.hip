@@ -660,15 +660,21 @@ size_t weight_k16s(size_t k) { return (k + 63) / 64 * 4; }
 bool planes_reach(size_t lda, size_t k) { return k > 0 && k <= ((size_t)1 << 20) && 127 * lda + k < ((size_t)1 << 29); }
 }
 
-// Planes where they are reckoned 5 % faster, about what the estimates are off by: from a few hundred rows on ([1024,768] x [768,768 / 3072]
-// 13.7 -> 12.0 us, 39.8 -> 32.5, [1024,3072] x [3072,768] 42.3 -> 36.4; [6304,768] x [768,768 / 2304 / 3072] 62 -> 51, 171 -> 128,
-// 225 -> 166, [6304,3072] x [3072,768] 223 -> 158; [12608,768] x [768,3072] 450 -> 315).  With fewer, a block's start and end and the 6 bytes a
-// weight takes instead of 4 outweigh the products ([256,768] x [768,768] 6.8 and 10.1, [512,384] x [384,384] 5.4 and 8.0).
+// Planes where they are reckoned 5 % faster, about what the estimates are off by, and where weights that come from HBM leave a gain: from a
+// few hundred rows on, with the same weights again and again ([1024,768] x [768,768 / 3072] 13.7 -> 12.0 us, 39.8 -> 32.5, [1024,3072] x
+// [3072,768] 42.3 -> 36.4; [6304,768] x [768,768 / 2304 / 3072] 62 -> 51, 171 -> 128, 225 -> 166, [6304,3072] x [3072,768] 223 -> 158;
+// [12608,768] x [768,3072] 450 -> 315).  With fewer, a block's start and end and the 6 bytes a weight takes instead of 4 outweigh the products
+// ([256,768] x [768,768] 6.8 and 10.1, [512,384] x [384,384] 5.4 and 8.0).
+// A graph's weights are other ones in each product, and a block's few wavefronts wait for them longer than the estimates, fitted to one
+// product alone, say: in chains of 24 to 40 products 0.3 us for 3.5 MB of planes and 2 to 6 for 14 MB, and about as much for 38 to 232 MB,
+// where later tiles' products hide it.  Without that [256,768] x [768,3072] lost 1.3 us of 15, [512,3072] x [3072,768] 1.7 of 25 and
+// [788,1536] x [1536,384] 1.1 of 15.  Of 66 sizes in such chains, none that is taken loses, and those left out would gain 1.9 us at most.
 bool gemm_takes_planes(const DeviceCtx &ctx, size_t m, size_t n, size_t k) {
     if (gemm_takes_split(ctx, m, n, k) || m < 64 || n < 64 || k < 64 || m >= ((size_t)1 << 31) || n >= ((size_t)1 << 31)) return false;
     const size_t cus = ctx.cus_per_xcd ? (size_t)ctx.cus_per_xcd : 32;
     const Choice ch = choose(1, m, n, k, cus, ctx.gemm_split_k, true);
-    return ch.us < 0.95 * choose(1, m, n, k, cus, ctx.gemm_split_k).us && Grid(ch, 1, m, n, true).fits(1);
+    const double us = choose(1, m, n, k, cus, ctx.gemm_split_k).us, from_hbm = std::min(1.5e-6 * (double)n * (double)k, 3.6);
+    return ch.us + std::max(0.05 * us, from_hbm) < us && Grid(ch, 1, m, n, true).fits(1);
 }
 
 int gemm_pack_weights(DeviceCtx &ctx, const float *b, size_t n, size_t k, size_t ld, bool k_contig) {

@@ -55,6 +55,19 @@ def test_as_close_as_the_fp32_kernel(case, rows, k, n):
     assert (np.abs(got[some] - want) <= bound).all()
 
 
+@pytest.mark.parametrize("rows,k,n", [(77, 768, 16384), (129, 771, 16390)])
+def test_few_rows_and_many_columns(case, rows, k, n):
+    test_as_close_as_the_fp32_kernel(case, rows, k, n)
+
+
+@pytest.mark.parametrize("rows,k,n", [(256, 768, 3072), (512, 3072, 768), (788, 1536, 384)])
+def test_sizes_that_weights_from_memory_hold_up_stay_on_the_fp32_kernel(case, rows, k, n):
+    case(f"[{rows},{k}] x [{k},{n}]")
+    rng = np.random.default_rng(rows)
+    a, w = (rng.standard_normal(s).astype(np.float32) for s in ((rows, k), (k, n)))
+    assert np.array_equal(product(rows, k, n, w).run([a])[0], fp32_kernel(a, w))
+
+
 @pytest.mark.parametrize("trans_b", [False, True])
 def test_gemm_with_bias(case, trans_b):
     case(f"Gemm, trans_b {trans_b}")
