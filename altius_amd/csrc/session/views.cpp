@@ -58,8 +58,13 @@ bool HipSession::rows_at_one_pitch(const DeviceTensor &t) {
     const size_t r = t.dims.len();
     const std::vector<int64_t> st = strides_of(t);
     if (r < 2 || t.dims[r - 2] < 2 || st[r - 1] != 1 || st[r - 2] < (int64_t)t.dims[r - 1]) return false;
-    for (size_t i = 0; i + 2 < r; i++)
-        if (t.dims[i] != 1 && st[i] != st[i + 1] * (int64_t)t.dims[i + 1]) return false;
+    // An axis of extent 1 may carry any stride: what an axis in front of one has to step is counted from the rows.
+    int64_t step = st[r - 2] * (int64_t)t.dims[r - 2];
+    for (size_t i = r - 2; i-- > 0;) {
+        if (t.dims[i] == 1) continue;
+        if (st[i] != step) return false;
+        step *= (int64_t)t.dims[i];
+    }
     return true;
 }
 

@@ -125,3 +125,32 @@ def test_a_view_has_the_bits_of_its_copy(case):
     in_place, copied = build(True).run([x])[0], build(False).run([x])[0]
     assert np.array_equal(in_place, copied)
     assert np.array_equal(in_place.reshape(1200, 768), product(1200, 768, 768, w).run([np.ascontiguousarray(x[..., 768:]).reshape(1200, 768)])[0])
+
+
+@pytest.mark.parametrize("shape,axis", [((4, 1, 600, 768), 2), ((4, 1, 1, 600, 768), 3), ((1, 4, 600, 768), 2), ((4, 600, 768), 1), ((2, 600, 1, 768), 1), ((4, 1, 300, 1536), 3),
+                                        ((1, 1, 1200, 1536), 3)])
+def test_parts_of_a_split_read_in_place(case, shape, axis):
+    """Parts along the rows, behind axes of extent 1 too, start further apart than their rows go; parts along the columns do not."""
+    case(f"both halves of a Split of {shape} along axis {axis}")
+    rng = np.random.default_rng(7)
+    x, w = rng.standard_normal(shape).astype(np.float32), (rng.standard_normal((768, 768)) * 0.05).astype(np.float32)
+    half = shape[axis] // 2
+
+    def build(views):
+        m = Model(opset_version=13)
+        v = m.new_val_named_and_shaped("x", list(shape))
+        m.add_input(v)
+        parts, products = [m.new_val(), m.new_val()], [m.new_val(), m.new_val()]
+        m.add_node(Op.Split, [v, m.new_initializer(np.array([half, half], np.int64))], parts, axis=axis)
+        for part, y in zip(parts, products):
+            m.add_node(Op.MatMul, [part, m.new_initializer(w)], [y])
+            m.add_output(y)
+        return HipSessionBuilder(m).with_strided_views(views).build()
+
+    in_place, copied = build(True), build(False)
+    got, plain = in_place.run([x]), copied.run([x])
+    assert in_place.copies_avoided() > copied.copies_avoided() == 0
+    for y, z, part in zip(got, plain, np.split(x, 2, axis)):
+        want, magnitude = part.astype(np.float64) @ w.astype(np.float64), np.abs(part).astype(np.float64) @ np.abs(w).astype(np.float64)
+        # fp32 arithmetic: k roundings of 2^-24 each
+        assert (np.abs(y - want) <= 768 * 2.0**-24 * magnitude).all() and (np.abs(z - want) <= 768 * 2.0**-24 * magnitude).all()
