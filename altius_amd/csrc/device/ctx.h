@@ -193,16 +193,18 @@ int launch_batchnorm(DeviceCtx &ctx, float *out, const float *x, const float *sc
 int launch_gemm(DeviceCtx &ctx, float *c, const float *a, const float *b, const float *c0, size_t batch, size_t m, size_t n,
                 size_t k, int trans_a, int trans_b, size_t lda, size_t ldb, size_t ldc, size_t a_batch_stride,
                 size_t b_batch_stride, size_t c_batch_stride, size_t c0_row_stride, size_t c0_col_stride, float alpha,
-                float beta);
+                float beta, const void *planes = nullptr);
 
 // The same with the batch index split in two, z = (z / batch_inner, z % batch_inner), each part with its own
 // stride per operand: operands that are strided views of a larger tensor (the heads of a [b, t, h, d] tensor
 // read in place as b x h matrices of t x d with row pitch h * d) need no copy.
-// post (may be null): GemmPost.
+// post (may be null): GemmPost.  planes (may be null): the second operand's as gemm_packed_weights has them, which the fp32 kernels' products
+// of one matrix with op(A) = A read instead.
 int launch_gemm_batch2(DeviceCtx &ctx, float *c, const float *a, const float *b, const float *c0, size_t batch_outer,
                        size_t batch_inner, size_t m, size_t n, size_t k, int trans_a, int trans_b, size_t lda, size_t ldb, size_t ldc,
                        const size_t a_batch_strides[2], const size_t b_batch_strides[2], const size_t c_batch_strides[2],
-                       size_t c0_row_stride, size_t c0_col_stride, float alpha, float beta, const GemmPost *post = nullptr);
+                       size_t c0_row_stride, size_t c0_col_stride, float alpha, float beta, const GemmPost *post = nullptr,
+                       const void *planes = nullptr);
 
 // The same, on the fp32 kernels whatever ctx.gemm_algorithm says; and about how long the tiled one takes, in us (vec: both operands
 // allow 16-byte loads).
@@ -210,12 +212,13 @@ int launch_gemm_f32(DeviceCtx &ctx, float *c, const float *a, const float *b, co
                     size_t n, size_t k, int trans_a, int trans_b, size_t lda, size_t ldb, size_t ldc, const size_t a_batch_strides[2],
                     const size_t b_batch_strides[2], const size_t c_batch_strides[2], size_t c0_row_stride, size_t c0_col_stride, float alpha,
                     float beta, const GemmPost *post = nullptr, const void *planes = nullptr);
-// planes: the second operand's as gemm_packed_weights has them (one batch, op(A) = A).
 // Makes planes of a weight matrix, which is not written to or freed while the context lasts: a product with as many rows as gemm_takes_planes
 // wants then runs on the bf16 matrix cores, every value as the exact sum of three bf16 numbers (gemm_planes.h).  AHIP_ERR_OOM: none made.
 int gemm_pack_weights(DeviceCtx &ctx, const float *b, size_t n, size_t k, size_t ld, bool k_contig);
 const void *gemm_packed_weights(const DeviceCtx &ctx, const float *b, size_t n, size_t k, size_t ld, bool k_contig);
-bool gemm_takes_planes(const DeviceCtx &ctx, size_t m, size_t n, size_t k);
+// operand, result: the m rows are those of so many `matrices`, which the fp32 kernel reads as a Transpose in front of the product has them, or
+// writes as one behind it wants them; by planes that is a copy.
+bool gemm_takes_planes(const DeviceCtx &ctx, size_t m, size_t n, size_t k, size_t matrices = 1, bool operand = false, bool result = false);
 double gemm_f32_us(const DeviceCtx &ctx, size_t batch, size_t m, size_t n, size_t k, bool vec);
 // How many chains of sums over k, 16 values each in turn, meet in an element of that product (1, 2 or 4); 0: it is no product of whole
 // tiles (many small matrices, or k cut into slices).

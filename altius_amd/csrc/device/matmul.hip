@@ -669,12 +669,17 @@ bool planes_reach(size_t lda, size_t k) { return k > 0 && k <= ((size_t)1 << 20)
 // product alone, say: in chains of 24 to 40 products 0.3 us for 3.5 MB of planes and 2 to 6 for 14 MB, and about as much for 38 to 232 MB,
 // where later tiles' products hide it.  Without that [256,768] x [768,3072] lost 1.3 us of 15, [512,3072] x [3072,768] 1.7 of 25 and
 // [788,1536] x [1536,384] 1.1 of 15.  Of 66 sizes in such chains, none that is taken loses, and those left out would gain 1.9 us at most.
-bool gemm_takes_planes(const DeviceCtx &ctx, size_t m, size_t n, size_t k) {
+// A view that is not one tall matrix is copied first, a Transpose behind that the fp32 kernel writes ahead of copies the result; against that the
+// fp32 kernel's tiles end with each matrix.  Copies of results take 2.5 us and 6 TB/s (58 products of 512 to 6304 rows and 192 to 3072 values of k
+// with Transpose(1,0,2) behind: none that is taken loses, those left out would gain 2 % at most), of operands that Transpose(0,2,1) turns 5 us
+// and 1.4 TB/s ([64,196,512] turned x [196,256] 36 us in place, 65 by planes; [16,1024,768] x [1024,256 / 2048] 54 and 107, 386 and 332).
+bool gemm_takes_planes(const DeviceCtx &ctx, size_t m, size_t n, size_t k, size_t matrices, bool operand, bool result) {
     if (gemm_takes_split(ctx, m, n, k) || m < 64 || n < 64 || k < 64 || m >= ((size_t)1 << 31) || n >= ((size_t)1 << 31)) return false;
-    const size_t cus = ctx.cus_per_xcd ? (size_t)ctx.cus_per_xcd : 32;
+    const size_t cus = ctx.cus_per_xcd ? (size_t)ctx.cus_per_xcd : 32, parts = operand || result ? std::max<size_t>(matrices, 1) : 1;
     const Choice ch = choose(1, m, n, k, cus, ctx.gemm_split_k, true);
-    const double us = choose(1, m, n, k, cus, ctx.gemm_split_k).us, from_hbm = std::min(1.5e-6 * (double)n * (double)k, 3.6);
-    return ch.us + std::max(0.05 * us, from_hbm) < us && Grid(ch, 1, m, n, true).fits(1);
+    const double us = choose(parts, m / parts, n, k, cus, ctx.gemm_split_k).us, from_hbm = std::min(1.5e-6 * (double)n * (double)k, 3.6);
+    const double copies = (operand ? 5.0 + 8.0 * (double)m * (double)k / 1.4e6 : 0.0) + (result ? 2.5 + 8.0 * (double)m * (double)n / 6e6 : 0.0);
+    return ch.us + copies + std::max(0.05 * us, from_hbm) < us && Grid(ch, 1, m, n, true).fits(1);
 }
 
 int gemm_pack_weights(DeviceCtx &ctx, const float *b, size_t n, size_t k, size_t ld, bool k_contig) {
@@ -709,10 +714,10 @@ bool gemm_takes_split(const DeviceCtx &ctx, size_t m, size_t n, size_t k) {
 int launch_gemm(DeviceCtx &ctx, float *c, const float *a, const float *b, const float *c0, size_t batch, size_t m, size_t n,
                 size_t k, int trans_a, int trans_b, size_t lda, size_t ldb, size_t ldc, size_t a_batch_stride,
                 size_t b_batch_stride, size_t c_batch_stride, size_t c0_row_stride, size_t c0_col_stride, float alpha,
-                float beta) {
+                float beta, const void *planes) {
     const size_t a_bs[2] = {a_batch_stride, 0}, b_bs[2] = {b_batch_stride, 0}, c_bs[2] = {c_batch_stride, 0};
     return launch_gemm_batch2(ctx, c, a, b, c0, batch, 1, m, n, k, trans_a, trans_b, lda, ldb, ldc, a_bs, b_bs, c_bs, c0_row_stride,
-                              c0_col_stride, alpha, beta);
+                              c0_col_stride, alpha, beta, nullptr, planes);
 }
 
 // The product in parts of at most `part` values of m (axis 0), n (1) or k (2; the parts' sums meet in C).
@@ -759,13 +764,11 @@ static int launch_gemm_far_rows(DeviceCtx &ctx, int axis, size_t part, float *c,
 int launch_gemm_batch2(DeviceCtx &ctx, float *c, const float *a, const float *b, const float *c0, size_t batch_outer,
                        size_t batch_inner, size_t m, size_t n, size_t k, int trans_a, int trans_b, size_t lda, size_t ldb, size_t ldc,
                        const size_t a_batch_strides[2], const size_t b_batch_strides[2], const size_t c_batch_strides[2],
-                       size_t c0_row_stride, size_t c0_col_stride, float alpha, float beta, const GemmPost *post) {
+                       size_t c0_row_stride, size_t c0_col_stride, float alpha, float beta, const GemmPost *post, const void *planes) {
     const bool has_post = post && (post->act != 0 || post->residual);
     if (!has_post && batch_outer * batch_inner == 1 && m && n && c && a && b && gemm_takes_split(ctx, m, n, k))
         return launch_gemm_split(ctx, c, a, b, c0, m, n, k, trans_a, trans_b, lda, ldb, ldc, c0_row_stride, c0_col_stride, alpha, beta);
-    const void *planes = nullptr;
-    if (batch_outer * batch_inner == 1 && !trans_a && !ctx.gemm_weights.empty() && gemm_takes_planes(ctx, m, n, k) && planes_reach(lda, k))
-        planes = gemm_packed_weights(ctx, b, n, k, ldb, trans_b != 0);
+    if (batch_outer * batch_inner != 1 || trans_a || !planes_reach(lda, k)) planes = nullptr;
     return launch_gemm_f32(ctx, c, a, b, c0, batch_outer, batch_inner, m, n, k, trans_a, trans_b, lda, ldb, ldc, a_batch_strides, b_batch_strides,
                            c_batch_strides, c0_row_stride, c0_col_stride, alpha, beta, post, planes);
 }

@@ -115,7 +115,12 @@ std::unique_ptr<HipSession> HipSessionBuilder::build(SessionError *err) {
         return nullptr;
     }
     s->plan_ = create_execution_plan(s->model_);
-    if (strided_views_) s->plan_views(fused_attention_);
+    const HipSession::ViewPlan views = s->find_views();
+    if (strided_views_) {
+        s->lazy_views_ = views.lazy;
+        s->matmul_out_perm_ = views.out_perm;
+        s->plan_views(fused_attention_);
+    }
     if (strided_views_ && !enable_profiling_) s->plan_norm_chains();  // a profile names every node
     if (strided_views_ && !enable_profiling_) s->plan_attention_rows();
 
@@ -154,6 +159,7 @@ std::unique_ptr<HipSession> HipSessionBuilder::build(SessionError *err) {
         if (t.elem_ty() == TensorElemType::F32 && d.ptr && d.nbytes()) gemm_register_constant(s->ctx_, d.ptr, d.nbytes());
         s->inits_[kv.first] = std::move(d);
     }
+    s->plan_planes(views);
     rc = s->pack_weights();
     if (!rc) rc = s->ctx_.check(hipStreamSynchronize(s->ctx_.stream), "hipStreamSynchronize(build)");
     if (rc) {
@@ -165,34 +171,25 @@ std::unique_ptr<HipSession> HipSessionBuilder::build(SessionError *err) {
 
 // ---- HipSession -------------------------------------------------------------------------
 
-// Planes of the weights whose products take them (gemm_takes_planes), where their shapes were inferred.  Where there is no room for them the
-// products read the weights as they are.
+// Planes of the weights whose products take them (plan_planes).  Where there is no room for them the products read the weights as they are.
 int HipSession::pack_weights() {
-    for (const NodeExecutionPlan &step : plan_) {
-        const Node &node = model_.graph.nodes[step.node_id];
-        if ((node.op.kind != OpKind::MatMul && node.op.kind != OpKind::Gemm) || node.op.trans_a || node.inputs.size() < 2) continue;
-        auto w = inits_.find(node.inputs[1]);
-        auto shape = inferred_.find(step.node_id);
-        if (w == inits_.end() || shape == inferred_.end() || w->second.elem_ty != TensorElemType::F32 || !w->second.ptr || w->second.dims.len() != 2) continue;
-        const FixedDimensions &wd = w->second.dims, &od = shape->second.second[0].dims;
-        const size_t k = node.op.trans_b ? wd[1] : wd[0], n = node.op.trans_b ? wd[0] : wd[1];
-        size_t rows = 1;
-        for (size_t i = 0; i + 1 < od.len(); i++) rows *= od[i];
-        if (!gemm_takes_planes(ctx_, rows, n, k)) continue;
-        const int rc = gemm_pack_weights(ctx_, static_cast<const float *>(w->second.ptr), n, k, wd[1], node.op.trans_b);
-        if (rc == AHIP_ERR_OOM) return AHIP_OK;
-        if (rc) return rc;
+    for (auto it = by_planes_.begin(); it != by_planes_.end();) {
+        const Node &node = model_.graph.nodes[*it];
+        const DeviceTensor &w = inits_.at(node.inputs[1]);
+        const bool k_contig = inferred_.at(*it).first.trans_b;
+        const size_t k = k_contig ? w.dims[1] : w.dims[0], n = k_contig ? w.dims[0] : w.dims[1];
+        const float *b = static_cast<const float *>(w.ptr);
+        const int rc = gemm_pack_weights(ctx_, b, n, k, w.dims[1], k_contig);
+        if (rc && rc != AHIP_ERR_OOM) return rc;
+        if (!rc) node_planes_[*it] = gemm_packed_weights(ctx_, b, n, k, w.dims[1], k_contig);
+        it = rc ? by_planes_.erase(it) : std::next(it);
     }
     return AHIP_OK;
 }
 
-bool HipSession::matmul_by_planes(const Op &op, const std::vector<DeviceTensor *> &in) const {
-    if (ctx_.gemm_weights.empty() || op.trans_a || in[1]->dims.len() != 2 || !in[1]->strides.empty() || in[0]->dims.len() < 2) return false;
-    const FixedDimensions &ad = in[0]->dims, &wd = in[1]->dims;
-    size_t rows = 1;
-    for (size_t i = 0; i + 1 < ad.len(); i++) rows *= ad[i];
-    const size_t k = ad[ad.len() - 1], n = op.trans_b ? wd[0] : wd[1];
-    return gemm_packed_weights(ctx_, static_cast<const float *>(in[1]->ptr), n, k, wd[1], op.trans_b) && gemm_takes_planes(ctx_, rows, n, k);
+const void *HipSession::weight_planes() const {
+    auto it = node_planes_.find(current_node_);
+    return it == node_planes_.end() ? nullptr : it->second;
 }
 
 HipSession::~HipSession() {
@@ -1586,10 +1583,9 @@ bool HipSession::run_device_op(const Node &node, const Op &op, const std::vector
                 return false;
             }
         }
-        // A product with weights kept as planes takes its first operand as one tall matrix, whichever way it is handed on: other tiles would
-        // add up in another order.
-        const bool by_planes = matmul_by_planes(op, in);
-        if (by_planes && !in[0]->strides.empty() && !rows_at_one_pitch(*in[0]) && !materialize(in[0], err)) return false;
+        // A product with weights kept as planes takes its first operand as one tall matrix.
+        const void *planes = weight_planes();
+        if (planes && !in[0]->strides.empty() && !rows_at_one_pitch(in[0]->dims, in[0]->strides) && !materialize(in[0], err)) return false;
         MatOperand A, B;
         if (!describe_operand(in[0], &A, err) || !describe_operand(in[1], &B, err)) return false;
         // trans_a / trans_b (fuse_transpose_matmul): the logical operand is the transpose of the tensor.
@@ -1612,14 +1608,14 @@ bool HipSession::run_device_op(const Node &node, const Op &op, const std::vector
         // transposed shape, and this node's value is a view of it.
         std::vector<int64_t> c_str = dense_strides(out.dims);
         auto pv = matmul_out_perm_.find(current_node_);
-        if (!by_planes && pv != matmul_out_perm_.end() && pv->second.size() == out.dims.len()) {
+        if (!planes && pv != matmul_out_perm_.end() && pv->second.size() == out.dims.len()) {
             FixedDimensions td = out.dims;
             for (size_t i = 0; i < td.len(); i++) td[i] = out.dims[(size_t)pv->second[i]];
             const std::vector<int64_t> ts = dense_strides(td);
             for (size_t i = 0; i < td.len(); i++) c_str[(size_t)pv->second[i]] = ts[i];
             if (!is_dense(out.dims, c_str)) out.strides = c_str;
         }
-        const bool plain = (in[0]->strides.empty() || by_planes) && in[1]->strides.empty() && out.strides.empty();
+        const bool plain = (in[0]->strides.empty() || planes) && in[1]->strides.empty() && out.strides.empty();
         if (plain && B.batch == 1 && A.batch == batch && !ta) {
             // [.., m, k] x [k, n]: one tall sgemm, as the reference does (session.rs:653-660)
             // On the fp32 kernel, the activation or the residual Add behind the product is done as it is written.
@@ -1629,7 +1625,7 @@ bool HipSession::run_device_op(const Node &node, const Op &op, const std::vector
                 if (post.act || post.residual) {
                     const size_t none[2] = {0, 0};
                     rc = launch_gemm_batch2(ctx_, o, f(in[0]), f(in[1]), bias, 1, 1, batch * m, n, k, 0, tb, A.ld, B.ld, n, none, none, none, 0, 1, 1.0f,
-                                            beta, &post);
+                                            beta, &post, planes);
                     if (!rc && post.act) out.applied_op = post.act;
                     if (!rc && post.residual) absorbed_[mp->second.add_node] = mp->second.add_input;
                     break;
@@ -1640,7 +1636,7 @@ bool HipSession::run_device_op(const Node &node, const Op &op, const std::vector
             if (!out.ptr && !take_act_planes(batch * m, n, &out, &c_planes, &c_op, err)) return false;
             if (a_op || c_planes)
                 rc = launch_gemm_split(ctx_, o, f(in[0]), f(in[1]), bias, batch * m, n, k, 0, tb, A.ld, B.ld, n, 0, 1, 1.0f, beta, a_op, nullptr, c_op, c_planes);
-            else rc = launch_gemm(ctx_, o, f(in[0]), f(in[1]), bias, 1, batch * m, n, k, 0, tb, A.ld, B.ld, n, 0, 0, 0, 0, 1, 1.0f, beta);
+            else rc = launch_gemm(ctx_, o, f(in[0]), f(in[1]), bias, 1, batch * m, n, k, 0, tb, A.ld, B.ld, n, 0, 0, 0, 0, 1, 1.0f, beta, planes);
             break;
         }
         if (a_op) return fail(err, SessionError::Message, "MatMul: an activation was left pending on a product that cannot fold it");
@@ -1719,14 +1715,14 @@ bool HipSession::run_device_op(const Node &node, const Op &op, const std::vector
             if (post.act || post.residual) {
                 const size_t none[2] = {0, 0};
                 rc = launch_gemm_batch2(ctx_, o, f(in[0]), f(in[1]), c0, 1, 1, m, n, k, op.trans_a, op.trans_b, a[1], b[1], n, none, none, none, rs, cs,
-                                        op.alpha, c0 ? op.beta : 0.0f, &post);
+                                        op.alpha, c0 ? op.beta : 0.0f, &post, weight_planes());
                 if (!rc && post.act) out.applied_op = post.act;
                 if (!rc && post.residual) absorbed_[mp->second.add_node] = mp->second.add_input;
                 break;
             }
         }
         rc = launch_gemm(ctx_, o, f(in[0]), f(in[1]), c0, 1, m, n, k, op.trans_a, op.trans_b, a[1], b[1], n, 0, 0, 0, rs, cs, op.alpha,
-                         c0 ? op.beta : 0.0f);
+                         c0 ? op.beta : 0.0f, weight_planes());
         break;
     }
     default: return fail(err, SessionError::Message, opname + ": Kernel not implemented");

@@ -209,12 +209,19 @@ private:
         std::vector<size_t> bdims;
         std::vector<int64_t> bstr;
     };
-    // Whether the tensor's rows follow each other at one pitch whatever axes they are counted by: one tall matrix.
-    static bool rows_at_one_pitch(const DeviceTensor &t);
-    // Planes for the weights of products that take them; at build, behind the initializers' upload.
+    // What may be a view or be written ahead of a Transpose, whether or not the session does so.
+    struct ViewPlan {
+        std::set<NodeId> lazy;                              // Split / Transpose nodes whose outputs are views
+        std::map<NodeId, std::vector<int64_t>> out_perm;    // MatMul nodes -> perm of the Transpose they feed
+    };
+    ViewPlan find_views() const;
+    // Products that read their weights' planes, and those planes; made at build, behind the initializers' upload.
+    std::set<NodeId> by_planes_;
+    std::map<NodeId, const void *> node_planes_;
+    void plan_planes(const ViewPlan &views);
     int pack_weights();
-    // Whether this MatMul's second operand is such a weight matrix, and the product takes its planes.
-    bool matmul_by_planes(const Op &op, const std::vector<DeviceTensor *> &in) const;
+    // The planes that the node being run reads its weights from, or null.
+    const void *weight_planes() const;
     // Fills *o; a view the GEMM's addressing cannot express is replaced by a dense copy first.
     bool describe_operand(DeviceTensor *t, MatOperand *o, SessionError *err);
     // MatMul -> Softmax -> MatMul as one kernel (plan_views finds the triples): the first MatMul leaves a
@@ -356,8 +363,8 @@ private:
     bool run_attention_rows(NodeId id, std::map<ValueId, DeviceTensor> &values, bool *done, SessionError *err);
     // Runs a deferred Add into the tensor's block.
     bool flush_add(DeviceTensor *t, SessionError *err);
-    std::set<NodeId> lazy_views_;                               // Split / Transpose nodes whose outputs are views
-    std::map<NodeId, std::vector<int64_t>> matmul_out_perm_;    // MatMul nodes -> perm of the Transpose they feed
+    std::set<NodeId> lazy_views_;                               // ViewPlan::lazy and out_perm, where the session hands out views
+    std::map<NodeId, std::vector<int64_t>> matmul_out_perm_;
 };
 
 class HipSessionBuilder {

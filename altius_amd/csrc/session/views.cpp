@@ -54,20 +54,6 @@ bool HipSession::apply_pending(DeviceTensor *t, SessionError *err) {
     return true;
 }
 
-bool HipSession::rows_at_one_pitch(const DeviceTensor &t) {
-    const size_t r = t.dims.len();
-    const std::vector<int64_t> st = strides_of(t);
-    if (r < 2 || t.dims[r - 2] < 2 || st[r - 1] != 1 || st[r - 2] < (int64_t)t.dims[r - 1]) return false;
-    // An axis of extent 1 may carry any stride: what an axis in front of one has to step is counted from the rows.
-    int64_t step = st[r - 2] * (int64_t)t.dims[r - 2];
-    for (size_t i = r - 2; i-- > 0;) {
-        if (t.dims[i] == 1) continue;
-        if (st[i] != step) return false;
-        step *= (int64_t)t.dims[i];
-    }
-    return true;
-}
-
 bool HipSession::describe_operand(DeviceTensor *t, MatOperand *o, SessionError *err) {
     for (int attempt = 0; attempt < 2; attempt++) {
         const size_t r = t->dims.len();
@@ -274,17 +260,10 @@ bool HipSession::run_attention_tail(const Op &op, const std::vector<DeviceTensor
 // A Split or Transpose hands out views when everything downstream of it can read them in place:
 // MatMul operands, possibly through reshapes and further transposes.  A MatMul whose only reader is
 // a Transpose that keeps the last axis writes its result directly in that Transpose's layout.
-void HipSession::plan_views(bool fused_attention) {
+HipSession::ViewPlan HipSession::find_views() const {
     const auto users = model_.get_value_users();
-    const auto parents = model_.get_value_parents();
     const Graph &g = model_.graph;
     auto is_output = [&](ValueId v) { return std::find(g.outputs.begin(), g.outputs.end(), v) != g.outputs.end(); };
-    // The [k, n] f32 weights of a product, which no input of the graph can stand in for.
-    auto weight_matrix = [&](const Node &product) -> const Tensor * {
-        auto w = product.inputs.size() > 1 ? g.inits.find(product.inputs[1]) : g.inits.end();
-        if (w == g.inits.end() || std::find(g.inputs.begin(), g.inputs.end(), product.inputs[1]) != g.inputs.end()) return nullptr;
-        return w->second.dims().len() == 2 && w->second.elem_ty() == TensorElemType::F32 ? &w->second : nullptr;
-    };
     std::function<bool(ValueId, int)> view_ok = [&](ValueId v, int depth) -> bool {
         if (depth > 8 || is_output(v)) return false;
         auto it = users.find(v);
@@ -303,6 +282,108 @@ void HipSession::plan_views(bool fused_attention) {
             }
         }
         return true;
+    };
+    ViewPlan plan;
+    for (const NodeExecutionPlan &step : plan_) {
+        const NodeId id = step.node_id;
+        const Node &n = g.nodes[id];
+        if (n.op.kind == OpKind::Split || n.op.kind == OpKind::Transpose) {
+            bool all = !n.outputs.empty();
+            for (ValueId v : n.outputs) all = all && view_ok(v, 0);
+            if (all) plan.lazy.insert(id);
+        } else if (n.op.kind == OpKind::MatMul && n.outputs.size() == 1 && !is_output(n.outputs[0])) {
+            auto it = users.find(n.outputs[0]);
+            if (it == users.end() || it->second.size() != 1) continue;
+            const Node &t = g.nodes[*it->second.begin()];
+            if (t.op.kind != OpKind::Transpose || t.inputs.size() != 1) continue;
+            const auto &perm = t.op.perm;
+            if (perm.size() < 3 || perm.back() != (int64_t)perm.size() - 1) continue;
+            plan.out_perm[id] = perm;
+        }
+    }
+    return plan;
+}
+
+// The strides in which a result of these dims is dense once it is transposed by perm.
+static std::vector<int64_t> strides_ahead_of(const FixedDimensions &dims, const std::vector<int64_t> &perm) {
+    FixedDimensions td = dims;
+    for (size_t i = 0; i < td.len(); i++) td[i] = dims[(size_t)perm[i]];
+    const std::vector<int64_t> ts = dense_strides(td);
+    std::vector<int64_t> s(td.len());
+    for (size_t i = 0; i < td.len(); i++) s[(size_t)perm[i]] = ts[i];
+    return s;
+}
+
+// Which products read their weights' planes, from the graph and its inferred shapes alone: with the views that a session may hand out
+// (`views`) and without, a product runs the same sums.  By planes the first operand is one tall matrix and the result dense; gemm_takes_planes
+// counts the copies that this takes of a view and ahead of a Transpose.
+void HipSession::plan_planes(const ViewPlan &views) {
+    struct View {
+        FixedDimensions dims;
+        std::vector<int64_t> strides;
+    };
+    std::map<ValueId, View> view_of;  // values that are views where views are handed out
+    const Graph &g = model_.graph;
+    for (const NodeExecutionPlan &step : plan_) {
+        const NodeId id = step.node_id;
+        const Node &n = g.nodes[id];
+        auto it = inferred_.find(id);
+        if (it == inferred_.end() || n.inputs.empty() || n.outputs.empty() || it->second.second.size() < n.outputs.size()) continue;
+        const Op &op = it->second.first;
+        const std::vector<TypedFixedShape> &shapes = it->second.second;
+        const FixedDimensions &od = shapes[0].dims;
+        auto in = view_of.find(n.inputs[0]);
+        auto hand_out = [&](size_t i, const std::vector<int64_t> &strides) {
+            if (!is_dense(shapes[i].dims, strides)) view_of[n.outputs[i]] = View{shapes[i].dims, strides};
+        };
+        if (is_alias_op(op.kind)) {
+            std::vector<int64_t> s;
+            if (in != view_of.end() && reshape_strides(in->second.dims, in->second.strides, od, &s)) hand_out(0, s);
+        } else if (op.kind == OpKind::Transpose && views.lazy.count(id) && op.perm.size() == od.len()) {
+            FixedDimensions d = od;
+            for (size_t i = 0; i < od.len(); i++) d[(size_t)op.perm[i]] = od[i];
+            const std::vector<int64_t> s = in != view_of.end() ? in->second.strides : dense_strides(d);
+            std::vector<int64_t> ps(od.len());
+            for (size_t i = 0; i < od.len(); i++) ps[i] = s[(size_t)op.perm[i]];
+            hand_out(0, ps);
+        } else if (op.kind == OpKind::Split && views.lazy.count(id)) {
+            const size_t axis = (size_t)(op.axis < 0 ? op.axis + (int64_t)od.len() : op.axis);
+            if (axis >= od.len()) continue;
+            FixedDimensions d = od;
+            d[axis] = 0;
+            for (size_t p = 0; p < n.outputs.size(); p++) d[axis] += shapes[p].dims[axis];
+            const std::vector<int64_t> s = in != view_of.end() ? in->second.strides : dense_strides(d);
+            for (size_t p = 0; p < n.outputs.size(); p++) hand_out(p, s);
+        } else if (op.kind == OpKind::MatMul || op.kind == OpKind::Gemm) {
+            auto pv = views.out_perm.find(id);
+            std::vector<int64_t> ahead;  // of a Transpose behind the product
+            if (pv != views.out_perm.end() && pv->second.size() == od.len()) ahead = strides_ahead_of(od, pv->second);
+            if (!ahead.empty() && is_dense(od, ahead)) ahead.clear();
+            auto w = n.inputs.size() > 1 ? g.inits.find(n.inputs[1]) : g.inits.end();
+            if (!op.trans_a && w != g.inits.end() && w->second.elem_ty() == TensorElemType::F32 && w->second.dims().len() == 2 && od.len() >= 2 &&
+                std::find(g.inputs.begin(), g.inputs.end(), n.inputs[1]) == g.inputs.end()) {
+                const FixedDimensions &wd = w->second.dims();
+                size_t matrices = 1;
+                for (size_t i = 0; i + 2 < od.len(); i++) matrices *= od[i];
+                const bool turned = op.kind == OpKind::MatMul && in != view_of.end() && !rows_at_one_pitch(in->second.dims, in->second.strides);
+                if (gemm_takes_planes(ctx_, matrices * od[od.len() - 2], op.trans_b ? wd[0] : wd[1], op.trans_b ? wd[1] : wd[0], matrices, turned, !ahead.empty()))
+                    by_planes_.insert(id);
+            }
+            if (!ahead.empty() && !by_planes_.count(id)) hand_out(0, ahead);
+        }
+    }
+}
+
+void HipSession::plan_views(bool fused_attention) {
+    const auto users = model_.get_value_users();
+    const auto parents = model_.get_value_parents();
+    const Graph &g = model_.graph;
+    auto is_output = [&](ValueId v) { return std::find(g.outputs.begin(), g.outputs.end(), v) != g.outputs.end(); };
+    // The [k, n] f32 weights of a product, which no input of the graph can stand in for.
+    auto weight_matrix = [&](const Node &product) -> const Tensor * {
+        auto w = product.inputs.size() > 1 ? g.inits.find(product.inputs[1]) : g.inits.end();
+        if (w == g.inits.end() || std::find(g.inputs.begin(), g.inputs.end(), product.inputs[1]) != g.inputs.end()) return nullptr;
+        return w->second.dims().len() == 2 && w->second.elem_ty() == TensorElemType::F32 ? &w->second : nullptr;
     };
     // Product or convolution -> activation, or -> Add(residual): done by its own kernel when that is an fp32 one.
     // v: the result as that node reads it.
@@ -325,11 +406,7 @@ void HipSession::plan_views(bool fused_attention) {
     for (const NodeExecutionPlan &step : plan_) {
         const NodeId id = step.node_id;
         const Node &n = g.nodes[id];
-        if (n.op.kind == OpKind::Split || n.op.kind == OpKind::Transpose) {
-            bool all = !n.outputs.empty();
-            for (ValueId v : n.outputs) all = all && view_ok(v, 0);
-            if (all) lazy_views_.insert(id);
-        } else if ((n.op.kind == OpKind::Gelu || n.op.kind == OpKind::ReLU) && n.outputs.size() == 1 && n.inputs.size() == 1 &&
+        if ((n.op.kind == OpKind::Gelu || n.op.kind == OpKind::ReLU) && n.outputs.size() == 1 && n.inputs.size() == 1 &&
                    !is_output(n.outputs[0])) {
             // The activation between two products: its only reader is a MatMul's first operand.
             auto it = users.find(n.outputs[0]);
@@ -452,11 +529,6 @@ void HipSession::plan_views(bool fused_attention) {
                     }
                 }
             }
-            const Node &t = g.nodes[*it->second.begin()];
-            if (t.op.kind != OpKind::Transpose || t.inputs.size() != 1) continue;
-            const auto &perm = t.op.perm;
-            if (perm.size() < 3 || perm.back() != (int64_t)perm.size() - 1) continue;
-            matmul_out_perm_[id] = perm;
         }
     }
     // An attention whose result goes, through the Transpose it is written ahead of and one Reshape, into a product with a

@@ -122,6 +122,20 @@ inline bool reshape_strides(const FixedDimensions &old_dims, const std::vector<i
     return oi == od.size();
 }
 
+// Whether a view's rows follow each other at one pitch whatever axes they are counted by: one tall matrix.
+inline bool rows_at_one_pitch(const FixedDimensions &dims, const std::vector<int64_t> &st) {
+    const size_t r = dims.len();
+    if (r < 2 || dims[r - 2] < 2 || st[r - 1] != 1 || st[r - 2] < (int64_t)dims[r - 1]) return false;
+    // An axis of extent 1 may carry any stride: what an axis in front of one has to step is counted from the rows.
+    int64_t step = st[r - 2] * (int64_t)dims[r - 2];
+    for (size_t i = r - 2; i-- > 0;) {
+        if (dims[i] == 1) continue;
+        if (st[i] != step) return false;
+        step *= (int64_t)dims[i];
+    }
+    return true;
+}
+
 // [outer, axis, inner] view of `dims` around `axis`.
 inline void split_at(const FixedDimensions &dims, size_t axis, size_t *outer, size_t *len, size_t *inner) {
     *outer = *inner = 1;

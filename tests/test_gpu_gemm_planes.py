@@ -154,3 +154,60 @@ def test_parts_of_a_split_read_in_place(case, shape, axis):
         want, magnitude = part.astype(np.float64) @ w.astype(np.float64), np.abs(part).astype(np.float64) @ np.abs(w).astype(np.float64)
         # fp32 arithmetic: k roundings of 2^-24 each
         assert (np.abs(y - want) <= 768 * 2.0**-24 * magnitude).all() and (np.abs(z - want) <= 768 * 2.0**-24 * magnitude).all()
+
+
+@pytest.mark.parametrize("b,t,c,n,planes", [(64, 196, 512, 256, False), (16, 1024, 768, 512, False), (32, 300, 1088, 770, False), (16, 1024, 768, 2048, True)])
+def test_a_transposed_first_operand_counts_its_copy(case, b, t, c, n, planes):
+    """Tokens mixed by a product over the middle axis: the fp32 kernel reads the Transpose's input where it lies, as it does with weights that
+    are an input of the graph; by planes the tall operand is copied first, which few products are worth."""
+    case(f"Transpose(0,2,1) of [{b},{t},{c}], then [{t},{n}]")
+    rng = np.random.default_rng(8)
+    x, w = rng.standard_normal((b, t, c)).astype(np.float32), (rng.standard_normal((t, n)) * 0.05).astype(np.float32)
+
+    def build(constant, views=True):
+        m = Model(opset_version=13)
+        v = m.new_val_named_and_shaped("x", [b, t, c])
+        m.add_input(v)
+        weights = m.new_initializer(w) if constant else m.new_val_named_and_shaped("w", [t, n])
+        if not constant:
+            m.add_input(weights)
+        turned, y = m.new_val(), m.new_val()
+        m.add_node(Op.Transpose, [v], [turned], perm=[0, 2, 1])
+        m.add_node(Op.MatMul, [turned, weights], [y])
+        m.add_output(y)
+        return HipSessionBuilder(m).with_strided_views(views).build()
+
+    (got,) = build(True).run([x])
+    assert np.array_equal(got, build(False).run([x, w])[0]) != planes
+    if planes:
+        assert np.array_equal(got, build(True, views=False).run([x])[0])
+    some = np.arange(0, c, 37)
+    assert np.abs(got[::7, some] - np.swapaxes(x[::7], 1, 2)[:, some].astype(np.float64) @ w).max() < 1e-4
+
+
+@pytest.mark.parametrize("b,t,k,n,planes", [(8, 128, 768, 768, False), (12, 256, 384, 768, False), (32, 197, 768, 768, True), (8, 128, 768, 3072, True)])
+def test_a_transpose_behind_counts_its_copy(case, b, t, k, n, planes):
+    """A product whose result a Transpose reads is written in that layout by the fp32 kernel; planes are taken where they save more than the copy costs."""
+    case(f"[{b},{t},{k}] x [{k},{n}], then Transpose(1,0,2)")
+    rng = np.random.default_rng(9)
+    x, w = rng.standard_normal((b, t, k)).astype(np.float32), (rng.standard_normal((k, n)) * 0.05).astype(np.float32)
+
+    def build(constant, views=True):
+        m = Model(opset_version=13)
+        v = m.new_val_named_and_shaped("x", [b, t, k])
+        m.add_input(v)
+        weights = m.new_initializer(w) if constant else m.new_val_named_and_shaped("w", [k, n])
+        if not constant:
+            m.add_input(weights)
+        y, turned = m.new_val(), m.new_val()
+        m.add_node(Op.MatMul, [v, weights], [y])
+        m.add_node(Op.Transpose, [y], [turned], perm=[1, 0, 2])
+        m.add_output(turned)
+        return HipSessionBuilder(m).with_strided_views(views).build()
+
+    session = build(True)
+    (got,), (plain,) = session.run([x]), build(False).run([x, w])
+    assert np.array_equal(got, plain) != planes and session.copies_avoided() == (0 if planes else 1)
+    if planes:
+        assert np.array_equal(got, build(True, views=False).run([x])[0])
+    assert np.abs(got[::5] - np.swapaxes(x, 0, 1)[::5].astype(np.float64) @ w).max() < 1e-4
