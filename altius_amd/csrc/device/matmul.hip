@@ -670,7 +670,7 @@ bool planes_reach(size_t lda, size_t k) { return k > 0 && k <= ((size_t)1 << 20)
 // where later tiles' products hide it.  Without that [256,768] x [768,3072] lost 1.3 us of 15, [512,3072] x [3072,768] 1.7 of 25 and
 // [788,1536] x [1536,384] 1.1 of 15.  Of 66 sizes in such chains, none that is taken loses, and those left out would gain 1.9 us at most.
 // A view that is not one tall matrix is copied first, a Transpose behind that the fp32 kernel writes ahead of copies the result; against that the
-// fp32 kernel's tiles end with each matrix.  Copies of results take 2.5 us and 6 TB/s (58 products of 512 to 6304 rows and 192 to 3072 values of k
+// fp32 kernel's tiles end with each matrix.  Copies of results take 2 us and 6 TB/s (58 products of 512 to 6304 rows and 192 to 3072 values of k
 // with Transpose(1,0,2) behind: none that is taken loses, those left out would gain 2 % at most), of operands that Transpose(0,2,1) turns 5 us
 // and 1.4 TB/s ([64,196,512] turned x [196,256] 36 us in place, 65 by planes; [16,1024,768] x [1024,256 / 2048] 54 and 107, 386 and 332).
 bool gemm_takes_planes(const DeviceCtx &ctx, size_t m, size_t n, size_t k, size_t matrices, bool operand, bool result) {
@@ -678,7 +678,7 @@ bool gemm_takes_planes(const DeviceCtx &ctx, size_t m, size_t n, size_t k, size_
     const size_t cus = ctx.cus_per_xcd ? (size_t)ctx.cus_per_xcd : 32, parts = operand || result ? std::max<size_t>(matrices, 1) : 1;
     const Choice ch = choose(1, m, n, k, cus, ctx.gemm_split_k, true);
     const double us = choose(parts, m / parts, n, k, cus, ctx.gemm_split_k).us, from_hbm = std::min(1.5e-6 * (double)n * (double)k, 3.6);
-    const double copies = (operand ? 5.0 + 8.0 * (double)m * (double)k / 1.4e6 : 0.0) + (result ? 2.5 + 8.0 * (double)m * (double)n / 6e6 : 0.0);
+    const double copies = (operand ? 5.0 + 8.0 * (double)m * (double)k / 1.4e6 : 0.0) + (result ? 2.0 + 8.0 * (double)m * (double)n / 6e6 : 0.0);
     return ch.us + copies + std::max(0.05 * us, from_hbm) < us && Grid(ch, 1, m, n, true).fits(1);
 }
 
