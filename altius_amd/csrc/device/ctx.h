@@ -28,14 +28,6 @@ struct PackedOperand {
     size_t bytes;
 };
 
-// A weight matrix [k, n] (k_contig: stored [n, k]) and its planes for the products that read it (device memory, owned).
-struct PackedWeights {
-    const float *b;
-    size_t n, k, ld;
-    bool k_contig;
-    void *planes;
-};
-
 // The streaming threshold of a session's context (see DeviceCtx::nt_threshold_bytes).
 constexpr size_t SESSION_NT_THRESHOLD_BYTES = (size_t)128 << 20;
 
@@ -86,7 +78,6 @@ struct DeviceCtx {
     bool gemm_in_kernel_k_cut = true;
     std::vector<ConstantBuffer> gemm_constants;
     std::vector<PackedOperand> gemm_packed;
-    std::vector<PackedWeights> gemm_weights;
     std::string last_error;
 
     bool streaming(size_t bytes) const { return bytes >= nt_threshold_bytes; }
@@ -198,7 +189,7 @@ int launch_gemm(DeviceCtx &ctx, float *c, const float *a, const float *b, const 
 // The same with the batch index split in two, z = (z / batch_inner, z % batch_inner), each part with its own
 // stride per operand: operands that are strided views of a larger tensor (the heads of a [b, t, h, d] tensor
 // read in place as b x h matrices of t x d with row pitch h * d) need no copy.
-// post (may be null): GemmPost.  planes (may be null): the second operand's as gemm_packed_weights has them, which the fp32 kernels' products
+// post (may be null): GemmPost.  planes (may be null): the second operand's as gemm_pack_weights leaves them, which the fp32 kernels' products
 // of one matrix with op(A) = A read instead.
 int launch_gemm_batch2(DeviceCtx &ctx, float *c, const float *a, const float *b, const float *c0, size_t batch_outer,
                        size_t batch_inner, size_t m, size_t n, size_t k, int trans_a, int trans_b, size_t lda, size_t ldb, size_t ldc,
@@ -212,10 +203,10 @@ int launch_gemm_f32(DeviceCtx &ctx, float *c, const float *a, const float *b, co
                     size_t n, size_t k, int trans_a, int trans_b, size_t lda, size_t ldb, size_t ldc, const size_t a_batch_strides[2],
                     const size_t b_batch_strides[2], const size_t c_batch_strides[2], size_t c0_row_stride, size_t c0_col_stride, float alpha,
                     float beta, const GemmPost *post = nullptr, const void *planes = nullptr);
-// Makes planes of a weight matrix, which is not written to or freed while the context lasts: a product with as many rows as gemm_takes_planes
-// wants then runs on the bf16 matrix cores, every value as the exact sum of three bf16 numbers (gemm_planes.h).  AHIP_ERR_OOM: none made.
-int gemm_pack_weights(DeviceCtx &ctx, const float *b, size_t n, size_t k, size_t ld, bool k_contig);
-const void *gemm_packed_weights(const DeviceCtx &ctx, const float *b, size_t n, size_t k, size_t ld, bool k_contig);
+// Planes of a weight matrix [k, n] (k_contig: stored [n, k]), gemm_weight_planes_bytes of device memory: a product with as many rows as
+// gemm_takes_planes wants runs by them on the bf16 matrix cores, every value as the exact sum of three bf16 numbers (gemm_planes.h).
+size_t gemm_weight_planes_bytes(size_t n, size_t k);
+int gemm_pack_weights(DeviceCtx &ctx, void *planes, const float *b, size_t n, size_t k, size_t ld, bool k_contig);
 // operand, result: the m rows are those of so many `matrices`, which the fp32 kernel reads as a Transpose in front of the product has them, or
 // writes as one behind it wants them; by planes that is a copy.
 bool gemm_takes_planes(const DeviceCtx &ctx, size_t m, size_t n, size_t k, size_t matrices = 1, bool operand = false, bool result = false);

@@ -790,8 +790,6 @@ int gemm_unregister_constant(DeviceCtx &ctx, const void *ptr) {
 void gemm_release_all(DeviceCtx &ctx) {
     for (PackedOperand &p : ctx.gemm_packed) (void)hipFree(p.planes);
     ctx.gemm_packed.clear();
-    for (PackedWeights &w : ctx.gemm_weights) (void)hipFree(w.planes);
-    ctx.gemm_weights.clear();
     ctx.gemm_constants.clear();
     if (ctx.gemm_ws) (void)hipFree(ctx.gemm_ws);
     ctx.gemm_ws = nullptr;

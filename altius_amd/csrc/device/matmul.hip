@@ -682,29 +682,13 @@ bool gemm_takes_planes(const DeviceCtx &ctx, size_t m, size_t n, size_t k, size_
     return ch.us + copies + std::max(0.05 * us, from_hbm) < us && Grid(ch, 1, m, n, true).fits(1);
 }
 
-int gemm_pack_weights(DeviceCtx &ctx, const float *b, size_t n, size_t k, size_t ld, bool k_contig) {
-    if (gemm_packed_weights(ctx, b, n, k, ld, k_contig)) return AHIP_OK;
+size_t gemm_weight_planes_bytes(size_t n, size_t k) { return (n + 31) / 32 * weight_k16s(k) * planes::SET; }
+
+int gemm_pack_weights(DeviceCtx &ctx, void *planes, const float *b, size_t n, size_t k, size_t ld, bool k_contig) {
     const size_t n32s = (n + 31) / 32, k16s = weight_k16s(k);
-    void *planes = nullptr;
-    if (hipMalloc(&planes, n32s * k16s * planes::SET) != hipSuccess) {
-        (void)hipGetLastError();
-        return ctx.fail(AHIP_ERR_OOM, "gemm: no memory for the planes of a weight matrix");
-    }
     hipLaunchKernelGGL(pack_planes, dim3((unsigned)((n32s * k16s + 3) / 4)), dim3(256), 0, ctx.stream, b, static_cast<u32x4 *>(planes), (uint32_t)n,
                        (uint32_t)k, k_contig ? (size_t)1 : ld, k_contig ? ld : (size_t)1, (uint32_t)n32s, (uint32_t)k16s);
-    const int rc = ctx.check(hipGetLastError(), "pack_planes launch");
-    if (rc) {
-        (void)hipFree(planes);
-        return rc;
-    }
-    ctx.gemm_weights.push_back(PackedWeights{b, n, k, ld, k_contig, planes});
-    return AHIP_OK;
-}
-
-const void *gemm_packed_weights(const DeviceCtx &ctx, const float *b, size_t n, size_t k, size_t ld, bool k_contig) {
-    for (const PackedWeights &w : ctx.gemm_weights)
-        if (w.b == b && w.n == n && w.k == k && w.ld == ld && w.k_contig == k_contig) return w.planes;
-    return nullptr;
+    return ctx.check(hipGetLastError(), "pack_planes launch");
 }
 
 bool gemm_takes_split(const DeviceCtx &ctx, size_t m, size_t n, size_t k) {

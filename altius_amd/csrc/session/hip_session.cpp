@@ -171,25 +171,59 @@ std::unique_ptr<HipSession> HipSessionBuilder::build(SessionError *err) {
 
 // ---- HipSession -------------------------------------------------------------------------
 
-// Planes of the weights whose products take them (plan_planes).  Where there is no room for them the products read the weights as they are.
+// Planes of the weights whose products take them (plan_planes), in a third of the memory that is free once the weights are there: what comes
+// behind, this session's runs or somebody else's, finds the rest.  A product whose planes have no room reads its weights as they are.
 int HipSession::pack_weights() {
-    for (auto it = by_planes_.begin(); it != by_planes_.end();) {
-        const Node &node = model_.graph.nodes[*it];
-        const DeviceTensor &w = inits_.at(node.inputs[1]);
-        const bool k_contig = inferred_.at(*it).first.trans_b;
-        const size_t k = k_contig ? w.dims[1] : w.dims[0], n = k_contig ? w.dims[0] : w.dims[1];
-        const float *b = static_cast<const float *>(w.ptr);
-        const int rc = gemm_pack_weights(ctx_, b, n, k, w.dims[1], k_contig);
-        if (rc && rc != AHIP_ERR_OOM) return rc;
-        if (!rc) node_planes_[*it] = gemm_packed_weights(ctx_, b, n, k, w.dims[1], k_contig);
-        it = rc ? by_planes_.erase(it) : std::next(it);
+    size_t left = 0, total = 0;
+    int rc = by_planes_.empty() ? AHIP_OK : ctx_.check(hipStreamSynchronize(ctx_.stream), "hipStreamSynchronize(weights)");
+    if (rc || by_planes_.empty()) return rc;
+    if (hipMemGetInfo(&left, &total) != hipSuccess) (void)hipGetLastError(), left = 0;
+    left /= 3;
+    auto made = std::make_unique<WeightPlanes>();
+    for (NodeId id : by_planes_) {
+        const ValueId v = model_.graph.nodes[id].inputs[1];
+        const DeviceTensor &w = inits_.at(v);
+        const bool k_contig = inferred_.at(id).first.trans_b;
+        const size_t k = k_contig ? w.dims[1] : w.dims[0], n = k_contig ? w.dims[0] : w.dims[1], bytes = gemm_weight_planes_bytes(n, k);
+        void *&planes = made->of[{v, k_contig}];
+        if (!planes && bytes <= left) {
+            if (hipMalloc(&planes, bytes) != hipSuccess) {
+                (void)hipGetLastError();
+                planes = nullptr, left = 0;
+            } else {
+                left -= bytes;
+                if ((rc = gemm_pack_weights(ctx_, planes, static_cast<const float *>(w.ptr), n, k, w.dims[1], k_contig))) return rc;
+            }
+        }
+        if (planes) node_planes_[id] = planes;
     }
+    if (!node_planes_.empty()) weight_planes_ = std::move(made);
     return AHIP_OK;
+}
+
+HipSession::WeightPlanes::~WeightPlanes() {
+    for (auto &p : of)
+        if (p.second) (void)hipFree(p.second);
 }
 
 const void *HipSession::weight_planes() const {
     auto it = node_planes_.find(current_node_);
     return it == node_planes_.end() ? nullptr : it->second;
+}
+
+// A run that finds no memory gives the planes of the weights back, which it can do without, and starts again.
+template <class F> bool HipSession::retry_without_planes(SessionError *err, F run) {
+    SessionError local;
+    SessionError *e = err ? err : &local;
+    if (run(e)) return true;
+    if (!weight_planes_ || e->kind != SessionError::OutOfMemory) return false;
+    (void)hipStreamSynchronize(ctx_.stream);
+    (void)hipGetLastError();
+    drop_graphs();  // recorded launches read the planes
+    eager_runs_.clear();
+    node_planes_.clear();
+    weight_planes_.reset();
+    return run(e);
 }
 
 HipSession::~HipSession() {
@@ -199,6 +233,7 @@ HipSession::~HipSession() {
         drop_graphs();
         if (span_begin_) (void)hipEventDestroy(span_begin_);
         if (span_end_) (void)hipEventDestroy(span_end_);
+        weight_planes_.reset();
         inits_.clear();  // blocks go back to the pool before it is destroyed
         pool_.reset();
         destroy_device_ctx(&ctx_);
@@ -297,6 +332,10 @@ bool HipSession::check_input(size_t i, TensorElemType elem_ty, const FixedDimens
 
 bool HipSession::run(const std::vector<Tensor> &inputs, std::vector<Tensor> *outputs, SessionError *err) {
     std::lock_guard<std::mutex> lock(mutex_);
+    return retry_without_planes(err, [&](SessionError *e) { return run_once(inputs, outputs, e); });
+}
+
+bool HipSession::run_once(const std::vector<Tensor> &inputs, std::vector<Tensor> *outputs, SessionError *err) {
     const auto t0 = std::chrono::steady_clock::now();
     if (!outputs) return fail(err, SessionError::Argument, "run: null output vector");
     outputs->clear();
@@ -422,6 +461,10 @@ bool HipSession::run(const std::vector<Tensor> &inputs, std::vector<Tensor> *out
 
 bool HipSession::run_device(const std::vector<DeviceTensor> &inputs, std::vector<DeviceTensor> *outputs, SessionError *err) {
     std::lock_guard<std::mutex> lock(mutex_);
+    return retry_without_planes(err, [&](SessionError *e) { return run_device_once(inputs, outputs, e); });
+}
+
+bool HipSession::run_device_once(const std::vector<DeviceTensor> &inputs, std::vector<DeviceTensor> *outputs, SessionError *err) {
     const auto t0 = std::chrono::steady_clock::now();
     if (!outputs) return fail(err, SessionError::Argument, "run_device: null output vector");
     outputs->clear();

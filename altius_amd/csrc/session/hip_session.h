@@ -216,10 +216,18 @@ private:
     };
     ViewPlan find_views() const;
     // Products that read their weights' planes, and those planes; made at build, behind the initializers' upload.
+    struct WeightPlanes {
+        std::map<std::pair<ValueId, bool>, void *> of;  // weights, whether k is contiguous
+        ~WeightPlanes();
+    };
     std::set<NodeId> by_planes_;
     std::map<NodeId, const void *> node_planes_;
+    std::unique_ptr<WeightPlanes> weight_planes_;
     void plan_planes(const ViewPlan &views);
     int pack_weights();
+    template <class F> bool retry_without_planes(SessionError *err, F run);
+    bool run_once(const std::vector<Tensor> &inputs, std::vector<Tensor> *outputs, SessionError *err);
+    bool run_device_once(const std::vector<DeviceTensor> &inputs, std::vector<DeviceTensor> *outputs, SessionError *err);
     // The planes that the node being run reads its weights from, or null.
     const void *weight_planes() const;
     // Fills *o; a view the GEMM's addressing cannot express is replaced by a dense copy first.

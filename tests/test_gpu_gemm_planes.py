@@ -1,11 +1,15 @@
 """Products of a session with weights kept as bf16 planes (csrc/device/gemm_planes.h) at the edges of their tiles, against float64: no
 further off than the fp32 kernel, and fp32 arithmetic's result for infinite, NaN, huge and denormal operand values."""
+import contextlib
+import ctypes
+
 import numpy as np
 import pytest
 
 from altius_amd import device as D
 from altius_amd.graph import Model, Op
 from altius_amd.session import HipSessionBuilder
+from test_gpu_graph_replay import hip_runtime
 
 pytestmark = pytest.mark.gpu
 
@@ -211,3 +215,60 @@ def test_a_transpose_behind_counts_its_copy(case, b, t, k, n, planes):
     if planes:
         assert np.array_equal(got, build(True, views=False).run([x])[0])
     assert np.abs(got[::5] - np.swapaxes(x, 0, 1)[::5].astype(np.float64) @ w).max() < 1e-4
+
+
+def weights_and_room(rows, k, n, w):
+    """rows of x times w, and the largest of `room` ones: a run that needs as much memory as its second input says."""
+    m = Model(opset_version=13)
+    x, shape = m.new_val_named_and_shaped("x", [rows, k]), m.new_val_named("shape")
+    y, ones, z = m.new_val(), m.new_val(), m.new_val()
+    m.add_input(x)
+    m.add_input(shape)
+    m.add_node(Op.MatMul, [x, m.new_initializer(w)], [y])
+    m.add_node(Op.Expand, [m.new_initializer(np.ones(1, np.float32)), shape], [ones])
+    m.add_node(Op.ReduceMax, [ones], [z], axes=[0, 1], keep_dims=1)
+    m.add_output(y)
+    m.add_output(z)
+    return HipSessionBuilder(m)
+
+
+def free_memory():
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert hip_runtime().hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
+
+
+@contextlib.contextmanager
+def memory_left(nbytes):
+    """All of the GPU's memory but that much is taken."""
+    with D.Context(0) as holder:
+        holder.alloc(free_memory() - nbytes)
+        yield
+
+
+def test_planes_give_way_to_what_a_run_needs(case):
+    """1 GiB of weights have 1.5 GiB of planes; a run that needs more than is left otherwise does without them, and so do later ones."""
+    case("planes go when a run finds no memory")
+    rng = np.random.default_rng(10)
+    rows, k, n = 128, 8192, 32768
+    x, w = rng.standard_normal((rows, k)).astype(np.float32), rng.standard_normal((k, n), dtype=np.float32)
+    plain = fp32_kernel(x, w)
+    session = weights_and_room(rows, k, n, w).build()
+    small = np.array([4, 256], np.int64)
+    assert not np.array_equal(session.run([x, small])[0], plain), "this size is meant to take the planes"
+    with memory_left(1 << 30):
+        for shape in (np.array([2048, 1 << 18], np.int64), small):  # 2 GiB
+            y, z = session.run([x, shape])
+            assert np.array_equal(y, plain) and np.array(z).ravel() == [1.0]
+
+
+def test_planes_leave_room_for_what_comes_behind(case):
+    """Planes take a third of what is free when a session is built, or are not made."""
+    case("planes are not made where memory is short")
+    rng = np.random.default_rng(11)
+    rows, k, n = 128, 8192, 32768
+    x, w = rng.standard_normal((rows, k)).astype(np.float32), rng.standard_normal((k, n), dtype=np.float32)
+    plain = fp32_kernel(x, w)
+    with memory_left(9 << 29):  # 4.5 GiB
+        y, _ = weights_and_room(rows, k, n, w).build().run([x, np.array([4, 256], np.int64)])
+    assert np.array_equal(y, plain)
