@@ -27,6 +27,7 @@ int global_fail(int code, const std::string &msg) {
 int global_check(hipError_t e, const char *what) {
     if (e == hipSuccess) return AHIP_OK;
     altius::set_global_error(std::string(what) + ": " + hipGetErrorString(e));
+    (void)hipGetLastError();
     return e == hipErrorOutOfMemory ? AHIP_ERR_OOM : AHIP_ERR_HIP;
 }
 

@@ -20,12 +20,14 @@ int DeviceCtx::fail(int code, const std::string &msg) {
 int DeviceCtx::check(hipError_t e, const char *what) {
     if (e == hipSuccess) return AHIP_OK;
     last_error = std::string(what) + ": " + hipGetErrorString(e);
+    (void)hipGetLastError();  // reported here, not behind this thread's next launch
     return e == hipErrorOutOfMemory ? AHIP_ERR_OOM : AHIP_ERR_HIP;
 }
 
 int create_device_ctx(int device, hipStream_t stream, bool own_stream, DeviceCtx *ctx, std::string *error) {
     auto fail = [&](hipError_t e, const char *what) {
         if (error) *error = std::string(what) + ": " + hipGetErrorString(e);
+        (void)hipGetLastError();
         return e == hipErrorOutOfMemory ? AHIP_ERR_OOM : AHIP_ERR_HIP;
     };
     int n = 0;

@@ -460,6 +460,29 @@ def test_softmax_with_absorbed_scale_and_mask(case, shape, mask_shape, scale_kin
     assert_close(got, O.softmax(z), what="vs oracle chain")
 
 
+def test_a_run_behind_one_that_found_no_memory(case):
+    """The failed allocation is that run's error: it does not come back from the next launch of the same thread."""
+    case("a run that fits behind one that does not")
+    m = Model()
+    x, shape = m.new_val_named_and_shaped("x", [64, 64]), m.new_val_named("shape")
+    ones, y, z = m.new_val(), m.new_val(), m.new_val()
+    m.add_input(x)
+    m.add_input(shape)
+    m.add_node(Op.MatMul, [x, m.new_initializer(np.eye(64, dtype=np.float32))], [y])
+    m.add_node(Op.Expand, [m.new_initializer(np.ones(1, np.float32)), shape], [ones])
+    m.add_node(Op.ReduceMax, [ones], [z], axes=[0, 1], keep_dims=True)
+    m.add_output(y)
+    m.add_output(z)
+    sess, a = HipSessionBuilder(m).build(), synth.normal(5, [64, 64])
+    for _ in range(2):
+        with pytest.raises(AltiusHipError) as e:
+            sess.run([a, np.array([1 << 20, 1 << 20], np.int64)])  # 4 TB
+        assert e.value.code == ERR_OOM
+        (got, one) = sess.run([a, np.array([2, 3], np.int64)])
+        assert_bits_equal(got, a, "x times the unit matrix")
+        assert np.array(one).ravel() == [1.0]
+
+
 def test_run_from_several_threads(case):
     """InterpreterSession::run takes &self and may be called from several threads at once (per-thread value maps,
     session.rs:52-58).  Here a session gives each of the calls that overlap a lane of its own (stream, buffer pool,
