@@ -79,7 +79,7 @@ int acquire_lane(ahip_session *session, size_t *index, std::shared_ptr<HipSessio
     const ahip_session_builder &b = session->settings;
     HipSessionBuilder hb(session->view.m);
     hb.with_intra_op_num_threads(b.threads).with_profiling_enabled(b.profiling).with_device(b.device).with_graph_replay(b.graph_replay).with_device_timing(b.device_timing)
-        .with_gemm_algorithm(b.gemm_algorithm).with_strided_views(b.strided_views).with_fused_attention(b.fused_attention);
+        .with_gemm_algorithm(b.gemm_algorithm).with_strided_views(b.strided_views).with_fused_attention(b.fused_attention).share_planes(*session->s);
     SessionError err;
     std::shared_ptr<HipSession> lane;
     try {

@@ -160,11 +160,19 @@ std::unique_ptr<HipSession> HipSessionBuilder::build(SessionError *err) {
         s->inits_[kv.first] = std::move(d);
     }
     s->plan_planes(views);
-    rc = s->pack_weights();
+    if (shares_planes_) s->weight_planes_ = planes_;
+    else rc = s->pack_weights();
     if (!rc) rc = s->ctx_.check(hipStreamSynchronize(s->ctx_.stream), "hipStreamSynchronize(build)");
     if (rc) {
         fail_code(err, rc, s->ctx_.last_error);
         return nullptr;
+    }
+    if (s->weight_planes_) {
+        std::lock_guard<std::mutex> lock(s->weight_planes_->mutex);
+        for (NodeId id : s->by_planes_) {
+            auto it = s->weight_planes_->of.find({s->model_.graph.nodes[id].inputs[1], s->inferred_.at(id).first.trans_b != 0});
+            if (it != s->weight_planes_->of.end() && it->second) s->node_planes_[id] = it->second;
+        }
     }
     return s;
 }
@@ -179,31 +187,55 @@ int HipSession::pack_weights() {
     if (rc || by_planes_.empty()) return rc;
     if (hipMemGetInfo(&left, &total) != hipSuccess) (void)hipGetLastError(), left = 0;
     left /= 3;
-    auto made = std::make_unique<WeightPlanes>();
+    auto made = std::make_shared<WeightPlanes>();
+    made->queued = ctx_.stream;
     for (NodeId id : by_planes_) {
         const ValueId v = model_.graph.nodes[id].inputs[1];
         const DeviceTensor &w = inits_.at(v);
         const bool k_contig = inferred_.at(id).first.trans_b;
         const size_t k = k_contig ? w.dims[1] : w.dims[0], n = k_contig ? w.dims[0] : w.dims[1], bytes = gemm_weight_planes_bytes(n, k);
         void *&planes = made->of[{v, k_contig}];
-        if (!planes && bytes <= left) {
-            if (hipMalloc(&planes, bytes) != hipSuccess) {
-                (void)hipGetLastError();
-                planes = nullptr, left = 0;
-            } else {
-                left -= bytes;
-                if ((rc = gemm_pack_weights(ctx_, planes, static_cast<const float *>(w.ptr), n, k, w.dims[1], k_contig))) return rc;
-            }
+        if (planes || bytes > left) continue;
+        if (hipMalloc(&planes, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            planes = nullptr, left = 0;
+            continue;
         }
-        if (planes) node_planes_[id] = planes;
+        left -= bytes;
+        if ((rc = gemm_pack_weights(ctx_, planes, static_cast<const float *>(w.ptr), n, k, w.dims[1], k_contig))) return rc;
     }
-    if (!node_planes_.empty()) weight_planes_ = std::move(made);
+    weight_planes_ = std::move(made);
     return AHIP_OK;
 }
 
-HipSession::WeightPlanes::~WeightPlanes() {
+void HipSession::WeightPlanes::release() {
     for (auto &p : of)
         if (p.second) (void)hipFree(p.second);
+    of.clear();
+}
+
+HipSession::PlanesInUse::PlanesInUse(HipSession *session) : s(session) {
+    if (!s->weight_planes_) return;
+    WeightPlanes &p = *s->weight_planes_;
+    std::unique_lock<std::mutex> lock(p.mutex);
+    while (p.going && !p.gone) p.left.wait(lock);
+    s->planes_there_ = !p.gone;
+    if (s->planes_there_) p.running++;
+    else s->forget_planes();
+}
+
+HipSession::PlanesInUse::~PlanesInUse() {
+    if (!s->planes_there_) return;
+    std::lock_guard<std::mutex> lock(s->weight_planes_->mutex);
+    s->weight_planes_->running--;
+    s->weight_planes_->left.notify_all();
+}
+
+void HipSession::forget_planes() {
+    if (node_planes_.empty()) return;
+    drop_graphs();  // recorded launches read them
+    eager_runs_.clear();
+    node_planes_.clear();
 }
 
 const void *HipSession::weight_planes() const {
@@ -215,14 +247,25 @@ const void *HipSession::weight_planes() const {
 template <class F> bool HipSession::retry_without_planes(SessionError *err, F run) {
     SessionError local;
     SessionError *e = err ? err : &local;
-    if (run(e)) return true;
-    if (!weight_planes_ || e->kind != SessionError::OutOfMemory) return false;
+    {
+        const PlanesInUse use(this);
+        if (run(e)) return true;
+    }
+    if (!planes_there_ || e->kind != SessionError::OutOfMemory) return false;
     (void)hipStreamSynchronize(ctx_.stream);
     (void)hipGetLastError();
-    drop_graphs();  // recorded launches read the planes
-    eager_runs_.clear();
-    node_planes_.clear();
-    weight_planes_.reset();
+    forget_planes();
+    planes_there_ = false;
+    {
+        WeightPlanes &p = *weight_planes_;
+        std::unique_lock<std::mutex> lock(p.mutex);
+        p.going = true;
+        while (p.running) p.left.wait(lock);
+        if (p.queued && !p.gone) (void)hipStreamSynchronize(p.queued);
+        p.release();
+        p.gone = true;
+        p.left.notify_all();
+    }
     return run(e);
 }
 
@@ -233,6 +276,10 @@ HipSession::~HipSession() {
         drop_graphs();
         if (span_begin_) (void)hipEventDestroy(span_begin_);
         if (span_end_) (void)hipEventDestroy(span_end_);
+        if (weight_planes_) {
+            std::lock_guard<std::mutex> lock(weight_planes_->mutex);
+            if (weight_planes_->queued == ctx_.stream) weight_planes_->queued = nullptr;
+        }
         weight_planes_.reset();
         inits_.clear();  // blocks go back to the pool before it is destroyed
         pool_.reset();

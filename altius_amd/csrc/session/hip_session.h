@@ -10,6 +10,7 @@
 // Failures come back as a SessionError value; nothing panics or aborts.
 #pragma once
 
+#include <condition_variable>
 #include <map>
 #include <set>
 #include <memory>
@@ -216,15 +217,29 @@ private:
     };
     ViewPlan find_views() const;
     // Products that read their weights' planes, and those planes; made at build, behind the initializers' upload.
+    // Shared by the sessions that share_planes joins: freed when none of them runs, and one that finds them gone drops what it has recorded.
     struct WeightPlanes {
         std::map<std::pair<ValueId, bool>, void *> of;  // weights, whether k is contiguous
-        ~WeightPlanes();
+        std::mutex mutex;
+        std::condition_variable left;
+        size_t running = 0;
+        bool going = false, gone = false;
+        hipStream_t queued = nullptr;  // of the session that made them, whose device runs end behind their call
+        ~WeightPlanes() { release(); }
+        void release();
+    };
+    struct PlanesInUse {  // for the length of a run
+        HipSession *s;
+        explicit PlanesInUse(HipSession *session);
+        ~PlanesInUse();
     };
     std::set<NodeId> by_planes_;
     std::map<NodeId, const void *> node_planes_;
-    std::unique_ptr<WeightPlanes> weight_planes_;
+    std::shared_ptr<WeightPlanes> weight_planes_;  // set at build
+    bool planes_there_ = false;                    // in this run
     void plan_planes(const ViewPlan &views);
     int pack_weights();
+    void forget_planes();
     template <class F> bool retry_without_planes(SessionError *err, F run);
     bool run_once(const std::vector<Tensor> &inputs, std::vector<Tensor> *outputs, SessionError *err);
     bool run_device_once(const std::vector<DeviceTensor> &inputs, std::vector<DeviceTensor> *outputs, SessionError *err);
@@ -428,6 +443,12 @@ public:
         device_ = device;
         return *this;
     }
+    // For a further session of the same model, switches and device: its products read the weights' planes that `first` has made.
+    HipSessionBuilder &share_planes(const HipSession &first) {
+        planes_ = first.weight_planes_;
+        shares_planes_ = true;
+        return *this;
+    }
     // Infers shapes, builds the execution plan, creates the device context and
     // uploads the initializers.  Returns nullptr and fills *err on failure.
     std::unique_ptr<HipSession> build(SessionError *err);
@@ -442,6 +463,8 @@ private:
     bool strided_views_ = true;
     bool fused_attention_ = false;
     bool device_timing_ = true;
+    std::shared_ptr<HipSession::WeightPlanes> planes_;
+    bool shares_planes_ = false;
 };
 
 }  // namespace altius

@@ -626,7 +626,7 @@ int ahip_session_builder_with_device_timing(ahip_session_builder *builder, int e
  * come out finite computed again on the fp32 matrix cores, so that every operand value has fp32 arithmetic's result; against
  * float64 it is 0.3 to 0.6 times as far off as the fp32 kernel.  Such a weight's planes (1.5 times its size) are made when the
  * session is built, in at most a third of the memory that is free then; a product whose planes have no room reads the weight as it is.
- * A run that finds no memory gives the planes back and starts again without them. */
+ * The session's lanes share them.  A run that finds no memory gives the planes back, once no lane runs, and starts again without them. */
 int ahip_session_builder_with_gemm_algorithm(ahip_session_builder *builder, int algorithm);
 /* Not in the reference, whose Split and Transpose always copy (session.rs:1179-1278, 1488-1548): with enable
  * != 0 (the default) a Split or Transpose whose result only MatMuls read, possibly through reshapes and further

@@ -2,6 +2,7 @@
 further off than the fp32 kernel, and fp32 arithmetic's result for infinite, NaN, huge and denormal operand values."""
 import contextlib
 import ctypes
+import threading
 
 import numpy as np
 import pytest
@@ -272,3 +273,47 @@ def test_planes_leave_room_for_what_comes_behind(case):
     with memory_left(9 << 29):  # 4.5 GiB
         y, _ = weights_and_room(rows, k, n, w).build().run([x, np.array([4, 256], np.int64)])
     assert np.array_equal(y, plain)
+
+
+def test_lanes_share_the_planes(case):
+    """A further lane has its own copy of the weights and reads the first one's planes; when one lane needs their memory, all go on without."""
+    case("planes of a session with lanes")
+    rng = np.random.default_rng(12)
+    rows, k, n = 128, 8192, 32768
+    x, w = rng.standard_normal((rows, k)).astype(np.float32), rng.standard_normal((k, n), dtype=np.float32)
+    small = np.array([4, 256], np.int64)
+    plain = fp32_kernel(x, w)
+    session = weights_and_room(rows, k, n, w).build()
+    (by_planes, _), wrong = session.run([x, small]), []
+    before = free_memory()
+
+    def several(runs, wanted):
+        together = threading.Barrier(2)
+
+        def work():
+            together.wait()
+            try:
+                for _ in range(runs):
+                    y, _ = session.run([x, small])
+                    if not any(np.array_equal(y, z) for z in wanted):
+                        wrong.append(y)
+            except Exception as e:  # noqa: BLE001 - reported below, in the main thread
+                wrong.append(repr(e))
+
+        threads = [threading.Thread(target=work) for _ in range(2)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+
+    several(10, [by_planes])
+    assert session.lanes() == 2 and not wrong, wrong
+    assert before - free_memory() < 1.5 * w.nbytes
+    with memory_left(1 << 30):
+        other = threading.Thread(target=several, args=(4, [by_planes, plain]))
+        other.start()
+        y, z = session.run([x, np.array([2048, 1 << 18], np.int64)])  # 2 GiB
+        other.join()
+        assert np.array_equal(y, plain) and not wrong, wrong
+        several(2, [plain])
+    assert not wrong, wrong
