@@ -234,6 +234,8 @@ __global__ __launch_bounds__(64 * WM * WN * WK, std::is_void<X>::value ? 1 : 2) 
         x.run(acc);
         // Where a sum is not finite an operand may have been infinite (inf - inf in the planes), or beyond 2^103, or the sum beyond 2^79: the
         // wavefront's sums over its values of k once more on the fp32 matrix cores, which have fp32 arithmetic's result for every value.
+        // [1024,768] x [768,768] takes 13 us, 22 with one row infinite and 24 with a NaN in every row, [1024,3072] x [3072,768] 40, 72 and 73,
+        // [6304,768] x [768,3072] 165, 225 and 446 (one value of k at a time: 60 and 70, 224 and 264, 336 and 910; the fp32 kernel 15, 42, 222).
         bool lost = false;
 #pragma unroll
         for (int i = 0; i < TA; i++)
@@ -248,23 +250,49 @@ __global__ __launch_bounds__(64 * WM * WN * WK, std::is_void<X>::value ? 1 : 2) 
                 for (int j = 0; j < TB; j++)
 #pragma unroll
                     for (int e = 0; e < 16; e++) acc[i][j][e] = 0.0f;
-            const uint32_t row0 = wm * (32 * TA) + lr, col0 = wn * (32 * TB) + lr;
-#pragma unroll 1
-            for (uint32_t set = wk; set / 4 * 64 < k; set += WK)
-#pragma unroll 1
-                for (uint32_t s = 0; s < 8; s++) {
-                    const uint32_t kk = planes::k_of(set, lk, s);
-                    float va[TA], vb[TB];
+            // A set's values all on their way at once, those of the next set beside its products.
+            const float *pa[TA], *pb[TB];
+            const size_t b_step = g.b_kc ? 1 : g.ldb;
 #pragma unroll
-                    for (int i = 0; i < TA; i++) va[i] = m0 + row0 + 32 * i < g.m && kk < k ? a[(size_t)(row0 + 32 * i) * g.lda + kk] : 0.0f;
+            for (int i = 0; i < TA; i++) pa[i] = a + (size_t)min(wm * (32 * TA) + lr + 32 * i, g.m - m0 - 1) * g.lda;
 #pragma unroll
-                    for (int j = 0; j < TB; j++)
-                        vb[j] = n0 + col0 + 32 * j < g.n && kk < k ? b[g.b_kc ? (size_t)(col0 + 32 * j) * g.ldb + kk : (size_t)kk * g.ldb + col0 + 32 * j] : 0.0f;
+            for (int j = 0; j < TB; j++) pb[j] = b + (size_t)min(wn * (32 * TB) + lr + 32 * j, g.n - n0 - 1) * (g.b_kc ? g.ldb : 1);
+            float va[2][8][TA], vb[2][8][TB];
+            auto fetch = [&](auto to, uint32_t set) __attribute__((always_inline)) {
+#pragma unroll
+                for (uint32_t s = 0; s < 8; s += VEC) {  // VEC values of k lie side by side, all in front of its end or none
+                    const uint32_t kk = planes::k_of(set, lk, s), at = min(kk, k - VEC);
+#pragma unroll
+                    for (int i = 0; i < TA; i++) {
+                        float row[VEC];
+                        __builtin_memcpy(row, __builtin_assume_aligned(pa[i] + at, VEC * sizeof(float)), sizeof(row));
+#pragma unroll
+                        for (uint32_t e = 0; e < VEC; e++) va[to][s + e][i] = kk < k ? row[e] : 0.0f;
+                    }
+#pragma unroll
+                    for (uint32_t e = 0; e < VEC; e++)
+#pragma unroll
+                        for (int j = 0; j < TB; j++) vb[to][s + e][j] = kk < k ? pb[j][(at + e) * b_step] : 0.0f;
+                }
+            };
+            auto multiply = [&](auto of) __attribute__((always_inline)) {
+#pragma unroll
+                for (int s = 0; s < 8; s++)
 #pragma unroll
                     for (int i = 0; i < TA; i++)
 #pragma unroll
-                        for (int j = 0; j < TB; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(va[i], vb[j], acc[i][j], 0, 0, 0);
-                }
+                        for (int j = 0; j < TB; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(va[of][s][i], vb[of][s][j], acc[i][j], 0, 0, 0);
+            };
+            constexpr std::integral_constant<int, 0> even = {};
+            constexpr std::integral_constant<int, 1> odd = {};
+            fetch(even, wk);
+#pragma unroll 1
+            for (uint32_t set = wk; set / 4 * 64 < k; set += 2 * WK) {
+                fetch(odd, set + WK);
+                multiply(even);
+                fetch(even, set + 2 * WK);
+                multiply(odd);  // behind the end of k: zeros
+            }
         } else {
 #pragma unroll
             for (int i = 0; i < TA; i++)
