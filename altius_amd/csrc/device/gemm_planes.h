@@ -76,15 +76,15 @@ struct Split4 {
 
 // The tile of a block: WM x WN x WK wavefronts, WK of them along k, with TA x TB tiles of 32 x 32 each.  A step is one set of k per
 // wavefront along k.  While step s multiplies, step s + 1's fragments of the first operand come out of LDS, step s + 2's values are split into
-// the buffer that step s has left, and memory is asked for the values of step s + 2 + NA and the weights of step s + NB - 1.  One barrier a step.
+// the buffer that step s has left, and memory is asked for the values of step s + 2 + NA and the weights of step s + 1.  One barrier a step.
 // Steps go in turns of U, the last turn with zeros behind the end of k.
-template <int WM, int WN, int WK, int TA, int TB, int VEC, int NB, int NA> struct Tile {
+template <int WM, int WN, int WK, int TA, int TB, int VEC, int NA> struct Tile {
     static constexpr int WAVES = WM * WN * WK, THREADS = 64 * WAVES, BM = 32 * WM * TA, BKT = 16 * WK;
     static constexpr int SETS = BM / 32 * WK, CH = BM * BKT / 8 / THREADS;
     static_assert(CH * THREADS * 8 == BM * BKT, "whole pieces");
     static constexpr int LDS_BYTES = 2 * SETS * (int)SET;
     static constexpr int U = 2;  // steps until registers and buffers are the same again
-    static_assert(U % NB == 0 && U % NA == 0, "whole turns");
+    static_assert(U % NA == 0, "whole turns");
 
     __amdgpu_buffer_rsrc_t rsrc;
     uint32_t off[CH], kp[CH], to[CH], from;
@@ -144,7 +144,7 @@ template <int WM, int WN, int WK, int TA, int TB, int VEC, int NB, int NA> struc
     __device__ __forceinline__ void run(floatx16 (&acc)[TA][TB]) {
         constexpr int BUF = SETS * (int)SET;
         f32x4 ra[NA][CH][2];
-        u32x4 xa[2][TA][3], xb[NB][TB][3];
+        u32x4 xa[2][TA][3], xb[2][TB][3];
         floatx16 low[TA][TB];
 #pragma unroll
         for (int i = 0; i < TA; i++)
@@ -168,8 +168,8 @@ template <int WM, int WN, int WK, int TA, int TB, int VEC, int NB, int NA> struc
 #pragma unroll
                 for (int c = 0; c < CH; c++) load_a(first[s][c], c, s);
             // In the order in which the steps load, so that a wait for one of them leaves as many of the others on their way as later ones do.
-            each<(NA > NB - 1 ? NA : NB - 1)>([&](auto t) __attribute__((always_inline)) {
-                constexpr int at = t - (NA > NB - 1 ? NA : NB - 1), sb = at + NB - 1, sa = at + 2 + NA;
+            each<NA>([&](auto t) __attribute__((always_inline)) {
+                constexpr int at = t - NA, sb = at + 1, sa = at + 2 + NA;
                 if constexpr (sb >= 0) {
 #pragma unroll
                     for (int j = 0; j < TB; j++)
@@ -203,19 +203,19 @@ template <int WM, int WN, int WK, int TA, int TB, int VEC, int NB, int NA> struc
 
         constexpr int Q = 6 * TA * TB, READS = 3 * TA, LOADS = 3 * TB, PARTS = 16 * CH, QR = Q / 3 > 0 ? Q / 3 : 1, QP = Q * 3 / 4;
         auto step = [&](auto at, uint32_t s) __attribute__((always_inline)) {
-            constexpr int now = at % 2, next = (at + 1) % 2, slot = (at + 2) % NA, bnow = at % NB, bnext = (at + NB - 1) % NB;
+            constexpr int now = at % 2, next = (at + 1) % 2, slot = (at + 2) % NA;
             Split4 sp[CH][2];
             each<Q>([&](auto q) __attribute__((always_inline)) {
                 constexpr int T = q / (TA * TB), i = q / TB % TA, j = q % TB;
                 constexpr int PA[6] = {2, 1, 0, 1, 0, 0}, PB[6] = {0, 1, 2, 0, 1, 0};  // smallest terms first
                 floatx16 &sum = T < 5 ? low[i][j] : acc[i][j];
-                sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, xa[now][i][PA[T]]), __builtin_bit_cast(bf16x8, xb[bnow][j][PB[T]]), sum, 0, 0, 0);
+                sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, xa[now][i][PA[T]]), __builtin_bit_cast(bf16x8, xb[now][j][PB[T]]), sum, 0, 0, 0);
                 __builtin_amdgcn_sched_barrier(0);
                 each<READS>([&](auto r) __attribute__((always_inline)) {
                     if constexpr (r * QR / READS == q) xa[next][r / 3][r % 3] = read(r / 3, r % 3, next);
                 });
                 each<LOADS>([&](auto l) __attribute__((always_inline)) {
-                    if constexpr (l * Q / LOADS == q) xb[bnext][l / 3][l % 3] = load_b(l / 3, l % 3, s + NB - 1);
+                    if constexpr (l * Q / LOADS == q) xb[next][l / 3][l % 3] = load_b(l / 3, l % 3, s + 1);
                 });
                 each<PARTS>([&](auto u) __attribute__((always_inline)) {
                     constexpr int c = u / 16, p = u / 2 % 8, h = u % 2;

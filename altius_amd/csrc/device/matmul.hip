@@ -642,18 +642,18 @@ template <bool AKC, bool BKC> void launch_tiles(const DeviceCtx &ctx, const Gemm
 
 void launch_plane_tiles(const DeviceCtx &ctx, const GemmArgs &g, int shape, bool vec) {
     const dim3 grid((g.full + (g.chunk - g.full) * g.slices) * 8), block(PLANE_SHAPES[shape].threads);
-#define TILES(WM, WN, WK, TA, TB, NB, NA)                                                                                               \
-    do {                                                                                                                                \
-        if (vec) hipLaunchKernelGGL((gemm_f32_tiles<true, true, WM, WN, WK, TA, TB, 4, planes::Tile<WM, WN, WK, TA, TB, 4, NB, NA>>),   \
-                                    grid, block, 0, ctx.stream, g);                                                                     \
-        else hipLaunchKernelGGL((gemm_f32_tiles<true, true, WM, WN, WK, TA, TB, 1, planes::Tile<WM, WN, WK, TA, TB, 1, NB, NA>>),       \
-                                grid, block, 0, ctx.stream, g);                                                                         \
+#define TILES(WM, WN, WK, TA, TB, NA)                                                                                               \
+    do {                                                                                                                            \
+        if (vec) hipLaunchKernelGGL((gemm_f32_tiles<true, true, WM, WN, WK, TA, TB, 4, planes::Tile<WM, WN, WK, TA, TB, 4, NA>>),   \
+                                    grid, block, 0, ctx.stream, g);                                                                 \
+        else hipLaunchKernelGGL((gemm_f32_tiles<true, true, WM, WN, WK, TA, TB, 1, planes::Tile<WM, WN, WK, TA, TB, 1, NA>>),       \
+                                grid, block, 0, ctx.stream, g);                                                                     \
     } while (0)
     switch (shape) {
-    case 0: TILES(1, 2, 4, 2, 1, 2, 2); break;
-    case 1: TILES(1, 2, 4, 2, 2, 2, 1); break;
-    case 2: TILES(2, 2, 2, 2, 2, 2, 1); break;
-    default: TILES(2, 2, 1, 2, 2, 2, 1); break;
+    case 0: TILES(1, 2, 4, 2, 1, 2); break;
+    case 1: TILES(1, 2, 4, 2, 2, 1); break;
+    case 2: TILES(2, 2, 2, 2, 2, 1); break;
+    default: TILES(2, 2, 1, 2, 2, 1); break;
     }
 #undef TILES
 }
@@ -702,7 +702,7 @@ bool planes_reach(size_t lda, size_t k) { return k > 0 && k <= ((size_t)1 << 20)
 // with Transpose(1,0,2) behind: none that is taken loses, those left out would gain 2 % at most), of operands that Transpose(0,2,1) turns 5 us
 // and 1.4 TB/s ([64,196,512] turned x [196,256] 36 us in place, 65 by planes; [16,1024,768] x [1024,256 / 2048] 54 and 107, 386 and 332).
 bool gemm_takes_planes(const DeviceCtx &ctx, size_t m, size_t n, size_t k, size_t matrices, bool operand, bool result) {
-    if (gemm_takes_split(ctx, m, n, k) || m < 64 || n < 64 || k < 64 || m >= ((size_t)1 << 31) || n >= ((size_t)1 << 31)) return false;
+    if (gemm_takes_split(ctx, m, n, k) || m < 64 || n < 64 || k < 64 || !planes_reach(k, k) || m >= ((size_t)1 << 31) || n >= ((size_t)1 << 31)) return false;
     const size_t cus = ctx.cus_per_xcd ? (size_t)ctx.cus_per_xcd : 32, parts = operand || result ? std::max<size_t>(matrices, 1) : 1;
     const Choice ch = choose(1, m, n, k, cus, ctx.gemm_split_k, true);
     const double us = choose(parts, m / parts, n, k, cus, ctx.gemm_split_k).us, from_hbm = std::min(1.5e-6 * (double)n * (double)k, 3.6);
@@ -897,7 +897,7 @@ int launch_gemm_f32(DeviceCtx &ctx, float *c, const float *a, const float *b, co
     // Up to the three blocks of 32 x 32 that a CU holds ([197,768] x [768,2304 / 3072] 10.4 -> 10.15 us, 13.6 -> 13.25, [1024,768] x [768,768]
     // 13.9 -> 13.5, [1024,3072] x [3072,768] 42.8 -> 41.8; of 4713 tiles the later ones starve, 82 -> 87, cut ones gain nothing, and
     // 64 x 64 tiles lose 7 % of three rounds and more).
-    g.apart = ch.slices == 1 && g.chunk <= 3 * cus;
+    g.apart = !planes && ch.slices == 1 && g.chunk <= 3 * cus;
     if (g.slices > 1) {
         g.partials = static_cast<float *>(ctx.gemm_partials);
         g.counters = ctx.gemm_counters;
@@ -907,9 +907,8 @@ int launch_gemm_f32(DeviceCtx &ctx, float *c, const float *a, const float *b, co
         const size_t span = (kc ? (rows - 1) * ld + sh.step : (sh.step - 1) * ld + rows) * 4;
         return span < end ? std::min<size_t>((end - span) / std::max<size_t>(step, 1), 0x7fffffff) : 0;
     };
-    g.window = (uint32_t)std::min(window(a_kc, std::min<size_t>(sh.bm, a_kc ? m : sh.bm), lda), window(b_kc, std::min<size_t>(sh.bn, b_kc ? n : sh.bn), ldb));
+    if (!planes) g.window = (uint32_t)std::min(window(a_kc, std::min<size_t>(sh.bm, a_kc ? m : sh.bm), lda), window(b_kc, std::min<size_t>(sh.bn, b_kc ? n : sh.bn), ldb));
     if (planes) {
-        g.window = (uint32_t)window(true, std::min<size_t>(sh.bm, m), lda);
         g.planes = static_cast<const char *>(planes);
         g.n32s = (uint32_t)((n + 31) / 32), g.k16s = (uint32_t)weight_k16s(k);
         g.b_kc = b_kc;

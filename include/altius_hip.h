@@ -276,7 +276,8 @@ int ahip_gemm(ahip_ctx *ctx, float *c, const float *a, const float *b, const flo
               float beta);
 
 /* The launch that ahip_gemm makes on the fp32 kernel's tiles for a product of this size (no GPU needed): how many blocks of 256 threads,
- * and into how many slices the tiles of a last, partly empty round are cut along k (1: none is cut).  AHIP_ERR_UNSUPPORTED: more
+ * and into how many slices the tiles of a last, partly empty round are cut along k (1: none is cut); a session's products by planes of
+ * their weights (ahip_session_builder_with_gemm_algorithm) have tiles of their own.  AHIP_ERR_UNSUPPORTED: more
  * tiles than a grid holds, which ahip_gemm refuses.  No counterpart in the reference. */
 int ahip_gemm_f32_grid(size_t batch, size_t m, size_t n, size_t k, size_t *blocks, int *slices);
 
