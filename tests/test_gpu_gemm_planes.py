@@ -60,6 +60,24 @@ def test_as_close_as_the_fp32_kernel(case, rows, k, n):
     assert (np.abs(got[some] - want) <= bound).all()
 
 
+# Sums of one sign, where roundings toward zero would add up: all four tiles (64 x 64, 64 x 128, 128 x 128 in two chains of k and in one).
+@pytest.mark.parametrize("rows,k,n", [(1024, 3072, 768), (6304, 768, 768), (6304, 3072, 768), (6304, 768, 3072)])
+@pytest.mark.parametrize("operands", ["unit", "relu", "equal"])
+def test_sums_of_one_sign(case, rows, k, n, operands):
+    case(f"{operands} operands, [{rows},{k}] x [{k},{n}]")
+    rng = np.random.default_rng(4)
+    if operands == "unit":
+        a, w = rng.random((rows, k), dtype=np.float32), rng.random((k, n), dtype=np.float32)
+    elif operands == "relu":
+        a, w = np.maximum(rng.standard_normal((rows, k), dtype=np.float32), 0), np.abs(rng.standard_normal((k, n), dtype=np.float32))
+    else:
+        a, w = np.full((rows, k), 1.1, np.float32), np.full((k, n), 1.3, np.float32)
+    some = np.unique(np.concatenate([np.arange(0, rows, 101), [rows - 1]]))
+    want = a[some].astype(np.float64) @ w.astype(np.float64)
+    got, plain = product(rows, k, n, w).run([a])[0][some], fp32_kernel(a, w)[some]
+    assert np.linalg.norm(got - want) <= np.linalg.norm(plain - want)
+
+
 @pytest.mark.parametrize("rows,k,n", [(77, 768, 16384), (129, 771, 16390)])
 def test_few_rows_and_many_columns(case, rows, k, n):
     test_as_close_as_the_fp32_kernel(case, rows, k, n)
@@ -120,15 +138,19 @@ def test_a_view_has_the_bits_of_its_copy(case):
         m = Model(opset_version=13)
         v = m.new_val_named_and_shaped("x", list(x.shape))
         m.add_input(v)
-        left, right, y = (m.new_val() for _ in range(3))
+        left, right, y, z = (m.new_val() for _ in range(4))
         m.add_node(Op.Split, [v, m.new_initializer(np.array([768, 768], np.int64))], [left, right], axis=2)
         m.add_node(Op.MatMul, [right, m.new_initializer(w)], [y])
+        m.add_node(Op.MatMul, [left, m.new_initializer(w)], [z])  # an output of the graph would have the Split copy
         m.add_output(y)
-        m.add_output(left)
+        m.add_output(z)
         return HipSessionBuilder(m).with_strided_views(views).build()
 
-    in_place, copied = build(True).run([x])[0], build(False).run([x])[0]
-    assert np.array_equal(in_place, copied)
+    views, copies = build(True), build(False)
+    (in_place, left), (copied, left_copied) = views.run([x]), copies.run([x])
+    assert views.copies_avoided() > copies.copies_avoided() == 0
+    assert np.array_equal(in_place, copied) and np.array_equal(left, left_copied)
+    assert not np.array_equal(left.reshape(1200, 768), fp32_kernel(np.ascontiguousarray(x[..., :768]).reshape(1200, 768), w)), "these sizes are meant to take the planes"
     assert np.array_equal(in_place.reshape(1200, 768), product(1200, 768, 768, w).run([np.ascontiguousarray(x[..., 768:]).reshape(1200, 768)])[0])
 
 
