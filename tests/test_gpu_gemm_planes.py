@@ -309,8 +309,8 @@ def test_lanes_share_the_planes(case):
     (by_planes, _), wrong = session.run([x, small]), []
     before = free_memory()
 
-    def several(runs, wanted):
-        together = threading.Barrier(2)
+    def several(callers, runs, wanted):
+        together = threading.Barrier(callers)
 
         def work():
             together.wait()
@@ -322,20 +322,21 @@ def test_lanes_share_the_planes(case):
             except Exception as e:  # noqa: BLE001 - reported below, in the main thread
                 wrong.append(repr(e))
 
-        threads = [threading.Thread(target=work) for _ in range(2)]
+        threads = [threading.Thread(target=work) for _ in range(callers)]
         for t in threads:
             t.start()
         for t in threads:
             t.join()
 
-    several(10, [by_planes])
+    several(2, 10, [by_planes])
     assert session.lanes() == 2 and not wrong, wrong
     assert before - free_memory() < 1.5 * w.nbytes
-    with memory_left(1 << 30):
-        other = threading.Thread(target=several, args=(4, [by_planes, plain]))
+    with memory_left(1 << 30):  # (a third caller's lane would take the memory for its weights)
+        other = threading.Thread(target=several, args=(1, 4, [by_planes, plain]))
         other.start()
         y, z = session.run([x, np.array([2048, 1 << 18], np.int64)])  # 2 GiB
         other.join()
         assert np.array_equal(y, plain) and not wrong, wrong
-        several(2, [plain])
+        several(2, 2, [plain])
+        assert session.lanes() == 2
     assert not wrong, wrong
