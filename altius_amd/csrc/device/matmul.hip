@@ -76,14 +76,14 @@ struct GemmArgs {
     float alpha, beta;
     int act;
     float act_alpha, act_beta;
-    // The second operand's planes where it has some, [n32s][k16s] sets (gemm_planes.h); b is the same operand as it lies in memory, b_kc: along k.
-    const char *planes;
-    uint32_t n32s, k16s;
-    int b_kc;
     // The blocks of a CU all start together, and go out of step by priorities: one's first loads and results beside another's products.
     // (Of 256 blocks dealt in turn each of the part's 256 CUs gets one, the next 256 are its second: with fewer CUs the priorities
     // would not differ where they should, and the results would be the same.)
     int apart;
+    // The second operand's planes where it has some, [n32s][k16s] sets (gemm_planes.h); b is the same operand as it lies in memory, b_kc: along k.
+    const char *planes;
+    uint32_t n32s, k16s;
+    int b_kc;
 };
 
 // Four floats that blocks on any XCD read and write.
