@@ -694,9 +694,13 @@ bool planes_reach(size_t lda, size_t k) { return k > 0 && k <= ((size_t)1 << 20)
 // [12608,768] x [768,3072] 450 -> 315).  With fewer, a block's start and end and the 6 bytes a weight takes instead of 4 outweigh the products
 // ([256,768] x [768,768] 6.8 and 10.1, [512,384] x [384,384] 5.4 and 8.0).
 // A graph's weights are other ones in each product, and a block's few wavefronts wait for them longer than the estimates, fitted to one
-// product alone, say: in chains of 24 to 40 products 0.3 us for 3.5 MB of planes and 2 to 6 for 14 MB, and about as much for 38 to 232 MB,
-// where later tiles' products hide it.  Without that [256,768] x [768,3072] lost 1.3 us of 15, [512,3072] x [3072,768] 1.7 of 25 and
-// [788,1536] x [1536,384] 1.1 of 15.  Of 66 sizes in such chains, none that is taken loses, and those left out would gain 1.9 us at most.
+// product alone, say.  In chains of 24 to 40 products planes took that much longer against the fp32 kernel than reckoned: -1.8 to 1.9 us for
+// 1 to 6 MB of them, -1.4 to 8.5 for 10.6 and -0.3 to 12.1 for 14, the most where k is long and the columns are few ([1576,3072] x [3072,768]:
+// 18.4 us reckoned, 6.2 gained); for 38 to 232 MB either kernel takes up to 50 us longer.  The estimates do not have that, so the line keeps a
+// distance instead, by the weights' size: without it [256,768] x [768,3072] lost 1.3 us of 15, [512,3072] x [3072,768] 1.7 of 25 and
+// [788,1536] x [1536,384] 1.1 of 15.  Of those 66 sizes none that is taken loses, and those left out would gain 1.9 us at most; of 216 more that
+// are taken, with weights from HBM (128 to 2048 rows, k of 1024 to 16384, 256 to 1536 columns; 1000 to 16448 rows, k of 64 to 1024), one loses:
+// [300,4096] x [4096,1024], 0.4 us of 31.
 // A view that is not one tall matrix is copied first, a Transpose behind that the fp32 kernel writes ahead of copies the result; against that the
 // fp32 kernel's tiles end with each matrix.  Copies of results take 2 us and 6 TB/s (58 products of 512 to 6304 rows and 192 to 3072 values of k
 // with Transpose(1,0,2) behind: none that is taken loses, those left out would gain 2 % at most), of operands that Transpose(0,2,1) turns 5 us

@@ -624,17 +624,20 @@ int ahip_session_builder_with_device_timing(ahip_session_builder *builder, int e
  * of a weight are made on its first use and kept until the session is freed.
  * On the default too a product of some hundred rows and more whose second operand is an initializer runs on the bf16 matrix
  * cores where that is reckoned faster: six products of the exact three-way split, the small ones summed apart, and what does not
- * come out finite computed again on the fp32 matrix cores, so that every operand value has fp32 arithmetic's result; against
- * float64 it is 0.3 to 0.6 times as far off as the fp32 kernel.  Such a weight's planes (1.5 times its size) are made when the
- * session is built, in at most a third of the memory that is free then; a product whose planes have no room reads the weight as it is.
- * The session's lanes share them.  A run that finds no memory gives the planes back, once no lane runs, and starts again without them. */
+ * come out finite computed again on the fp32 matrix cores, so that every operand value has fp32 arithmetic's result (such a product
+ * takes up to three times as long).  Against float64 it is at most 0.6 times as far off as the fp32 kernel, on operands of both
+ * signs or of one; where no more than two products of a sum are not zero, up to 1.04 times.  Such a weight's planes (1.5 times its
+ * size) are made when the session is built, in at most a third of the memory that is free then; a product whose planes have no room
+ * reads the weight as it is.  The session's lanes share them.  A run that finds no memory gives the planes back, once no lane runs,
+ * and starts again without them. */
 int ahip_session_builder_with_gemm_algorithm(ahip_session_builder *builder, int algorithm);
 /* Not in the reference, whose Split and Transpose always copy (session.rs:1179-1278, 1488-1548): with enable
  * != 0 (the default) a Split or Transpose whose result only MatMuls read, possibly through reshapes and further
  * transposes, hands out a strided view of its input, which the MatMul reads in place (ahip_gemm_batch2), and
  * a MatMul read only by a Transpose that keeps the last axis writes that Transpose's layout directly.  The
  * products are the same kernels on the same values: results do not change by a bit.  A view that some other
- * reader needs, or that the GEMM's addressing cannot express, is copied as before. */
+ * reader needs, that the GEMM's addressing cannot express, or that a product by planes has to read as one tall
+ * matrix and is faster for it, is copied as before. */
 int ahip_session_builder_with_strided_views(ahip_session_builder *builder, int enable);
 /* Not in the reference, which runs MatMul, Softmax and MatMul as three kernels (session.rs:621-684, 990-1026):
  * with enable != 0 (default 0; needs strided views) a MatMul -> Softmax(last axis, with the scale and per-key
