@@ -171,7 +171,7 @@ std::unique_ptr<HipSession> HipSessionBuilder::build(SessionError *err) {
         std::lock_guard<std::mutex> lock(s->weight_planes_->mutex);
         for (NodeId id : s->by_planes_) {
             auto it = s->weight_planes_->of.find({s->model_.graph.nodes[id].inputs[1], s->inferred_.at(id).first.trans_b != 0});
-            if (it != s->weight_planes_->of.end() && it->second) s->node_planes_[id] = it->second;
+            if (it != s->weight_planes_->of.end()) s->node_planes_[id] = it->second;
         }
     }
     return s;
@@ -204,7 +204,8 @@ int HipSession::pack_weights() {
         left -= bytes;
         if ((rc = gemm_pack_weights(ctx_, planes, static_cast<const float *>(w.ptr), n, k, w.dims[1], k_contig))) return rc;
     }
-    weight_planes_ = std::move(made);
+    for (auto it = made->of.begin(); it != made->of.end();) it = it->second ? std::next(it) : made->of.erase(it);
+    if (!made->of.empty()) weight_planes_ = std::move(made);
     return AHIP_OK;
 }
 
